@@ -30,7 +30,7 @@ EXPORTS = [
 
 EXT_EXPORTS = ["fastKronGetLastPlan", "fastKronSetTunedDB", "fastKronSetPlanOnly", "fastKronGetLastLaunches",
                "sgemkmStaticScratch", "fastKronGetSyncError", "fastKronSetSyncHelpAfter",
-               "fastKronProbeCopyPattern"]     # include/fastkron_ext.h
+               "fastKronProbeCopyPattern", "fastKronGradSizes", "fastKronGradForward", "fastKronGradBackward"]     # include/fastkron_ext.h
 
 _lib = None
 
@@ -96,6 +96,10 @@ def load():
     lib.fastKronGetSyncError.argtypes = [vp, u32p]
     lib.fastKronSetSyncHelpAfter.argtypes = [u32]
     lib.fastKronProbeCopyPattern.argtypes = [vp, cint, vp, vp, vp, vp, u32]
+    lib.fastKronGradSizes.argtypes = [vp, cint, cint, u32, u32, u32p, u32p, cint, u64, cint, u32, szp, szp]
+    lib.fastKronGradForward.argtypes = [vp, cint, cint, u32, u32, u32p, u32p, vp, cint, u64, vpp, cint, cint, u32, vp, vp]
+    lib.fastKronGradBackward.argtypes = [vp, cint, cint, u32, u32, u32p, u32p, vp, cint, u64, vpp, cint, cint, u32, vp, vp,
+                                         vp, vpp, vp]
     lib.fastKronSetPlanOnly.argtypes = [vp, cint]
     lib.fastKronGetLastLaunches.argtypes = [vp, ctypes.c_char_p, ctypes.c_size_t]
     lib.fastKronGetLastLaunches.restype = ctypes.c_size_t

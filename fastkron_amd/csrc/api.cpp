@@ -290,4 +290,35 @@ FK_FWD_SB(dkmmForwardStridedBatched, double, DType::F64, MMType::KMM,
            uint64_t strideX, double* Z, uint64_t strideZ, uint32_t batchCount, double* Intermediates[],
            uint64_t strideIntermediates[]))
 
+static Handle::GradProblem gradProblem(int mkm, int dbl, uint32_t M, uint32_t N, const uint32_t* Ps, const uint32_t* Qs,
+                                       const void* X, fastKronOp opX, uint64_t strideX, const void* const* Fs, fastKronOp opFs,
+                                       int perBatchFs, uint32_t batchCount) {
+  return Handle::GradProblem{mkm ? MMType::MKM : MMType::KMM, dbl ? DType::F64 : DType::F32, M, N, Ps, Qs, X, opX, strideX,
+                             Fs, opFs, perBatchFs != 0, batchCount};
+}
+
+fastKronError fastKronGradSizes(fastKronHandle handle, int mkm, int dbl, uint32_t M, uint32_t N, const uint32_t Ps[],
+                                const uint32_t Qs[], fastKronOp opX, uint64_t strideX, int perBatchFs, uint32_t batchCount,
+                                size_t* saveElems, size_t* workElems) {
+  if (!handle) return fastKronInvalidArgument;
+  return H(handle)->gradSizes(gradProblem(mkm, dbl, M, N, Ps, Qs, nullptr, opX, strideX, nullptr, fastKronOp_N, perBatchFs,
+                                          batchCount), saveElems, workElems);
+}
+
+fastKronError fastKronGradForward(fastKronHandle handle, int mkm, int dbl, uint32_t M, uint32_t N, const uint32_t Ps[],
+                                  const uint32_t Qs[], const void* X, fastKronOp opX, uint64_t strideX, const void* const Fs[],
+                                  fastKronOp opFs, int perBatchFs, uint32_t batchCount, void* Z, void* save) {
+  if (!handle) return fastKronInvalidArgument;
+  return H(handle)->gradForward(gradProblem(mkm, dbl, M, N, Ps, Qs, X, opX, strideX, Fs, opFs, perBatchFs, batchCount), Z, save);
+}
+
+fastKronError fastKronGradBackward(fastKronHandle handle, int mkm, int dbl, uint32_t M, uint32_t N, const uint32_t Ps[],
+                                   const uint32_t Qs[], const void* X, fastKronOp opX, uint64_t strideX, const void* const Fs[],
+                                   fastKronOp opFs, int perBatchFs, uint32_t batchCount, const void* gZ, void* save, void* gX,
+                                   void* const gFs[], void* work) {
+  if (!handle) return fastKronInvalidArgument;
+  return H(handle)->gradBackward(gradProblem(mkm, dbl, M, N, Ps, Qs, X, opX, strideX, Fs, opFs, perBatchFs, batchCount), gZ,
+                                 save, gX, gFs, work);
+}
+
 }  // extern "C"

@@ -80,6 +80,17 @@ class Handle {
   // kernels for those sizes apply.  Returns false when nothing is merged; on true `out` is the merged problem.
   bool mergeSmallFactors(const KronProblem& p, KronProblem* out, const CallWorkspace* ws = nullptr);
 
+  // Forward pass that keeps what the backward pass needs, and the backward pass (gradient.cpp).
+  struct GradProblem {
+    MMType mm; DType dt; uint32_t M, N; const uint32_t* P; const uint32_t* Q;
+    const void* X; int opX; uint64_t strideX;
+    const void* const* F; int opF; bool perBatchF;
+    uint32_t batch;
+  };
+  fastKronError gradSizes(const GradProblem& p, size_t* saveElems, size_t* workElems) const;
+  fastKronError gradForward(const GradProblem& p, void* Z, void* save);
+  fastKronError gradBackward(const GradProblem& p, const void* gZ, void* save, void* gX, void* const* gF, void* work);
+
   const std::string& lastPlan() const { return lastPlan_; }
   void setTunedDB(const char* path);
 

@@ -20,7 +20,8 @@ __global__ __launch_bounds__(256) void kron_merge_kernel(const MergeArgs a) {
   const MergeGroup g = a.g[blockIdx.x];
   uint32_t P = 1, Q = 1;
   for (uint32_t j = 0; j < g.count; j++) { P *= g.p[j]; Q *= g.q[j]; }
-  T* dst = (T*)g.dst;
+  const uint32_t b = blockIdx.y;
+  T* dst = (T*)g.dst + (size_t)b * P * Q;
   for (uint32_t e = threadIdx.x; e < P * Q; e += 256) {
     uint32_t p = e / Q, q = e % Q;
     const uint32_t p0 = p, q0 = q;
@@ -28,7 +29,7 @@ __global__ __launch_bounds__(256) void kron_merge_kernel(const MergeArgs a) {
     for (int j = (int)g.count - 1; j >= 0; j--) {          // the last source owns the fastest digit
       const uint32_t pj = p % g.p[j], qj = q % g.q[j];
       p /= g.p[j]; q /= g.q[j];
-      v *= ((const T*)g.src[j])[(int64_t)pj * g.sp[j] + (int64_t)qj * g.sq[j]];
+      v *= ((const T*)g.src[j])[(int64_t)b * (g.p[j] * g.q[j]) + (int64_t)pj * g.sp[j] + (int64_t)qj * g.sq[j]];
     }
     dst[(int64_t)p0 * g.dsp + (int64_t)q0 * g.dsq] = v;
   }
@@ -55,9 +56,9 @@ hipError_t launchFill(void* dst, size_t elems, DType dt, hipStream_t stream) {
 }
 
 hipError_t launchMergeFactors(const MergeArgs& a, DType dt, hipStream_t stream) {
-  if (a.groups == 0 || a.groups > kMaxMergeGroups) return hipErrorInvalidValue;
-  if (dt == DType::F32) hipLaunchKernelGGL(kron_merge_kernel<float>, dim3(a.groups), dim3(256), 0, stream, a);
-  else                  hipLaunchKernelGGL(kron_merge_kernel<double>, dim3(a.groups), dim3(256), 0, stream, a);
+  if (a.groups == 0 || a.groups > kMaxMergeGroups || a.batch == 0 || a.batch > 65535) return hipErrorInvalidValue;
+  if (dt == DType::F32) hipLaunchKernelGGL(kron_merge_kernel<float>, dim3(a.groups, a.batch), dim3(256), 0, stream, a);
+  else                  hipLaunchKernelGGL(kron_merge_kernel<double>, dim3(a.groups, a.batch), dim3(256), 0, stream, a);
   return hipGetLastError();
 }
 

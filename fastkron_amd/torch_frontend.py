@@ -10,12 +10,12 @@ broadcast and batching rules):
 * a tensor whose last two dimensions are a transposed view of a row-major buffer is passed as that buffer
   with `fastKronOp_T` instead of being copied (reference fastkrontorch.py:66-76);
 * 1-D X is a single row (MKM) or column (KMM);
-* with gradients required, the forward family of the library keeps every step's output and `backward`
-  chains through the saved intermediates (reference fastkrontorch.py:160-217); when only X needs a gradient
-  the backward pass is one fused library call with the transposed factors.
+* with gradients of factors required, the library's gradient functions (include/fastkron_ext.h) run the forward
+  pass keeping every step's input and the backward pass through the steps (reference fastkrontorch.py:160-217);
+  when only X needs a gradient the backward pass is one fused library call with the transposed factors.
 
-PyTorch supplies memory, streams and, in `backward` for factor gradients, the per-step GEMMs (as in the
-reference); the forward arithmetic is always the library's HIP kernels.  CPU tensors and dtypes other than
+PyTorch supplies memory and streams; the arithmetic of both passes is the library's HIP kernels (a backward pass that
+is itself differentiated, create_graph=True, is composed of PyTorch operations).  CPU tensors and dtypes other than
 float32 / float64 are errors: there is no fallback path (the reference falls back to a shuffle algorithm
 built from `torch.matmul`, fastkronbase.py:478-518).
 """
@@ -154,8 +154,13 @@ def _batch_plan(zbatch, shapes):
     return inner, plans, steps
 
 
-def _run(mm, x, fs, alpha, beta, y, keep_intermediates):
-    """Returns (z, intermediates); intermediates is [] unless keep_intermediates."""
+def _check(e, where):
+    if e != SUCCESS:
+        from . import FastKronError
+        raise FastKronError(e, where)
+
+
+def _run(mm, x, fs, alpha, beta, y):
     _validate(mm, x, fs, y)
     if beta != 0.0 and y is None:
         raise ValueError(f"When beta != 0 ({beta}) then y should not be None")
@@ -172,40 +177,19 @@ def _run(mm, x, fs, alpha, beta, y, keep_intermediates):
     fold = (mm == "mkm" and len(p.zbatch) > 0 and p.fbatch == () and p.opX == OP_N and
             (p.yb is None or p.ybatch == p.zbatch))
     M = p.M * nb if fold else p.M
-    if keep_intermediates:
-        widths = h.sizes_forward(p.M, p.Ps, p.Qs)[1]          # elements per problem, one per kept step
-        inter = [torch.empty(p.zbatch + ((p.M, w // p.M) if mm == "mkm" else (w // p.M, p.M)),
-                             dtype=x.dtype, device=x.device) for w in widths]
-        t1 = t2 = None
-    else:
-        inter = []
-        te = h.sizes(M, p.Ps, p.Qs)[1]
-        inner = 1 if (fold or not p.zbatch) else p.zbatch[-1]
-        t1, t2 = new(te * inner), new(te * inner)
-
-    def check(e, where):
-        if e != SUCCESS:
-            from . import FastKronError
-            raise FastKronError(e, where)
+    te = h.sizes(M, p.Ps, p.Qs)[1]
+    inner = 1 if (fold or not p.zbatch) else p.zbatch[-1]
+    t1, t2 = new(te * inner), new(te * inner)
 
     if fold or not p.zbatch:
         fptr = capi.arr_ptr([f.data_ptr() for f in p.fb])
-        if keep_intermediates:
-            ip = capi.arr_ptr([t.data_ptr() for t in inter]) if inter else None
-            if mm == "mkm":
-                check(getattr(lib, pre + "mkmForward")(h.h, BACKEND_HIP, M, N, Ps, Qs, _address(p.xb), p.opX, fptr, p.opF,
-                                                       _address(z), ip), "mkmForward")
-            else:
-                check(getattr(lib, pre + "kmmForward")(h.h, BACKEND_HIP, N, Qs, Ps, M, fptr, p.opF, _address(p.xb), p.opX,
-                                                       _address(z), ip), "kmmForward")
+        yp = _address(p.yb) if p.yb is not None else None
+        if mm == "mkm":
+            _check(getattr(lib, pre + "gemkm")(h.h, BACKEND_HIP, M, N, Ps, Qs, _address(p.xb), p.opX, fptr, p.opF,
+                                              _address(z), alpha, beta, yp, _address(t1), _address(t2)), "gemkm")
         else:
-            yp = _address(p.yb) if p.yb is not None else None
-            if mm == "mkm":
-                check(getattr(lib, pre + "gemkm")(h.h, BACKEND_HIP, M, N, Ps, Qs, _address(p.xb), p.opX, fptr, p.opF,
-                                                  _address(z), alpha, beta, yp, _address(t1), _address(t2)), "gemkm")
-            else:
-                check(getattr(lib, pre + "gekmm")(h.h, BACKEND_HIP, N, Qs, Ps, M, fptr, p.opF, _address(p.xb), p.opX,
-                                                  _address(z), alpha, beta, yp, _address(t1), _address(t2)), "gekmm")
+            _check(getattr(lib, pre + "gekmm")(h.h, BACKEND_HIP, N, Qs, Ps, M, fptr, p.opF, _address(p.xb), p.opX,
+                                              _address(z), alpha, beta, yp, _address(t1), _address(t2)), "gekmm")
     else:
         shapes = [p.xbatch, p.fbatch, p.ybatch if p.yb is not None else p.zbatch, p.zbatch]
         inner, plans, steps = _batch_plan(p.zbatch, shapes)
@@ -215,31 +199,19 @@ def _run(mm, x, fs, alpha, beta, y, keep_intermediates):
         for xo, fo, yo, zo in plans:
             fptr = capi.arr_ptr([f.data_ptr() + fo * b * f.element_size() for f, b in zip(p.fb, fblk)])
             xp, zp = _address(p.xb, xo * xblk), _address(z, zo * zblk)
-            if keep_intermediates:
-                ip = capi.arr_ptr([t.data_ptr() + zo * (w) * t.element_size() for t, w in zip(inter, widths)]) if inter else None
-                sI = capi.arr_u64(list(widths)) if inter else None
-                if mm == "mkm":
-                    check(getattr(lib, pre + "mkmForwardStridedBatched")(
-                        h.h, BACKEND_HIP, p.M, N, Ps, Qs, xp, p.opX, steps[0] * xblk, fptr, p.opF, sF, zp, zblk, inner,
-                        ip, sI), "mkmForwardStridedBatched")
-                else:
-                    check(getattr(lib, pre + "kmmForwardStridedBatched")(
-                        h.h, BACKEND_HIP, N, Qs, Ps, p.M, fptr, p.opF, sF, xp, p.opX, steps[0] * xblk, zp, zblk, inner,
-                        ip, sI), "kmmForwardStridedBatched")
+            yp = _address(p.yb, yo * zblk) if p.yb is not None else None
+            sY = steps[2] * zblk if p.yb is not None else 0
+            if mm == "mkm":
+                _check(getattr(lib, pre + "gemkmStridedBatched")(
+                    h.h, BACKEND_HIP, p.M, N, Ps, Qs, xp, p.opX, steps[0] * xblk, fptr, p.opF, sF, zp, zblk,
+                    alpha, beta, inner, yp, sY, _address(t1), _address(t2)), "gemkmStridedBatched")
             else:
-                yp = _address(p.yb, yo * zblk) if p.yb is not None else None
-                sY = steps[2] * zblk if p.yb is not None else 0
-                if mm == "mkm":
-                    check(getattr(lib, pre + "gemkmStridedBatched")(
-                        h.h, BACKEND_HIP, p.M, N, Ps, Qs, xp, p.opX, steps[0] * xblk, fptr, p.opF, sF, zp, zblk,
-                        alpha, beta, inner, yp, sY, _address(t1), _address(t2)), "gemkmStridedBatched")
-                else:
-                    check(getattr(lib, pre + "gekmmStridedBatched")(
-                        h.h, BACKEND_HIP, N, Qs, Ps, p.M, fptr, p.opF, sF, xp, p.opX, steps[0] * xblk, zp, zblk,
-                        alpha, beta, inner, yp, sY, _address(t1), _address(t2)), "gekmmStridedBatched")
+                _check(getattr(lib, pre + "gekmmStridedBatched")(
+                    h.h, BACKEND_HIP, N, Qs, Ps, p.M, fptr, p.opF, sF, xp, p.opX, steps[0] * xblk, zp, zblk,
+                    alpha, beta, inner, yp, sY, _address(t1), _address(t2)), "gekmmStridedBatched")
     if p.is_vec:
         z = z.reshape(z.shape[:-2] + (-1,))
-    return z, inter
+    return z
 
 
 def _sum_to(g, shape):
@@ -247,28 +219,126 @@ def _sum_to(g, shape):
     return g.sum_to_size(shape) if tuple(g.shape) != tuple(shape) else g
 
 
-def _mkm_backward(grad_z, x, fs, inter, need_x, need_f):
-    """Gradients of Z = X (F_0 (x) ... (x) F_{N-1}) (logical MKM shapes).  inter[j] is the input of the step of
-    factor j (the output of the step of factor j+1); the input of the last factor's step is X itself.
-    Step of factor i maps rows (m, s) of its input, reshaped (M*S, P_i), through F_i and stores column q at
-    q*S + s; its backward therefore un-shuffles the output gradient to (M*S, Q_i) first."""
-    inputs = list(inter) + [x]
-    M = grad_z.shape[-2]
+class _GradCall:
+    """One differentiable call as the library's gradient functions take it; holds shapes only, so that it can be kept
+    from the forward to the backward pass.  Batches are flattened to one dimension of nb entries; an operand that is
+    broadcast over a part of it only is expanded first."""
+
+    def __init__(self, mm, p, h, dtype):
+        self.mkm, self.nb = mm == "mkm", _prod(p.zbatch)
+        nx, nf = _prod(p.xbatch), _prod(p.fbatch)
+        self.expand_x, self.expand_f, self.per_batch = nx not in (1, self.nb), nf not in (1, self.nb), nf > 1
+        self.zbatch, self.zshape, self.is_vec, self.opX, self.opF = p.zbatch, p.zshape, p.is_vec, p.opX, p.opF
+        self.xshape = p.zbatch + ((p.M, p.K) if self.mkm else (p.K, p.M))
+        fbatch = p.zbatch if self.per_batch else ()
+        self.fshapes = [fbatch + ((P, Q) if self.mkm else (Q, P)) for P, Q in zip(p.Ps, p.Qs)]
+        self.stride_x = p.M * p.K if nx > 1 else 0
+        self.shape = (1 if self.mkm else 0, 1 if dtype == torch.float64 else 0, p.M, len(p.Ps), capi.arr_u32(p.Ps), capi.arr_u32(p.Qs))
+        save, work = ctypes.c_size_t(), ctypes.c_size_t()
+        _check(h.lib.fastKronGradSizes(h.h, *self.shape, self.opX, self.stride_x, int(self.per_batch), self.nb,
+                                       ctypes.byref(save), ctypes.byref(work)), "fastKronGradSizes")
+        self.save, self.work = save.value, work.value
+
+    def buffers(self, x, fs):
+        """The operands' row-major buffers (the swapped ones where the call says fastKronOp_T)."""
+        if self.is_vec:
+            x = x.reshape(1, -1) if self.mkm else x.reshape(-1, 1)
+        x = (x.mT if self.opX == OP_T else x).contiguous()
+        fs = [(f.mT if self.opF == OP_T else f).contiguous() for f in fs]
+        if self.expand_x:
+            x = x.expand(self.zbatch + x.shape[-2:]).contiguous()
+        if self.expand_f:
+            fs = [f.expand(self.zbatch + f.shape[-2:]).contiguous() for f in fs]
+        return x, fs
+
+    def args(self, x, fs):
+        return self.shape + (x.data_ptr(), self.opX, self.stride_x, capi.arr_ptr([f.data_ptr() for f in fs]), self.opF,
+                             int(self.per_batch), self.nb)
+
+
+def _grad_forward(mm, x, fs):
+    """(z, what the backward pass needs beside the operands, the call)"""
+    h = _handle()
+    c = _GradCall(mm, _Problem(mm, x, fs, None), h, x.dtype)
+    xb, fb = c.buffers(x, fs)
+    z, save = x.new_empty(c.zshape), x.new_empty(c.save)
+    _check(h.lib.fastKronGradForward(h.h, *c.args(xb, fb), z.data_ptr(), save.data_ptr()), "fastKronGradForward")
+    if c.is_vec:
+        z = z.reshape(z.shape[:-2] + (-1,))
+    return z, save, c
+
+
+def _grad_backward(c, grad_z, x, fs, save, need_x, need_f):
+    h = _handle()
+    gz = grad_z.contiguous()
+    xb, fb = c.buffers(x, fs)
+    gx = x.new_empty(c.xshape) if need_x else None
+    gfs = [x.new_empty(s) if n else None for s, n in zip(c.fshapes, need_f)]
+    work = x.new_empty(c.work)
+    _check(h.lib.fastKronGradBackward(h.h, *c.args(xb, fb), gz.data_ptr(), save.data_ptr(), gx.data_ptr() if need_x else None,
+                                      capi.arr_ptr([g.data_ptr() if g is not None else None for g in gfs]), work.data_ptr()),
+           "fastKronGradBackward")
+    if gx is not None:
+        gx = _sum_to(gx, c.xshape[-2:]).reshape(x.shape) if c.is_vec else _sum_to(gx, x.shape)
+    return gx, [None if g is None else _sum_to(g, f.shape) if c.per_batch else g.reshape(f.shape) for g, f in zip(gfs, fs)]
+
+
+def _differentiable_backward(grad_z, x, fs, need_x, need_f):
+    """Gradients of Z = X (F_0 (x) ... (x) F_{N-1}) from PyTorch operations, for backward passes that are themselves
+    differentiated (create_graph).  Step of factor i maps rows (m, s) of its input, reshaped (M*S, P_i), through F_i and
+    stores column q at q*S + s; its backward un-shuffles the output gradient to (M*S, Q_i) first."""
+    M = x.shape[-2]
+    inputs = [x]                                          # of the steps, last factor first
+    for f in reversed(fs[1:]):
+        P, Q = f.shape[-2:]
+        t = inputs[-1]
+        S = t.shape[-1] // P
+        o = t.reshape(t.shape[:-2] + (M * S, P)) @ f
+        inputs.append(o.reshape(o.shape[:-2] + (M, S, Q)).transpose(-1, -2).reshape(o.shape[:-2] + (M, S * Q)))
+    inputs.reverse()
     g = grad_z
     grad_fs = []
     for i, f in enumerate(fs):
         P, Q = f.shape[-2], f.shape[-1]
         S = g.shape[-1] // Q
         a = g.reshape(g.shape[:-2] + (M, Q, S)).transpose(-1, -2).reshape(g.shape[:-2] + (M * S, Q))
-        if need_f[i]:
-            inp = inputs[i]
-            inp = inp.reshape(inp.shape[:-2] + (M * S, P))
-            grad_fs.append(_sum_to(inp.mT @ a, f.shape))
-        else:
-            grad_fs.append(None)
+        inp = inputs[i].reshape(inputs[i].shape[:-2] + (M * S, P))
+        grad_fs.append(_sum_to((inp.mT.contiguous() @ a), f.shape) if need_f[i] else None)
         if i + 1 < len(fs) or need_x:
-            g = (a @ f.mT).reshape(a.shape[:-2] + (M, S * P))
+            g = (a @ f.mT.contiguous()).reshape(a.shape[:-2] + (M, S * P))
     return (_sum_to(g, x.shape) if need_x else None), grad_fs
+
+
+def _forward(mm, ctx, x, fs):
+    ctx.nf, ctx.kept = len(fs), any(f.requires_grad for f in fs)
+    if ctx.kept:
+        _validate(mm, x, fs, None)
+        z, save, ctx.call = _grad_forward(mm, x, fs)
+        ctx.save_for_backward(x, *fs, save)
+    else:
+        z = _run(mm, x, fs, 1.0, 0.0, None)
+        ctx.save_for_backward(x, *fs)
+    return z
+
+
+def _backward(mm, ctx, grad_z):
+    x, fs = ctx.saved_tensors[0], ctx.saved_tensors[1:ctx.nf + 1]
+    need_x, need_f = ctx.needs_input_grad[0], ctx.needs_input_grad[1:ctx.nf + 1]
+    if not any(need_f):
+        # one fused library call on the transposed views: dX = dZ (F_0^T (x) ...) for MKM, (F_0^T (x) ...) dZ for KMM
+        gx = _run(mm, grad_z, [f.mT for f in fs], 1.0, 0.0, None) if need_x else None
+        return (_sum_to(gx, x.shape) if gx is not None else None,) + (None,) * ctx.nf
+    if not torch.is_grad_enabled():
+        gx, gfs = _grad_backward(ctx.call, grad_z, x, fs, ctx.saved_tensors[-1], need_x, need_f)
+        return (gx,) + tuple(gfs)
+    if mm == "mkm":
+        row = lambda t: t.reshape(1, -1) if x.ndim == 1 else t
+        gx, gfs = _differentiable_backward(row(grad_z), row(x), fs, need_x, need_f)
+        return (gx.reshape(x.shape) if gx is not None else None,) + tuple(gfs)
+    # Z^T = X^T (F_0^T (x) ...): the MKM rule on the transposed tensors
+    col = lambda t: t.reshape(-1, 1) if x.ndim == 1 else t
+    gx, gfs = _differentiable_backward(col(grad_z).mT, col(x).mT, [f.mT for f in fs], need_x, need_f)
+    return (gx.mT.reshape(x.shape) if gx is not None else None,) + tuple(g.mT if g is not None else None for g in gfs)
 
 
 class MKM(torch.autograd.Function):
@@ -276,26 +346,11 @@ class MKM(torch.autograd.Function):
 
     @staticmethod
     def forward(ctx, x, *fs):
-        need_f = any(f.requires_grad for f in fs)
-        z, inter = _run("mkm", x, fs, 1.0, 0.0, None, keep_intermediates=need_f)
-        ctx.save_for_backward(x, *fs, *inter)
-        ctx.nf, ctx.kept = len(fs), need_f
-        return z
+        return _forward("mkm", ctx, x, fs)
 
     @staticmethod
     def backward(ctx, grad_z):
-        x, fs, inter = ctx.saved_tensors[0], ctx.saved_tensors[1:ctx.nf + 1], ctx.saved_tensors[ctx.nf + 1:]
-        need_x, need_f = ctx.needs_input_grad[0], ctx.needs_input_grad[1:ctx.nf + 1]
-        if not any(need_f):
-            # dX = dZ (F_0^T (x) ... (x) F_{N-1}^T): one fused library call on the transposed views
-            gx = _run("mkm", grad_z, [f.mT for f in fs], 1.0, 0.0, None, False)[0] if need_x else None
-            return (_sum_to(gx, x.shape) if gx is not None else None,) + (None,) * ctx.nf
-        xv = x.reshape(1, -1) if x.ndim == 1 else x
-        gz = grad_z.reshape(1, -1) if grad_z.ndim == 1 else grad_z
-        gx, gfs = _mkm_backward(gz, xv, fs, inter, need_x, need_f)
-        if gx is not None and x.ndim == 1:
-            gx = gx.reshape(x.shape)
-        return (gx,) + tuple(gfs)
+        return _backward("mkm", ctx, grad_z)
 
 
 class KMM(torch.autograd.Function):
@@ -304,27 +359,11 @@ class KMM(torch.autograd.Function):
 
     @staticmethod
     def forward(ctx, x, *fs):
-        need_f = any(f.requires_grad for f in fs)
-        z, inter = _run("kmm", x, fs, 1.0, 0.0, None, keep_intermediates=need_f)
-        ctx.save_for_backward(x, *fs, *inter)
-        ctx.nf = len(fs)
-        return z
+        return _forward("kmm", ctx, x, fs)
 
     @staticmethod
     def backward(ctx, grad_z):
-        x, fs, inter = ctx.saved_tensors[0], ctx.saved_tensors[1:ctx.nf + 1], ctx.saved_tensors[ctx.nf + 1:]
-        need_x, need_f = ctx.needs_input_grad[0], ctx.needs_input_grad[1:ctx.nf + 1]
-        if not any(need_f):
-            # dX = (F_0^T (x) ... (x) F_{N-1}^T) dZ
-            gx = _run("kmm", grad_z, [f.mT for f in fs], 1.0, 0.0, None, False)[0] if need_x else None
-            return (_sum_to(gx, x.shape) if gx is not None else None,) + (None,) * ctx.nf
-        # Z^T = X^T (F_0^T (x) ...): the MKM rule on the transposed tensors
-        xv = x.reshape(-1, 1) if x.ndim == 1 else x
-        gz = grad_z.reshape(-1, 1) if grad_z.ndim == 1 else grad_z
-        gx, gfs = _mkm_backward(gz.mT, xv.mT, [f.mT for f in fs], [t.mT for t in inter], need_x, need_f)
-        if gx is not None:
-            gx = gx.mT.reshape(x.shape)
-        return (gx,) + tuple(g.mT if g is not None else None for g in gfs)
+        return _backward("kmm", ctx, grad_z)
 
 
 def _wants_grad(x, fs):
@@ -347,7 +386,7 @@ def gemkm(x, fs, alpha=1.0, beta=0.0, y=None):
     if _wants_grad(x, fs):
         _no_epilogue_with_grad(alpha, beta, y)
         return MKM.apply(x, *fs)
-    return _run("mkm", x, fs, float(alpha), float(beta), y, False)[0]
+    return _run("mkm", x, fs, float(alpha), float(beta), y)
 
 
 def gekmm(fs, x, alpha=1.0, beta=0.0, y=None):
@@ -357,4 +396,4 @@ def gekmm(fs, x, alpha=1.0, beta=0.0, y=None):
     if _wants_grad(x, fs):
         _no_epilogue_with_grad(alpha, beta, y)
         return KMM.apply(x, *fs)
-    return _run("kmm", x, fs, float(alpha), float(beta), y, False)[0]
+    return _run("kmm", x, fs, float(alpha), float(beta), y)

@@ -78,6 +78,30 @@ fastKronError fastKronSetSyncHelpAfter(uint32_t polls);
 fastKronError fastKronProbeCopyPattern(fastKronHandle handle, int pattern, const float* X, const float* Y, float* Z,
                                        float* T, uint32_t M);
 
+/*
+ * Gradients.  fastKronGradForward computes Z like the forward family of include/fastkron.h (alpha = 1, no Y) and keeps in
+ * `save` what the backward pass needs; fastKronGradBackward takes the gradient gZ of Z (laid out like Z, batch entries
+ * one after the other) and writes the gradient of X to gX (row-major M x K for MKM, K x M for KMM, one per batch entry,
+ * also when X is shared by the batch) unless gX is NULL, and the gradient of every factor whose entry of gFs is not
+ * NULL (row-major P x Q for MKM, Q x P for KMM whatever opFs; with perBatchFs one per batch entry, otherwise one, summed
+ * over the batch).  Equal calls give equal bits.
+ * mkm: 1 for Z = X (F_0 x ...), 0 for Z = (F_0 x ...) X; dbl: 0 for float, 1 for double operands.  A batch has batchCount
+ * entries; X's are strideX elements apart (0: shared), the factors' P*Q elements (perBatchFs) or shared, Z's M*L.
+ * fastKronGradSizes gives the elements of `save` (kept from the forward to the backward pass, with the same shapes) and
+ * of `work` (scratch of the backward pass).  Both calls run on the handle's stream, allocate nothing and never synchronise.
+ * The reference has the forward family only and leaves gradients to PyTorch (reference pyfastkron/fastkrontorch.py:160-217).
+ */
+fastKronError fastKronGradSizes(fastKronHandle handle, int mkm, int dbl, uint32_t M, uint32_t N, const uint32_t Ps[],
+                                const uint32_t Qs[], fastKronOp opX, uint64_t strideX, int perBatchFs, uint32_t batchCount,
+                                size_t* saveElems, size_t* workElems);
+fastKronError fastKronGradForward(fastKronHandle handle, int mkm, int dbl, uint32_t M, uint32_t N, const uint32_t Ps[],
+                                  const uint32_t Qs[], const void* X, fastKronOp opX, uint64_t strideX, const void* const Fs[],
+                                  fastKronOp opFs, int perBatchFs, uint32_t batchCount, void* Z, void* save);
+fastKronError fastKronGradBackward(fastKronHandle handle, int mkm, int dbl, uint32_t M, uint32_t N, const uint32_t Ps[],
+                                   const uint32_t Qs[], const void* X, fastKronOp opX, uint64_t strideX, const void* const Fs[],
+                                   fastKronOp opFs, int perBatchFs, uint32_t batchCount, const void* gZ, void* save, void* gX,
+                                   void* const gFs[], void* work);
+
 #ifdef __cplusplus
 }
 #endif

@@ -1,0 +1,112 @@
+"""Gradients of gemkm / gekmm (kernels/gradient_mfma.hip) against PyTorch's autograd of the dense Kronecker product in
+float64 on the CPU.  Bounds: a factor gradient is a sum of n = rows products of random sign; with u the unit roundoff a
+sum of n terms in blocks of 16 and then pairs of waves has an error of about sqrt(n) * u in the norm of the result, here
+n <= 2^14: 128 u (fp32 7.6e-6, fp64 1.4e-14), doubled for the steps in front of it."""
+import numpy as np
+import pytest
+
+pytestmark = pytest.mark.gpu
+BOUND = {"float32": 2 * 128 * 2.0 ** -24, "float64": 2 * 128 * 2.0 ** -53}
+
+CASES = [
+    # mm, m, (P, Q) of every factor, batch of x, of the factors, x transposed, factors transposed
+    ("mkm", 64, [(16, 16), (16, 16)], (), (), False, False),          # whole tiles, one block
+    ("mkm", 5, [(3, 3), (5, 2), (4, 7)], (), (), False, False),       # merged, ragged
+    ("kmm", 7, [(3, 3), (5, 2), (4, 7)], (), (), False, True),        # rows of 7: no 16-byte accesses
+    ("kmm", 64, [(8, 8), (8, 8), (8, 8)], (), (), True, False),       # merged 64x64, X copied transposed
+    ("mkm", 33, [(32, 32), (32, 32)], (), (), False, False),          # two blocks, last tile incomplete
+    ("mkm", 9, [(31, 17), (18, 33)], (), (), True, True),             # padded blocks
+    ("mkm", 3, [(64, 64), (50, 64)], (), (), False, False),           # 64x64 block
+    ("mkm", 4, [(100, 70)], (), (), False, False),                    # several blocks of the factor, one step
+    ("kmm", 20, [(128, 128), (2, 2)], (), (), False, False),
+    ("mkm", 3, [(2, 3), (260, 300)], (), (), False, False),           # F beyond LDS in fp64
+    ("kmm", 1, [(16, 16), (4, 4)], (), (), False, False),             # a single column
+    ("mkm", 1, [(4, 4)] * 6, (), (), False, False),                   # one row, merged groups of three
+    ("mkm", 6, [(8, 8), (8, 8)], (3,), (), False, False),             # batch of X, shared factors
+    ("kmm", 6, [(12, 12), (9, 9)], (3,), (), False, False),
+    ("mkm", 6, [(16, 8), (8, 16)], (), (4,), False, False),           # shared X, factors per entry
+    ("kmm", 5, [(6, 6), (4, 4), (5, 5)], (2, 1), (3,), False, True),  # broadcast both ways, merged per entry
+    ("mkm", 8, [(16, 16), (16, 16)], (2, 3), (2, 3), True, False),
+]
+
+
+def reference(mm, x, fs, gz):
+    """Gradients from dense products in float64 on the CPU."""
+    import torch
+    x = x.detach().cpu().double().requires_grad_(True)
+    fs = [f.detach().cpu().double().requires_grad_(True) for f in fs]
+    k = fs[0]
+    for f in fs[1:]:
+        k = (k[..., :, None, :, None] * f[..., None, :, None, :]).reshape(k.shape[:-2] + (k.shape[-2] * f.shape[-2], k.shape[-1] * f.shape[-1]))
+    z = x @ k if mm == "mkm" else k @ x
+    return z.detach(), torch.autograd.grad(z, [x, *fs], gz.cpu().double())
+
+
+def operands(mm, m, shapes, xb, fb, trx, trf, dtype, seed=1):
+    import torch
+    g = torch.Generator().manual_seed(seed)
+    k, l = int(np.prod([p for p, _ in shapes])), int(np.prod([q for _, q in shapes]))
+
+    def rand(shape, tr):
+        t = torch.randn(shape[:-2] + (shape[-1], shape[-2]) if tr else shape, generator=g, dtype=dtype).cuda()
+        return t.mT if tr else t
+    x = rand(xb + ((m, k) if mm == "mkm" else (k, m)), trx)
+    fs = [rand(fb + ((p, q) if mm == "mkm" else (q, p)), trf) for p, q in shapes]
+    zb = tuple(torch.broadcast_shapes(xb, fb))
+    return x, fs, rand(zb + ((m, l) if mm == "mkm" else (l, m)), False)
+
+
+def rel(a, b):
+    return float((a.cpu().double() - b).norm() / b.norm())
+
+
+@pytest.mark.parametrize("dt", ["float32", "float64"])
+@pytest.mark.parametrize("case", CASES, ids=lambda c: f"{c[0]}_{c[1]}_{'_'.join('%dx%d' % s for s in c[2])}_{c[3]}_{c[4]}_{int(c[5])}{int(c[6])}")
+def test_gradients(case, dt):
+    import torch
+    import fastkron_amd as fk
+    mm, m, shapes, xb, fb, trx, trf = case
+    x, fs, gz = operands(mm, m, shapes, xb, fb, trx, trf, getattr(torch, dt))
+    zr, want = reference(mm, x, fs, gz)
+    x.requires_grad_(True)
+    for f in fs:
+        f.requires_grad_(True)
+    z = fk.gemkm(x, fs) if mm == "mkm" else fk.gekmm(fs, x)
+    assert rel(z.detach(), zr) <= BOUND[dt]
+    got = torch.autograd.grad(z, [x, *fs], gz, retain_graph=True)
+    for a, b in zip(got, want):
+        assert a.shape == b.shape and rel(a, b) <= BOUND[dt]
+    again = torch.autograd.grad(z, [x, *fs], gz, retain_graph=True)
+    assert all(torch.equal(a, b) for a, b in zip(got, again))
+    # a single factor's gradient, the chain cut short
+    only = torch.autograd.grad(z, [fs[0]], gz)[0]
+    assert rel(only, want[1]) <= BOUND[dt]
+
+
+@pytest.mark.parametrize("mm", ["mkm", "kmm"])
+def test_many_rows(mm):
+    """Every workgroup takes several tiles and the partial sums of all of them are added: 2^18 rows of integers, exact."""
+    import torch
+    import fastkron_amd as fk
+    g = torch.Generator().manual_seed(3)
+    x = torch.randint(-2, 3, (2 ** 15, 64) if mm == "mkm" else (64, 2 ** 15), generator=g).float().cuda()
+    fs = [torch.randint(-2, 3, s, generator=g).float().cuda().requires_grad_(True) for s in ((8, 8), (8, 8))]
+    gz = torch.randint(-1, 2, x.shape, generator=g).float().cuda()
+    z = fk.gemkm(x, fs) if mm == "mkm" else fk.gekmm(fs, x)
+    got = torch.autograd.grad(z, fs, gz)
+    _, want = reference(mm, x, fs, gz)
+    for a, b in zip(got, want[1:]):
+        assert torch.equal(a.cpu().double(), b)
+
+
+def test_backward_of_a_backward_pass():
+    """create_graph: the backward pass is differentiated once more."""
+    import torch
+    import fastkron_amd as fk
+    for mm in ("mkm", "kmm"):
+        x, fs, _ = operands(mm, 3, [(3, 2), (2, 4)], (), (), False, False, torch.float64)
+        x.requires_grad_(True)
+        for f in fs:
+            f.requires_grad_(True)
+        fn = fk.MKM.apply if mm == "mkm" else fk.KMM.apply
+        assert torch.autograd.gradgradcheck(fn, (x, *fs), eps=1e-6, atol=1e-5)
