@@ -73,6 +73,28 @@ static hipError_t fusedSmallLaunch(const KernelInfo& k, const StepArgs& a, hipSt
 }
 static bool fusedSmallCheck(const KernelInfo& k, const StepArgs& a) { return fusedSmallSupported(a, k.dt); }
 
+// ---- whole rows of small square factors, in place in LDS ----
+static bool smallInplaceCanRun(const KernelInfo& k, const KronProblem& p, uint32_t lo, uint32_t hi, bool first, bool,
+                               const DeviceInfo& dev) {
+  const uint32_t nf = hi - lo + 1;
+  if (k.dt != p.dt || p.mm != MMType::MKM || nf < 2 || nf > kMaxFused || p.forward) return false;
+  if (first && p.opX == 2) return false;
+  uint32_t ps[kMaxFused], qs[kMaxFused];
+  // Ahead of the kernel with two LDS buffers at every shape measured (1.1 to 3.2 times, 1 to 10000 rows), except few rows
+  // of more than 64 KB in passes of one digit (mixed chains, wide fp64 factors): one CU per row then takes longer than
+  // the other kernel's pieces of a row on many (10 x 40320, 2x2 ... 8x8: 34 us against 21; dgemkm 40 x 7^5: 26 against
+  // 23; from 100 rows on it is ahead, 36 against 47).
+  bool oneDigit = p.dt == DType::F64 && p.P[hi] >= 6;
+  for (uint32_t j = 0; j < nf; j++) {
+    ps[j] = p.P[hi - j]; qs[j] = p.Q[hi - j];
+    if (ps[j] != ps[0]) oneDigit = true;
+  }
+  if (dev.rulesOfThumb && oneDigit && p.colsBefore(hi) * dtypeSize(p.dt) > 65536 && (uint64_t)p.M * p.batch < 96) return false;
+  return dev.ldsPerBlock >= 160 * 1024 && smallInplaceFits(nf, ps, qs, p.colsBefore(hi), p.M, p.batch, p.dt);
+}
+static hipError_t smallInplaceLaunch(const KernelInfo& k, const StepArgs& a, hipStream_t s) { return launchSmallInplace(a, k.dt, s); }
+static bool smallInplaceCheck(const KernelInfo& k, const StepArgs& a) { return smallInplaceSupported(a, k.dt); }
+
 // ---- one factor of any shape up to 256x512 on the matrix cores (zero padded) ----
 static bool stepAnyCanRun(const KernelInfo& k, const KronProblem& p, uint32_t lo, uint32_t hi, bool first, bool,
                           const DeviceInfo& dev) {
@@ -104,6 +126,14 @@ void registerGenericKernels(std::vector<KernelInfo>& out) {
     k.name = std::string("gekmm_hip_gfx950_512_") + (dt == DType::F32 ? "f" : "d") + "_anyxany_256x512_1_16xany_mfma16x16x4";
     k.dt = dt; k.P = 1; k.Q = 1; k.fused = 1; k.tileM = 0; k.tileK = 0; k.threads = 256; k.variant = 0;
     k.canRun = stepAnyCanRun; k.launch = stepAnyLaunch; k.check = stepAnyCheck;
+    out.push_back(k);
+  }
+  for (DType dt : {DType::F32, DType::F64}) {
+    // ahead of the kernel with two LDS buffers: chosen first where both take the same factors
+    KernelInfo k{};
+    k.name = std::string("mkm_hip_gfx950_640_") + (dt == DType::F32 ? "f" : "d") + "_small_fused_inplace_8";
+    k.dt = dt; k.P = 1; k.Q = 1; k.fused = kMaxFused; k.tileM = 0; k.tileK = 0; k.threads = 640; k.variant = 0;
+    k.canRun = smallInplaceCanRun; k.launch = smallInplaceLaunch; k.check = smallInplaceCheck;
     out.push_back(k);
   }
   for (DType dt : {DType::F32, DType::F64}) {

@@ -161,6 +161,11 @@ bool fusedSmallFits(uint32_t nf, const uint32_t* p, const uint32_t* q, uint64_t 
 bool fusedSmallSupported(const StepArgs& a, DType dt);
 hipError_t launchFusedSmall(const StepArgs& a, DType dt, hipStream_t stream);
 
+// Whole rows of small square factors (2 <= P <= 8, any mix, at most 160 KB per row) in place in LDS, MKM layout.
+bool smallInplaceFits(uint32_t nf, const uint32_t* p, const uint32_t* q, uint64_t Kin, uint32_t M, uint32_t batch, DType dt);
+bool smallInplaceSupported(const StepArgs& a, DType dt);
+hipError_t launchSmallInplace(const StepArgs& a, DType dt, hipStream_t stream);
+
 // Kronecker products of adjacent small factors into the handle's workspace, one workgroup per product.
 hipError_t launchMergeFactors(const MergeArgs& a, DType dt, hipStream_t stream);
 // Transposed copy: in is R x C row-major per batch entry, out is C x R.

@@ -1,0 +1,391 @@
+// Whole rows of small square factors in one launch (MKM layout, 2 <= P <= 8, any mix, fp32 or fp64): 3^n, 5^n, 6^n,
+// 7^n, 8^n with row counts the 8x8 matrix-core kernel does not take, 2x3x5x7 ...
+//
+// When the factors of a launch cover whole rows, the sliced multiply of all of them leaves every digit of the column
+// index where it was, and with square factors also its extent.  The factors are therefore applied in place to rows
+// kept in LDS: a pass takes one to three adjacent digits, a thread reads the P^D values of a digit group into
+// registers, applies the D factors there and writes the values back to where they came from.  One copy of the rows
+// (not two buffers), one barrier per pass, nf / D passes.  Factor values are the same in all lanes and enter the FMAs
+// as scalar operands.
+//
+//   load     one contiguous piece of memory, 16 bytes per lane whatever its alignment: the LDS copy is shifted by
+//            the 0 .. 3 elements that the piece starts behind a 16-byte boundary;
+//   passes   last digits first; lanes run over the faster digits, the first pass (digit groups contiguous) reads with
+//            an odd lane stride (no bank conflicts) or, for even P, with 16-byte accesses;
+//   store    straight from the registers of the last pass where its lanes cover runs of 64 elements or more,
+//            otherwise from LDS.
+//
+// Bound: memory in principle; with two workgroups of 62.5 KB per CU (5^6) their load, arithmetic and store phases
+// overlap little: 4 us of FMAs and 6 us of memory per row and CU.  Measured against two launches of the kernel with two LDS
+// buffers and one factor per pass (fused_small.hip): sgemkm 1001 x 5^6 90.6 -> 45.4 us (2.8 TB/s), 4096 x 5^5 62.4 ->
+// 28.6, 1000 x 7^5 128 -> 58, dgemkm 1000 x 3^8 89 -> 28 (3.8 TB/s), 1000 x 6^5 112 -> 48.  Tried and slower: a
+// persistent form with the next rows in registers (45 -> 53 us, spills), a start delay of the CU's second workgroup
+// (no change).
+// The reference fuses factors in shared memory between two buffers (reference src/kernels/cuda/kernel.cuh:165-219).
+#include <hip/hip_runtime.h>
+#include <type_traits>
+#include "../problem.h"
+#include "launch.h"
+
+namespace fk {
+
+constexpr uint32_t kIpMaxP = 8;
+constexpr uint32_t kIpMaxThreads = 640;      // 625 digit groups of 5^6 in one round
+constexpr size_t kIpLdsMax = 160 * 1024;
+
+struct InplacePass { uint32_t f0, p, d, s, magic; };     // factors f0 .. f0+d-1, distance s between values of the first
+struct InplaceTile {
+  uint32_t P, K, rows, passes, direct, threads, tiles;            // P: of all factors, 0 if they differ
+  InplacePass ps[kMaxFused];
+};
+
+constexpr int ipPow(int p, int d) { return d == 0 ? 1 : p * ipPow(p, d - 1); }
+
+template <typename T> __device__ __forceinline__ T ipLoad(__amdgpu_buffer_rsrc_t from, uint32_t lane, uint32_t uniform) {
+  if constexpr (sizeof(T) == 4) return __builtin_bit_cast(T, __builtin_amdgcn_raw_buffer_load_b32(from, (int)lane, (int)uniform, 0));
+  else return __builtin_bit_cast(T, __builtin_amdgcn_raw_buffer_load_b64(from, (int)lane, (int)uniform, 0));
+}
+template <typename T> __device__ __forceinline__ void ipStore(T v, __amdgpu_buffer_rsrc_t to, uint32_t lane, uint32_t uniform) {
+  typedef unsigned int U2 __attribute__((ext_vector_type(2)));
+  if constexpr (sizeof(T) == 4) __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(unsigned int, v), to, (int)lane, (int)uniform, 0);
+  else __builtin_amdgcn_raw_buffer_store_b64(__builtin_bit_cast(U2, v), to, (int)lane, (int)uniform, 0);
+}
+
+// out = alpha * v (+ beta * y)
+template <typename T, bool HAS_Y>
+struct IpOut {
+  T* out; const T* y; T alpha, beta;
+  __amdgpu_buffer_rsrc_t target, yTarget;                    // the same as buffer descriptors
+  __device__ __forceinline__ void put(uint32_t e, T v) const {
+    v *= alpha;
+    if (HAS_Y) v += beta * y[e];
+    out[e] = v;
+  }
+};
+
+// S: the distance between the values of the fastest digit when it is known at compile time (the values' addresses are
+// then offsets of one register), 0 otherwise.
+template <typename T, int P, int D, int S, bool HAS_Y>
+__device__ __forceinline__ void ipPass(T* __restrict__ rows, const StepArgs& a, const InplacePass& ps, const uint32_t b,
+                                       const uint32_t E, const bool vec, const bool toMemory, const IpOut<T, HAS_Y>& o) {
+  constexpr int N = ipPow(P, D), VE = 16 / (int)sizeof(T);
+  constexpr int U = N >= 16 ? 1 : N >= 6 ? 2 : 4;            // digit groups per thread and round
+  constexpr int kScalars = 64;                               // scalar registers for factor values
+  constexpr bool kHoist = D * P * P * (int)sizeof(T) / 4 <= kScalars;
+  constexpr int TQ0 = kScalars * 4 / (int)sizeof(T) / P, TQ = TQ0 < P ? TQ0 : P;      // columns of a factor at a time
+  static_assert(TQ == P || D == 1, "the values read are overwritten after all columns");
+  typedef T VT __attribute__((ext_vector_type(VE)));
+  typedef const __attribute__((address_space(4))) T* ConstPtr;
+  const uint32_t s = S ? S : ps.s, groups = E / N, nth = blockDim.x;
+  // (read-only for the whole launch, the same address in every lane: the constant address space makes these scalar loads)
+  auto loadF = [&](int d, int q0, T (&F_)[P][TQ]) {
+    uint64_t fa = (uint64_t)((const T*)a.f[ps.f0 + d] + (size_t)b * a.f_batch[ps.f0 + d]);
+    if (!kHoist) {
+      // all factor values of a pass do not fit the scalar registers: opaque, so that they are not kept for the next round
+      asm volatile("" : "+s"(fa));
+      __builtin_amdgcn_sched_barrier(0);
+    }
+    const ConstPtr F = (ConstPtr)(uintptr_t)fa;
+    // (a factor is stored P x P one way or the other: constant offsets become wide scalar loads)
+    const bool pMajor = a.f_sq[ps.f0 + d] == 1;
+    if constexpr (TQ == P) {
+      // (selected as whole numbers: selections of floating-point values would move them to vector registers)
+      typedef std::conditional_t<sizeof(T) == 4, uint32_t, uint64_t> W;
+      W m[P * P];
+#pragma unroll
+      for (int i = 0; i < P * P; i++) m[i] = __builtin_bit_cast(W, (T)F[i]);
+#pragma unroll
+      for (int p = 0; p < P; p++)
+#pragma unroll
+        for (int q = 0; q < P; q++) F_[p][q] = __builtin_bit_cast(T, p == q || pMajor ? m[p * P + q] : m[q * P + p]);
+    } else if (pMajor) {
+#pragma unroll
+      for (int p = 0; p < P; p++)
+#pragma unroll
+        for (int q = 0; q < TQ; q++) if (q0 + q < P) F_[p][q] = F[p * P + q0 + q];
+    } else {
+#pragma unroll
+      for (int q = 0; q < TQ; q++)
+#pragma unroll
+        for (int p = 0; p < P; p++) if (q0 + q < P) F_[p][q] = F[p + (q0 + q) * P];
+    }
+  };
+  T Fk[kHoist ? D : 1][P][TQ];
+  if constexpr (kHoist) {
+#pragma unroll
+    for (int d = 0; d < D; d++) loadF(d, 0, Fk[d]);
+  }
+  for (uint32_t g0 = threadIdx.x; g0 < groups; g0 += U * nth) {
+    uint32_t step = s;
+    asm volatile("" : "+s"(step));                             // (its multiples would fill the registers)
+    uint32_t e0[U];
+    T x[U][N];
+    const bool v16 = S == 1 && N % VE == 0 && vec;
+#pragma unroll
+    for (int k = 0; k < U; k++) {
+      const uint32_t g = g0 + k * nth;
+      const uint32_t hi = S == 1 ? g : S ? g / (uint32_t)(S ? S : 1) : __umulhi(g, ps.magic);
+      e0[k] = hi * (s * N) + (g - hi * s);
+      if (U > 1 && g >= groups) continue;
+      if (v16) {
+#pragma unroll
+        for (int i = 0; i < N / VE; i++) {
+          const VT t = *(const VT*)(rows + e0[k] + i * VE);
+#pragma unroll
+          for (int j = 0; j < VE; j++) x[k][i * VE + j] = t[j];
+        }
+      } else {
+        uint32_t at = e0[k];
+#pragma unroll
+        for (int i = 0; i < N; i++, at += step) x[k][i] = rows[S ? e0[k] + i * S : at];
+      }
+    }
+#pragma unroll
+    for (int d = 0; d < D; d++) {
+      const int st = ipPow(P, d);
+      T u[TQ == P ? 1 : U][TQ == P ? 1 : P];
+      if constexpr (TQ < P) {
+#pragma unroll
+        for (int k = 0; k < U; k++)
+#pragma unroll
+          for (int p = 0; p < P; p++) u[k][p] = x[k][p];
+      }
+#pragma unroll
+      for (int q0 = 0; q0 < P; q0 += TQ) {
+        T Fl[P][TQ];
+        if constexpr (!kHoist) loadF(d, q0, Fl);
+#pragma unroll
+        for (int k = 0; k < U; k++)
+#pragma unroll
+          for (int r = 0; r < N / P; r++) {
+            const int i0 = r / st * (st * P) + r % st;
+            T v[P];
+#pragma unroll
+            for (int p = 0; p < P; p++) v[p] = TQ < P ? u[TQ == P ? 0 : k][TQ == P ? 0 : p] : x[k][i0 + p * st];
+#pragma unroll
+            for (int q = 0; q < TQ; q++) {
+              if (q0 + q >= P) continue;
+              T acc = v[0] * (kHoist ? Fk[kHoist ? d : 0][0][q] : Fl[0][q]);
+#pragma unroll
+              for (int p = 1; p < P; p++) acc += v[p] * (kHoist ? Fk[kHoist ? d : 0][p][q] : Fl[p][q]);
+              x[k][i0 + (q0 + q) * st] = acc;
+            }
+          }
+      }
+    }
+#pragma unroll
+    for (int k = 0; k < U; k++) {
+      if (U > 1 && g0 + k * nth >= groups) continue;
+      uint32_t at = e0[k];
+      if (toMemory) {
+        // through buffer descriptors: one address register per group, the values' distances as scalar offsets
+        T yv[HAS_Y ? N : 1];
+        if constexpr (HAS_Y) {
+#pragma unroll
+          for (uint32_t i = 0; i < N; i++) yv[i] = ipLoad<T>(o.yTarget, e0[k] * sizeof(T), i * step * sizeof(T));
+        }
+#pragma unroll
+        for (uint32_t i = 0; i < N; i++) {
+          T v = x[k][i] * o.alpha;
+          if constexpr (HAS_Y) v += o.beta * yv[i];
+          ipStore<T>(v, o.target, e0[k] * sizeof(T), i * step * sizeof(T));
+        }
+      } else if (v16) {
+#pragma unroll
+        for (int i = 0; i < N / VE; i++) {
+          VT t;
+#pragma unroll
+          for (int j = 0; j < VE; j++) t[j] = x[k][i * VE + j];
+          *(VT*)(rows + e0[k] + i * VE) = t;
+        }
+      } else {
+#pragma unroll
+        for (int i = 0; i < N; i++, at += step) rows[S ? e0[k] + i * S : at] = x[k][i];
+      }
+    }
+  }
+}
+
+// The pass with its distance as a constant where the chain is one of equal factors (1, P^D, P^2D) or begins it.
+template <typename T, int P, int D, bool HAS_Y>
+__device__ __forceinline__ void ipPassAny(T* __restrict__ rows, const StepArgs& a, const InplacePass& ps, const uint32_t b,
+                                          const uint32_t E, const bool vec, const bool toMemory, const IpOut<T, HAS_Y>& o) {
+  constexpr int N = ipPow(P, D);
+  if (ps.s == 1) return ipPass<T, P, D, 1, HAS_Y>(rows, a, ps, b, E, vec, false, o);
+  if constexpr (N >= 25) {
+    if (ps.s == N) return ipPass<T, P, D, N, HAS_Y>(rows, a, ps, b, E, false, toMemory, o);
+    if constexpr (P < 7) { if (ps.s == N * N) return ipPass<T, P, D, N * N, HAS_Y>(rows, a, ps, b, E, false, toMemory, o); }
+  }
+  ipPass<T, P, D, 0, HAS_Y>(rows, a, ps, b, E, false, toMemory, o);
+}
+
+// Digits per pass: as many as their values fit the registers.
+constexpr int ipDepth(int p, size_t es) { return p <= 3 ? 3 : p <= 5 || (p <= 7 && es == 4) ? 2 : 1; }
+// Waves per SIMD: fp32 rows of up to 80 KB run as two workgroups of ten waves per CU; the wider groups have fewer
+// threads (6^5: 216 groups, 7^5: 343) and take more registers.
+constexpr int ipWaves(int p, size_t es) { return es == 8 || p == 7 ? 3 : p == 6 || p == 8 || p == 0 ? 4 : 5; }
+
+// P: all factors are PxP; 0: any mix, one digit per pass.
+template <typename T, int P, bool HAS_Y>
+__global__ __launch_bounds__(kIpMaxThreads, ipWaves(P, sizeof(T)))
+void kron_small_inplace_kernel(const StepArgs a, const InplaceTile t) {
+  constexpr uint32_t VE = 16 / sizeof(T);
+  typedef T VT __attribute__((ext_vector_type(VE)));
+  extern __shared__ __align__(16) unsigned char ipLds[];
+  const uint32_t tid = threadIdx.x, nth = blockDim.x, b = blockIdx.y;
+  const uint32_t m0 = blockIdx.x * t.rows;
+  const uint32_t E = (a.M - m0 < t.rows ? a.M - m0 : t.rows) * t.K;
+  const T* src = (const T*)a.in + (size_t)b * a.in_batch + (size_t)m0 * t.K;
+  const uint32_t shift = (uint32_t)((uintptr_t)src / sizeof(T)) & (VE - 1);
+  VT* chunks = (VT*)ipLds;
+  T* rows = (T*)ipLds + shift;
+  IpOut<T, HAS_Y> o;
+  o.out = (T*)a.out + (size_t)b * a.out_batch + (size_t)m0 * t.K;
+  o.y = HAS_Y ? (const T*)a.y + (size_t)b * a.y_batch + (size_t)m0 * t.K : nullptr;
+  o.target = streamTarget(o.out, E * (uint32_t)sizeof(T));
+  if (HAS_Y) o.yTarget = streamTarget((void*)o.y, E * (uint32_t)sizeof(T));
+  o.alpha = a.epilogue ? (T)a.alpha : T(1); o.beta = (T)a.beta;
+
+  // 16-byte pieces that lie inside the rows, then the elements before the first and behind the last of them
+  const uint32_t first = shift ? 1 : 0, last = (shift + E) / VE;
+  constexpr int LU = 8;
+  for (uint32_t c0 = first + tid; c0 < last; c0 += LU * nth) {
+    VT v[LU];
+#pragma unroll
+    for (int k = 0; k < LU; k++) if (c0 + k * nth < last) v[k] = *(const VT*)(src + ((int64_t)(c0 + k * nth) * VE - shift));
+#pragma unroll
+    for (int k = 0; k < LU; k++) if (c0 + k * nth < last) chunks[c0 + k * nth] = v[k];
+  }
+  if (tid < 2 * VE) {
+    const uint32_t e = tid < VE ? tid : E - 1 - (tid - VE);
+    if (e < E) {
+      const uint32_t c = (shift + e) / VE;
+      if (c < first || c >= last) rows[e] = src[e];
+    }
+  }
+  __syncthreads();
+
+  for (uint32_t i = 0; i < t.passes; i++) {
+    const InplacePass ps = t.ps[i];
+    const bool toMemory = t.direct && i + 1 == t.passes;
+    if constexpr (P == 0) {
+      switch (ps.p) {
+#define IP_CASE(PV) case PV: ipPassAny<T, PV, 1, HAS_Y>(rows, a, ps, b, E, shift == 0, toMemory, o); break;
+        IP_CASE(2) IP_CASE(3) IP_CASE(4) IP_CASE(5) IP_CASE(6) IP_CASE(7) IP_CASE(8)
+#undef IP_CASE
+        default: break;
+      }
+    } else {
+      constexpr int D = ipDepth(P, sizeof(T));
+      if (ps.d == D) ipPassAny<T, P, D, HAS_Y>(rows, a, ps, b, E, shift == 0, toMemory, o);
+      else if (ps.d == 1) ipPassAny<T, P, 1, HAS_Y>(rows, a, ps, b, E, shift == 0, toMemory, o);
+      else if constexpr (D == 3) ipPassAny<T, P, 2, HAS_Y>(rows, a, ps, b, E, shift == 0, toMemory, o);
+    }
+    if (!toMemory) __syncthreads();
+  }
+  if (t.direct) return;
+
+  const bool v16 = shift == 0 && (uintptr_t)o.out % 16 == 0 && (!HAS_Y || (uintptr_t)o.y % 16 == 0);
+  const uint32_t whole = v16 ? E / VE : 0;
+  for (uint32_t c = tid; c < whole; c += nth) {
+    VT v = chunks[c] * o.alpha;
+    if (HAS_Y) v += ((const VT*)o.y)[c] * o.beta;
+    ((VT*)o.out)[c] = v;
+  }
+  for (uint32_t e = whole * VE + tid; e < E; e += nth) o.put(e, rows[e]);
+}
+
+static bool ipTile(uint32_t nf, const uint32_t* p, const uint32_t* q, uint64_t Kin, uint32_t M, uint32_t batch, DType dt,
+                   InplaceTile* t) {
+  if (nf < 1 || nf > kMaxFused || M == 0) return false;
+  const size_t es = dtypeSize(dt);
+  uint64_t K = 1;
+  bool mixed = false;
+  for (uint32_t j = 0; j < nf; j++) {
+    if (p[j] < 2 || p[j] > kIpMaxP || q[j] != p[j]) return false;
+    K *= p[j];
+    if (p[j] != p[0]) mixed = true;
+  }
+  if (K != Kin || K * es + 16 > kIpLdsMax) return false;
+  *t = InplaceTile{};
+  t->K = (uint32_t)K; t->P = mixed ? 0 : p[0];
+  // several short rows per workgroup: up to 32 KB while that leaves two workgroups per CU and more
+  t->rows = 1;
+  while (2 * t->rows * K * es <= 32768 && (uint64_t)M * batch / (2 * t->rows) >= 512) t->rows *= 2;
+  t->tiles = (M + t->rows - 1) / t->rows;
+  uint32_t s = 1, widest = 1;
+  for (uint32_t j = 0; j < nf;) {
+    InplacePass& ps = t->ps[t->passes++];
+    const uint32_t dmax = mixed ? 1 : ipDepth(p[j], es);
+    uint32_t d = 1, n = p[j];
+    while (d < dmax && j + d < nf && p[j + d] == p[j]) { d++; n *= p[j]; }
+    ps.f0 = j; ps.p = p[j]; ps.d = d; ps.s = s;
+    // floor(g / s) = mulhi(g, magic) for g * s < 2^32: g and s are below the rows' element count, at most 40960, over n
+    ps.magic = s == 1 ? 0 : (uint32_t)((1ull << 32) / s) + 1;
+    const uint32_t groups = (uint32_t)(t->rows * K / n);
+    if (groups > widest) widest = groups;
+    j += d;
+    t->direct = s >= 64;
+    s *= n;
+  }
+  // One group per thread; with enough tiles to fill the device rather 256 threads (and more rounds) than fewer workgroups
+  // per CU than their LDS allows.
+  uint32_t most = kIpMaxThreads;
+  if ((uint64_t)t->tiles * batch >= 512) {
+    const uint32_t perCU = (uint32_t)(kIpLdsMax / (t->rows * K * es + 16));
+    const uint32_t fit = 64 * (4 * ipWaves(t->P, es) / perCU);
+    most = fit > kIpMaxThreads ? kIpMaxThreads : fit < 256 ? 256 : fit;
+  }
+  const uint32_t rounds = (widest + most - 1) / most;
+  t->threads = ((widest + rounds - 1) / rounds + 63) / 64 * 64;
+  return true;
+}
+
+bool smallInplaceFits(uint32_t nf, const uint32_t* p, const uint32_t* q, uint64_t Kin, uint32_t M, uint32_t batch, DType dt) {
+  InplaceTile t;
+  return ipTile(nf, p, q, Kin, M, batch, dt, &t);
+}
+
+bool smallInplaceSupported(const StepArgs& a, DType dt) {
+  if (a.batch == 0 || a.batch > 65535 || a.Kin != a.Kout) return false;
+  if (a.in_ldc != 1 || a.out_ldc != 1 || a.in_ldm != (int64_t)a.Kin || a.out_ldm != (int64_t)a.Kin) return false;
+  if (a.y && (a.y_ldc != 1 || a.y_ldm != (int64_t)a.Kin)) return false;
+  for (uint32_t j = 0; j < a.nf && j < kMaxFused; j++)
+    if (!(a.f_sq[j] == 1 && a.f_sp[j] == (int64_t)a.q[j]) && !(a.f_sp[j] == 1 && a.f_sq[j] == (int64_t)a.p[j])) return false;
+  return smallInplaceFits(a.nf, a.p, a.q, a.Kin, a.M, a.batch, dt);
+}
+
+template <typename T, int P, bool HAS_Y>
+static hipError_t launchIpP(const StepArgs& a, const InplaceTile& t, hipStream_t stream) {
+  static PerDeviceOnce attrOnce;
+  const int dev = launchDeviceIndex();
+  const size_t lds = (size_t)t.rows * t.K * sizeof(T) + 16;
+  if (lds > 65536 && !attrOnce.done(dev)) {
+    hipError_t e = hipFuncSetAttribute((const void*)kron_small_inplace_kernel<T, P, HAS_Y>, hipFuncAttributeMaxDynamicSharedMemorySize,
+                                       (int)kIpLdsMax);
+    if (e != hipSuccess) return e;
+    attrOnce.mark(dev);
+  }
+  hipLaunchKernelGGL((kron_small_inplace_kernel<T, P, HAS_Y>), dim3(t.tiles, a.batch), dim3(t.threads), lds,
+                     stream, a, t);
+  return hipGetLastError();
+}
+
+template <typename T>
+static hipError_t launchIpT(const StepArgs& a, const InplaceTile& t, hipStream_t stream) {
+  const bool y = a.y && a.epilogue;
+  switch (t.P) {
+#define IP_CASE(P) case P: return y ? launchIpP<T, P, true>(a, t, stream) : launchIpP<T, P, false>(a, t, stream);
+    IP_CASE(0) IP_CASE(2) IP_CASE(3) IP_CASE(4) IP_CASE(5) IP_CASE(6) IP_CASE(7) IP_CASE(8)
+#undef IP_CASE
+    default: return hipErrorInvalidValue;
+  }
+}
+
+hipError_t launchSmallInplace(const StepArgs& a, DType dt, hipStream_t stream) {
+  InplaceTile t;
+  if (!smallInplaceSupported(a, dt) || !ipTile(a.nf, a.p, a.q, a.Kin, a.M, a.batch, dt, &t)) return hipErrorInvalidValue;
+  return dt == DType::F32 ? launchIpT<float>(a, t, stream) : launchIpT<double>(a, t, stream);
+}
+
+}  // namespace fk

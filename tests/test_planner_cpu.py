@@ -441,6 +441,25 @@ def test_lds_fused_groups_get_balanced_depth(online_planner):
     assert e == capi.SUCCESS and len(names) == 1 and "small_fused" in names[0], names
 
 
+def test_whole_rows_of_small_square_factors_run_in_place(online_planner):
+    """One launch where the factors cover whole rows of at most 160 KB, are square and X is not transposed; few long rows in
+    passes of one digit stay with the kernel that spreads a row over workgroups."""
+    def inplace(mm, dt, M, Ps, Qs=None, **kw):
+        e, names, _ = plan(online_planner, mm, dt, M, Ps, Qs or Ps, **kw)
+        assert e == capi.SUCCESS
+        return len(names) == 1 and "inplace" in names[0]
+    mixed = [2, 3, 4, 5, 6, 7, 8]
+    for dt in ("s", "d"):
+        assert inplace("mkm", dt, 1, [5] * 6) and inplace("mkm", dt, 1001, [5] * 6, beta=0.5, with_y=True)
+        assert inplace("mkm", dt, 7, [7, 3, 8], opF=capi.OP_T, offs={"x": 4 if dt == "s" else 8, "z": 8})
+        assert inplace("mkm", dt, 9, [5, 5, 5], batch=3) and inplace("kmm", dt, 1, [5] * 4)
+        assert not inplace("mkm", dt, 9, [5, 5, 5], opX=capi.OP_T) and not inplace("kmm", dt, 2, [5] * 4)
+        assert not inplace("mkm", dt, 9, [5, 5], [5, 4]) and not inplace("mkm", dt, 9, [5] * 7)
+    assert not inplace("mkm", "s", 95, mixed) and inplace("mkm", "s", 96, mixed)
+    assert not inplace("mkm", "d", 95, [7] * 5) and inplace("mkm", "d", 96, [7] * 5) and inplace("mkm", "s", 1, [7] * 5)
+    assert not inplace("mkm", "d", 1000, mixed)                       # 315 KB
+
+
 def test_padded_step_rules_for_rectangular_and_large_odd_factors(online_planner):
     planner = online_planner
     # shrinking factors with 16 rows: padded matrix-core step, not the plain kernel

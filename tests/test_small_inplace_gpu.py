@@ -1,0 +1,65 @@
+"""Rows of small square factors applied in place in LDS (kernels/small_inplace.hip) against the oracle, at the edges of
+its tiles: one row and several per workgroup, a last workgroup that is not full, rows that start off a 16-byte
+boundary, single digits and groups of them, stores from registers and from LDS.  TOL of gpu_util: normwise 1e-5 / 1e-12;
+the sums have at most 8 terms per factor and nine factors, so u * 72 = 4.3e-6 / 8e-15 bounds the error."""
+import numpy as np
+import pytest
+
+from oracle import kron_oracle as ko
+from tests.gpu_util import TOL, make_case, normwise, oracle_answer, run_gpu
+
+pytestmark = pytest.mark.gpu
+
+CASES = [
+    # rows, factors
+    (1, [5] * 6),            # one row
+    (7, [5] * 6),            # odd row length: every alignment of a row
+    (2, [5] * 5), (3, [3] * 8), (3, [7] * 5), (2, [6] * 5), (5, [6, 6, 6]),
+    (1100, [3, 3]),          # several rows per workgroup, last one not full
+    (2051, [5, 5, 5]), (1031, [7, 7]), (1029, [2, 2, 2, 2, 2]), (4111, [6, 2]), (1057, [4, 4, 4]),
+    (13, [8, 8, 8]), (9, [8] * 4), (4, [2, 3, 5, 7, 8]), (3, [8, 7, 5, 3, 2]), (2, [4, 4, 8, 3, 3, 3, 3]),
+    (2, [2, 3, 4, 5, 6, 7, 8]),      # 40320 columns: a whole CU's LDS in fp32
+]
+
+
+@pytest.fixture(scope="module")
+def fk():
+    import fastkron_amd
+    h = fastkron_amd.FastKron()
+    yield h
+    h.close()
+
+
+@pytest.mark.parametrize("dt", [np.float32, np.float64], ids=["f", "d"])
+@pytest.mark.parametrize("M,Ps", CASES, ids=lambda v: str(v) if isinstance(v, int) else "x".join(map(str, v)))
+def test_small_factors_in_place(fk, M, Ps, dt):
+    for seed, kw in enumerate([dict(alpha=1.5, beta=0.5), dict(alpha=1.0, beta=0.0, opFs=ko.OP_T),
+                               dict(alpha=1.0, beta=0.0, batch=3), dict(alpha=-2.0, beta=1.0, batch=2, share_f=True)]):
+        alpha, beta = kw.pop("alpha"), kw.pop("beta")
+        batch, share = kw.get("batch", 1), dict(share_f=True) if kw.get("share_f") else {}
+        X, Fs, Y = make_case(ko.MKM, M, Ps, Ps, dt, seed=7 + 50 * seed, with_y=beta != 0.0, batch=batch, **share)
+        want = oracle_answer(ko.MKM, M, Ps, Ps, X, Fs, Y, alpha, beta, **kw)
+        got, e = run_gpu(fk, ko.MKM, M, Ps, Ps, X, Fs, Y, alpha, beta, **kw)
+        assert e == 0 and normwise(got, want) <= TOL[dt], (fk.last_plan(), kw)
+
+
+def test_rows_off_a_16_byte_boundary(fk):
+    """Base addresses that are only 4-byte aligned, of X and of Z, and the in-place epilogue (Y is Z)."""
+    import torch
+    M, Ps = 6, [5, 5, 5, 5]
+    K = 625
+    X, Fs, Y = make_case(ko.MKM, M, Ps, Ps, np.float32, seed=3)
+    want = oracle_answer(ko.MKM, M, Ps, Ps, X, Fs, Y, 1.5, 0.5).reshape(-1)
+    fs = [torch.from_numpy(f).cuda() for f in Fs]
+    for off in (1, 2, 3):
+        x = torch.full((M * K + 8,), float("nan"), device="cuda")
+        z = torch.full((M * K + 8,), 77.0, device="cuda")
+        x[off:off + M * K] = torch.from_numpy(X).cuda().reshape(-1)
+        z[off:off + M * K] = torch.from_numpy(Y).cuda().reshape(-1)
+        t1, t2 = torch.empty(M * K, device="cuda"), torch.empty(M * K, device="cuda")
+        zv = z[off:off + M * K]
+        assert fk.xgemkm(M, Ps, Ps, x[off:off + M * K], fs, zv, 1.5, 0.5, zv, t1, t2) == 0
+        torch.cuda.synchronize()
+        assert "inplace" in fk.last_plan()[0][2]
+        assert normwise(zv.cpu().numpy(), want) <= TOL[np.float32]
+        assert bool((z[:off] == 77.0).all()) and bool((z[off + M * K:] == 77.0).all())
