@@ -24,3 +24,14 @@ done
 for p in "${pids[@]}"; do wait "$p"; done
 "$HIPCC" -shared -fPIC --offload-arch=gfx950 -o "$OUT/libFastKron.so" "${objs[@]}"
 echo "built $OUT/libFastKron.so"
+# the PyTorch front end's host path: host code only, against the headers of the PyTorch that runs it
+read -r -a TORCH < <(python3 - <<'PY'
+import os, sysconfig, torch
+from torch.utils import cpp_extension
+print(*(f"-isystem {p}" for p in cpp_extension.include_paths() + [sysconfig.get_paths()["include"]]),
+      f"-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}", f"-L{os.path.join(os.path.dirname(torch.__file__), 'lib')}")
+PY
+)
+g++ -O2 -std=c++17 -fPIC -shared -fvisibility=hidden -Wall -I"$HERE/../../include" "$HERE/frontend.cpp" -o "$OUT/_frontend.so" \
+    "${TORCH[@]}" -ltorch_python -ltorch_cpu -ltorch -lc10
+echo "built $OUT/_frontend.so"

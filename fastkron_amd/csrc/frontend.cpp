@@ -1,0 +1,367 @@
+// The PyTorch front end's host path in native code: from tensors to one library call (fastkron_amd/torch_frontend.py has
+// the entry points, the autograd functions and the messages of refused operands).
+//
+// A product of small operands costs what the host spends on it: in Python the shape rules, three allocations, a dozen
+// ctypes objects and the stream look-up took 27 of the 34.5 us of a vector against 8x8 (x) 8x8 (x) 8x8 (now 7.7 us with
+// its kernel of 5 us; sgemkm 4096 x 32x32^2 with all gradients 175 -> 95 us, dgekmm 8x8^5 x 16 with factor gradients 255
+// -> 123 us).  Everything between the Python call and the C API happens here instead; nothing is kept between calls.
+// A function returns None for operands that it does not take (the Python side then says why), a fastKronError as a
+// whole number where the library refuses the call, and otherwise its tensors; product returns False for a call that is
+// to be recorded for gradients.  The interpreter's lock is held throughout: threads share the default handle.
+//
+// Rules (reference pyfastkron/fastkronbase.py:104-518): leading dimensions are batches, broadcast between X, the factors
+// and Y; the innermost batch dimension is one strided-batched call (stride 0 = shared operand), outer ones a loop; a
+// batch of X against shared factors is more rows of one problem (MKM); transposed views are passed as their buffer.
+#include <Python.h>
+#include <torch/csrc/Exceptions.h>
+#include <torch/csrc/autograd/python_variable.h>
+#include <ATen/ATen.h>
+#include <c10/core/GradMode.h>
+
+#include <cstdint>
+#include <vector>
+
+#include "../../include/fastkron.h"
+#include "../../include/fastkron_ext.h"
+
+namespace {
+
+using at::Tensor;
+using Dims = c10::SmallVector<int64_t, 8>;
+
+constexpr int kMaxFactors = 64;
+
+// Entry points of the library that Python has loaded.
+struct Api {
+  decltype(&sgemkm) sgemkm_; decltype(&dgemkm) dgemkm_; decltype(&sgekmm) sgekmm_; decltype(&dgekmm) dgekmm_;
+  decltype(&sgemkmStridedBatched) sgemkmB; decltype(&dgemkmStridedBatched) dgemkmB;
+  decltype(&sgekmmStridedBatched) sgekmmB; decltype(&dgekmmStridedBatched) dgekmmB;
+  decltype(&gekmmSizes) sizes; decltype(&fastKronSetStream) setStream;
+  decltype(&fastKronGradSizes) gradSizes; decltype(&fastKronGradForward) gradForward; decltype(&fastKronGradBackward) gradBackward;
+} api;
+
+int64_t prod(at::IntArrayRef d) { int64_t n = 1; for (int64_t v : d) n *= v; return n; }
+Dims batchOf(const Tensor& t) { return t.dim() > 2 ? Dims(t.sizes().begin(), t.sizes().end() - 2) : Dims(); }
+
+bool broadcast(const Dims& a, const Dims& b, Dims* out) {
+  const size_t n = std::max(a.size(), b.size());
+  out->assign(n, 1);
+  for (size_t i = 0; i < n; i++) {
+    const int64_t x = i < n - a.size() ? 1 : a[i - (n - a.size())], y = i < n - b.size() ? 1 : b[i - (n - b.size())];
+    if (x != y && x != 1 && y != 1) return false;
+    (*out)[i] = x == 1 ? y : x;
+  }
+  return true;
+}
+
+// X and factors as the library takes them: row-major buffers (the swapped one of a transposed view, op T).
+struct Operands {
+  bool mkm, vec;                              // vec: X has one dimension
+  fastKronOp opX, opF;
+  Tensor x, f[kMaxFactors];
+  uint32_t N, Ps[kMaxFactors], Qs[kMaxFactors];
+  int64_t M, K, L;
+  Dims xb, fb, zb, zshape;                    // batch dimensions of X, of the factors and of the result
+
+  void setZShape() {
+    zshape = zb;
+    zshape.push_back(mkm ? M : L); zshape.push_back(mkm ? L : M);
+  }
+  bool f64() const { return x.scalar_type() == at::kDouble; }
+};
+
+bool usable(const Tensor& t) { return t.defined() && t.is_cuda() && t.layout() == at::kStrided; }
+
+bool swapped(const Tensor& t) { return !t.is_contiguous() && t.dim() >= 2 && t.mT().is_contiguous(); }
+Tensor buffer(const Tensor& t, fastKronOp op) { return (op == fastKronOp_T ? t.mT() : t).contiguous(); }
+
+// ops: the storage to use (0: as the tensors are stored)
+bool makeOperands(bool mkm, PyObject* px, PyObject* pfs, int opX, int opF, Operands* o) {
+  if (!THPVariable_Check(px) || !(PyList_Check(pfs) || PyTuple_Check(pfs))) return false;
+  const Py_ssize_t n = PySequence_Fast_GET_SIZE(pfs);
+  if (n == 0 || n > kMaxFactors) return false;
+  Tensor x = THPVariable_Unpack(px);
+  if (!usable(x) || (x.scalar_type() != at::kFloat && x.scalar_type() != at::kDouble) || x.dim() == 0) return false;
+  o->mkm = mkm; o->N = (uint32_t)n; o->vec = x.dim() == 1;
+  if (o->vec) x = mkm ? x.reshape({1, -1}) : x.reshape({-1, 1});
+  bool anyT = false, anyN = false;
+  for (Py_ssize_t i = 0; i < n; i++) {
+    PyObject* pf = PySequence_Fast_GET_ITEM(pfs, i);
+    if (!THPVariable_Check(pf)) return false;
+    const Tensor& f = THPVariable_Unpack(pf);
+    if (!usable(f) || f.dim() < 2 || f.scalar_type() != x.scalar_type() || f.device() != x.device()) return false;
+    if (i && f.sizes().slice(0, f.dim() - 2) != o->f[0].sizes().slice(0, o->f[0].dim() - 2)) return false;
+    o->f[i] = f;
+    (swapped(f) ? anyT : anyN) = true;
+    const int64_t a = f.size(-2), b = f.size(-1);
+    if (a == 0 || b == 0) return false;
+    o->Ps[i] = (uint32_t)(mkm ? a : b); o->Qs[i] = (uint32_t)(mkm ? b : a);
+  }
+  o->fb = batchOf(o->f[0]);
+  o->xb = batchOf(x);
+  o->M = mkm ? x.size(-2) : x.size(-1); o->K = mkm ? x.size(-1) : x.size(-2);
+  int64_t k = 1;
+  o->L = 1;
+  for (Py_ssize_t i = 0; i < n; i++) { k *= o->Ps[i]; o->L *= o->Qs[i]; }
+  if (k != o->K || !broadcast(o->xb, o->fb, &o->zb)) return false;
+  o->setZShape();
+  o->opX = opX ? (fastKronOp)opX : swapped(x) ? fastKronOp_T : fastKronOp_N;
+  o->opF = opF ? (fastKronOp)opF : anyT && !anyN ? fastKronOp_T : fastKronOp_N;      // one op is passed for all factors
+  o->x = buffer(x, o->opX);
+  for (Py_ssize_t i = 0; i < n; i++) o->f[i] = buffer(o->f[i], o->opF);
+  return true;
+}
+
+struct Call { fastKronHandle handle; void* stream; };
+
+// handle, stream, mkm: the first arguments of every function
+bool callOf(PyObject* const* args, Call* c, bool* mkm) {
+  c->handle = (fastKronHandle)PyLong_AsVoidPtr(args[0]);
+  c->stream = PyLong_AsVoidPtr(args[1]);
+  *mkm = PyObject_IsTrue(args[2]) == 1;
+  return !PyErr_Occurred();
+}
+
+PyObject* failed(fastKronError e) { return PyLong_FromLong((long)e); }
+
+fastKronError call(const Call& c, const Operands& o, uint32_t M, const void* x, const void* const* f, void* z, double alpha,
+                   double beta, const void* y, void* t1, void* t2) {
+  const fastKronBackend B = fastKronBackend_HIP;
+  if (o.f64()) {
+    if (o.mkm) return api.dgemkm_(c.handle, B, M, o.N, (uint32_t*)o.Ps, (uint32_t*)o.Qs, (double*)x, o.opX, (const double**)f, o.opF, (double*)z,
+                                  alpha, beta, (const double*)y, (double*)t1, (double*)t2);
+    return api.dgekmm_(c.handle, B, o.N, (uint32_t*)o.Qs, (uint32_t*)o.Ps, M, (const double**)f, o.opF, (double*)x, o.opX, (double*)z, alpha, beta,
+                       (const double*)y, (double*)t1, (double*)t2);
+  }
+  if (o.mkm) return api.sgemkm_(c.handle, B, M, o.N, (uint32_t*)o.Ps, (uint32_t*)o.Qs, (float*)x, o.opX, (const float**)f, o.opF, (float*)z,
+                                (float)alpha, (float)beta, (const float*)y, (float*)t1, (float*)t2);
+  return api.sgekmm_(c.handle, B, o.N, (uint32_t*)o.Qs, (uint32_t*)o.Ps, M, (const float**)f, o.opF, (float*)x, o.opX, (float*)z, (float)alpha,
+                     (float)beta, (const float*)y, (float*)t1, (float*)t2);
+}
+
+fastKronError callBatched(const Call& c, const Operands& o, const void* x, uint64_t sx, const void* const* f, uint64_t* sf, void* z,
+                          uint64_t sz, double alpha, double beta, uint32_t batch, const void* y, uint64_t sy, void* t1, void* t2) {
+  const fastKronBackend B = fastKronBackend_HIP;
+  const uint32_t M = (uint32_t)o.M;
+  if (o.f64()) {
+    if (o.mkm) return api.dgemkmB(c.handle, B, M, o.N, (uint32_t*)o.Ps, (uint32_t*)o.Qs, (double*)x, o.opX, sx, (const double**)f, o.opF, sf,
+                                  (double*)z, sz, alpha, beta, batch, (const double*)y, sy, (double*)t1, (double*)t2);
+    return api.dgekmmB(c.handle, B, o.N, (uint32_t*)o.Qs, (uint32_t*)o.Ps, M, (const double**)f, o.opF, sf, (double*)x, o.opX, sx, (double*)z, sz,
+                       alpha, beta, batch, (const double*)y, sy, (double*)t1, (double*)t2);
+  }
+  if (o.mkm) return api.sgemkmB(c.handle, B, M, o.N, (uint32_t*)o.Ps, (uint32_t*)o.Qs, (float*)x, o.opX, sx, (const float**)f, o.opF, sf,
+                                (float*)z, sz, (float)alpha, (float)beta, batch, (const float*)y, sy, (float*)t1, (float*)t2);
+  return api.sgekmmB(c.handle, B, o.N, (uint32_t*)o.Qs, (uint32_t*)o.Ps, M, (const float**)f, o.opF, sf, (float*)x, o.opX, sx, (float*)z, sz,
+                     (float)alpha, (float)beta, batch, (const float*)y, sy, (float*)t1, (float*)t2);
+}
+
+// product(handle, stream, mkm, x, fs, alpha, beta, y) -> z, or False
+PyObject* product(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
+  HANDLE_TH_ERRORS
+  Call c; bool mkm;
+  if (nargs != 8 || !callOf(args, &c, &mkm)) { if (!PyErr_Occurred()) PyErr_SetString(PyExc_TypeError, "product: 8 arguments"); return nullptr; }
+  const double alpha = PyFloat_AsDouble(args[5]), beta = PyFloat_AsDouble(args[6]);
+  if (PyErr_Occurred()) return nullptr;
+  Operands o;
+  if (!makeOperands(mkm, args[3], args[4], 0, 0, &o)) Py_RETURN_NONE;
+  if (c10::GradMode::is_enabled()) {
+    bool wanted = THPVariable_Unpack(args[3]).requires_grad();
+    for (uint32_t i = 0; i < o.N; i++) wanted = wanted || THPVariable_Unpack(PySequence_Fast_GET_ITEM(args[4], i)).requires_grad();
+    if (wanted) Py_RETURN_FALSE;
+  }
+  Tensor y;
+  Dims yb;
+  if (args[7] != Py_None) {
+    if (!THPVariable_Check(args[7])) Py_RETURN_NONE;
+    y = THPVariable_Unpack(args[7]);
+    if (!usable(y) || y.scalar_type() != o.x.scalar_type() || y.device() != o.x.device()) Py_RETURN_NONE;
+    if (o.vec && y.dim() == 1) y = mkm ? y.reshape({1, -1}) : y.reshape({-1, 1});
+    if (y.dim() < 2 || y.size(-2) != o.zshape[o.zshape.size() - 2] || y.size(-1) != o.zshape.back()) Py_RETURN_NONE;
+    yb = batchOf(y);
+    Dims both;
+    if (!broadcast(yb, o.zb, &both) || both != o.zb) Py_RETURN_NONE;
+    y = y.contiguous();
+  } else if (beta != 0.0) Py_RETURN_NONE;
+
+  Tensor z = at::empty(o.zshape, o.x.options());
+  const size_t es = z.element_size();
+  // batch of X against shared factors: more rows of the same problem (MKM, X stored row-major)
+  const bool fold = mkm && !o.zb.empty() && o.fb.empty() && o.opX == fastKronOp_N && (!y.defined() || yb == o.zb);
+  const int64_t M = fold ? o.M * prod(o.zb) : o.M;
+  const bool one = fold || o.zb.empty();
+  const int64_t inner = one ? 1 : o.zb.back();
+  size_t ye = 0, te = 0;
+  fastKronError e = api.sizes(c.handle, (uint32_t)M, o.N, o.Ps, o.Qs, &ye, &te);
+  if (e != fastKronSuccess) return failed(e);
+  // both temporaries in one allocation, each on a 256-byte boundary
+  const size_t tn = te * (size_t)inner, off = (tn * es + 255) / 256 * 256 / es;
+  Tensor temp = at::empty({(int64_t)(off + tn)}, o.x.options());
+  char* t1 = (char*)temp.data_ptr();
+  char* t2 = t1 ? t1 + off * es : nullptr;
+  e = api.setStream(c.handle, fastKronBackend_HIP, &c.stream);
+  if (e != fastKronSuccess) return failed(e);
+
+  const void* f[kMaxFactors];
+  if (one) {
+    for (uint32_t i = 0; i < o.N; i++) f[i] = o.f[i].data_ptr();
+    e = call(c, o, (uint32_t)M, o.x.data_ptr(), f, z.data_ptr(), alpha, beta, y.defined() ? y.data_ptr() : nullptr, t1, t2);
+    if (e != fastKronSuccess) return failed(e);
+  } else {
+    const size_t d = o.zb.size();
+    // element offset of the entry `idx` (innermost index 0) of an operand with batch dimensions `b` broadcast to zb's
+    auto entry = [&](const Dims& b, const Dims& idx) {
+      int64_t lin = 0;
+      for (size_t i = 0; i < b.size(); i++) lin = lin * b[i] + (b[i] > 1 ? idx[d - b.size() + i] : 0);
+      return lin;
+    };
+    auto step = [&](const Dims& b) { return !b.empty() && b.back() > 1 ? 1 : 0; };
+    const int64_t xblk = o.M * o.K, zblk = o.M * o.L;
+    uint64_t sf[kMaxFactors];
+    for (uint32_t i = 0; i < o.N; i++) sf[i] = step(o.fb) ? (uint64_t)o.Ps[i] * o.Qs[i] : 0;
+    const int64_t outer = prod(at::IntArrayRef(o.zb.data(), d - 1));
+    Dims idx(d, 0);
+    for (int64_t lin = 0; lin < outer; lin++) {
+      int64_t rem = lin;
+      for (size_t i = d - 1; i-- > 0;) { idx[i] = rem % o.zb[i]; rem /= o.zb[i]; }
+      const int64_t fo = entry(o.fb, idx);
+      for (uint32_t i = 0; i < o.N; i++) f[i] = (char*)o.f[i].data_ptr() + (size_t)fo * o.Ps[i] * o.Qs[i] * es;
+      e = callBatched(c, o, (char*)o.x.data_ptr() + (size_t)(entry(o.xb, idx) * xblk) * es, step(o.xb) ? xblk : 0, f, sf,
+                      (char*)z.data_ptr() + (size_t)(entry(o.zb, idx) * zblk) * es, zblk, alpha, beta, (uint32_t)inner,
+                      y.defined() ? (char*)y.data_ptr() + (size_t)(entry(yb, idx) * zblk) * es : nullptr, y.defined() && step(yb) ? zblk : 0, t1,
+                      t2);
+      if (e != fastKronSuccess) return failed(e);
+    }
+  }
+  if (o.vec) {
+    Dims s = o.zb;
+    s.push_back(-1);
+    z = z.reshape(s);
+  }
+  return THPVariable_Wrap(std::move(z));
+  END_HANDLE_TH_ERRORS
+}
+
+// The operands of a differentiated call as the library's gradient functions take them: batches flattened to one dimension
+// of nb entries; an operand that is broadcast over a part of it only is expanded first.
+struct GradOperands {
+  bool perBatch; int64_t nb; uint64_t strideX; const void* f[kMaxFactors];
+};
+void gradOperands(Operands* o, GradOperands* g) {
+  g->nb = prod(o->zb);
+  const int64_t nx = prod(o->xb), nf = prod(o->fb);
+  g->perBatch = nf > 1;
+  g->strideX = nx > 1 ? (uint64_t)(o->M * o->K) : 0;
+  auto expand = [&](Tensor& t) {
+    Dims s = o->zb;
+    s.push_back(t.size(-2)); s.push_back(t.size(-1));
+    t = t.expand(s).contiguous();
+  };
+  if (nx != 1 && nx != g->nb) expand(o->x);
+  if (nf != 1 && nf != g->nb) for (uint32_t i = 0; i < o->N; i++) expand(o->f[i]);
+  for (uint32_t i = 0; i < o->N; i++) g->f[i] = o->f[i].data_ptr();
+}
+
+// grad_forward(handle, stream, mkm, x, fs) -> (z, kept for the backward pass, storage of X, of the factors)
+PyObject* gradForward(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
+  HANDLE_TH_ERRORS
+  Call c; bool mkm;
+  if (nargs != 5 || !callOf(args, &c, &mkm)) { if (!PyErr_Occurred()) PyErr_SetString(PyExc_TypeError, "grad_forward: 5 arguments"); return nullptr; }
+  Operands o; GradOperands g;
+  if (!makeOperands(mkm, args[3], args[4], 0, 0, &o)) Py_RETURN_NONE;
+  gradOperands(&o, &g);
+  size_t save = 0, work = 0;
+  fastKronError e = api.gradSizes(c.handle, mkm, o.f64(), (uint32_t)o.M, o.N, o.Ps, o.Qs, o.opX, g.strideX, g.perBatch, (uint32_t)g.nb, &save, &work);
+  if (e == fastKronSuccess) e = api.setStream(c.handle, fastKronBackend_HIP, &c.stream);
+  if (e != fastKronSuccess) return failed(e);
+  Tensor z = at::empty(o.zshape, o.x.options()), kept = at::empty({(int64_t)save}, o.x.options());
+  e = api.gradForward(c.handle, mkm, o.f64(), (uint32_t)o.M, o.N, o.Ps, o.Qs, o.x.data_ptr(), o.opX, g.strideX, g.f, o.opF, g.perBatch,
+                      (uint32_t)g.nb, z.data_ptr(), kept.data_ptr());
+  if (e != fastKronSuccess) return failed(e);
+  if (o.vec) {
+    Dims s = o.zb;
+    s.push_back(-1);
+    z = z.reshape(s);
+  }
+  return Py_BuildValue("NNii", THPVariable_Wrap(std::move(z)), THPVariable_Wrap(std::move(kept)), (int)o.opX, (int)o.opF);
+  END_HANDLE_TH_ERRORS
+}
+
+// grad_backward(handle, stream, mkm, x, fs, opX, opF, grad of z, kept, need x, need fs) -> (grad of x, of every factor)
+PyObject* gradBackward(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
+  HANDLE_TH_ERRORS
+  Call c; bool mkm;
+  if (nargs != 11 || !callOf(args, &c, &mkm)) { if (!PyErr_Occurred()) PyErr_SetString(PyExc_TypeError, "grad_backward: 11 arguments"); return nullptr; }
+  const long opX = PyLong_AsLong(args[5]), opF = PyLong_AsLong(args[6]);
+  if (PyErr_Occurred()) return nullptr;
+  Operands o; GradOperands g;
+  // (the storage of the forward pass: what was kept depends on it, also if the operands come back stored another way)
+  if (!THPVariable_Check(args[7]) || !THPVariable_Check(args[8]) || !PyTuple_Check(args[10]) ||
+      !makeOperands(mkm, args[3], args[4], (int)opX, (int)opF, &o) || PyTuple_GET_SIZE(args[10]) != (Py_ssize_t)o.N) Py_RETURN_NONE;
+  gradOperands(&o, &g);
+  const Tensor gz = THPVariable_Unpack(args[7]).contiguous(), kept = THPVariable_Unpack(args[8]).contiguous();
+  size_t save = 0, work = 0;
+  fastKronError e = api.gradSizes(c.handle, mkm, o.f64(), (uint32_t)o.M, o.N, o.Ps, o.Qs, o.opX, g.strideX, g.perBatch, (uint32_t)g.nb, &save, &work);
+  if (e == fastKronSuccess) e = api.setStream(c.handle, fastKronBackend_HIP, &c.stream);
+  if (e != fastKronSuccess) return failed(e);
+  if (gz.numel() != prod(o.zshape) || gz.scalar_type() != o.x.scalar_type() || kept.numel() != (int64_t)save) Py_RETURN_NONE;
+  const bool needX = PyObject_IsTrue(args[9]) == 1;
+  Tensor gx, gf[kMaxFactors];
+  void* gfp[kMaxFactors];
+  Dims xs = o.zb;
+  xs.push_back(mkm ? o.M : o.K); xs.push_back(mkm ? o.K : o.M);
+  if (needX) gx = at::empty(xs, o.x.options());
+  for (uint32_t i = 0; i < o.N; i++) {
+    gfp[i] = nullptr;
+    if (PyObject_IsTrue(PyTuple_GET_ITEM(args[10], i)) != 1) continue;
+    Dims s = g.perBatch ? o.zb : Dims();
+    s.push_back(mkm ? o.Ps[i] : o.Qs[i]); s.push_back(mkm ? o.Qs[i] : o.Ps[i]);
+    gf[i] = at::empty(s, o.x.options());
+    gfp[i] = gf[i].data_ptr();
+  }
+  const Tensor scratch = at::empty({(int64_t)work}, o.x.options());
+  e = api.gradBackward(c.handle, mkm, o.f64(), (uint32_t)o.M, o.N, o.Ps, o.Qs, o.x.data_ptr(), o.opX, g.strideX, g.f, o.opF, g.perBatch,
+                       (uint32_t)g.nb, gz.data_ptr(), kept.data_ptr(), needX ? gx.data_ptr() : nullptr, gfp, scratch.data_ptr());
+  if (e != fastKronSuccess) return failed(e);
+  PyObject* out = PyTuple_New(1 + (Py_ssize_t)o.N);
+  if (!out) return nullptr;
+  auto put = [&](Py_ssize_t at, Tensor t) {
+    if (!t.defined()) { Py_INCREF(Py_None); PyTuple_SET_ITEM(out, at, Py_None); }
+    else PyTuple_SET_ITEM(out, at, THPVariable_Wrap(std::move(t)));
+  };
+  // gradients are summed over the dimensions that were broadcast
+  if (needX) {
+    const Tensor& x = THPVariable_Unpack(args[3]);
+    gx = o.vec ? gx.sum_to_size({xs[xs.size() - 2], xs.back()}).reshape(x.sizes()) : gx.sizes() == x.sizes() ? gx : gx.sum_to_size(x.sizes());
+  }
+  put(0, needX ? gx : Tensor());
+  for (uint32_t i = 0; i < o.N; i++) {
+    const Tensor& f = THPVariable_Unpack(PySequence_Fast_GET_ITEM(args[4], i));
+    if (gf[i].defined() && gf[i].sizes() != f.sizes()) gf[i] = g.perBatch ? gf[i].sum_to_size(f.sizes()) : gf[i].reshape(f.sizes());
+    put(1 + i, gf[i]);
+  }
+  return out;
+  END_HANDLE_TH_ERRORS
+}
+
+// use(addresses of the entry points, in the order of Api)
+PyObject* use(PyObject*, PyObject* addresses) {
+  void* a[sizeof(Api) / sizeof(void*)];
+  constexpr Py_ssize_t n = sizeof(Api) / sizeof(void*);
+  if (!PyTuple_Check(addresses) || PyTuple_GET_SIZE(addresses) != n) { PyErr_SetString(PyExc_TypeError, "use: a tuple of addresses"); return nullptr; }
+  for (Py_ssize_t i = 0; i < n; i++) a[i] = PyLong_AsVoidPtr(PyTuple_GET_ITEM(addresses, i));
+  if (PyErr_Occurred()) return nullptr;
+  memcpy((void*)&api, a, sizeof(api));
+  Py_RETURN_NONE;
+}
+
+PyMethodDef methods[] = {
+    {"use", (PyCFunction)use, METH_O, nullptr},
+    {"product", (PyCFunction)(void (*)(void))product, METH_FASTCALL, nullptr},
+    {"grad_forward", (PyCFunction)(void (*)(void))gradForward, METH_FASTCALL, nullptr},
+    {"grad_backward", (PyCFunction)(void (*)(void))gradBackward, METH_FASTCALL, nullptr},
+    {nullptr, nullptr, 0, nullptr}};
+PyModuleDef module = {PyModuleDef_HEAD_INIT, "_frontend", nullptr, -1, methods};
+
+}  // namespace
+
+extern "C" __attribute__((visibility("default"))) PyObject* PyInit__frontend(void) { return PyModule_Create(&module); }

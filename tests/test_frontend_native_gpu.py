@@ -1,0 +1,91 @@
+"""The native host path of the PyTorch front end (csrc/frontend.cpp): operands that are stored in unusual ways against the
+same call on plain copies (equal bits: the same kernels on the same values; where a transposed view takes another kernel,
+TOL of gpu_util), refused operands, streams, and operands that come back from saved-tensor hooks stored another way."""
+import numpy as np
+import pytest
+
+from tests.gpu_util import TOL, normwise
+
+pytestmark = pytest.mark.gpu
+
+
+def rand(*shape, dtype=None):
+    import torch
+    return torch.randn(*shape, dtype=dtype or torch.float32, device="cuda")
+
+
+@pytest.mark.parametrize("mm", ["mkm", "kmm"])
+def test_unusual_storage(mm):
+    import torch
+    import fastkron_amd as fk
+    call = (lambda x, fs, **k: fk.gemkm(x, fs, **k)) if mm == "mkm" else (lambda x, fs, **k: fk.gekmm(fs, x, **k))
+    torch.manual_seed(1)
+    shape = (6, 30) if mm == "mkm" else (30, 6)
+    fs = [rand(5, 5), rand(6, 6)]
+    x = rand(*shape)
+    want = call(x, fs)
+    wide = rand(shape[0], 2 * shape[1])
+    wide[:, ::2] = x
+    assert torch.equal(call(wide[:, ::2], fs), want)                            # neither contiguous nor transposed
+    assert normwise(call(x.t().contiguous().t(), fs).cpu(), want.cpu()) <= TOL[np.float32]
+    mixed = [fs[0], fs[1].t().contiguous().t()]                                 # factors stored differently
+    assert torch.equal(call(x, mixed), want)
+    assert torch.equal(call(x, tuple(fs)), want) and torch.equal(call(torch.nn.Parameter(x, requires_grad=False), fs), want)
+    y = rand(3, 1, *shape)                                                      # Y broadcast over a part of the batch
+    xb = rand(3, 2, *shape)
+    got = call(xb, fs, alpha=2.0, beta=0.5, y=y)
+    for i in range(3):
+        for j in range(2):
+            assert normwise(got[i, j].cpu(), (2.0 * call(xb[i, j], fs) + 0.5 * y[i, 0]).cpu()) <= TOL[np.float32]
+    v = rand(60)[::2]                                                           # a strided vector
+    assert torch.equal(call(v, fs), call(v.contiguous(), fs)) and call(v, fs).shape == (30,)
+    bf = [rand(4, 5, 5), rand(4, 6, 6)]                                         # shared X, factors per entry
+    got = call(x, bf)
+    for i in range(4):
+        assert normwise(got[i].cpu(), call(x, [f[i] for f in bf]).cpu()) <= TOL[np.float32]
+
+
+def test_refused_operands():
+    import torch
+    import fastkron_amd as fk
+    x, fs = rand(4, 16), [rand(4, 4), rand(4, 4)]
+    for bad, kind in [((x, []), ValueError), ((x, fs[0]), ValueError), (("x", fs), ValueError), ((x, [fs[0], 3]), ValueError),
+                      ((x, [fs[0], rand(4)]), ValueError), ((x, [fs[0], fs[1].cpu()]), RuntimeError),
+                      ((x, [fs[0], rand(2, 4, 4)]), ValueError), ((rand(3, 4, 16), [rand(2, 4, 4)] * 2), ValueError),
+                      ((x, fs, 1.0, 1.0, rand(4, 15)), ValueError), ((x, fs, 1.0, 1.0, rand(2, 4, 16)), ValueError),
+                      ((x, fs, 1.0, 1.0, rand(4, 16).double()), ValueError), ((x[:0], fs), fk.FastKronError),
+                      ((rand(4, 1), [rand(1, 1)] * 65), fk.FastKronError), ((rand(4, 0), [rand(0, 4), rand(4, 4)]), fk.FastKronError)]:
+        with pytest.raises(kind):
+            fk.gemkm(*bad)
+    f = [t.clone().requires_grad_(True) for t in fs]
+    with pytest.raises(ValueError):
+        fk.MKM.apply(rand(4, 15), *f)
+
+
+def test_calls_follow_the_current_stream():
+    import torch
+    import fastkron_amd as fk
+    x, fs = rand(512, 4096), [rand(16, 16) for _ in range(3)]
+    want = fk.gemkm(x, fs)
+    side = torch.cuda.Stream()
+    side.wait_stream(torch.cuda.current_stream())
+    with torch.cuda.stream(side):
+        torch.cuda._sleep(2_000_000)
+        x2 = x * 2.0
+        z = fk.gemkm(x2, fs)                                                    # has to wait for x2
+    side.synchronize()
+    assert torch.equal(z, fk.gemkm(x2, fs)) and normwise(z.cpu(), 2.0 * want.cpu()) <= TOL[np.float32]
+
+
+@pytest.mark.parametrize("mm", ["mkm", "kmm"])
+def test_saved_tensors_may_come_back_stored_another_way(mm):
+    import torch
+    import fastkron_amd as fk
+    fn = fk.MKM.apply if mm == "mkm" else fk.KMM.apply
+    x = rand(24, 7).t() if mm == "mkm" else rand(7, 24).t()                     # transposed views
+    fs = [rand(6, 6).t().requires_grad_(True), rand(4, 4).t().requires_grad_(True)]
+    gz = rand(*((7, 24) if mm == "mkm" else (24, 7)))
+    want = torch.autograd.grad(fn(x, *fs), fs, gz)
+    with torch.autograd.graph.saved_tensors_hooks(lambda t: t.cpu(), lambda t: t.cuda().contiguous()):
+        z = fn(x, *fs)
+    assert all(torch.equal(a, b) for a, b in zip(torch.autograd.grad(z, fs, gz), want))
