@@ -56,14 +56,17 @@ StepShape stepShape(const KronProblem& q, uint32_t g) {
   return q.mm == MMType::MKM ? StepShape{q.M, S} : StepShape{S, q.M};
 }
 
-// Estimated seconds of the forward and backward launches of one factor of P x Q on `rows` rows: bytes at 6 TB/s, the
+// Estimated seconds of the forward and backward launches of one factor of P x Q on `rows` rows: bytes at 6 TB/s; the
 // matrix instructions of both passes (4 + 8 per 16x16 block of the factor and 16 rows; 32 cycles each in fp32, about
-// 100 measured for the fp64 form) on 1024 SIMDs at 2.4 GHz, and 9 us for the launches.
+// 100 measured for the fp64 form) on 1024 SIMDs at 2.4 GHz; and what the launches take however few rows there are, 10 us
+// and the chain of one wave's tile (64x64: 5 us in fp32, 8 in fp64).  Measured, small chains of 8x8: 11 us per factor,
+// as pairs of 64x64 17 us in fp32 and 21 to 30 in fp64, and 14 us for forming the products and splitting their gradients.
 double stepCost(uint64_t rows, uint32_t P, uint32_t Q, DType dt) {
   const double bytes = (double)rows * (3.0 * P + 2.0 * Q) * (double)dtypeSize(dt);
-  const double blocks = (double)((P + 15) / 16) * (double)((Q + 15) / 16);
+  const uint32_t big = std::max(P, Q), zb = big <= 16 ? 1 : big <= 32 ? 2 : 4;      // the kernel's block of the factor
+  const double blocks = (double)((P + 16 * zb - 1) / (16 * zb)) * (double)((Q + 16 * zb - 1) / (16 * zb)) * zb * zb;
   const double cycles = (double)rows / 16.0 * blocks * 12.0 * (dt == DType::F32 ? 32.0 : 100.0);
-  return bytes / 6e12 + cycles / (1024.0 * 2.4e9) + 9e-6;
+  return bytes / 6e12 + cycles / (1024.0 * 2.4e9) + 10e-6 + (dt == DType::F32 ? 5e-6 : 8e-6) * zb * zb / 16.0;
 }
 
 // Groups of adjacent factors with the least estimated time; a group of several factors becomes one of at most 64x64.
@@ -86,8 +89,14 @@ void groupFactors(const KronProblem& p, GradPlan* gp) {
   }
   double plain = 0;
   for (uint32_t i = 0; i < N; i++) plain += stepCost((uint64_t)p.M * p.batch * (p.colsBefore(i) / p.P[i]), p.P[i], p.Q[i], p.dt);
-  // (merging costs two more small launches)
-  const bool merge = best[N] + 8e-6 < plain;
+  // Forming the products and splitting their gradients are two more launches, 14 us together.  A program that goes through
+  // autograd spends about 75 us of host time on the two passes and 3.6 us per launch besides, on which short launches
+  // wait: the longer of the two decides (dgekmm 8x8^5 x 16: plain, 11 launches, 70 us on the device, 130 us a pass;
+  // merged, 9 launches, 80 and 123 us).
+  uint32_t groups = 0;
+  for (uint32_t end = N; end > 0; end = from[end]) groups++;
+  auto pass = [](double device, uint32_t launches) { return std::max(device, 75e-6 + 3.6e-6 * launches); };
+  const bool merge = groups < N && pass(best[N] + 14e-6, 2 * groups + 3) < pass(plain, 2 * N + 1);
   uint32_t n = 0;
   for (uint32_t end = N; end > 0; n++) {
     const uint32_t lo = merge ? from[end] : end - 1;

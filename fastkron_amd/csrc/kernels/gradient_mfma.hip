@@ -14,7 +14,7 @@
 //        second time in this order, from the first-level cache.  The rows of F are permuted in fp64 so that a lane ends
 //        up with four consecutive p in either type: one 16-byte store (two in fp64) in the MKM layout.
 // A wave takes tiles of 16 u; dF stays in its accumulators over all of them, is summed over the four waves of the
-// workgroup in LDS and written as one partial sum per workgroup; kron_grad_reduce_kernel adds the partial sums in a
+// workgroup by a tree in LDS and written as one partial sum per workgroup; kron_grad_reduce_kernel adds the partial sums in a
 // fixed order (no atomics: repeated calls give the same bits).
 //
 // A workgroup handles at most 64x64 of the factor; larger factors run as one launch for dF, one 64x64 block of it per
@@ -81,11 +81,27 @@ void kron_grad_step_kernel(const GradStepArgs a) {
   const uint32_t pitch = a.fPitch;                         // LDS elements per row of F (0: F is read from memory)
 
   if (GA && pitch) {
-    // rows p0 .. p0 + 16*ZB of F, zero beyond P and Q
-    const uint32_t cols = nqb * 16;
-    for (uint32_t e = tid; e < 16 * ZB * cols; e += kGradThreads) {
-      const uint32_t pl = e / cols, q = e - pl * cols, p = p0 + pl;
-      fs[pl * pitch + q] = (p < P && q < Q) ? F[(int64_t)p * a.f_sp + (int64_t)q * a.f_sq] : (T)0;
+    // rows p0 .. p0 + 16*ZB of F, zero beyond P and Q; the loads of eight elements in flight (one at a time, 64x64 took
+    // 16 round trips to memory, more than the tile of a wave)
+    const uint32_t cols = DF ? 16 * ZB : nqb * 16, total = 16 * ZB * cols;
+    constexpr int LU = 8;
+    // along the contiguous dimension of F
+    const bool pFast = a.f_sp == 1;
+    for (uint32_t e0 = tid; e0 < total; e0 += LU * kGradThreads) {
+      T v[LU];
+#pragma unroll
+      for (int k = 0; k < LU; k++) {
+        const uint32_t e = e0 + k * kGradThreads;
+        const uint32_t pl = pFast ? e % (16 * ZB) : e / cols, q = pFast ? e / (16 * ZB) : e - e / cols * cols, p = p0 + pl;
+        v[k] = (T)0;
+        if (e < total && p < P && q < Q) v[k] = F[(int64_t)p * a.f_sp + (int64_t)q * a.f_sq];
+      }
+#pragma unroll
+      for (int k = 0; k < LU; k++) {
+        const uint32_t e = e0 + k * kGradThreads;
+        const uint32_t pl = pFast ? e % (16 * ZB) : e / cols, q = pFast ? e / (16 * ZB) : e - e / cols * cols;
+        if (e < total) fs[pl * pitch + q] = v[k];
+      }
     }
     __syncthreads();
   }
@@ -267,28 +283,53 @@ void kron_grad_step_kernel(const GradStepArgs a) {
   }
 
   if (DF) {
-    // the four waves' sums, one after the other, in one LDS copy of the block
+    // the four waves' sums as a tree in LDS: (0 + 2) + (1 + 3), a lane's values side by side for all lanes
     constexpr int N = 16 * ZB;
+    static_assert(kGradWaves == 4, "two levels");
+    auto slot = [&](int half, int i, int j, int r) { return fs + half * (N * N) + ((i * ZB + j) * 4 + r) * 64 + l; };
     __syncthreads();                                       // everyone is done with the factor in LDS
-#pragma unroll 1
-    for (int ww = 0; ww < kGradWaves; ww++) {
-      if (w == ww) {
+    if (w >= 2) {
 #pragma unroll
-        for (int i = 0; i < ZB; i++)
+      for (int i = 0; i < ZB; i++)
 #pragma unroll
-          for (int j = 0; j < ZB; j++)
+        for (int j = 0; j < ZB; j++)
 #pragma unroll
-            for (int r = 0; r < 4; r++) {
-              T* d = fs + (16 * i + MF::row(r, hi)) * N + 16 * j + lo;
-              *d = ww == 0 ? acc[i][j][r] : *d + acc[i][j][r];
-            }
-      }
-      __syncthreads();
+          for (int r = 0; r < 4; r++) *slot(w - 2, i, j, r) = acc[i][j][r];
     }
+    __syncthreads();
+    if (w < 2) {
+#pragma unroll
+      for (int i = 0; i < ZB; i++)
+#pragma unroll
+        for (int j = 0; j < ZB; j++)
+#pragma unroll
+          for (int r = 0; r < 4; r++) acc[i][j][r] += *slot(w, i, j, r);
+    }
+    __syncthreads();
+    if (w == 1) {
+#pragma unroll
+      for (int i = 0; i < ZB; i++)
+#pragma unroll
+        for (int j = 0; j < ZB; j++)
+#pragma unroll
+          for (int r = 0; r < 4; r++) *slot(0, i, j, r) = acc[i][j][r];
+    }
+    __syncthreads();
+    if (w == 0) {
+      // (the second half holds the block row by row for the store)
+#pragma unroll
+      for (int i = 0; i < ZB; i++)
+#pragma unroll
+        for (int j = 0; j < ZB; j++)
+#pragma unroll
+          for (int r = 0; r < 4; r++)
+            fs[N * N + (16 * i + MF::row(r, hi)) * N + 16 * j + lo] = acc[i][j][r] + *slot(0, i, j, r);
+    }
+    __syncthreads();
     T* part = (T*)a.partial + ((size_t)bt * a.partStride + a.partFirst + blockIdx.x) * ((size_t)P * Q);
     for (uint32_t e = tid; e < N * N; e += kGradThreads) {
       const uint32_t p = p0 + e / N, q = q0 + e % N;
-      if (p < P && q < Q) part[(size_t)p * Q + q] = fs[e];
+      if (p < P && q < Q) part[(size_t)p * Q + q] = fs[N * N + e];
     }
   }
 }
@@ -328,13 +369,15 @@ __global__ __launch_bounds__(256) void kron_grad_reduce_kernel(const GradReduceA
   }
 }
 
-// One workgroup per source of a merged factor: thread = (entry of the source, share of the other digits).
+// One workgroup per source of a merged factor: thread = (entry of the source, share of the other digits).  Bound by the
+// chain of loads of a share's terms, hence as many shares as a workgroup has threads for.
+constexpr uint32_t kUnmergeThreads = 1024;
 template <typename T>
-__global__ __launch_bounds__(256) void kron_grad_unmerge_kernel(const GradUnmergeArgs a) {
+__global__ __launch_bounds__(kUnmergeThreads) void kron_grad_unmerge_kernel(const GradUnmergeArgs a) {
   const MergeGroup& g = a.g[blockIdx.x];
   const uint32_t j = blockIdx.y, b = blockIdx.z;
   if (j >= g.count || !a.out[blockIdx.x][j]) return;
-  __shared__ T s[256];
+  __shared__ T s[kUnmergeThreads];
   uint32_t P = 1, Q = 1, sufP = 1, sufQ = 1;               // digits behind source j are the fast ones
   for (uint32_t i = 0; i < g.count; i++) {
     P *= g.p[i]; Q *= g.q[i];
@@ -343,9 +386,9 @@ __global__ __launch_bounds__(256) void kron_grad_unmerge_kernel(const GradUnmerg
   const uint32_t pj = g.p[j], qj = g.q[j], n = pj * qj, restP = P / pj, restQ = Q / qj;
   const T* dG = (const T*)g.dst + (size_t)b * P * Q;
   T* out = (T*)a.out[blockIdx.x][j] + (size_t)b * n;
-  uint32_t shares = 256 / n;
+  uint32_t shares = kUnmergeThreads / n;
   if (shares == 0) shares = 1;
-  const uint32_t step = 256 / shares;                       // entries per round
+  const uint32_t step = kUnmergeThreads / shares;                       // entries per round
   const uint32_t share = threadIdx.x / step, en = threadIdx.x % step;
   for (uint32_t e0 = 0; e0 < n; e0 += step) {
     const uint32_t e = e0 + en;
@@ -413,7 +456,7 @@ static hipError_t launchGradStepT(GradStepArgs a, hipStream_t stream) {
   const int zb = big <= 16 ? 1 : big <= 32 ? 2 : 4;
   const uint32_t pChunks = (a.P + 16 * zb - 1) / (16 * zb), qBlocks = (a.Q + 15) / 16;
   a.qChunks = (a.Q + 16 * zb - 1) / (16 * zb);
-  const size_t red = (size_t)256 * zb * zb * sizeof(T);
+  const size_t red = (size_t)2 * 256 * zb * zb * sizeof(T);           // two halves of the tree
   auto run = [&](auto df, auto ga, uint32_t gridX, uint32_t gridZ) -> hipError_t {
     constexpr bool D = decltype(df)::value, G = decltype(ga)::value;
     const uint32_t cols = D ? 16 * zb : 16 * qBlocks;
@@ -461,8 +504,8 @@ hipError_t launchGradReduce(const GradReduceArgs& a, uint32_t batch, DType dt, h
 hipError_t launchGradUnmerge(const GradUnmergeArgs& a, uint32_t batch, DType dt, hipStream_t stream) {
   if (a.groups == 0) return hipSuccess;
   const dim3 grid(a.groups, kMaxMergeSources, batch);
-  if (dt == DType::F32) hipLaunchKernelGGL(kron_grad_unmerge_kernel<float>, grid, dim3(256), 0, stream, a);
-  else                  hipLaunchKernelGGL(kron_grad_unmerge_kernel<double>, grid, dim3(256), 0, stream, a);
+  if (dt == DType::F32) hipLaunchKernelGGL(kron_grad_unmerge_kernel<float>, grid, dim3(kUnmergeThreads), 0, stream, a);
+  else                  hipLaunchKernelGGL(kron_grad_unmerge_kernel<double>, grid, dim3(kUnmergeThreads), 0, stream, a);
   return hipGetLastError();
 }
 

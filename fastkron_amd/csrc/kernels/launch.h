@@ -166,7 +166,7 @@ bool smallInplaceFits(uint32_t nf, const uint32_t* p, const uint32_t* q, uint64_
 bool smallInplaceSupported(const StepArgs& a, DType dt);
 hipError_t launchSmallInplace(const StepArgs& a, DType dt, hipStream_t stream);
 
-// Kronecker products of adjacent small factors into the handle's workspace, one workgroup per product.
+// Kronecker products of adjacent small factors into the handle's workspace, 256 entries per workgroup.
 hipError_t launchMergeFactors(const MergeArgs& a, DType dt, hipStream_t stream);
 // Transposed copy: in is R x C row-major per batch entry, out is C x R.
 hipError_t launchTranspose(const void* in, void* out, uint32_t R, uint32_t C, uint32_t batch, uint64_t inBatch,
