@@ -52,7 +52,7 @@ constexpr int kK2Win = 3;              // k0 slices of a tile in flight
 // one; the two columns go through the matrix cores as two column blocks.
 template <typename T, bool HAS_Y, bool EXACT, int JW>
 __global__ __launch_bounds__(256, 2) void kron_kmm16x2_kernel(const StepArgs a, const uint32_t mTiles,
-                                                              const uint32_t totalTiles) {
+                                                              const uint32_t totalTiles, const uint32_t qSplit) {
   using MF = K2Mfma<T>;
   using Acc = typename MF::Acc;
   typedef T V2 __attribute__((ext_vector_type(2)));
@@ -91,7 +91,9 @@ __global__ __launch_bounds__(256, 2) void kron_kmm16x2_kernel(const StepArgs a, 
   const T* YB = HAS_Y ? (const T*)a.y + (size_t)bt * a.y_batch : nullptr;
   const T alpha = a.epilogue ? (T)a.alpha : (T)1, beta = (T)a.beta;
 
-  const uint32_t nWaves = gridDim.x * kK2Waves;
+  // qSplit neighbouring waves share a tile: each computes its T, and its share of the output rows q0
+  const uint32_t nWaves = gridDim.x * kK2Waves / qSplit, waveId = (blockIdx.x * kK2Waves + w) / qSplit;
+  const int share = (int)(w % qSplit), q0First = share * P / (int)qSplit, q0End = (share + 1) * P / (int)qSplit;
   // x[c] = X[(s, k0, k1 = 4*c + hi), m]; columns beyond M are clamped to the tile's first one (computed, not stored)
   // The rows are read in the order (k0, c): row k0*P + 4*c + hi, four rows further with every load and P - 16
   // back at the end of a slice, so one running pointer serves the whole tile.  Rows 4*c + hi >= P are not read.
@@ -121,7 +123,7 @@ __global__ __launch_bounds__(256, 2) void kron_kmm16x2_kernel(const StepArgs a, 
   // (the window's registers are free from the last matrix product on): a tile that requested them at its own start
   // sat out a memory round trip, behind the stores of the tile before, with nothing else in flight.
   T xw[kK2Win][JW][4];
-  uint32_t t = blockIdx.x * kK2Waves + w;
+  uint32_t t = waveId;
   if (t >= totalTiles) return;
   const T* xp = tileRows(t);
 #pragma unroll
@@ -162,10 +164,10 @@ __global__ __launch_bounds__(256, 2) void kron_kmm16x2_kernel(const StepArgs a, 
     // output row (q0, q1 = row(r, hi)): a running pointer per lane, 16 rows further with every q0
     const uint64_t oq = S * (uint64_t)a.out_ldc, yq = HAS_Y ? S * (uint64_t)a.y_ldc : 0;   // stride of one output row q
     const uint64_t rs = (uint64_t)(MF::row(1, 0) - MF::row(0, 0));                        // rows between two registers
-    T* op = outB + m + s * (uint64_t)a.out_ldc + (uint64_t)MF::row(0, hi) * oq;
-    const T* yp = HAS_Y ? YB + m + s * (uint64_t)a.y_ldc + (uint64_t)MF::row(0, hi) * yq : nullptr;
+    T* op = outB + m + s * (uint64_t)a.out_ldc + ((uint64_t)MF::row(0, hi) + (uint64_t)(q0First * P)) * oq;
+    const T* yp = HAS_Y ? YB + m + s * (uint64_t)a.y_ldc + ((uint64_t)MF::row(0, hi) + (uint64_t)(q0First * P)) * yq : nullptr;
 #pragma unroll 1
-    for (int q0 = 0; q0 < P; q0++) {
+    for (int q0 = q0First; q0 < q0End; q0++) {
       T yv[JW][4];
       if (HAS_Y) {
 #pragma unroll
@@ -247,14 +249,19 @@ static hipError_t launchKmm16x2T(const StepArgs& a, hipStream_t stream) {
   // persistent waves: two workgroups of four waves per CU (two waves per SIMD)
   uint32_t wgs = (uint32_t)cus * 2;
   if (a.batch > 1) wgs = (wgs + a.batch - 1) / a.batch;
-  const uint32_t need = (totalTiles + kK2Waves - 1) / kK2Waves;
+  // Few tiles: two or four waves per tile while every SIMD has at most one wave.  A tile is a chain of 16 k0 products and
+  // 16 rows q0 on the vector ALU, about half of the wave's time each, whatever the number of tiles (1000 x 16^2 fp64
+  // 9.3 -> 6.8 us, 20 x 14^2 fp64 10.4 -> 8.0, 2 x 12^4 fp64 in two launches 21.1 -> 15.4).
+  uint32_t qSplit = 1;
+  while (qSplit < 4 && (uint64_t)totalTiles * a.batch * qSplit * 2 <= 4ull * cus) qSplit *= 2;
+  const uint32_t need = (totalTiles * qSplit + kK2Waves - 1) / kK2Waves;
   if (wgs > need) wgs = need;
   if (wgs == 0) wgs = 1;
   dim3 grid(wgs, a.batch), block(256);
   if (a.y && a.epilogue)
-    hipLaunchKernelGGL((kron_kmm16x2_kernel<T, true, EXACT, JW>), grid, block, 0, stream, a, mTiles, totalTiles);
+    hipLaunchKernelGGL((kron_kmm16x2_kernel<T, true, EXACT, JW>), grid, block, 0, stream, a, mTiles, totalTiles, qSplit);
   else
-    hipLaunchKernelGGL((kron_kmm16x2_kernel<T, false, EXACT, JW>), grid, block, 0, stream, a, mTiles, totalTiles);
+    hipLaunchKernelGGL((kron_kmm16x2_kernel<T, false, EXACT, JW>), grid, block, 0, stream, a, mTiles, totalTiles, qSplit);
   return hipGetLastError();
 }
 
