@@ -61,6 +61,7 @@ struct StepAnyGeom {
   uint32_t qbSlab, nSlabs;             // 16-column blocks per slab of output columns, slabs per factor
   uint32_t vecLoad;                    // elements per vector load of the input (0: element by element)
   uint32_t nJ, jBlocks, totalTiles;
+  uint32_t magicPerK, magicQp;         // floor(x / d) = mulhi(x, magic) for x * d < 2^32: elements per lane group, per row of the slab
   int64_t inLine, inJ, inP, outLine, outJ, outQ, yLine, yJ, yQ;
 };
 
@@ -87,30 +88,36 @@ __global__ __launch_bounds__(kSaThreads, 2) void kron_step_any_kernel(const Step
   const T alpha = a.epilogue ? (T)a.alpha : (T)1, beta = (T)a.beta;
 
   // the zero-padded slab of the factor: fl[k*kStride + c*Qp + q] = F[k*pc + c][16*ib0 + q]
-  {
+  auto stageFactor = [&]() {
     const T* F = (const T*)a.f[0] + (size_t)bt * a.f_batch[0];
     const uint32_t perK = g.pcPad * Qp;                // rows pc .. pcPad-1 of a lane group are zero
     // eight loads of a thread go out before the first LDS write waits for one: a loop of load, wait, write would
-    // put one memory round trip per element of a thread in front of the first product
+    // put one memory round trip per element of a thread in front of the first product.  Divisions by multiplication, and the
+    // first tile's loads ahead: on short launches the indexes and the tile's round trip cost as much as the products (two
+    // steps each: 1003 x 31x63^2 fp32 23.1 -> 20.6 us, 100 rows 15.0 -> 12.4, dgekmm 20^2 x 50 13.0 -> 10.5; 3000 x 24x48^2
+    // 31.2 -> 27.5).
     constexpr int kBatch = 8;
-    for (uint32_t base = tid; base < 4 * perK; base += kBatch * kSaThreads) {
+    for (uint32_t base = 0; base < 4 * perK; base += kBatch * kSaThreads) {
       T v[kBatch];
       uint32_t dst[kBatch];
 #pragma unroll
       for (int u = 0; u < kBatch; u++) {
-        const uint32_t idx = base + u * kSaThreads;
-        const uint32_t k = idx / perK, rem = idx - k * perK, c = rem / Qp, q = rem - c * Qp;
+        if (base + u * kSaThreads >= 4 * perK) break;
+        const uint32_t idx = base + u * kSaThreads + tid;
+        const uint32_t k = __umulhi(idx, g.magicPerK), rem = idx - k * perK, c = __umulhi(rem, g.magicQp), q = rem - c * Qp;
         const uint32_t p = k * pc + c, qq = 16 * ib0 + q;
         v[u] = (T)0;
         if (idx < 4 * perK && c < pc && p < g.P && qq < g.Q) v[u] = F[(int64_t)p * a.f_sp[0] + (int64_t)qq * a.f_sq[0]];
         dst[u] = k * g.kStride + c * Qp + q;
       }
 #pragma unroll
-      for (int u = 0; u < kBatch; u++)
-        if (base + u * kSaThreads < 4 * perK) fl[dst[u]] = v[u];
+      for (int u = 0; u < kBatch; u++) {
+        if (base + u * kSaThreads >= 4 * perK) break;
+        if (base + u * kSaThreads + tid < 4 * perK) fl[dst[u]] = v[u];
+      }
     }
-  }
-  __syncthreads();
+    __syncthreads();
+  };
 
   const uint32_t nWaves = gridDim.x * kSaWaves;
   const uint32_t wave = blockIdx.x * kSaWaves + w;
@@ -208,8 +215,9 @@ __global__ __launch_bounds__(kSaThreads, 2) void kron_step_any_kernel(const Step
         }
       }
     };
+    if (wave < g.totalTiles) loadTile(wave, xn);           // (in flight while the factor is staged)
+    stageFactor();
     if (wave >= g.totalTiles) return;
-    loadTile(wave, xn);
     computeTile(wave);
     for (uint32_t t = wave + nWaves; t < g.totalTiles; t += nWaves) computeTile(t);
     return;
@@ -217,6 +225,7 @@ __global__ __launch_bounds__(kSaThreads, 2) void kron_step_any_kernel(const Step
 
   T xn[PREFETCH ? PCMAX : 1];
   if (PREFETCH && wave < g.totalTiles) loadTile(wave, (T(&)[PCMAX])xn);
+  stageFactor();
   for (uint32_t t = wave; t < g.totalTiles; t += nWaves) {
     T x[PCMAX];
     if (PREFETCH) {
@@ -281,6 +290,9 @@ static bool stepAnyGeometry(const StepArgs& a, DType dt, StepAnyGeom* g) {
   if (slab > g->qb) slab = g->qb;
   g->qbSlab = slab; g->nSlabs = (g->qb + slab - 1) / slab;
   g->kStride = g->pcPad * slab * 16 + 16;
+  // (at most 4 * pcPad * 16 * slab elements, 64 KB of them or one 16-column block of 256 rows: products below 2^28)
+  g->magicPerK = (uint32_t)((1ull << 32) / (g->pcPad * slab * 16)) + 1;
+  g->magicQp = (uint32_t)((1ull << 32) / (slab * 16)) + 1;
   uint64_t nLines;
   if (saOutRowsContiguous(a)) {        // KMM: lanes along the rows of one slice
     nLines = S; g->nJ = a.M;
