@@ -733,7 +733,7 @@ fastKronError Handle::trySplitLeadingTrailing(const KronProblem& p, void* temp1,
   if (!temp1 || !temp2 || p.N < 3) return fastKronKernelNotFound;
   // trailing run of identical square factors that one whole-row kernel fuses:
   // fp32 8x8 (five), 16x16 (four), 32x32 (three), 64x64 (two); fp64 16x16 (three), 32x32 or 64x64 (two);
-  // 9x9 ... 15x15 (three, either type)
+  // 9x9 ... 15x15 (three, either type); 3x3, 5x5, 6x6, 7x7 (eight, six, five, five, either type)
   const uint32_t tp = p.P[p.N - 1], tq = p.Q[p.N - 1];
   if (tq != tp) {
     // two trailing rectangular factors of a shape the pair kernel has exact tiles for (32x64, 64x32)
@@ -759,10 +759,26 @@ fastKronError Handle::trySplitLeadingTrailing(const KronProblem& p, void* temp1,
   if (p.dt == DType::F32 && tp == 16 && p.N >= 4 && (uint64_t)p.M * (p.K() / 65536) * p.batch < 96) maxT = 3;
   if (maxT == 0 && tp >= 9 && tp <= 15) maxT = 3;       // zero-padded form of the 16x16x3 wave-per-block kernel
   if (maxT == 0 && tp >= 17 && tp <= 31) maxT = 2;      // zero-padded form of the 32x32 pair kernel
+  bool inplace = false;
+  if (maxT == 0 && (tp == 3 || tp == 5 || tp == 6 || tp == 7)) {
+    // rows longer than the in-place kernel's LDS: as many trailing factors as it holds (3^8, 5^6, 6^5, 7^5), which are blocks
+    // of 6561 columns and more for the leading ones
+    inplace = true;
+    for (uint64_t bytes = dtypeSize(p.dt) * tp; bytes + 16 <= 160 * 1024 && maxT < kMaxFused; bytes *= tp) maxT++;
+  }
   if (maxT == 0) return fastKronKernelNotFound;
   uint32_t nT = 0;
   while (nT < maxT && nT < p.N && p.P[p.N - 1 - nT] == tp && p.Q[p.N - 1 - nT] == tp) nT++;
   if (nT < 2 || nT == p.N) return fastKronKernelNotFound;         // a chain of nT factors alone is a whole-row problem
+  // (sgemkm 1000 x 5^7 527 -> 342 us, 1 x 5^7 26 -> 14, 1000 x 3^9 128 -> 76, 1000 x 6^6 313 -> 177, 200 x 7^6 183 -> 120,
+  // dgemkm 100 x 7^6 185 -> 126, all against groups of the kernel with two LDS buffers.  Three and more leading factors lose,
+  // 50 x 3^11 87 -> 125, and few long fp64 blocks in passes of one digit gain nothing, 2 x 6^6 19.0 -> 19.6.)
+  if (inplace && (nT != maxT || p.N - nT > 2)) return fastKronKernelNotFound;
+  if (inplace && p.dt == DType::F64 && tp >= 6) {
+    uint64_t blocks = (uint64_t)p.M * p.batch;
+    for (uint32_t i = 0; i < p.N - nT; i++) blocks *= p.P[i];
+    if (blocks < 96) return fastKronKernelNotFound;
+  }
   if (p.dt == DType::F64 && tp == 8 && nT != 5) return fastKronKernelNotFound;   // (that kernel takes exactly five)
   const uint32_t g = p.N - nT;
   KronProblem q1, q2;

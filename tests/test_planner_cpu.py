@@ -459,6 +459,17 @@ def test_whole_rows_of_small_square_factors_run_in_place(online_planner):
     assert not inplace("mkm", "d", 95, [7] * 5) and inplace("mkm", "d", 96, [7] * 5) and inplace("mkm", "s", 1, [7] * 5)
     assert not inplace("mkm", "d", 1000, mixed)                       # 315 KB
 
+    # longer rows: blocks of as many trailing factors as the kernel holds, at most two factors across the blocks
+    def blocks(dt, M, Ps, **kw):
+        e, names, launches = plan(online_planner, "mkm", dt, M, Ps, Ps, **kw)
+        assert e == capi.SUCCESS
+        return int(launches[0]["M"]) if "inplace" in names[0] and int(launches[0]["lo"]) == 0 and len(names) > 1 else None
+    assert blocks("s", 3, [5] * 7) == 15 and blocks("d", 3, [5] * 8) == 75 and blocks("s", 2, [6] * 6) == 12
+    assert blocks("s", 1, [7] * 6) == 7 and blocks("s", 2, [9, 2] + [3] * 8) == 36 and blocks("s", 9, [5] * 7, beta=0.5, y_is_z=True) == 45
+    assert blocks("s", 3, [3] * 11) is None and blocks("s", 3, [64] + [5] * 3) is None      # three leading ones; short blocks
+    assert blocks("d", 15, [6] * 6) is None and blocks("d", 16, [6] * 6) == 96
+    assert blocks("s", 3, [5] * 7, batch=2) is None and blocks("s", 3, [5] * 7, batch=2, strideF=[0] * 7) == 15
+
 
 def test_padded_step_rules_for_rectangular_and_large_odd_factors(online_planner):
     planner = online_planner

@@ -43,6 +43,22 @@ def test_small_factors_in_place(fk, M, Ps, dt):
         assert e == 0 and normwise(got, want) <= TOL[dt], (fk.last_plan(), kw)
 
 
+@pytest.mark.parametrize("dt", [np.float32, np.float64], ids=["f", "d"])
+@pytest.mark.parametrize("M,Ps", [(3, [5] * 7), (1, [3] * 9), (2, [6] * 6), (2, [7] * 6), (5, [4, 2] + [5] * 6), (100, [2] + [7] * 5)],
+                         ids=lambda v: str(v) if isinstance(v, int) else "x".join(map(str, v)))
+def test_rows_beyond_the_lds_run_their_trailing_factors_in_place(fk, M, Ps, dt):
+    """A two-part plan: blocks of 3^8, 5^6, 6^5 or 7^5 columns in place, the leading factors across the blocks."""
+    few_long_rows = dt is np.float64 and Ps[-1] >= 6 and M < 20       # (fewer than 96 blocks in passes of one digit)
+    for seed, kw in enumerate([dict(alpha=1.5, beta=0.5), dict(alpha=1.0, beta=0.0, opFs=ko.OP_T, batch=2, share_f=True)]):
+        alpha, beta = kw.pop("alpha"), kw.pop("beta")
+        batch, share = kw.get("batch", 1), dict(share_f=True) if kw.get("share_f") else {}
+        X, Fs, Y = make_case(ko.MKM, M, Ps, Ps, dt, seed=5 + 50 * seed, with_y=beta != 0.0, batch=batch, **share)
+        want = oracle_answer(ko.MKM, M, Ps, Ps, X, Fs, Y, alpha, beta, **kw)
+        got, e = run_gpu(fk, ko.MKM, M, Ps, Ps, X, Fs, Y, alpha, beta, **kw)
+        assert e == 0 and normwise(got, want) <= TOL[dt], (fk.last_plan(), kw)
+        assert few_long_rows or "inplace" in fk.last_plan()[0][2], fk.last_plan()
+
+
 def test_rows_off_a_16_byte_boundary(fk):
     """Base addresses that are only 4-byte aligned, of X and of Z, and the in-place epilogue (Y is Z)."""
     import torch
