@@ -2,9 +2,9 @@
 // steps in the opposite order, one launch per step for the gradients of the step's input and of its factor
 // (kernels/gradient_mfma.hip), one launch that adds the partial sums of all factors.
 //
-// Adjacent small factors are replaced by their Kronecker product first (exact algebra), so that a chain of n small
-// factors takes fewer passes over the data; the gradients of the product's sources follow from its own gradient
-// (one small launch for all of them).
+// Every factor keeps a step of its own: merged to products of up to 64x64, chains of small factors took fewer launches
+// (dgekmm 8x8^5 x 16 nine instead of eleven, 125 against 130 us), but Z and the gradient of X came out with twice the
+// rounding error (8x8^4 in fp32 2.0e-7 against 1.1e-7).
 // The reference chains PyTorch matmuls through the intermediates of its forward family, one factor at a time
 // (reference pyfastkron/fastkrontorch.py:160-217).
 #include "handle.h"
@@ -26,16 +26,15 @@ size_t roundUp(size_t v) { return (v + 63) & ~(size_t)63; }       // elements: 2
 
 // The chain as the two passes run it.
 struct GradPlan {
-  KronProblem q;                    // merged chain, MKM or KMM, op(X) = N; F, X, Z, inter not set
-  uint32_t lo[kMaxFactors], hi[kMaxFactors];      // sources of factor g of q
-  bool pMajor;                      // storage of the sources: element (p, q) at p*Q + q
+  KronProblem q;                    // MKM or KMM, op(X) = N; F, X, Z, inter not set
+  bool pMajor;                      // storage of the factors: element (p, q) at p*Q + q
   bool outTransposed;               // gradients of the factors are Q x P (KMM)
   bool copyX;                       // op(X) = T: X is copied transposed
   uint32_t xBatch;                  // entries of that copy
   // offsets into `save`, in elements
-  size_t saveX, saveF[kMaxFactors], saveI[kMaxFactors], saveTotal;
+  size_t saveX, saveI[kMaxFactors], saveTotal;
   // offsets into `work`
-  size_t workG[2], workP[kMaxFactors], workD[kMaxFactors], workTotal;
+  size_t workG[2], workP[kMaxFactors], workTotal;
   uint32_t parts[kMaxFactors];      // partial sums of factor g per batch entry
 };
 
@@ -54,63 +53,6 @@ struct StepShape { uint64_t O, Tn; };               // rows u = o*Tn + t
 StepShape stepShape(const KronProblem& q, uint32_t g) {
   const uint64_t S = q.colsBefore(g) / q.P[g];
   return q.mm == MMType::MKM ? StepShape{q.M, S} : StepShape{S, q.M};
-}
-
-// Estimated seconds of the forward and backward launches of one factor of P x Q on `rows` rows: bytes at 6 TB/s; the
-// matrix instructions of both passes (4 + 8 per 16x16 block of the factor and 16 rows; 32 cycles each in fp32, about
-// 100 measured for the fp64 form) on 1024 SIMDs at 2.4 GHz; and what the launches take however few rows there are, 10 us
-// and the chain of one wave's tile (64x64: 5 us in fp32, 8 in fp64).  Measured, small chains of 8x8: 11 us per factor,
-// as pairs of 64x64 17 us in fp32 and 21 to 30 in fp64, and 14 us for forming the products and splitting their gradients.
-double stepCost(uint64_t rows, uint32_t P, uint32_t Q, DType dt) {
-  const double bytes = (double)rows * (3.0 * P + 2.0 * Q) * (double)dtypeSize(dt);
-  const uint32_t big = std::max(P, Q), zb = big <= 16 ? 1 : big <= 32 ? 2 : 4;      // the kernel's block of the factor
-  const double blocks = (double)((P + 16 * zb - 1) / (16 * zb)) * (double)((Q + 16 * zb - 1) / (16 * zb)) * zb * zb;
-  const double cycles = (double)rows / 16.0 * blocks * 12.0 * (dt == DType::F32 ? 32.0 : 100.0);
-  return bytes / 6e12 + cycles / (1024.0 * 2.4e9) + 10e-6 + (dt == DType::F32 ? 5e-6 : 8e-6) * zb * zb / 16.0;
-}
-
-// Groups of adjacent factors with the least estimated time; a group of several factors becomes one of at most 64x64.
-void groupFactors(const KronProblem& p, GradPlan* gp) {
-  const uint32_t N = p.N;
-  double best[kMaxFactors + 1];
-  uint32_t from[kMaxFactors + 1];
-  best[0] = 0;
-  for (uint32_t end = 1; end <= N; end++) {
-    best[end] = 1e300;
-    uint64_t P = 1, Q = 1;
-    const uint64_t cols = p.colsBefore(end - 1);
-    for (uint32_t lo = end; lo-- > 0;) {
-      P *= p.P[lo]; Q *= p.Q[lo];
-      const uint32_t n = end - lo;
-      if (n > 1 && (P > 64 || Q > 64 || n > kMaxMergeSources)) break;
-      const double c = best[lo] + stepCost((uint64_t)p.M * p.batch * (cols / P), (uint32_t)P, (uint32_t)Q, p.dt);
-      if (c < best[end]) { best[end] = c; from[end] = lo; }
-    }
-  }
-  double plain = 0;
-  for (uint32_t i = 0; i < N; i++) plain += stepCost((uint64_t)p.M * p.batch * (p.colsBefore(i) / p.P[i]), p.P[i], p.Q[i], p.dt);
-  // Forming the products and splitting their gradients are two more launches, 14 us together.  A program that goes through
-  // autograd spends about 75 us of host time on the two passes and 3.6 us per launch besides, on which short launches
-  // wait: the longer of the two decides (dgekmm 8x8^5 x 16: plain, 11 launches, 70 us on the device, 130 us a pass;
-  // merged, 9 launches, 80 and 123 us).
-  uint32_t groups = 0;
-  for (uint32_t end = N; end > 0; end = from[end]) groups++;
-  auto pass = [](double device, uint32_t launches) { return std::max(device, 75e-6 + 3.6e-6 * launches); };
-  const bool merge = groups < N && pass(best[N] + 14e-6, 2 * groups + 3) < pass(plain, 2 * N + 1);
-  uint32_t n = 0;
-  for (uint32_t end = N; end > 0; n++) {
-    const uint32_t lo = merge ? from[end] : end - 1;
-    gp->lo[n] = lo; gp->hi[n] = end - 1;
-    end = lo;
-  }
-  std::reverse(gp->lo, gp->lo + n);
-  std::reverse(gp->hi, gp->hi + n);
-  KronProblem& q = gp->q;
-  q.N = n;
-  for (uint32_t g = 0; g < n; g++) {
-    q.P[g] = q.Q[g] = 1;
-    for (uint32_t i = gp->lo[g]; i <= gp->hi[g]; i++) { q.P[g] *= p.P[i]; q.Q[g] *= p.Q[i]; }
-  }
 }
 
 fastKronError makePlan(const Handle::GradProblem& p, GradPlan* gp) {
@@ -138,14 +80,10 @@ fastKronError makePlan(const Handle::GradProblem& p, GradPlan* gp) {
       (uint64_t)q.M * q.batch < (1ull << 32)) {
     q.M *= q.batch; q.batch = 1;
   }
-  const KronProblem single = q;
-  groupFactors(single, gp);
   const size_t nb = q.batch;
   size_t off = 0;
   auto take = [&](size_t elems) { const size_t o = off; off += roundUp(elems); return o; };
   gp->saveX = gp->copyX ? take((size_t)gp->xBatch * p.M * K) : 0;
-  for (uint32_t g = 0; g < q.N; g++)
-    gp->saveF[g] = gp->lo[g] < gp->hi[g] ? take((p.perBatchF ? nb : 1) * (size_t)q.P[g] * q.Q[g]) : 0;
   for (uint32_t g = 1; g < q.N; g++) gp->saveI[g] = take(nb * q.M * q.colsAfter(g));      // output of step g
   gp->saveTotal = off;
   off = 0;
@@ -158,21 +96,9 @@ fastKronError makePlan(const Handle::GradProblem& p, GradPlan* gp) {
     forRowChunks(s.O, s.Tn, [&](uint64_t, uint64_t on, uint64_t, uint64_t tn) { parts += gradWorkgroups(q.P[g], q.Q[g], on * tn, q.batch); });
     gp->parts[g] = parts;
     gp->workP[g] = take(nb * parts * q.P[g] * q.Q[g]);
-    gp->workD[g] = gp->lo[g] < gp->hi[g] ? take((p.perBatchF ? nb : 1) * (size_t)q.P[g] * q.Q[g]) : 0;
   }
   gp->workTotal = off;
   return fastKronSuccess;
-}
-
-// Sources of merged factor g, as the merging kernel reads them.
-void mergeGroupOf(const Handle::GradProblem& p, const GradPlan& gp, uint32_t g, MergeGroup* mg) {
-  mg->count = gp.hi[g] - gp.lo[g] + 1;
-  for (uint32_t j = 0; j < mg->count; j++) {
-    const uint32_t fi = gp.lo[g] + j;
-    mg->src[j] = p.F[fi]; mg->p[j] = p.P[fi]; mg->q[j] = p.Q[fi];
-    mg->sp[j] = gp.pMajor ? (int64_t)p.Q[fi] : 1;
-    mg->sq[j] = gp.pMajor ? 1 : (int64_t)p.P[fi];
-  }
 }
 
 }  // namespace
@@ -209,23 +135,10 @@ fastKronError Handle::gradForward(const GradProblem& p, void* Z, void* save) {
     q.X = xt; q.strideX = q.batch > 1 && gp.xBatch > 1 ? (uint64_t)p.M * t.K() : 0;
     q.xJustWritten = true;
   }
-  MergeArgs ma{};
-  ma.batch = p.perBatchF ? q.batch : 1;
-  auto flush = [&]() { const hipError_t he = ma.groups ? launchMergeFactors(ma, p.dt, stream_) : hipSuccess; ma.groups = 0; return he; };
   for (uint32_t g = 0; g < q.N; g++) {
-    const size_t pq = (size_t)q.P[g] * q.Q[g];
-    q.strideF[g] = p.perBatchF && q.batch > 1 ? pq : 0;
-    q.F[g] = p.F[gp.lo[g]];
-    if (gp.lo[g] == gp.hi[g]) continue;
-    MergeGroup& mg = ma.g[ma.groups++];
-    mergeGroupOf(p, gp, g, &mg);
-    mg.dst = sv + gp.saveF[g] * es;
-    mg.dsp = gp.pMajor ? (int64_t)q.Q[g] : 1;
-    mg.dsq = gp.pMajor ? 1 : (int64_t)q.P[g];
-    q.F[g] = mg.dst;
-    if (ma.groups == kMaxMergeGroups && flush() != hipSuccess) return fastKronInvalidArgument;
+    q.strideF[g] = p.perBatchF && q.batch > 1 ? (uint64_t)q.P[g] * q.Q[g] : 0;
+    q.F[g] = p.F[g];
   }
-  if (flush() != hipSuccess) return fastKronInvalidArgument;
   q.forward = true; q.strided = q.batch > 1; q.haveStrideInter = true;
   for (uint32_t g = 1; g < q.N; g++) {
     q.inter[g - 1] = sv + gp.saveI[g] * es;
@@ -256,8 +169,7 @@ fastKronError Handle::gradBackward(const GradProblem& p, const void* gZ, void* s
   int lastWanted = -1;
   bool wanted[kMaxFactors];
   for (uint32_t g = 0; g < q.N; g++) {
-    wanted[g] = false;
-    for (uint32_t i = gp.lo[g]; i <= gp.hi[g]; i++) wanted[g] = wanted[g] || gF[i];
+    wanted[g] = gF[g] != nullptr;
     if (wanted[g]) lastWanted = (int)g;
   }
   if (gX) lastWanted = (int)q.N - 1;
@@ -269,8 +181,7 @@ fastKronError Handle::gradBackward(const GradProblem& p, const void* gZ, void* s
     const bool lastStep = i + 1 == (int)q.N;
     GradStepArgs a{};
     a.P = q.P[i]; a.Q = q.Q[i];
-    const bool merged = gp.lo[i] < gp.hi[i];
-    const char* F = merged ? sv + gp.saveF[i] * es : (const char*)p.F[gp.lo[i]];
+    const char* F = (const char*)p.F[i];
     a.f_sp = gp.pMajor ? (int64_t)a.Q : 1;
     a.f_sq = gp.pMajor ? 1 : (int64_t)a.P;
     a.f_batch = p.perBatchF && q.batch > 1 ? (uint64_t)a.P * a.Q : 0;
@@ -332,10 +243,8 @@ fastKronError Handle::gradBackward(const GradProblem& p, const void* gZ, void* s
     g = gin; gBatch = ginBatch;
   }
 
-  // sum the partial sums of all factors, then split the gradients of merged factors
+  // sum the partial sums of all factors
   GradReduceArgs ra{};
-  GradUnmergeArgs ua{};
-  ua.perBatch = p.perBatchF; ua.outTransposed = gp.outTransposed;
   const uint32_t fBatch = p.perBatchF ? q.batch : 1;
   auto reduceNow = [&]() -> hipError_t {
     for (uint32_t b0 = 0; b0 < fBatch && ra.count; b0 += kMaxGridBatch) {
@@ -357,41 +266,11 @@ fastKronError Handle::gradBackward(const GradProblem& p, const void* gZ, void* s
     r.P = q.P[i]; r.Q = q.Q[i];
     r.count = gp.parts[i] * (p.perBatchF ? 1 : q.batch);
     r.partial = wk + gp.workP[i] * es;
-    const bool merged = gp.lo[i] < gp.hi[i];
-    r.out = merged ? (void*)(wk + gp.workD[i] * es) : gF[gp.lo[i]];
-    const bool tr = !merged && gp.outTransposed;
-    r.osp = tr ? 1 : r.Q; r.osq = tr ? r.P : 1;
+    r.out = gF[i];
+    r.osp = gp.outTransposed ? 1 : r.Q; r.osq = gp.outTransposed ? r.P : 1;
     if (ra.count == kMaxGradReduce && reduceNow() != hipSuccess) return fastKronInvalidArgument;
   }
   if (reduceNow() != hipSuccess) return fastKronInvalidArgument;
-  auto unmergeNow = [&]() -> hipError_t {
-    for (uint32_t b0 = 0; b0 < fBatch && ua.groups; b0 += kMaxGridBatch) {
-      GradUnmergeArgs c = ua;
-      for (uint32_t k = 0; k < c.groups; k++) {
-        uint64_t pq = 1;
-        for (uint32_t j = 0; j < c.g[k].count; j++) {
-          const uint64_t n = (uint64_t)c.g[k].p[j] * c.g[k].q[j];
-          pq *= n;
-          c.g[k].src[j] = (const char*)c.g[k].src[j] + (p.perBatchF ? (size_t)b0 * n * es : 0);
-          if (c.out[k][j]) c.out[k][j] = (char*)c.out[k][j] + (size_t)b0 * n * es;
-        }
-        c.g[k].dst = (char*)c.g[k].dst + (size_t)b0 * pq * es;
-      }
-      const hipError_t he = launchGradUnmerge(c, std::min(fBatch - b0, kMaxGridBatch), p.dt, stream_);
-      if (he != hipSuccess) return he;
-    }
-    ua.groups = 0;
-    return hipSuccess;
-  };
-  for (int i = 0; i <= lastWanted; i++) {
-    if (!wanted[i] || gp.lo[i] == gp.hi[i]) continue;
-    const uint32_t k = ua.groups++;
-    mergeGroupOf(p, gp, i, &ua.g[k]);
-    ua.g[k].dst = wk + gp.workD[i] * es;
-    for (uint32_t j = 0; j < kMaxMergeSources; j++) ua.out[k][j] = j < ua.g[k].count ? gF[gp.lo[i] + j] : nullptr;
-    if (ua.groups == kMaxUnmergeGroups && unmergeNow() != hipSuccess) return fastKronInvalidArgument;
-  }
-  if (unmergeNow() != hipSuccess) return fastKronInvalidArgument;
   return fastKronSuccess;
 }
 

@@ -28,23 +28,11 @@ struct GradReduce {
 constexpr uint32_t kMaxGradReduce = 32;
 struct GradReduceArgs { GradReduce r[kMaxGradReduce]; uint32_t count; };
 
-// Gradients of the sources of merged factors: with G = F_0 (x) F_1 (x) ... and dG given,
-// dF_j[p_j, q_j] = sum over the other digits of dG[p, q] * prod_{i != j} F_i[p_i, q_i].
-constexpr uint32_t kMaxUnmergeGroups = 8;
-struct GradUnmergeArgs {
-  MergeGroup g[kMaxUnmergeGroups];                             // dst: dG, row-major P x Q
-  void* out[kMaxUnmergeGroups][kMaxMergeSources];              // null: not wanted; element (p, q) at p*q_j + q, or transposed
-  uint32_t groups;
-  uint32_t perBatch;                                           // sources differ per batch entry
-  uint32_t outTransposed;
-};
-
 constexpr size_t kGradLdsMax = 140 * 1024;
 
 // Workgroups (partial sums) a step is given.
 uint32_t gradWorkgroups(uint32_t P, uint32_t Q, uint64_t U, uint32_t batch);
 hipError_t launchGradStep(const GradStepArgs& a, DType dt, hipStream_t stream);
 hipError_t launchGradReduce(const GradReduceArgs& a, uint32_t batch, DType dt, hipStream_t stream);
-hipError_t launchGradUnmerge(const GradUnmergeArgs& a, uint32_t batch, DType dt, hipStream_t stream);
 
 }  // namespace fk

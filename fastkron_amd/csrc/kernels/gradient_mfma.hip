@@ -369,58 +369,6 @@ __global__ __launch_bounds__(256) void kron_grad_reduce_kernel(const GradReduceA
   }
 }
 
-// One workgroup per source of a merged factor: thread = (entry of the source, share of the other digits).  Bound by the
-// chain of loads of a share's terms, hence as many shares as a workgroup has threads for.
-constexpr uint32_t kUnmergeThreads = 1024;
-template <typename T>
-__global__ __launch_bounds__(kUnmergeThreads) void kron_grad_unmerge_kernel(const GradUnmergeArgs a) {
-  const MergeGroup& g = a.g[blockIdx.x];
-  const uint32_t j = blockIdx.y, b = blockIdx.z;
-  if (j >= g.count || !a.out[blockIdx.x][j]) return;
-  __shared__ T s[kUnmergeThreads];
-  uint32_t P = 1, Q = 1, sufP = 1, sufQ = 1;               // digits behind source j are the fast ones
-  for (uint32_t i = 0; i < g.count; i++) {
-    P *= g.p[i]; Q *= g.q[i];
-    if (i > j) { sufP *= g.p[i]; sufQ *= g.q[i]; }
-  }
-  const uint32_t pj = g.p[j], qj = g.q[j], n = pj * qj, restP = P / pj, restQ = Q / qj;
-  const T* dG = (const T*)g.dst + (size_t)b * P * Q;
-  T* out = (T*)a.out[blockIdx.x][j] + (size_t)b * n;
-  uint32_t shares = kUnmergeThreads / n;
-  if (shares == 0) shares = 1;
-  const uint32_t step = kUnmergeThreads / shares;                       // entries per round
-  const uint32_t share = threadIdx.x / step, en = threadIdx.x % step;
-  for (uint32_t e0 = 0; e0 < n; e0 += step) {
-    const uint32_t e = e0 + en;
-    T v = (T)0;
-    if (e < n && share < shares) {
-      const uint32_t p = e / qj, q = e - p * qj;
-      for (uint32_t r = share; r < restP * restQ; r += shares) {
-        const uint32_t rp = r / restQ, rq = r - rp * restQ;
-        // positions in G: the digit of source j goes between the slower and the faster ones
-        const uint32_t ip = (rp / sufP * pj + p) * sufP + rp % sufP, iq = (rq / sufQ * qj + q) * sufQ + rq % sufQ;
-        T wgt = dG[(size_t)ip * Q + iq];
-        uint32_t xp = rp, xq = rq;
-        for (int i = (int)g.count - 1; i >= 0; i--) {
-          if (i == (int)j) continue;
-          const uint32_t dp = xp % g.p[i], dq = xq % g.q[i];
-          xp /= g.p[i]; xq /= g.q[i];
-          wgt *= ((const T*)g.src[i])[(a.perBatch ? (int64_t)b * (g.p[i] * g.q[i]) : 0) + (int64_t)dp * g.sp[i] + (int64_t)dq * g.sq[i]];
-        }
-        v += wgt;
-      }
-    }
-    __syncthreads();
-    s[threadIdx.x] = v;
-    __syncthreads();
-    if (share == 0 && e < n) {
-      for (uint32_t k = 1; k < shares; k++) v += s[k * step + en];
-      const uint32_t p = e / qj, q = e - p * qj;
-      out[a.outTransposed ? (size_t)q * pj + p : (size_t)e] = v;
-    }
-  }
-}
-
 template <typename T, int ZB, bool DF, bool GA, bool FULL>
 static hipError_t launchGradF(const GradStepArgs& a, uint32_t gridX, uint32_t gridZ, size_t lds, hipStream_t stream) {
   static PerDeviceOnce attrOnce;
@@ -498,14 +446,6 @@ hipError_t launchGradReduce(const GradReduceArgs& a, uint32_t batch, DType dt, h
   const dim3 grid(gx, a.count, batch);
   if (dt == DType::F32) hipLaunchKernelGGL(kron_grad_reduce_kernel<float>, grid, dim3(256), 0, stream, a);
   else                  hipLaunchKernelGGL(kron_grad_reduce_kernel<double>, grid, dim3(256), 0, stream, a);
-  return hipGetLastError();
-}
-
-hipError_t launchGradUnmerge(const GradUnmergeArgs& a, uint32_t batch, DType dt, hipStream_t stream) {
-  if (a.groups == 0) return hipSuccess;
-  const dim3 grid(a.groups, kMaxMergeSources, batch);
-  if (dt == DType::F32) hipLaunchKernelGGL(kron_grad_unmerge_kernel<float>, grid, dim3(kUnmergeThreads), 0, stream, a);
-  else                  hipLaunchKernelGGL(kron_grad_unmerge_kernel<double>, grid, dim3(kUnmergeThreads), 0, stream, a);
   return hipGetLastError();
 }
 

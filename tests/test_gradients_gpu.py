@@ -11,9 +11,9 @@ BOUND = {"float32": 2 * 128 * 2.0 ** -24, "float64": 2 * 128 * 2.0 ** -53}
 CASES = [
     # mm, m, (P, Q) of every factor, batch of x, of the factors, x transposed, factors transposed
     ("mkm", 64, [(16, 16), (16, 16)], (), (), False, False),          # whole tiles, one block
-    ("mkm", 5, [(3, 3), (5, 2), (4, 7)], (), (), False, False),       # merged, ragged
+    ("mkm", 5, [(3, 3), (5, 2), (4, 7)], (), (), False, False),       # small, ragged
     ("kmm", 7, [(3, 3), (5, 2), (4, 7)], (), (), False, True),        # rows of 7: no 16-byte accesses
-    ("kmm", 64, [(8, 8), (8, 8), (8, 8)], (), (), True, False),       # merged 64x64, X copied transposed
+    ("kmm", 64, [(8, 8), (8, 8), (8, 8)], (), (), True, False),       # X copied transposed
     ("mkm", 33, [(32, 32), (32, 32)], (), (), False, False),          # two blocks, last tile incomplete
     ("mkm", 9, [(31, 17), (18, 33)], (), (), True, True),             # padded blocks
     ("mkm", 3, [(64, 64), (50, 64)], (), (), False, False),           # 64x64 block
@@ -21,11 +21,11 @@ CASES = [
     ("kmm", 20, [(128, 128), (2, 2)], (), (), False, False),
     ("mkm", 3, [(2, 3), (260, 300)], (), (), False, False),           # F beyond LDS in fp64
     ("kmm", 1, [(16, 16), (4, 4)], (), (), False, False),             # a single column
-    ("mkm", 1, [(4, 4)] * 6, (), (), False, False),                   # one row, merged groups of three
+    ("mkm", 1, [(4, 4)] * 6, (), (), False, False),                   # one row
     ("mkm", 6, [(8, 8), (8, 8)], (3,), (), False, False),             # batch of X, shared factors
     ("kmm", 6, [(12, 12), (9, 9)], (3,), (), False, False),
     ("mkm", 6, [(16, 8), (8, 16)], (), (4,), False, False),           # shared X, factors per entry
-    ("kmm", 5, [(6, 6), (4, 4), (5, 5)], (2, 1), (3,), False, True),  # broadcast both ways, merged per entry
+    ("kmm", 5, [(6, 6), (4, 4), (5, 5)], (2, 1), (3,), False, True),  # broadcast both ways
     ("mkm", 8, [(16, 16), (16, 16)], (2, 3), (2, 3), True, False),
 ]
 
