@@ -261,6 +261,13 @@ void gradOperands(Operands* o, GradOperands* g) {
   for (uint32_t i = 0; i < o->N; i++) g->f[i] = o->f[i].data_ptr();
 }
 
+// The kernels know a tensor by its address only: one that comes back from a saved-tensors hook, or as a gradient, of another
+// type or on another device would be read beyond its end or not be there at all.
+void requireLike(const Tensor& t, const Tensor& x, const char* what) {
+  TORCH_CHECK(usable(t) && t.device() == x.device() && t.scalar_type() == x.scalar_type(), "Expected ", what, " to be ", x.scalar_type(),
+              " on ", x.device(), " like the operands, but it is ", t.defined() ? t.toString() : std::string("undefined"));
+}
+
 // grad_forward(handle, stream, mkm, x, fs) -> (z, kept for the backward pass, storage of X, of the factors)
 PyObject* gradForward(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
   HANDLE_TH_ERRORS
@@ -298,12 +305,15 @@ PyObject* gradBackward(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
   if (!THPVariable_Check(args[7]) || !THPVariable_Check(args[8]) || !PyTuple_Check(args[10]) ||
       !makeOperands(mkm, args[3], args[4], (int)opX, (int)opF, &o) || PyTuple_GET_SIZE(args[10]) != (Py_ssize_t)o.N) Py_RETURN_NONE;
   gradOperands(&o, &g);
+  requireLike(THPVariable_Unpack(args[7]), o.x, "the gradient");
+  requireLike(THPVariable_Unpack(args[8]), o.x, "the buffer kept by the forward pass");
   const Tensor gz = THPVariable_Unpack(args[7]).contiguous(), kept = THPVariable_Unpack(args[8]).contiguous();
   size_t save = 0, work = 0;
   fastKronError e = api.gradSizes(c.handle, mkm, o.f64(), (uint32_t)o.M, o.N, o.Ps, o.Qs, o.opX, g.strideX, g.perBatch, (uint32_t)g.nb, &save, &work);
   if (e == fastKronSuccess) e = api.setStream(c.handle, fastKronBackend_HIP, &c.stream);
   if (e != fastKronSuccess) return failed(e);
-  if (gz.numel() != prod(o.zshape) || gz.scalar_type() != o.x.scalar_type() || kept.numel() != (int64_t)save) Py_RETURN_NONE;
+  TORCH_CHECK(gz.numel() == prod(o.zshape), "Expected a gradient of ", prod(o.zshape), " elements, got ", gz.numel());
+  TORCH_CHECK(kept.numel() == (int64_t)save, "Expected a buffer of ", save, " elements from the forward pass, got ", kept.numel());
   const bool needX = PyObject_IsTrue(args[9]) == 1;
   Tensor gx, gf[kMaxFactors];
   void* gfp[kMaxFactors];

@@ -89,3 +89,23 @@ def test_saved_tensors_may_come_back_stored_another_way(mm):
     with torch.autograd.graph.saved_tensors_hooks(lambda t: t.cpu(), lambda t: t.cuda().contiguous()):
         z = fn(x, *fs)
     assert all(torch.equal(a, b) for a, b in zip(torch.autograd.grad(z, fs, gz), want))
+
+
+@pytest.mark.parametrize("mm", ["mkm", "kmm"])
+@pytest.mark.parametrize("change", ["half", "double", "cpu", "short", "sparse"])
+def test_the_kept_buffer_has_to_come_back_as_it_was(mm, change):
+    """The one saved tensor of one dimension is the buffer that the forward pass keeps; the kernels would read beyond a
+    buffer of another type, or through a host address."""
+    import torch
+    import fastkron_amd as fk
+    fn = fk.MKM.apply if mm == "mkm" else fk.KMM.apply
+    x = rand(*((7, 24) if mm == "mkm" else (24, 7)))
+    fs = [rand(6, 6).requires_grad_(True), rand(4, 4).requires_grad_(True)]
+    unpack = {"half": lambda t: t.half(), "double": lambda t: t.double(), "cpu": lambda t: t.cpu(), "short": lambda t: t[:-1],
+              "sparse": lambda t: t.to_sparse()}[change]
+    seen = []
+    with torch.autograd.graph.saved_tensors_hooks(lambda t: t, lambda t: (seen.append(t), unpack(t))[1] if t.ndim == 1 else t):
+        z = fn(x, *fs)
+    with pytest.raises(RuntimeError, match="forward pass"):
+        torch.autograd.grad(z, fs, torch.ones_like(z))
+    assert len(seen) == 1
