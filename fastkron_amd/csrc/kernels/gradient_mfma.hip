@@ -235,7 +235,8 @@ void kron_grad_step_kernel(const GradStepArgs a) {
             else {
               const uint32_t pl = 16 * i + MF::perm(lo);
               const uint32_t p = p0 + pl < P ? p0 + pl : P - 1;
-              f = F[(int64_t)p * a.f_sp + (int64_t)(q < Q ? q : Q - 1) * a.f_sq];
+              f = (T)0;                                    // (as in LDS: zero beyond Q, or an infinity there would count as 0 * inf)
+              if (q < Q) f = F[(int64_t)p * a.f_sp + (int64_t)q * a.f_sq];
             }
             ga[i] = MF::mma(f, xv, ga[i]);
           }

@@ -110,3 +110,44 @@ def test_backward_of_a_backward_pass():
             f.requires_grad_(True)
         fn = fk.MKM.apply if mm == "mkm" else fk.KMM.apply
         assert torch.autograd.gradgradcheck(fn, (x, *fs), eps=1e-6, atol=1e-5)
+
+
+def library_gradients(mm, x, fs, gz):
+    """Z and the gradients of X and of every factor through the C functions, operands stored row-major, no batch."""
+    import ctypes
+    import torch
+    import fastkron_amd as fk
+    from fastkron_amd import capi
+    h = fk.default_handle()
+    h.set_stream(torch.cuda.current_stream())
+    mkm, dbl = int(mm == "mkm"), int(x.dtype == torch.float64)
+    M = x.shape[0] if mkm else x.shape[1]
+    shape = (M, len(fs), capi.arr_u32([f.shape[0 if mkm else 1] for f in fs]), capi.arr_u32([f.shape[1 if mkm else 0] for f in fs]))
+    save, work = ctypes.c_size_t(), ctypes.c_size_t()
+    assert h.lib.fastKronGradSizes(h.h, mkm, dbl, *shape, capi.OP_N, 0, 0, 1, ctypes.byref(save), ctypes.byref(work)) == 0
+    new = lambda *s: torch.full(s, float("nan"), dtype=x.dtype, device="cuda")
+    kept, scratch, z, gx, gf = new(save.value), new(work.value), torch.empty_like(gz), torch.empty_like(x), [torch.empty_like(f) for f in fs]
+    ptr = lambda t: ctypes.c_void_p(t.data_ptr())
+    args = (h.h, mkm, dbl, *shape, ptr(x), capi.OP_N, 0, capi.arr_ptr([f.data_ptr() for f in fs]), capi.OP_N, 0, 1)
+    assert h.lib.fastKronGradForward(*args, ptr(z), ptr(kept)) == 0
+    assert h.lib.fastKronGradBackward(*args, ptr(gz), ptr(kept), ptr(gx), capi.arr_ptr([g.data_ptr() for g in gf]), ptr(scratch)) == 0
+    torch.cuda.synchronize()
+    return z, gx, gf
+
+
+@pytest.mark.parametrize("dt", ["float32", "float64"])
+@pytest.mark.parametrize("mm", ["mkm", "kmm"])
+@pytest.mark.parametrize("Q", [17, 70, 281, 553])                   # one block, several, F beyond LDS in fp64, in either type
+def test_infinities_stay_where_they_are(Q, mm, dt):
+    """Blocks of 16 are padded: what stands beside the padding must not enter it as 0 * inf."""
+    import torch
+    x, fs, gz = operands(mm, 5, [(20, Q)], (), (), False, False, getattr(torch, dt))
+    (fs[0] if mm == "mkm" else fs[0].t())[3, Q - 1] = float("inf")
+    (x if mm == "mkm" else x.t())[2, 19] = float("-inf")
+    _, gx, gf = library_gradients(mm, x, fs, gz)
+    X, F, G = (t.cpu().double() if mm == "mkm" else t.cpu().double().t() for t in (x, fs[0], gz))
+    for got, want in ((gx, G @ F.t()), (gf[0], X.t() @ G)):
+        got = got.cpu().double() if mm == "mkm" else got.cpu().double().t()
+        assert torch.equal(got.isinf(), want.isinf()) and torch.equal(got[got.isinf()], want[want.isinf()])
+        fin = want.isfinite()
+        assert float((got[fin] - want[fin]).norm() / want[fin].norm()) <= BOUND[dt]
