@@ -147,6 +147,11 @@ def _sum_to(g, shape):
     return g.sum_to_size(shape) if tuple(g.shape) != tuple(shape) else g
 
 
+def _matrix(mm, v):
+    """Vectors as matrices of one row (MKM) or column (KMM)."""
+    return v.unsqueeze(-2 if mm == "mkm" else -1)
+
+
 def _differentiable_backward(grad_z, x, fs, need_x, need_f):
     """Gradients of Z = X (F_0 (x) ... (x) F_{N-1}) from PyTorch operations, for backward passes that are themselves
     differentiated (create_graph).  Step of factor i maps rows (m, s) of its input, reshaped (M*S, P_i), through F_i and
@@ -193,20 +198,21 @@ def _backward(mm, ctx, grad_z):
         # one fused library call on the transposed views: dX = dZ (F_0^T (x) ...) for MKM, (F_0^T (x) ...) dZ for KMM
         if not need_x:
             return (None,) * (ctx.nf + 1)
+        # (a vector against a batch of factors has one result per entry: each a matrix of one row / column)
+        vec = x.ndim == 1 and grad_z.ndim > 1
         with torch.no_grad():
-            gx = _run(mm, grad_z, [f.mT for f in fs], 1.0, 0.0, None)
-        return (_sum_to(gx, x.shape),) + (None,) * ctx.nf
+            gx = _run(mm, _matrix(mm, grad_z) if vec else grad_z, [f.mT for f in fs], 1.0, 0.0, None)
+        return (_sum_to(gx, _matrix(mm, x).shape).reshape(x.shape) if vec else _sum_to(gx, x.shape),) + (None,) * ctx.nf
     if not torch.is_grad_enabled():
         h, stream = _handle()
         return _result(_native.grad_backward(h, stream, mm == "mkm", x, fs, ctx.opX, ctx.opF, grad_z, saved[-1], need_x, need_f), mm, x, fs,
                        0.0, None, "fastKronGradBackward")
+    matrix = lambda t: _matrix(mm, t) if x.ndim == 1 else t
     if mm == "mkm":
-        row = lambda t: t.reshape(1, -1) if x.ndim == 1 else t
-        gx, gfs = _differentiable_backward(row(grad_z), row(x), fs, need_x, need_f)
+        gx, gfs = _differentiable_backward(matrix(grad_z), matrix(x), fs, need_x, need_f)
         return (gx.reshape(x.shape) if gx is not None else None,) + tuple(gfs)
     # Z^T = X^T (F_0^T (x) ...): the MKM rule on the transposed tensors
-    col = lambda t: t.reshape(-1, 1) if x.ndim == 1 else t
-    gx, gfs = _differentiable_backward(col(grad_z).mT, col(x).mT, [f.mT for f in fs], need_x, need_f)
+    gx, gfs = _differentiable_backward(matrix(grad_z).mT, matrix(x).mT, [f.mT for f in fs], need_x, need_f)
     return (gx.mT.reshape(x.shape) if gx is not None else None,) + tuple(g.mT if g is not None else None for g in gfs)
 
 

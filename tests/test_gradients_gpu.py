@@ -151,3 +151,25 @@ def test_infinities_stay_where_they_are(Q, mm, dt):
         assert torch.equal(got.isinf(), want.isinf()) and torch.equal(got[got.isinf()], want[want.isinf()])
         fin = want.isfinite()
         assert float((got[fin] - want[fin]).norm() / want[fin].norm()) <= BOUND[dt]
+
+
+@pytest.mark.parametrize("create_graph", [False, True])
+@pytest.mark.parametrize("need", ["x", "factors", "all"])
+@pytest.mark.parametrize("mm", ["mkm", "kmm"])
+@pytest.mark.parametrize("fb", [(), (3,), (2, 3)])
+def test_gradients_of_a_vector(fb, mm, need, create_graph):
+    """X of one dimension; against a batch of factors its gradient is the sum over the entries, each with its own result."""
+    import torch
+    import fastkron_amd as fk
+    g = torch.Generator().manual_seed(1)
+    x = torch.randn(12, generator=g, dtype=torch.float64).cuda()
+    fs = [torch.randn(fb + ((p, q) if mm == "mkm" else (q, p)), generator=g, dtype=torch.float64).cuda() for p, q in ((3, 2), (4, 5))]
+    gz = torch.randn(fb + (10,), generator=g, dtype=torch.float64).cuda()
+    _, want = reference(mm, x, fs, gz)
+    needed = [need != "factors"] + [need != "x"] * 2
+    for t, n in zip([x, *fs], needed):
+        t.requires_grad_(n)
+    z = fk.gemkm(x, fs) if mm == "mkm" else fk.gekmm(fs, x)
+    got = torch.autograd.grad(z, [t for t, n in zip([x, *fs], needed) if n], gz, create_graph=create_graph)
+    for a, b in zip(got, [w for w, n in zip(want, needed) if n]):
+        assert a.shape == b.shape and rel(a.detach(), b) <= BOUND["float64"]
