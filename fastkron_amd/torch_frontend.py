@@ -196,12 +196,13 @@ def _backward(mm, ctx, grad_z):
     need_x, need_f = ctx.needs_input_grad[0], ctx.needs_input_grad[1:ctx.nf + 1]
     if not any(need_f):
         # one fused library call on the transposed views: dX = dZ (F_0^T (x) ...) for MKM, (F_0^T (x) ...) dZ for KMM
+        # (itself recorded where the backward pass is differentiated)
         if not need_x:
             return (None,) * (ctx.nf + 1)
         # (a vector against a batch of factors has one result per entry: each a matrix of one row / column)
         vec = x.ndim == 1 and grad_z.ndim > 1
-        with torch.no_grad():
-            gx = _run(mm, _matrix(mm, grad_z) if vec else grad_z, [f.mT for f in fs], 1.0, 0.0, None)
+        gz, fts = _matrix(mm, grad_z) if vec else grad_z, [f.mT for f in fs]
+        gx = gemkm(gz, fts) if mm == "mkm" else gekmm(fts, gz)
         return (_sum_to(gx, _matrix(mm, x).shape).reshape(x.shape) if vec else _sum_to(gx, x.shape),) + (None,) * ctx.nf
     if not torch.is_grad_enabled():
         h, stream = _handle()

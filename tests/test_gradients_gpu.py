@@ -99,6 +99,25 @@ def test_many_rows(mm):
         assert torch.equal(a.cpu().double(), b)
 
 
+@pytest.mark.parametrize("need", ["x", "factors"])
+@pytest.mark.parametrize("mm", ["mkm", "kmm"])
+def test_gradient_of_a_gradient(mm, need):
+    """create_graph with gradients of X alone or of the factors alone: the norm of the gradient is differentiated, in float64
+    against the dense product on the CPU."""
+    import torch
+    import fastkron_amd as fk
+    x, fs, _ = operands(mm, 3, [(3, 2), (2, 4)], (), (), False, True, torch.float64)
+
+    def second(x, fs, product):
+        w = [t.requires_grad_(True) for t in ([x] if need == "x" else fs)]
+        first = torch.autograd.grad((product(x, fs) ** 2).sum(), w, create_graph=True)
+        return torch.autograd.grad(sum((g ** 2).sum() for g in first), w)
+    got = second(x, fs, lambda x, fs: fk.gemkm(x, fs) if mm == "mkm" else fk.gekmm(fs, x))
+    want = second(x.detach().cpu(), [f.detach().cpu() for f in fs], lambda x, fs: x @ torch.kron(*fs) if mm == "mkm" else torch.kron(*fs) @ x)
+    for a, b in zip(got, want):
+        assert rel(a, b) <= BOUND["float64"]
+
+
 def test_backward_of_a_backward_pass():
     """create_graph: the backward pass is differentiated once more."""
     import torch
