@@ -30,6 +30,7 @@ using at::Tensor;
 using Dims = c10::SmallVector<int64_t, 8>;
 
 constexpr int kMaxFactors = 64;
+constexpr int64_t kMaxCount = UINT32_MAX;                      // rows, batch entries and factor extents are 32-bit numbers in the C API
 
 // Entry points of the library that Python has loaded.
 struct Api {
@@ -94,12 +95,13 @@ bool makeOperands(bool mkm, PyObject* px, PyObject* pfs, int opX, int opF, Opera
     o->f[i] = f;
     (swapped(f) ? anyT : anyN) = true;
     const int64_t a = f.size(-2), b = f.size(-1);
-    if (a == 0 || b == 0) return false;
+    if (a == 0 || b == 0 || a > kMaxCount || b > kMaxCount) return false;
     o->Ps[i] = (uint32_t)(mkm ? a : b); o->Qs[i] = (uint32_t)(mkm ? b : a);
   }
   o->fb = batchOf(o->f[0]);
   o->xb = batchOf(x);
   o->M = mkm ? x.size(-2) : x.size(-1); o->K = mkm ? x.size(-1) : x.size(-2);
+  if (o->M > kMaxCount) return false;
   int64_t k = 1;
   o->L = 1;
   for (Py_ssize_t i = 0; i < n; i++) { k *= o->Ps[i]; o->L *= o->Qs[i]; }
@@ -186,10 +188,11 @@ PyObject* product(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
   Tensor z = at::empty(o.zshape, o.x.options());
   const size_t es = z.element_size();
   // batch of X against shared factors: more rows of the same problem (MKM, X stored row-major)
-  const bool fold = mkm && !o.zb.empty() && o.fb.empty() && o.opX == fastKronOp_N && (!y.defined() || yb == o.zb);
+  const bool fold = mkm && !o.zb.empty() && o.fb.empty() && o.opX == fastKronOp_N && (!y.defined() || yb == o.zb) && prod(o.zb) <= kMaxCount / std::max<int64_t>(o.M, 1);
   const int64_t M = fold ? o.M * prod(o.zb) : o.M;
   const bool one = fold || o.zb.empty();
   const int64_t inner = one ? 1 : o.zb.back();
+  if (inner > kMaxCount) return failed(fastKronInvalidKMMProblem);
   size_t ye = 0, te = 0;
   fastKronError e = api.sizes(c.handle, (uint32_t)M, o.N, o.Ps, o.Qs, &ye, &te);
   if (e != fastKronSuccess) return failed(e);
@@ -246,8 +249,9 @@ PyObject* product(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
 struct GradOperands {
   bool perBatch; int64_t nb; uint64_t strideX; const void* f[kMaxFactors];
 };
-void gradOperands(Operands* o, GradOperands* g) {
+bool gradOperands(Operands* o, GradOperands* g) {
   g->nb = prod(o->zb);
+  if (g->nb > kMaxCount) return false;
   const int64_t nx = prod(o->xb), nf = prod(o->fb);
   g->perBatch = nf > 1;
   g->strideX = nx > 1 ? (uint64_t)(o->M * o->K) : 0;
@@ -259,6 +263,7 @@ void gradOperands(Operands* o, GradOperands* g) {
   if (nx != 1 && nx != g->nb) expand(o->x);
   if (nf != 1 && nf != g->nb) for (uint32_t i = 0; i < o->N; i++) expand(o->f[i]);
   for (uint32_t i = 0; i < o->N; i++) g->f[i] = o->f[i].data_ptr();
+  return true;
 }
 
 // The kernels know a tensor by its address only: one that comes back from a saved-tensors hook, or as a gradient, of another
@@ -275,7 +280,7 @@ PyObject* gradForward(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
   if (nargs != 5 || !callOf(args, &c, &mkm)) { if (!PyErr_Occurred()) PyErr_SetString(PyExc_TypeError, "grad_forward: 5 arguments"); return nullptr; }
   Operands o; GradOperands g;
   if (!makeOperands(mkm, args[3], args[4], 0, 0, &o)) Py_RETURN_NONE;
-  gradOperands(&o, &g);
+  if (!gradOperands(&o, &g)) Py_RETURN_NONE;
   size_t save = 0, work = 0;
   fastKronError e = api.gradSizes(c.handle, mkm, o.f64(), (uint32_t)o.M, o.N, o.Ps, o.Qs, o.opX, g.strideX, g.perBatch, (uint32_t)g.nb, &save, &work);
   if (e == fastKronSuccess) e = api.setStream(c.handle, fastKronBackend_HIP, &c.stream);
@@ -303,8 +308,7 @@ PyObject* gradBackward(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
   Operands o; GradOperands g;
   // (the storage of the forward pass: what was kept depends on it, also if the operands come back stored another way)
   if (!THPVariable_Check(args[7]) || !THPVariable_Check(args[8]) || !PyTuple_Check(args[10]) ||
-      !makeOperands(mkm, args[3], args[4], (int)opX, (int)opF, &o) || PyTuple_GET_SIZE(args[10]) != (Py_ssize_t)o.N) Py_RETURN_NONE;
-  gradOperands(&o, &g);
+      !makeOperands(mkm, args[3], args[4], (int)opX, (int)opF, &o) || PyTuple_GET_SIZE(args[10]) != (Py_ssize_t)o.N || !gradOperands(&o, &g)) Py_RETURN_NONE;
   requireLike(THPVariable_Unpack(args[7]), o.x, "the gradient");
   requireLike(THPVariable_Unpack(args[8]), o.x, "the buffer kept by the forward pass");
   const Tensor gz = THPVariable_Unpack(args[7]).contiguous(), kept = THPVariable_Unpack(args[8]).contiguous();

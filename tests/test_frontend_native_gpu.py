@@ -109,3 +109,27 @@ def test_the_kept_buffer_has_to_come_back_as_it_was(mm, change):
     with pytest.raises(RuntimeError, match="forward pass"):
         torch.autograd.grad(z, fs, torch.ones_like(z))
     assert len(seen) == 1
+
+
+def test_row_counts_beyond_32_bits():
+    """The C API counts rows in 32 bits: a folded batch of more rows goes entry by entry, one entry of more is refused (before
+    anything of its size is allocated)."""
+    import torch
+    import fastkron_amd as fk
+    f = [torch.full((1, 1), 3.0, device="cuda")]
+    with pytest.raises(fk.FastKronError):
+        fk.gemkm(rand(1, 1).expand(2 ** 32 + 4, 1), f)
+    with pytest.raises(fk.FastKronError):
+        fk.gekmm(f, rand(1, 1).expand(1, 2 ** 32 + 4))
+    with pytest.raises(fk.FastKronError):
+        fk.MKM.apply(rand(1, 1).expand(2 ** 32 + 4, 1), f[0].clone().requires_grad_(True))
+    if torch.cuda.mem_get_info()[0] < 110 << 30:
+        pytest.skip("needs 110 GB")
+    x = torch.ones((2 ** 20 + 1, 4096, 1), device="cuda")                       # 2^32 + 4096 rows, 17 GB
+    x[-1, -1] = 2.0
+    z = fk.gemkm(x, f)
+    x *= 3.0
+    same = torch.equal(z, x)
+    del x, z
+    torch.cuda.empty_cache()
+    assert same
