@@ -154,11 +154,11 @@ def _matrix(mm, v):
 
 def _differentiable_backward(grad_z, x, fs, need_x, need_f):
     """Gradients of Z = X (F_0 (x) ... (x) F_{N-1}) from PyTorch operations, for backward passes that are themselves
-    differentiated (create_graph).  Step of factor i maps rows (m, s) of its input, reshaped (M*S, P_i), through F_i and
+    differentiated (create_graph) or take a batch of gradients at once (vmap).  Step of factor i maps rows (m, s) of its input, reshaped (M*S, P_i), through F_i and
     stores column q at q*S + s; its backward un-shuffles the output gradient to (M*S, Q_i) first."""
     M = x.shape[-2]
     inputs = [x]                                          # of the steps, last factor first
-    for f in reversed(fs[1:]):
+    for f in reversed(fs[1:] if any(need_f) else ()):
         P, Q = f.shape[-2:]
         t = inputs[-1]
         S = t.shape[-1] // P
@@ -171,8 +171,11 @@ def _differentiable_backward(grad_z, x, fs, need_x, need_f):
         P, Q = f.shape[-2], f.shape[-1]
         S = g.shape[-1] // Q
         a = g.reshape(g.shape[:-2] + (M, Q, S)).transpose(-1, -2).reshape(g.shape[:-2] + (M * S, Q))
-        inp = inputs[i].reshape(inputs[i].shape[:-2] + (M * S, P))
-        grad_fs.append(_sum_to((inp.mT.contiguous() @ a), f.shape) if need_f[i] else None)
+        if need_f[i]:
+            inp = inputs[i].reshape(inputs[i].shape[:-2] + (M * S, P))
+            grad_fs.append(_sum_to((inp.mT.contiguous() @ a), f.shape))
+        else:
+            grad_fs.append(None)
         if i + 1 < len(fs) or need_x:
             g = (a @ f.mT.contiguous()).reshape(a.shape[:-2] + (M, S * P))
     return (_sum_to(g, x.shape) if need_x else None), grad_fs
@@ -194,7 +197,9 @@ def _backward(mm, ctx, grad_z):
     saved = ctx.saved_tensors
     x, fs = saved[0], saved[1:ctx.nf + 1]
     need_x, need_f = ctx.needs_input_grad[0], ctx.needs_input_grad[1:ctx.nf + 1]
-    if not any(need_f):
+    # is_grads_batched, jacobian(vectorize=True): tensors with no address to pass on
+    batched = torch._C._functorch.is_legacy_batchedtensor(grad_z) or torch._C._functorch.is_batchedtensor(grad_z)
+    if not any(need_f) and not batched:
         # one fused library call on the transposed views: dX = dZ (F_0^T (x) ...) for MKM, (F_0^T (x) ...) dZ for KMM
         # (itself recorded where the backward pass is differentiated)
         if not need_x:
@@ -204,7 +209,7 @@ def _backward(mm, ctx, grad_z):
         gz, fts = _matrix(mm, grad_z) if vec else grad_z, [f.mT for f in fs]
         gx = gemkm(gz, fts) if mm == "mkm" else gekmm(fts, gz)
         return (_sum_to(gx, _matrix(mm, x).shape).reshape(x.shape) if vec else _sum_to(gx, x.shape),) + (None,) * ctx.nf
-    if not torch.is_grad_enabled():
+    if not torch.is_grad_enabled() and not batched:
         h, stream = _handle()
         return _result(_native.grad_backward(h, stream, mm == "mkm", x, fs, ctx.opX, ctx.opF, grad_z, saved[-1], need_x, need_f), mm, x, fs,
                        0.0, None, "fastKronGradBackward")

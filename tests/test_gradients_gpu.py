@@ -192,3 +192,27 @@ def test_gradients_of_a_vector(fb, mm, need, create_graph):
     got = torch.autograd.grad(z, [t for t, n in zip([x, *fs], needed) if n], gz, create_graph=create_graph)
     for a, b in zip(got, [w for w, n in zip(want, needed) if n]):
         assert a.shape == b.shape and rel(a.detach(), b) <= BOUND["float64"]
+
+
+@pytest.mark.parametrize("need", ["x", "factors", "all"])
+@pytest.mark.parametrize("mm", ["mkm", "kmm"])
+@pytest.mark.parametrize("xb,fb", [((), ()), ((2, 1), (3,)), (None, (3,))])           # None: X of one dimension
+def test_batches_of_gradients(xb, fb, mm, need):
+    """is_grads_batched and jacobian(vectorize=True) against one gradient at a time."""
+    import torch
+    import fastkron_amd as fk
+    x, fs, _ = operands(mm, 3 if xb is not None else 1, [(3, 2), (2, 4)], xb or (), fb, False, False, torch.float64)
+    x = x.reshape(-1) if xb is None else x
+    needed = [need != "factors"] + [need != "x"] * 2
+    for t, n in zip([x, *fs], needed):
+        t.requires_grad_(n)
+    product = lambda *t: fk.gemkm(t[0], t[1:]) if mm == "mkm" else fk.gekmm(t[1:], t[0])
+    z, w = product(x, *fs), [t for t, n in zip([x, *fs], needed) if n]
+    gz = torch.randn((4,) + z.shape, dtype=z.dtype, device="cuda")
+    one = [torch.autograd.grad(z, w, g, retain_graph=True) for g in gz]
+    for i, a in enumerate(torch.autograd.grad(z, w, gz, is_grads_batched=True)):
+        assert rel(a, torch.stack([g[i] for g in one]).cpu()) <= BOUND["float64"]
+    at = lambda *t: product(*[t[needed[:i].count(True)] if n else u for i, (u, n) in enumerate(zip([x, *fs], needed))])
+    jacobian = lambda v: torch.autograd.functional.jacobian(at, tuple(t.detach() for t in w), vectorize=v)
+    for a, b in zip(jacobian(True), jacobian(False)):
+        assert a.shape == b.shape and rel(a, b.cpu()) <= BOUND["float64"]
