@@ -10,6 +10,7 @@
 #include "handle.h"
 
 #include <algorithm>
+#include <cstdio>
 #include <cstring>
 
 #include "kernels/gradient.h"
@@ -119,7 +120,7 @@ fastKronError Handle::gradForward(const GradProblem& p, void* Z, void* save) {
   fastKronError e = makePlan(p, &gp);
   if (e != fastKronSuccess) return e;
   if (gp.saveTotal && !save) return fastKronInvalidArgument;
-  e = ensureDevice();
+  e = planOnly_ ? fastKronSuccess : ensureDevice();
   if (e != fastKronSuccess) return e;
   launchLog_.clear();
   const size_t es = dtypeSize(p.dt);
@@ -131,7 +132,7 @@ fastKronError Handle::gradForward(const GradProblem& p, void* Z, void* save) {
     t.mm = p.mm; t.dt = p.dt; t.M = p.M; t.N = p.N; t.batch = p.batch; t.X = p.X; t.strideX = p.strideX;
     for (uint32_t i = 0; i < p.N; i++) { t.P[i] = p.P[i]; t.Q[i] = p.Q[i]; }
     void* xt = sv + gp.saveX * es;
-    if (launchTransposeX(t, xt, (uint64_t)p.M * t.K()) != hipSuccess) return fastKronInvalidArgument;
+    if (!planOnly_ && launchTransposeX(t, xt, (uint64_t)p.M * t.K()) != hipSuccess) return fastKronInvalidArgument;
     q.X = xt; q.strideX = q.batch > 1 && gp.xBatch > 1 ? (uint64_t)p.M * t.K() : 0;
     q.xJustWritten = true;
   }
@@ -157,8 +158,9 @@ fastKronError Handle::gradBackward(const GradProblem& p, const void* gZ, void* s
   fastKronError e = makePlan(p, &gp);
   if (e != fastKronSuccess) return e;
   if ((gp.saveTotal && !save) || (gp.workTotal && !work)) return fastKronInvalidArgument;
-  e = ensureDevice();
+  e = planOnly_ ? fastKronSuccess : ensureDevice();
   if (e != fastKronSuccess) return e;
+  launchLog_.clear();
   const KronProblem& q = gp.q;
   const size_t es = dtypeSize(p.dt);
   const uint32_t ve = (uint32_t)(16 / es);
@@ -236,7 +238,12 @@ fastKronError Handle::gradBackward(const GradProblem& p, const void* gZ, void* s
         c.vecG = t4 && aligned(c.g, c.g_o, c.g_q, gBatch);
         c.vecIn = t4 && c.in_t == 1 && aligned(c.in, c.in_o, c.in_p, inBatch);
         c.vecOut = c.gin && c.in_p == 1 && c.P % 4 == 0 && aligned(c.gin, c.in_o, c.in_t, ginBatch);
-        he = launchGradStep(c, p.dt, stream_);
+        if (planOnly_) {
+          char line[192];
+          const int n = snprintf(line, sizeof(line), "kernel=gradient_step lo=%d hi=%d rows=%u batch=%u in=%p g=%p gin=%p partial=%p\n", i, i, c.U,
+                                 c.batch, c.in, c.g, c.gin, c.partial);
+          launchLog_.append(line, n > 0 ? (size_t)n : 0);
+        } else he = launchGradStep(c, p.dt, stream_);
       }
     });
     if (he != hipSuccess) return fastKronInvalidArgument;
@@ -254,8 +261,9 @@ fastKronError Handle::gradBackward(const GradProblem& p, const void* gZ, void* s
         c.r[i].partial = (const char*)c.r[i].partial + (size_t)b0 * c.r[i].count * pq * es;
         c.r[i].out = (char*)c.r[i].out + (size_t)b0 * pq * es;
       }
-      const hipError_t he = launchGradReduce(c, std::min(fBatch - b0, kMaxGridBatch), p.dt, stream_);
-      if (he != hipSuccess) return he;
+      const uint32_t n = std::min(fBatch - b0, kMaxGridBatch);
+      if (planOnly_) launchLog_ += "kernel=gradient_sum factors=" + std::to_string(c.count) + " batch=" + std::to_string(n) + "\n";
+      else if (const hipError_t he = launchGradReduce(c, n, p.dt, stream_); he != hipSuccess) return he;
     }
     ra.count = 0;
     return hipSuccess;

@@ -33,6 +33,8 @@ fastKronError fastKronSetTunedDB(fastKronHandle handle, const char* path);
  * fastKronGetLastLaunches lists the launches the call would have made, one text line per launch:
  *   "kernel=<name> lo=<lo> hi=<hi> M=<rows> batch=<n> Kin=<cols> Kout=<cols> in=<ptr> out=<ptr> y=<ptr>
  *    in_batch=<elems> out_batch=<elems> y_batch=<elems> f_batch=<elems>,<elems>,..."
+ * fastKronGradForward is such a call; for fastKronGradBackward the lines are kernel=gradient_step, one per step of the chain,
+ * and kernel=gradient_sum.
  * Meant for host-side tests of the planner and for inspecting what a call will do.  The reference has no such
  * mode; its nearest counterpart is the kernel series printed under FASTKRON_LOG=INFO
  * (reference src/kernel_db/kernel_db.cpp:282-285).

@@ -619,3 +619,25 @@ def test_a_refusing_kernel_is_replaced_by_the_next_in_line(planner, which, expec
     e, names, launches = plan(planner, "mkm", "s", 8, [128] * 2, [128] * 2, beta=0.5, with_y=True, offs={which: 4})
     assert e == capi.SUCCESS and len(launches) == 2
     assert all(expect in n for n in names), names
+
+
+@pytest.mark.parametrize("mm", ["mkm", "kmm"])
+@pytest.mark.parametrize("opX", [capi.OP_N, capi.OP_T])
+def test_gradient_functions_launch_nothing_in_plan_only_mode(planner, mm, opX):
+    """Without a GPU any launch, and any look at the device, would be an error."""
+    lib, h = planner
+    M, Ps, Qs = 6, [3, 4, 8], [5, 4, 8]
+    shape = (int(mm == "mkm"), 0, M, 3, capi.arr_u32(Ps), capi.arr_u32(Qs))
+    save, work = ctypes.c_size_t(), ctypes.c_size_t()
+    assert lib.fastKronGradSizes(h, *shape, opX, M * 96, 1, 2, ctypes.byref(save), ctypes.byref(work)) == capi.SUCCESS
+    ptr = [ctypes.c_void_p(BASE + i * GAP) for i in range(8)]
+    fs, gf = (capi.arr_ptr([BASE + (n + i) * GAP for i in range(3)]) for n in (10, 13))
+    args = (h, *shape, ptr[0], opX, M * 96, fs, capi.OP_N, 1, 2)
+    assert lib.fastKronGradForward(*args, ptr[1], ptr[2]) == capi.SUCCESS
+    buf = ctypes.create_string_buffer(1 << 14)
+    lib.fastKronGetLastLaunches(h, buf, len(buf))
+    assert [l.split()[1] for l in buf.value.decode().splitlines()] == ["lo=2", "lo=1", "lo=0"]
+    assert lib.fastKronGradBackward(*args, ptr[3], ptr[2], ptr[4], gf, ptr[5]) == capi.SUCCESS
+    lib.fastKronGetLastLaunches(h, buf, len(buf))
+    assert [l.split()[0] for l in buf.value.decode().splitlines()] == ["kernel=gradient_step"] * 3 + ["kernel=gradient_sum"]
+    assert lib.fastKronGradBackward(*args, None, ptr[2], ptr[4], gf, ptr[5]) != capi.SUCCESS
