@@ -69,6 +69,12 @@ struct Operands {
     zshape.push_back(mkm ? M : L); zshape.push_back(mkm ? L : M);
   }
   bool f64() const { return x.scalar_type() == at::kDouble; }
+  // batch of X against shared factors: more rows of the same problem (MKM, X stored row-major)
+  bool folds() const {
+    return mkm && !zb.empty() && fb.empty() && opX == fastKronOp_N && prod(zb) <= kMaxCount / std::max<int64_t>(M, 1);
+  }
+  // no entry along an outer batch dimension: a loop of no calls (an innermost dimension of no entries is refused by the call)
+  bool noCalls() const { return zb.size() > 1 && prod(at::IntArrayRef(zb.data(), zb.size() - 1)) == 0 && !folds(); }
 };
 
 bool usable(const Tensor& t) { return t.defined() && t.is_cuda() && t.layout() == at::kStrided; }
@@ -187,8 +193,7 @@ PyObject* product(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
 
   Tensor z = at::empty(o.zshape, o.x.options());
   const size_t es = z.element_size();
-  // batch of X against shared factors: more rows of the same problem (MKM, X stored row-major)
-  const bool fold = mkm && !o.zb.empty() && o.fb.empty() && o.opX == fastKronOp_N && (!y.defined() || yb == o.zb) && prod(o.zb) <= kMaxCount / std::max<int64_t>(o.M, 1);
+  const bool fold = o.folds() && (!y.defined() || yb == o.zb);
   const int64_t M = fold ? o.M * prod(o.zb) : o.M;
   const bool one = fold || o.zb.empty();
   const int64_t inner = one ? 1 : o.zb.back();
@@ -280,6 +285,8 @@ PyObject* gradForward(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
   if (nargs != 5 || !callOf(args, &c, &mkm)) { if (!PyErr_Occurred()) PyErr_SetString(PyExc_TypeError, "grad_forward: 5 arguments"); return nullptr; }
   Operands o; GradOperands g;
   if (!makeOperands(mkm, args[3], args[4], 0, 0, &o)) Py_RETURN_NONE;
+  if (o.noCalls() && !o.vec)
+    return Py_BuildValue("NNii", THPVariable_Wrap(at::empty(o.zshape, o.x.options())), THPVariable_Wrap(at::empty({0}, o.x.options())), (int)o.opX, (int)o.opF);
   if (!gradOperands(&o, &g)) Py_RETURN_NONE;
   size_t save = 0, work = 0;
   fastKronError e = api.gradSizes(c.handle, mkm, o.f64(), (uint32_t)o.M, o.N, o.Ps, o.Qs, o.opX, g.strideX, g.perBatch, (uint32_t)g.nb, &save, &work);
@@ -308,7 +315,19 @@ PyObject* gradBackward(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
   Operands o; GradOperands g;
   // (the storage of the forward pass: what was kept depends on it, also if the operands come back stored another way)
   if (!THPVariable_Check(args[7]) || !THPVariable_Check(args[8]) || !PyTuple_Check(args[10]) ||
-      !makeOperands(mkm, args[3], args[4], (int)opX, (int)opF, &o) || PyTuple_GET_SIZE(args[10]) != (Py_ssize_t)o.N || !gradOperands(&o, &g)) Py_RETURN_NONE;
+      !makeOperands(mkm, args[3], args[4], (int)opX, (int)opF, &o) || PyTuple_GET_SIZE(args[10]) != (Py_ssize_t)o.N) Py_RETURN_NONE;
+  const bool needX = PyObject_IsTrue(args[9]) == 1;
+  auto needF = [&](uint32_t i) { return PyObject_IsTrue(PyTuple_GET_ITEM(args[10], i)) == 1; };
+  if (o.noCalls()) {
+    PyObject* out = PyTuple_New(1 + (Py_ssize_t)o.N);
+    for (uint32_t i = 0; out && i <= o.N; i++) {
+      const Tensor& t = THPVariable_Unpack(i ? PySequence_Fast_GET_ITEM(args[4], i - 1) : args[3]);
+      if (i ? needF(i - 1) : needX) PyTuple_SET_ITEM(out, i, THPVariable_Wrap(at::zeros(t.sizes(), o.x.options())));
+      else { Py_INCREF(Py_None); PyTuple_SET_ITEM(out, i, Py_None); }
+    }
+    return out;
+  }
+  if (!gradOperands(&o, &g)) Py_RETURN_NONE;
   requireLike(THPVariable_Unpack(args[7]), o.x, "the gradient");
   requireLike(THPVariable_Unpack(args[8]), o.x, "the buffer kept by the forward pass");
   const Tensor gz = THPVariable_Unpack(args[7]).contiguous(), kept = THPVariable_Unpack(args[8]).contiguous();
@@ -318,7 +337,6 @@ PyObject* gradBackward(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
   if (e != fastKronSuccess) return failed(e);
   TORCH_CHECK(gz.numel() == prod(o.zshape), "Expected a gradient of ", prod(o.zshape), " elements, got ", gz.numel());
   TORCH_CHECK(kept.numel() == (int64_t)save, "Expected a buffer of ", save, " elements from the forward pass, got ", kept.numel());
-  const bool needX = PyObject_IsTrue(args[9]) == 1;
   Tensor gx, gf[kMaxFactors];
   void* gfp[kMaxFactors];
   Dims xs = o.zb;
@@ -326,7 +344,7 @@ PyObject* gradBackward(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
   if (needX) gx = at::empty(xs, o.x.options());
   for (uint32_t i = 0; i < o.N; i++) {
     gfp[i] = nullptr;
-    if (PyObject_IsTrue(PyTuple_GET_ITEM(args[10], i)) != 1) continue;
+    if (!needF(i)) continue;
     Dims s = g.perBatch ? o.zb : Dims();
     s.push_back(mkm ? o.Ps[i] : o.Qs[i]); s.push_back(mkm ? o.Qs[i] : o.Ps[i]);
     gf[i] = at::empty(s, o.x.options());

@@ -133,3 +133,30 @@ def test_row_counts_beyond_32_bits():
     del x, z
     torch.cuda.empty_cache()
     assert same
+
+
+@pytest.mark.parametrize("mm,xb,fb,taken", [
+    ("mkm", (), (0, 3), True), ("mkm", (0, 3), (0, 3), True), ("mkm", (0, 3), (1, 3), True), ("mkm", (0, 2, 0), (0, 2, 0), True),
+    ("kmm", (), (0, 3), True), ("kmm", (0, 3), (), True), ("kmm", (2, 0, 3), (), True),
+    ("mkm", (0, 3), (), False), ("mkm", (3, 0), (3, 0), False), ("kmm", (3, 0), (3, 0), False), ("mkm", (0,), (0,), False), ("kmm", (), (0,), False)])
+@pytest.mark.parametrize("need", ["", "x", "factors", "all"])
+def test_empty_batches(mm, xb, fb, taken, need):
+    """No entry along an outer batch dimension: an empty result and gradients of zeros, with every kind of gradient.  An
+    empty innermost dimension, or rows folded to none, are refused, as the library refuses M = 0."""
+    import torch
+    import fastkron_amd as fk
+    rows = lambda a, b: (a, b) if mm == "mkm" else (b, a)
+    x, fs = rand(*xb, *rows(3, 6)), [rand(*fb, *rows(3, 2)), rand(*fb, *rows(2, 4))]
+    x.requires_grad_(need in ("x", "all"))
+    for f in fs:
+        f.requires_grad_(need in ("factors", "all"))
+    call = lambda: fk.gemkm(x, fs) if mm == "mkm" else fk.gekmm(fs, x)
+    if not taken:
+        with pytest.raises(fk.FastKronError):
+            call()
+        return
+    z = call()
+    assert z.shape == tuple(torch.broadcast_shapes(xb, fb)) + rows(3, 8)
+    w = [t for t in [x, *fs] if t.requires_grad]
+    for t, g in zip(w, torch.autograd.grad(z, w, torch.ones_like(z)) if w else []):
+        assert g.shape == t.shape and not g.any()
