@@ -82,8 +82,9 @@ bool usable(const Tensor& t) { return t.defined() && t.is_cuda() && t.layout() =
 bool swapped(const Tensor& t) { return !t.is_contiguous() && t.dim() >= 2 && t.mT().is_contiguous(); }
 Tensor buffer(const Tensor& t, fastKronOp op) { return (op == fastKronOp_T ? t.mT() : t).contiguous(); }
 
-// ops: the storage to use (0: as the tensors are stored)
-bool makeOperands(bool mkm, PyObject* px, PyObject* pfs, int opX, int opF, Operands* o) {
+// Shapes and storage only, nothing is copied before all of a call's rules have been looked at (a call that is recorded for
+// gradients comes back through the autograd function); ops: the storage to use (0: as the tensors are stored).
+bool describe(bool mkm, PyObject* px, PyObject* pfs, int opX, int opF, Operands* o) {
   if (!THPVariable_Check(px) || !(PyList_Check(pfs) || PyTuple_Check(pfs))) return false;
   const Py_ssize_t n = PySequence_Fast_GET_SIZE(pfs);
   if (n == 0 || n > kMaxFactors) return false;
@@ -115,9 +116,13 @@ bool makeOperands(bool mkm, PyObject* px, PyObject* pfs, int opX, int opF, Opera
   o->setZShape();
   o->opX = opX ? (fastKronOp)opX : swapped(x) ? fastKronOp_T : fastKronOp_N;
   o->opF = opF ? (fastKronOp)opF : anyT && !anyN ? fastKronOp_T : fastKronOp_N;      // one op is passed for all factors
-  o->x = buffer(x, o->opX);
-  for (Py_ssize_t i = 0; i < n; i++) o->f[i] = buffer(o->f[i], o->opF);
+  o->x = x;
   return true;
+}
+// ... and the buffers
+void makeBuffers(Operands* o) {
+  o->x = buffer(o->x, o->opX);
+  for (uint32_t i = 0; i < o->N; i++) o->f[i] = buffer(o->f[i], o->opF);
 }
 
 struct Call { fastKronHandle handle; void* stream; };
@@ -171,7 +176,7 @@ PyObject* product(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
   const double alpha = PyFloat_AsDouble(args[5]), beta = PyFloat_AsDouble(args[6]);
   if (PyErr_Occurred()) return nullptr;
   Operands o;
-  if (!makeOperands(mkm, args[3], args[4], 0, 0, &o)) Py_RETURN_NONE;
+  if (!describe(mkm, args[3], args[4], 0, 0, &o)) Py_RETURN_NONE;
   if (c10::GradMode::is_enabled()) {
     bool wanted = THPVariable_Unpack(args[3]).requires_grad();
     for (uint32_t i = 0; i < o.N; i++) wanted = wanted || THPVariable_Unpack(PySequence_Fast_GET_ITEM(args[4], i)).requires_grad();
@@ -190,6 +195,7 @@ PyObject* product(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
     if (!broadcast(yb, o.zb, &both) || both != o.zb) Py_RETURN_NONE;
     y = y.contiguous();
   } else if (beta != 0.0) Py_RETURN_NONE;
+  makeBuffers(&o);
 
   Tensor z = at::empty(o.zshape, o.x.options());
   const size_t es = z.element_size();
@@ -257,6 +263,7 @@ struct GradOperands {
 bool gradOperands(Operands* o, GradOperands* g) {
   g->nb = prod(o->zb);
   if (g->nb > kMaxCount) return false;
+  makeBuffers(o);
   const int64_t nx = prod(o->xb), nf = prod(o->fb);
   g->perBatch = nf > 1;
   g->strideX = nx > 1 ? (uint64_t)(o->M * o->K) : 0;
@@ -284,7 +291,7 @@ PyObject* gradForward(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
   Call c; bool mkm;
   if (nargs != 5 || !callOf(args, &c, &mkm)) { if (!PyErr_Occurred()) PyErr_SetString(PyExc_TypeError, "grad_forward: 5 arguments"); return nullptr; }
   Operands o; GradOperands g;
-  if (!makeOperands(mkm, args[3], args[4], 0, 0, &o)) Py_RETURN_NONE;
+  if (!describe(mkm, args[3], args[4], 0, 0, &o)) Py_RETURN_NONE;
   if (o.noCalls() && !o.vec)
     return Py_BuildValue("NNii", THPVariable_Wrap(at::empty(o.zshape, o.x.options())), THPVariable_Wrap(at::empty({0}, o.x.options())), (int)o.opX, (int)o.opF);
   if (!gradOperands(&o, &g)) Py_RETURN_NONE;
@@ -315,7 +322,7 @@ PyObject* gradBackward(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
   Operands o; GradOperands g;
   // (the storage of the forward pass: what was kept depends on it, also if the operands come back stored another way)
   if (!THPVariable_Check(args[7]) || !THPVariable_Check(args[8]) || !PyTuple_Check(args[10]) ||
-      !makeOperands(mkm, args[3], args[4], (int)opX, (int)opF, &o) || PyTuple_GET_SIZE(args[10]) != (Py_ssize_t)o.N) Py_RETURN_NONE;
+      !describe(mkm, args[3], args[4], (int)opX, (int)opF, &o) || PyTuple_GET_SIZE(args[10]) != (Py_ssize_t)o.N) Py_RETURN_NONE;
   const bool needX = PyObject_IsTrue(args[9]) == 1;
   auto needF = [&](uint32_t i) { return PyObject_IsTrue(PyTuple_GET_ITEM(args[10], i)) == 1; };
   if (o.noCalls()) {

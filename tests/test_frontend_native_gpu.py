@@ -160,3 +160,22 @@ def test_empty_batches(mm, xb, fb, taken, need):
     w = [t for t in [x, *fs] if t.requires_grad]
     for t, g in zip(w, torch.autograd.grad(z, w, torch.ones_like(z)) if w else []):
         assert g.shape == t.shape and not g.any()
+
+
+@pytest.mark.parametrize("mm", ["mkm", "kmm"])
+def test_a_recorded_call_copies_its_operands_once(mm):
+    """A strided X and strided factors are copied by the autograd function, not by the call that finds it has to be recorded
+    as well: gemkm allocates what the autograd function alone does."""
+    import torch
+    import fastkron_amd as fk
+    x = rand(64, 2 * 4096)[:, ::2] if mm == "mkm" else rand(4096, 2 * 64)[:, ::2]
+    fs = [rand(16, 32)[:, ::2].requires_grad_(True) for _ in range(3)]
+
+    def allocated(call):
+        before = torch.cuda.memory_stats()["allocated_bytes.all.allocated"]
+        call()
+        return torch.cuda.memory_stats()["allocated_bytes.all.allocated"] - before
+    call = (lambda: fk.gemkm(x, fs)) if mm == "mkm" else (lambda: fk.gekmm(fs, x))
+    fn = fk.MKM.apply if mm == "mkm" else fk.KMM.apply
+    call()
+    assert allocated(call) == allocated(lambda: fn(x, *fs))
