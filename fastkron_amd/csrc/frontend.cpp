@@ -7,7 +7,7 @@
 // -> 123 us).  Everything between the Python call and the C API happens here instead; nothing is kept between calls.
 // A function returns None for operands that it does not take (the Python side then says why), a fastKronError as a
 // whole number where the library refuses the call, and otherwise its tensors; product returns False for a call that is
-// to be recorded for gradients.  The interpreter's lock is held throughout: threads share the default handle.
+// to be recorded for gradients.
 //
 // Rules (reference pyfastkron/fastkronbase.py:104-518): leading dimensions are batches, broadcast between X, the factors
 // and Y; the innermost batch dimension is one strided-batched call (stride 0 = shared operand), outer ones a loop; a
@@ -19,7 +19,7 @@
 #include <c10/core/GradMode.h>
 
 #include <cstdint>
-#include <vector>
+#include <mutex>
 
 #include "../../include/fastkron.h"
 #include "../../include/fastkron_ext.h"
@@ -135,6 +135,19 @@ bool callOf(PyObject* const* args, Call* c, bool* mkm) {
   return !PyErr_Occurred();
 }
 
+// While the library runs, without the interpreter's lock: other Python threads go on while it tunes or waits for room in the
+// launch queue (they stood still through the 18 ms in which a first call was tuned).  Threads share the default handle and
+// each call sets its stream, so one call at a time.  No Python object is touched in its scope.
+class LibraryCall {
+ public:
+  LibraryCall() : thread_(PyEval_SaveThread()) { one().lock(); }
+  ~LibraryCall() { one().unlock(); PyEval_RestoreThread(thread_); }
+  LibraryCall(const LibraryCall&) = delete;
+ private:
+  static std::mutex& one() { static std::mutex m; return m; }
+  PyThreadState* thread_;
+};
+
 PyObject* failed(fastKronError e) { return PyLong_FromLong((long)e); }
 
 fastKronError call(const Call& c, const Operands& o, uint32_t M, const void* x, const void* const* f, void* z, double alpha,
@@ -212,15 +225,15 @@ PyObject* product(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
   Tensor temp = at::empty({(int64_t)(off + tn)}, o.x.options());
   char* t1 = (char*)temp.data_ptr();
   char* t2 = t1 ? t1 + off * es : nullptr;
-  e = api.setStream(c.handle, fastKronBackend_HIP, &c.stream);
-  if (e != fastKronSuccess) return failed(e);
-
-  const void* f[kMaxFactors];
-  if (one) {
-    for (uint32_t i = 0; i < o.N; i++) f[i] = o.f[i].data_ptr();
-    e = call(c, o, (uint32_t)M, o.x.data_ptr(), f, z.data_ptr(), alpha, beta, y.defined() ? y.data_ptr() : nullptr, t1, t2);
-    if (e != fastKronSuccess) return failed(e);
-  } else {
+  auto run = [&]() -> fastKronError {
+    LibraryCall unlocked;
+    fastKronError e = api.setStream(c.handle, fastKronBackend_HIP, &c.stream);
+    if (e != fastKronSuccess) return e;
+    const void* f[kMaxFactors];
+    if (one) {
+      for (uint32_t i = 0; i < o.N; i++) f[i] = o.f[i].data_ptr();
+      return call(c, o, (uint32_t)M, o.x.data_ptr(), f, z.data_ptr(), alpha, beta, y.defined() ? y.data_ptr() : nullptr, t1, t2);
+    }
     const size_t d = o.zb.size();
     // element offset of the entry `idx` (innermost index 0) of an operand with batch dimensions `b` broadcast to zb's
     auto entry = [&](const Dims& b, const Dims& idx) {
@@ -243,9 +256,12 @@ PyObject* product(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
                       (char*)z.data_ptr() + (size_t)(entry(o.zb, idx) * zblk) * es, zblk, alpha, beta, (uint32_t)inner,
                       y.defined() ? (char*)y.data_ptr() + (size_t)(entry(yb, idx) * zblk) * es : nullptr, y.defined() && step(yb) ? zblk : 0, t1,
                       t2);
-      if (e != fastKronSuccess) return failed(e);
+      if (e != fastKronSuccess) return e;
     }
-  }
+    return e;
+  };
+  e = run();
+  if (e != fastKronSuccess) return failed(e);
   if (o.vec) {
     Dims s = o.zb;
     s.push_back(-1);
@@ -297,11 +313,15 @@ PyObject* gradForward(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
   if (!gradOperands(&o, &g)) Py_RETURN_NONE;
   size_t save = 0, work = 0;
   fastKronError e = api.gradSizes(c.handle, mkm, o.f64(), (uint32_t)o.M, o.N, o.Ps, o.Qs, o.opX, g.strideX, g.perBatch, (uint32_t)g.nb, &save, &work);
-  if (e == fastKronSuccess) e = api.setStream(c.handle, fastKronBackend_HIP, &c.stream);
   if (e != fastKronSuccess) return failed(e);
   Tensor z = at::empty(o.zshape, o.x.options()), kept = at::empty({(int64_t)save}, o.x.options());
-  e = api.gradForward(c.handle, mkm, o.f64(), (uint32_t)o.M, o.N, o.Ps, o.Qs, o.x.data_ptr(), o.opX, g.strideX, g.f, o.opF, g.perBatch,
-                      (uint32_t)g.nb, z.data_ptr(), kept.data_ptr());
+  {
+    LibraryCall unlocked;
+    e = api.setStream(c.handle, fastKronBackend_HIP, &c.stream);
+    if (e == fastKronSuccess)
+      e = api.gradForward(c.handle, mkm, o.f64(), (uint32_t)o.M, o.N, o.Ps, o.Qs, o.x.data_ptr(), o.opX, g.strideX, g.f, o.opF, g.perBatch,
+                          (uint32_t)g.nb, z.data_ptr(), kept.data_ptr());
+  }
   if (e != fastKronSuccess) return failed(e);
   if (o.vec) {
     Dims s = o.zb;
@@ -340,7 +360,6 @@ PyObject* gradBackward(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
   const Tensor gz = THPVariable_Unpack(args[7]).contiguous(), kept = THPVariable_Unpack(args[8]).contiguous();
   size_t save = 0, work = 0;
   fastKronError e = api.gradSizes(c.handle, mkm, o.f64(), (uint32_t)o.M, o.N, o.Ps, o.Qs, o.opX, g.strideX, g.perBatch, (uint32_t)g.nb, &save, &work);
-  if (e == fastKronSuccess) e = api.setStream(c.handle, fastKronBackend_HIP, &c.stream);
   if (e != fastKronSuccess) return failed(e);
   TORCH_CHECK(gz.numel() == prod(o.zshape), "Expected a gradient of ", prod(o.zshape), " elements, got ", gz.numel());
   TORCH_CHECK(kept.numel() == (int64_t)save, "Expected a buffer of ", save, " elements from the forward pass, got ", kept.numel());
@@ -358,8 +377,13 @@ PyObject* gradBackward(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
     gfp[i] = gf[i].data_ptr();
   }
   const Tensor scratch = at::empty({(int64_t)work}, o.x.options());
-  e = api.gradBackward(c.handle, mkm, o.f64(), (uint32_t)o.M, o.N, o.Ps, o.Qs, o.x.data_ptr(), o.opX, g.strideX, g.f, o.opF, g.perBatch,
-                       (uint32_t)g.nb, gz.data_ptr(), kept.data_ptr(), needX ? gx.data_ptr() : nullptr, gfp, scratch.data_ptr());
+  {
+    LibraryCall unlocked;
+    e = api.setStream(c.handle, fastKronBackend_HIP, &c.stream);
+    if (e == fastKronSuccess)
+      e = api.gradBackward(c.handle, mkm, o.f64(), (uint32_t)o.M, o.N, o.Ps, o.Qs, o.x.data_ptr(), o.opX, g.strideX, g.f, o.opF, g.perBatch,
+                           (uint32_t)g.nb, gz.data_ptr(), kept.data_ptr(), needX ? gx.data_ptr() : nullptr, gfp, scratch.data_ptr());
+  }
   if (e != fastKronSuccess) return failed(e);
   PyObject* out = PyTuple_New(1 + (Py_ssize_t)o.N);
   if (!out) return nullptr;

@@ -179,3 +179,59 @@ def test_a_recorded_call_copies_its_operands_once(mm):
     fn = fk.MKM.apply if mm == "mkm" else fk.KMM.apply
     call()
     assert allocated(call) == allocated(lambda: fn(x, *fs))
+
+
+def test_other_threads_run_during_a_call(monkeypatch):
+    """A call that tunes keeps the host busy for milliseconds; a thread that ticks every half of one goes on meanwhile."""
+    import threading
+    import time
+    import torch
+    import fastkron_amd as fk
+    handle = fk.FastKron(tune=True)
+    handle.set_tuned_db("")
+    monkeypatch.setattr(fk, "_default", handle)
+    x, fs = rand(500, 21 ** 3), [rand(21, 21) for _ in range(3)]
+    ticks, stop = [], threading.Event()
+
+    def tick():
+        while not stop.wait(0.0005):
+            ticks.append(time.perf_counter())
+    thread = threading.Thread(target=tick)
+    thread.start()
+    begin = time.perf_counter()
+    fk.gemkm(x, fs)
+    end = time.perf_counter()
+    stop.set()
+    thread.join()
+    inside = [begin] + [t for t in ticks if begin <= t <= end] + [end]
+    longest = max(b - a for a, b in zip(inside, inside[1:]))
+    assert end - begin > 0.004 and longest < 0.5 * (end - begin), (end - begin, longest)
+
+
+def test_threads_with_streams_of_their_own():
+    """Each call sets the shared handle's stream: two threads must not get in between, products and gradients alike."""
+    import threading
+    import torch
+    import fastkron_amd as fk
+    shapes = [(64, [4] * 5), (33, [5] * 4), (100, [16] * 3), (7, [31, 31])]
+    errors = []
+
+    def work(i):
+        m, ps = shapes[i]
+        g = torch.Generator(device="cuda").manual_seed(i)
+        stream = torch.cuda.Stream()
+        with torch.cuda.stream(stream):
+            fs = [torch.randn(p, p, device="cuda", generator=g).requires_grad_(True) for p in ps]
+            x = torch.randn(m, int(np.prod(ps)), device="cuda", generator=g)
+            want = fk.gemkm(x, [f.detach() for f in fs])
+            grads = torch.autograd.grad(fk.gemkm(x, fs), fs, x)
+            for n in range(40):
+                y = x * 1.0                                                     # written on this stream just before it is read
+                if not torch.equal(fk.gemkm(y, [f.detach() for f in fs]), want):
+                    errors.append((i, n, "product"))
+                if not all(torch.equal(a, b) for a, b in zip(torch.autograd.grad(fk.gemkm(y, fs), fs, y), grads)):
+                    errors.append((i, n, "gradients"))
+    threads = [threading.Thread(target=work, args=(i,)) for i in range(len(shapes))]
+    [t.start() for t in threads]
+    [t.join() for t in threads]
+    assert not errors, errors
