@@ -7,6 +7,7 @@ pyfastkron/fastkrontorch.py:340-465) for tensors that live in HBM.  PyTorch is u
 library's HIP kernels, and a missing library or a CPU tensor is an error, never a fallback.
 """
 import ctypes
+import threading
 
 from . import capi
 from .capi import (BACKEND_HIP, OP_N, OP_T, OPT_NONE, OPT_TUNE, OPT_USE_FUSION, SUCCESS)
@@ -188,12 +189,16 @@ class FastKron:
 
 
 _default = None
+_default_lock = threading.Lock()
 
 
 def default_handle():
     global _default
     if _default is None:
-        _default = FastKron()
+        # (one handle for all threads: the front end passes its address on, so a second one must not replace it)
+        with _default_lock:
+            if _default is None:
+                _default = FastKron()
     return _default
 
 

@@ -127,3 +127,22 @@ def test_tuned_plan_file_round_trip(tmp_path, handle):
     f = tmp_path / "tuned.db"
     f.write_text("# comment\n8x64*(8x8^2)_NN_f 0.01 1 0 1 no_such_kernel\n")
     assert lib.fastKronSetTunedDB(h, str(f).encode()) == capi.SUCCESS
+
+
+def test_first_calls_of_several_threads_share_one_handle(monkeypatch):
+    """The front end passes the default handle's address on: a second handle that replaced the first would free it under a
+    call that is still running."""
+    import threading
+    import time
+    import fastkron_amd
+
+    class Slow:
+        def __init__(self):
+            time.sleep(0.05)
+    monkeypatch.setattr(fastkron_amd, "FastKron", Slow)
+    monkeypatch.setattr(fastkron_amd, "_default", None)
+    got = []
+    threads = [threading.Thread(target=lambda: got.append(fastkron_amd.default_handle())) for _ in range(4)]
+    [t.start() for t in threads]
+    [t.join() for t in threads]
+    assert len(got) == 4 and len(set(map(id, got))) == 1
