@@ -30,12 +30,12 @@ struct GradPlan {
   KronProblem q;                    // MKM or KMM, op(X) = N; F, X, Z, inter not set
   bool pMajor;                      // storage of the factors: element (p, q) at p*Q + q
   bool outTransposed;               // gradients of the factors are Q x P (KMM)
-  bool copyX;                       // op(X) = T: X is copied transposed
+  bool copyX;                       // op(X) = T: each pass reads a transposed copy of X, which is not kept between them
   uint32_t xBatch;                  // entries of that copy
   // offsets into `save`, in elements
-  size_t saveX, saveI[kMaxFactors], saveTotal;
+  size_t saveI[kMaxFactors], saveTotal;
   // offsets into `work`
-  size_t workG[2], workP[kMaxFactors], workTotal;
+  size_t workX, workG[2], workP[kMaxFactors], workTotal;
   uint32_t parts[kMaxFactors];      // partial sums of factor g per batch entry
 };
 
@@ -84,10 +84,10 @@ fastKronError makePlan(const Handle::GradProblem& p, GradPlan* gp) {
   const size_t nb = q.batch;
   size_t off = 0;
   auto take = [&](size_t elems) { const size_t o = off; off += roundUp(elems); return o; };
-  gp->saveX = gp->copyX ? take((size_t)gp->xBatch * p.M * K) : 0;
   for (uint32_t g = 1; g < q.N; g++) gp->saveI[g] = take(nb * q.M * q.colsAfter(g));      // output of step g
   gp->saveTotal = off;
   off = 0;
+  gp->workX = gp->copyX ? take((size_t)gp->xBatch * p.M * K) : 0;
   size_t widest = 0;
   for (uint32_t g = 0; g + 1 < q.N; g++) widest = std::max<size_t>(widest, q.colsBefore(g));
   for (int i = 0; i < 2; i++) gp->workG[i] = q.N > 1u + i ? take(nb * q.M * widest) : 0;
@@ -113,6 +113,14 @@ fastKronError Handle::gradSizes(const GradProblem& p, size_t* saveElems, size_t*
   return fastKronSuccess;
 }
 
+// X (op T) of every batch entry with a stride of its own, transposed to `to`.
+hipError_t Handle::transposeX(const GradProblem& p, void* to) {
+  KronProblem t{};
+  t.mm = p.mm; t.dt = p.dt; t.M = p.M; t.N = p.N; t.batch = p.batch; t.X = p.X; t.strideX = p.strideX;
+  for (uint32_t i = 0; i < p.N; i++) { t.P[i] = p.P[i]; t.Q[i] = p.Q[i]; }
+  return launchTransposeX(t, to, (uint64_t)p.M * t.K());
+}
+
 fastKronError Handle::gradForward(const GradProblem& p, void* Z, void* save) {
   if (!Z || !p.X || !p.F) return fastKronInvalidArgument;
   for (uint32_t i = 0; i < p.N; i++) if (!p.F[i]) return fastKronInvalidKMMProblem;
@@ -128,13 +136,16 @@ fastKronError Handle::gradForward(const GradProblem& p, void* Z, void* save) {
   KronProblem q = gp.q;
   q.X = p.X; q.strideX = q.batch > 1 ? p.strideX : 0;
   if (gp.copyX) {
-    KronProblem t{};
-    t.mm = p.mm; t.dt = p.dt; t.M = p.M; t.N = p.N; t.batch = p.batch; t.X = p.X; t.strideX = p.strideX;
-    for (uint32_t i = 0; i < p.N; i++) { t.P[i] = p.P[i]; t.Q[i] = p.Q[i]; }
-    void* xt = sv + gp.saveX * es;
-    if (!planOnly_ && launchTransposeX(t, xt, (uint64_t)p.M * t.K()) != hipSuccess) return fastKronInvalidArgument;
-    q.X = xt; q.strideX = q.batch > 1 && gp.xBatch > 1 ? (uint64_t)p.M * t.K() : 0;
-    q.xJustWritten = true;
+    if (q.N > 1 && (uint64_t)gp.xBatch * p.M * q.K() <= (uint64_t)q.batch * q.M * q.L()) {
+      // the copy stands in Z, which only the last of the launches writes
+      if (!planOnly_ && transposeX(p, Z) != hipSuccess) return fastKronInvalidArgument;
+      q.X = Z; q.strideX = q.batch > 1 && gp.xBatch > 1 ? (uint64_t)p.M * q.K() : 0;
+      q.xJustWritten = true;
+    } else {
+      // no room for it: the first launch reads X as it is stored (entry by entry: not as rows of one problem)
+      q.M = p.M; q.batch = p.batch;
+      q.opX = fastKronOp_T; q.strideX = q.batch > 1 ? p.strideX : 0;
+    }
   }
   for (uint32_t g = 0; g < q.N; g++) {
     q.strideF[g] = p.perBatchF && q.batch > 1 ? (uint64_t)q.P[g] * q.Q[g] : 0;
@@ -175,6 +186,7 @@ fastKronError Handle::gradBackward(const GradProblem& p, const void* gZ, void* s
     if (wanted[g]) lastWanted = (int)g;
   }
   if (gX) lastWanted = (int)q.N - 1;
+  if (gp.copyX && wanted[q.N - 1] && !planOnly_ && transposeX(p, wk + gp.workX * es) != hipSuccess) return fastKronInvalidArgument;
 
   const void* g = gZ;
   uint64_t gBatch = q.batch > 1 ? (uint64_t)q.M * q.L() : 0;
@@ -189,7 +201,7 @@ fastKronError Handle::gradBackward(const GradProblem& p, const void* gZ, void* s
     a.f_batch = p.perBatchF && q.batch > 1 ? (uint64_t)a.P * a.Q : 0;
     const char* in; uint64_t inBatch;
     if (lastStep) {
-      in = gp.copyX ? sv + gp.saveX * es : (const char*)p.X;
+      in = gp.copyX ? wk + gp.workX * es : (const char*)p.X;
       inBatch = q.batch > 1 ? (gp.copyX ? (gp.xBatch > 1 ? (uint64_t)q.M * Kin : 0) : p.strideX) : 0;
     } else {
       in = sv + gp.saveI[i + 1] * es;

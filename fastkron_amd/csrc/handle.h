@@ -90,6 +90,7 @@ class Handle {
   fastKronError gradSizes(const GradProblem& p, size_t* saveElems, size_t* workElems) const;
   fastKronError gradForward(const GradProblem& p, void* Z, void* save);
   fastKronError gradBackward(const GradProblem& p, const void* gZ, void* save, void* gX, void* const* gF, void* work);
+  hipError_t transposeX(const GradProblem& p, void* to);
 
   const std::string& lastPlan() const { return lastPlan_; }
   void setTunedDB(const char* path);

@@ -27,6 +27,12 @@ CASES = [
     ("mkm", 6, [(16, 8), (8, 16)], (), (4,), False, False),           # shared X, factors per entry
     ("kmm", 5, [(6, 6), (4, 4), (5, 5)], (2, 1), (3,), False, True),  # broadcast both ways
     ("mkm", 8, [(16, 16), (16, 16)], (2, 3), (2, 3), True, False),
+    ("mkm", 6, [(8, 3), (5, 5)], (3,), (), True, False),              # a transposed X larger than Z: read as it is stored
+    ("kmm", 6, [(8, 3), (5, 5)], (2,), (2,), True, True),
+    ("mkm", 9, [(20, 30)], (2,), (), True, False),                    # ... and in a single step
+    ("kmm", 9, [(20, 30)], (), (), True, False),
+    ("mkm", 6, [(3, 8), (5, 5)], (3,), (), True, False),              # ... copied to Z, batch folded into rows
+    ("kmm", 6, [(3, 8), (5, 5)], (2, 1), (3,), True, False),
 ]
 
 
@@ -216,3 +222,20 @@ def test_batches_of_gradients(xb, fb, mm, need):
     jacobian = lambda v: torch.autograd.functional.jacobian(at, tuple(t.detach() for t in w), vectorize=v)
     for a, b in zip(jacobian(True), jacobian(False)):
         assert a.shape == b.shape and rel(a, b.cpu()) <= BOUND["float64"]
+
+
+@pytest.mark.parametrize("mm", ["mkm", "kmm"])
+def test_a_transposed_x_is_not_kept_as_a_copy(mm):
+    """Between the passes a call holds its result and the steps' outputs, however X is stored."""
+    import torch
+    import fastkron_amd as fk
+
+    def held(transposed, n):
+        fs = [torch.randn(16, 16, device="cuda", requires_grad=True) for _ in range(n)]
+        rows, cols = (512, 16 ** n) if mm == "mkm" else (16 ** n, 512)
+        x = torch.randn(cols, rows, device="cuda").t() if transposed else torch.randn(rows, cols, device="cuda")
+        before = torch.cuda.memory_allocated()
+        z = fk.gemkm(x, fs) if mm == "mkm" else fk.gekmm(fs, x)
+        return torch.cuda.memory_allocated() - before
+    for n in (1, 3):
+        assert held(True, n) == held(False, n)
