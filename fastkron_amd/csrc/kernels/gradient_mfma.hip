@@ -235,8 +235,9 @@ void kron_grad_step_kernel(const GradStepArgs a) {
             else {
               const uint32_t pl = 16 * i + MF::perm(lo);
               const uint32_t p = p0 + pl < P ? p0 + pl : P - 1;
-              f = (T)0;                                    // (as in LDS: zero beyond Q, or an infinity there would count as 0 * inf)
-              if (q < Q) f = F[(int64_t)p * a.f_sp + (int64_t)q * a.f_sq];
+              // (as in LDS, zero beyond Q: an infinity in the last column would count as 0 * inf)
+              const T v = F[(int64_t)p * a.f_sp + (int64_t)(q < Q ? q : Q - 1) * a.f_sq];
+              f = FULL || q < Q ? v : (T)0;
             }
             ga[i] = MF::mma(f, xv, ga[i]);
           }
