@@ -252,8 +252,8 @@ fastKronError Handle::gradBackward(const GradProblem& p, const void* gZ, void* s
         c.vecOut = c.gin && c.in_p == 1 && c.P % 4 == 0 && aligned(c.gin, c.in_o, c.in_t, ginBatch);
         if (planOnly_) {
           char line[192];
-          const int n = snprintf(line, sizeof(line), "kernel=gradient_step lo=%d hi=%d rows=%u batch=%u in=%p g=%p gin=%p partial=%p\n", i, i, c.U,
-                                 c.batch, c.in, c.g, c.gin, c.partial);
+          const int n = snprintf(line, sizeof(line), "kernel=gradient_step lo=%d hi=%d rows=%u batch=%u sums=%u in=%p g=%p gin=%p partial=%p\n", i, i, c.U,
+                                 c.batch, c.gridX, c.in, c.g, c.gin, c.partial);
           launchLog_.append(line, n > 0 ? (size_t)n : 0);
         } else he = launchGradStep(c, p.dt, stream_);
       }

@@ -394,9 +394,17 @@ static hipError_t launchGradT(const GradStepArgs& a, uint32_t gridX, uint32_t gr
 uint32_t gradWorkgroups(uint32_t P, uint32_t Q, uint64_t U, uint32_t batch) {
   const uint64_t tiles = (U + 15) / 16, need = (tiles + kGradWaves - 1) / kGradWaves;
   const uint32_t big = P > Q ? P : Q;
-  uint64_t cap = big <= 32 ? 512 : 256;
   const uint64_t share = (uint64_t)batch * ((P + 63) / 64) * ((Q + 63) / 64);
-  cap = (cap + share - 1) / share;
+  uint64_t cap = 1;
+  if (big <= 32) {
+    if (share < 512) cap = 512 / share;
+  } else {
+    // The number for which the last round over 256 CUs is fullest, the smallest of equal ones, within four rounds.  Rounded up
+    // from 256 / blocks, 3x3 blocks had 261 workgroups, which took two rounds (forward pass and factor gradient alone, us:
+    // sgekmm 192x192 x 83333 484 -> 353, 96x192 x 83333 271 -> 191, 640x640 x 6250 367 -> 279).
+    for (uint64_t c = 1; c * share <= 1024; c++)
+      if ((c * share + 255) / 256 * cap < (cap * share + 255) / 256 * c) cap = c;
+  }
   return (uint32_t)(need < cap ? need : cap);
 }
 

@@ -641,3 +641,23 @@ def test_gradient_functions_launch_nothing_in_plan_only_mode(planner, mm, opX):
     lib.fastKronGetLastLaunches(h, buf, len(buf))
     assert [l.split()[0] for l in buf.value.decode().splitlines()] == ["kernel=gradient_step"] * 3 + ["kernel=gradient_sum"]
     assert lib.fastKronGradBackward(*args, None, ptr[2], ptr[4], gf, ptr[5]) != capi.SUCCESS
+
+
+@pytest.mark.parametrize("P,Q", [(96, 192), (192, 96), (192, 192), (384, 384), (640, 640), (100, 100), (512, 512), (64, 64), (33, 40), (2048, 128)])
+@pytest.mark.parametrize("batch", [1, 5])
+def test_the_last_round_of_the_backward_kernel_is_not_nearly_empty(planner, P, Q, batch):
+    """Workgroups of one launch for a factor's gradient (64x64 blocks of it, by partial sums, by batch entries) on 256 CUs, with
+    rows enough for any number of them: at most a quarter of the rounds' places stay empty."""
+    lib, h = planner
+    M = 2 ** 20
+    shape = (0, 0, M, 1, capi.arr_u32([P]), capi.arr_u32([Q]))
+    ptr = [ctypes.c_void_p(BASE + i * GAP) for i in range(8)]
+    one = lambda i: capi.arr_ptr([BASE + i * GAP])
+    assert lib.fastKronGradBackward(h, *shape, ptr[0], capi.OP_N, M * P, one(10), capi.OP_N, 1, batch, ptr[3], ptr[2], None, one(11),
+                                    ptr[5]) == capi.SUCCESS
+    buf = ctypes.create_string_buffer(1 << 14)
+    lib.fastKronGetLastLaunches(h, buf, len(buf))
+    step = dict(kv.split("=") for kv in buf.value.decode().splitlines()[0].split())
+    groups = int(step["sums"]) * -(-P // 64) * -(-Q // 64) * batch
+    rounds = -(-groups // 256)
+    assert groups >= 0.75 * 256 * rounds, (groups, rounds)
