@@ -30,7 +30,8 @@ EXPORTS = [
 
 EXT_EXPORTS = ["fastKronGetLastPlan", "fastKronSetTunedDB", "fastKronSetPlanOnly", "fastKronGetLastLaunches",
                "sgemkmStaticScratch", "fastKronGetSyncError", "fastKronSetSyncHelpAfter",
-               "fastKronProbeCopyPattern", "fastKronGradSizes", "fastKronGradForward", "fastKronGradBackward"]     # include/fastkron_ext.h
+               "fastKronProbeCopyPattern", "fastKronGradSizes", "fastKronGradForward", "fastKronGradBackward",
+               "fastKronGradBackwardSteps"]     # include/fastkron_ext.h
 
 _lib = None
 
@@ -100,6 +101,8 @@ def load():
     lib.fastKronGradForward.argtypes = [vp, cint, cint, u32, u32, u32p, u32p, vp, cint, u64, vpp, cint, cint, u32, vp, vp]
     lib.fastKronGradBackward.argtypes = [vp, cint, cint, u32, u32, u32p, u32p, vp, cint, u64, vpp, cint, cint, u32, vp, vp,
                                          vp, vpp, vp]
+    lib.fastKronGradBackwardSteps.argtypes = [vp, cint, cint, u32, u32, u32p, u32p, vp, cint, u64, vpp, cint, cint, u32, u32, u32, vp, vp,
+                                              vp, vpp, vp]
     lib.fastKronSetPlanOnly.argtypes = [vp, cint]
     lib.fastKronGetLastLaunches.argtypes = [vp, ctypes.c_char_p, ctypes.c_size_t]
     lib.fastKronGetLastLaunches.restype = ctypes.c_size_t

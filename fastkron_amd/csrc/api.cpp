@@ -316,9 +316,18 @@ fastKronError fastKronGradBackward(fastKronHandle handle, int mkm, int dbl, uint
                                    const uint32_t Qs[], const void* X, fastKronOp opX, uint64_t strideX, const void* const Fs[],
                                    fastKronOp opFs, int perBatchFs, uint32_t batchCount, const void* gZ, void* save, void* gX,
                                    void* const gFs[], void* work) {
+  if (N == 0) return fastKronInvalidKMMProblem;
+  return fastKronGradBackwardSteps(handle, mkm, dbl, M, N, Ps, Qs, X, opX, strideX, Fs, opFs, perBatchFs, batchCount, 0, N - 1, gZ, save, gX,
+                                   gFs, work);
+}
+
+fastKronError fastKronGradBackwardSteps(fastKronHandle handle, int mkm, int dbl, uint32_t M, uint32_t N, const uint32_t Ps[],
+                                        const uint32_t Qs[], const void* X, fastKronOp opX, uint64_t strideX, const void* const Fs[],
+                                        fastKronOp opFs, int perBatchFs, uint32_t batchCount, uint32_t first, uint32_t last,
+                                        const void* gOut, void* save, void* gIn, void* const gFs[], void* work) {
   if (!handle) return fastKronInvalidArgument;
-  return H(handle)->gradBackward(gradProblem(mkm, dbl, M, N, Ps, Qs, X, opX, strideX, Fs, opFs, perBatchFs, batchCount), gZ,
-                                 save, gX, gFs, work);
+  return H(handle)->gradBackward(gradProblem(mkm, dbl, M, N, Ps, Qs, X, opX, strideX, Fs, opFs, perBatchFs, batchCount), first, last, gOut,
+                                 save, gIn, gFs, work);
 }
 
 }  // extern "C"

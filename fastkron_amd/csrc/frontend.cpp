@@ -38,7 +38,7 @@ struct Api {
   decltype(&sgemkmStridedBatched) sgemkmB; decltype(&dgemkmStridedBatched) dgemkmB;
   decltype(&sgekmmStridedBatched) sgekmmB; decltype(&dgekmmStridedBatched) dgekmmB;
   decltype(&gekmmSizes) sizes; decltype(&fastKronSetStream) setStream;
-  decltype(&fastKronGradSizes) gradSizes; decltype(&fastKronGradForward) gradForward; decltype(&fastKronGradBackward) gradBackward;
+  decltype(&fastKronGradSizes) gradSizes; decltype(&fastKronGradForward) gradForward; decltype(&fastKronGradBackwardSteps) gradSteps;
 } api;
 
 int64_t prod(at::IntArrayRef d) { int64_t n = 1; for (int64_t v : d) n *= v; return n; }
@@ -332,6 +332,38 @@ PyObject* gradForward(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
   END_HANDLE_TH_ERRORS
 }
 
+// Where the gradient of a step's input is PyTorch's product instead of the library's backward kernel, which takes 64 rows of
+// the factor per workgroup with all of Q contracted in one chain of loads, reads the gradient again for every 64 rows, and has
+// one workgroup per CU (or the factor in memory, from Q = 273 in fp64 on) for wide factors.  Measured, the launch alone
+// against the product with its copies and its host time, of which some 10 us are the share of a call from here, in us:
+//   Q > 384 (fp64 272): 64x4096, 15 rows fp32 485 / 26, 16x1024, 3906 columns 79 / 34, 1024x1024, 3906 rows fp32 555 / 64 and
+//   244 rows fp64 203 / 34, 512x512, 122 columns fp32 37 / 32, 64x512, 122 rows 59 / 33 (the smallest measured);
+//   otherwise P or Q above 128 from 2^27 multiply-adds on: 256x256, 15625 columns fp32 70 / 34, 224x224, 17857 rows fp32
+//   94 / 28, 160x160, 12500 rows fp64 84 / 24; below, the kernel: 384x384, 162 columns fp32 16 / 31, 256x256, 1953 columns
+//   fp32 11 / 34, 160x160, 3125 rows 26 / 25, 224x224, 1116 columns fp64 33 / 21.
+// Up to 128 the kernel's launches for both gradients are never behind in all.  The gradient of the factor is the kernel's
+// everywhere, also where the product is up to 1.5 times faster (512x512 and more, fp32 columns): its sums are 2 to 7 times
+// closer to 64-bit ones.
+bool wideStep(const Operands& o, uint32_t i, int64_t rows) {
+  const int64_t P = o.Ps[i], Q = o.Qs[i];
+  return std::max(P, Q) > 128 && (Q > (o.f64() ? 272 : 384) || (double)rows * P * Q >= 134217728.0);
+}
+
+// The gradient of the input of step i (S slices of P): g M x (Q, S) -> M x (S, P) for MKM, (Q, S) x M -> (S, P) x M for KMM.
+Tensor wideInputGradient(const Operands& o, const GradOperands& gr, uint32_t i, int64_t S, const Tensor& g) {
+  const int64_t P = o.Ps[i], Q = o.Qs[i], M = o.M, nb = gr.nb;
+  const bool pMajor = o.mkm == (o.opF == fastKronOp_N);                  // stored P x Q, else Q x P
+  const Tensor f = gr.perBatch ? (pMajor ? o.f[i].view({nb, P, Q}).mT() : o.f[i].view({nb, Q, P}))           // Q x P
+                               : (pMajor ? o.f[i].view({P, Q}).t() : o.f[i].view({Q, P}));
+  if (o.mkm || M == 1) {
+    const Tensor a = g.view({nb, M, Q, S}).transpose(2, 3);
+    return gr.perBatch ? at::bmm(a.reshape({nb, M * S, Q}), f) : at::mm(a.reshape({nb * M * S, Q}), f);
+  }
+  const Tensor a = g.view({nb, Q, S * M});
+  const Tensor r = gr.perBatch || nb > 1 ? at::bmm(gr.perBatch ? f.mT() : f.t().expand({nb, P, Q}), a) : at::mm(f.t(), a[0]);
+  return r.view({nb, P, S, M}).transpose(1, 2).contiguous();
+}
+
 // grad_backward(handle, stream, mkm, x, fs, opX, opF, grad of z, kept, need x, need fs) -> (grad of x, of every factor)
 PyObject* gradBackward(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
   HANDLE_TH_ERRORS
@@ -367,7 +399,6 @@ PyObject* gradBackward(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
   void* gfp[kMaxFactors];
   Dims xs = o.zb;
   xs.push_back(mkm ? o.M : o.K); xs.push_back(mkm ? o.K : o.M);
-  if (needX) gx = at::empty(xs, o.x.options());
   for (uint32_t i = 0; i < o.N; i++) {
     gfp[i] = nullptr;
     if (!needF(i)) continue;
@@ -377,14 +408,36 @@ PyObject* gradBackward(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
     gfp[i] = gf[i].data_ptr();
   }
   const Tensor scratch = at::empty({(int64_t)work}, o.x.options());
-  {
+  auto steps = [&](uint32_t first, uint32_t last, const Tensor& gOut, const Tensor& gIn) {
     LibraryCall unlocked;
-    e = api.setStream(c.handle, fastKronBackend_HIP, &c.stream);
-    if (e == fastKronSuccess)
-      e = api.gradBackward(c.handle, mkm, o.f64(), (uint32_t)o.M, o.N, o.Ps, o.Qs, o.x.data_ptr(), o.opX, g.strideX, g.f, o.opF, g.perBatch,
-                           (uint32_t)g.nb, gz.data_ptr(), kept.data_ptr(), needX ? gx.data_ptr() : nullptr, gfp, scratch.data_ptr());
+    fastKronError r = api.setStream(c.handle, fastKronBackend_HIP, &c.stream);
+    if (r == fastKronSuccess)
+      r = api.gradSteps(c.handle, mkm, o.f64(), (uint32_t)o.M, o.N, o.Ps, o.Qs, o.x.data_ptr(), o.opX, g.strideX, g.f, o.opF, g.perBatch,
+                        (uint32_t)g.nb, first, last, gOut.data_ptr(), kept.data_ptr(), gIn.defined() ? gIn.data_ptr() : nullptr, gfp, scratch.data_ptr());
+    return r;
+  };
+  // columns behind step i, and whether the gradient of its input is needed
+  int64_t cols = o.L;
+  uint32_t lastWanted = 0;
+  for (uint32_t i = 0; i < o.N; i++) if (gfp[i]) lastWanted = i;
+  auto inputWanted = [&](uint32_t i) { return i + 1 == o.N ? needX : i < lastWanted || needX; };
+  auto wide = [&](uint32_t i, int64_t k) { return inputWanted(i) && wideStep(o, i, g.nb * o.M * (k / o.Qs[i])); };
+  Tensor gNow = gz;
+  for (uint32_t i = 0; i < o.N && (i <= lastWanted || needX);) {
+    uint32_t last = i;
+    int64_t k = cols / o.Qs[i] * o.Ps[i];                                // columns of the input of step `last`
+    const bool product = wide(i, cols);
+    if (!product) for (; last + 1 < o.N && !wide(last + 1, k); last++) k = k / o.Qs[last + 1] * o.Ps[last + 1];
+    Tensor gIn;
+    if (!product && inputWanted(last)) {
+      gIn = last + 1 == o.N ? at::empty(xs, o.x.options()) : at::empty({g.nb * o.M * k}, o.x.options());
+    }
+    e = steps(i, last, gNow, gIn);
+    if (e != fastKronSuccess) return failed(e);
+    if (product) gIn = wideInputGradient(o, g, i, cols / o.Qs[i], gNow);
+    gNow = gIn; cols = k; i = last + 1;
   }
-  if (e != fastKronSuccess) return failed(e);
+  if (needX) gx = gNow.view(xs);
   PyObject* out = PyTuple_New(1 + (Py_ssize_t)o.N);
   if (!out) return nullptr;
   auto put = [&](Py_ssize_t at, Tensor t) {

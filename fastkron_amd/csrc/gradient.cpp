@@ -162,8 +162,9 @@ fastKronError Handle::gradForward(const GradProblem& p, void* Z, void* save) {
   return runOnline(q, nullptr, nullptr, nullptr);
 }
 
-fastKronError Handle::gradBackward(const GradProblem& p, const void* gZ, void* save, void* gX, void* const* gF, void* work) {
-  if (!gZ || !p.X || !p.F || !gF) return fastKronInvalidArgument;
+fastKronError Handle::gradBackward(const GradProblem& p, uint32_t first, uint32_t last, const void* gOut, void* save, void* gIn, void* const* gF,
+                                   void* work) {
+  if (!gOut || !p.X || !p.F || !gF || first > last || last >= p.N) return fastKronInvalidArgument;
   for (uint32_t i = 0; i < p.N; i++) if (!p.F[i]) return fastKronInvalidKMMProblem;
   GradPlan gp;
   fastKronError e = makePlan(p, &gp);
@@ -178,19 +179,19 @@ fastKronError Handle::gradBackward(const GradProblem& p, const void* gZ, void* s
   char* sv = (char*)save;
   char* wk = (char*)work;
   const bool mkm = q.mm == MMType::MKM;
-  // the last factor (in chain order) whose gradient is wanted: nothing behind it is computed unless gX is
+  // the last factor (in chain order) whose gradient is wanted: nothing behind it is computed unless gIn is
   int lastWanted = -1;
-  bool wanted[kMaxFactors];
-  for (uint32_t g = 0; g < q.N; g++) {
+  bool wanted[kMaxFactors] = {};
+  for (uint32_t g = first; g <= last; g++) {
     wanted[g] = gF[g] != nullptr;
     if (wanted[g]) lastWanted = (int)g;
   }
-  if (gX) lastWanted = (int)q.N - 1;
+  if (gIn) lastWanted = (int)last;
   if (gp.copyX && wanted[q.N - 1] && !planOnly_ && transposeX(p, wk + gp.workX * es) != hipSuccess) return fastKronInvalidArgument;
 
-  const void* g = gZ;
-  uint64_t gBatch = q.batch > 1 ? (uint64_t)q.M * q.L() : 0;
-  for (int i = 0; i <= lastWanted; i++) {
+  const void* g = gOut;
+  uint64_t gBatch = q.batch > 1 ? (uint64_t)q.M * q.colsAfter(first) : 0;
+  for (int i = (int)first; i <= lastWanted; i++) {
     const uint64_t Kin = q.colsBefore(i), S = Kin / q.P[i];
     const bool lastStep = i + 1 == (int)q.N;
     GradStepArgs a{};
@@ -208,7 +209,7 @@ fastKronError Handle::gradBackward(const GradProblem& p, const void* gZ, void* s
       inBatch = (uint64_t)q.M * Kin;
     }
     void* gin = nullptr;
-    if (lastStep) gin = gX;
+    if (i == (int)last) gin = gIn;
     else if (i < lastWanted) gin = wk + gp.workG[i & 1] * es;
     const uint64_t ginBatch = (uint64_t)q.M * Kin;
     if (mkm) {
@@ -280,7 +281,7 @@ fastKronError Handle::gradBackward(const GradProblem& p, const void* gZ, void* s
     ra.count = 0;
     return hipSuccess;
   };
-  for (int i = 0; i <= lastWanted; i++) {
+  for (int i = (int)first; i <= lastWanted; i++) {
     if (!wanted[i]) continue;
     GradReduce& r = ra.r[ra.count++];
     r.P = q.P[i]; r.Q = q.Q[i];

@@ -89,7 +89,8 @@ class Handle {
   };
   fastKronError gradSizes(const GradProblem& p, size_t* saveElems, size_t* workElems) const;
   fastKronError gradForward(const GradProblem& p, void* Z, void* save);
-  fastKronError gradBackward(const GradProblem& p, const void* gZ, void* save, void* gX, void* const* gF, void* work);
+  // the steps of the factors first .. last: from the gradient of the first one's output to that of the last one's input
+  fastKronError gradBackward(const GradProblem& p, uint32_t first, uint32_t last, const void* gOut, void* save, void* gIn, void* const* gF, void* work);
   hipError_t transposeX(const GradProblem& p, void* to);
 
   const std::string& lastPlan() const { return lastPlan_; }

@@ -44,7 +44,7 @@ def _load_native():
     lib = capi.load()
     names = ["sgemkm", "dgemkm", "sgekmm", "dgekmm", "sgemkmStridedBatched", "dgemkmStridedBatched", "sgekmmStridedBatched",
              "dgekmmStridedBatched", "gekmmSizes", "fastKronSetStream", "fastKronGradSizes", "fastKronGradForward",
-             "fastKronGradBackward"]                      # the order of csrc/frontend.cpp
+             "fastKronGradBackwardSteps"]                 # the order of csrc/frontend.cpp
     m.use(tuple(ctypes.cast(getattr(lib, n), ctypes.c_void_p).value for n in names))
     return m
 

@@ -103,6 +103,17 @@ fastKronError fastKronGradBackward(fastKronHandle handle, int mkm, int dbl, uint
                                    const uint32_t Qs[], const void* X, fastKronOp opX, uint64_t strideX, const void* const Fs[],
                                    fastKronOp opFs, int perBatchFs, uint32_t batchCount, const void* gZ, void* save, void* gX,
                                    void* const gFs[], void* work);
+/*
+ * A part of the backward pass, for callers that compute the gradient of some step's input by a product of their own: the
+ * steps of the factors first .. last (fastKronGradBackward: 0 .. N-1).  gOut is the gradient of the output of the step of
+ * factor `first` (gZ for 0), gIn receives the gradient of the input of the step of factor `last` (gX for N-1) unless it is
+ * NULL; both are M x columns (MKM) or columns x M (KMM), batch entries one after the other.  Entries of gFs outside the
+ * range are not looked at.
+ */
+fastKronError fastKronGradBackwardSteps(fastKronHandle handle, int mkm, int dbl, uint32_t M, uint32_t N, const uint32_t Ps[],
+                                        const uint32_t Qs[], const void* X, fastKronOp opX, uint64_t strideX, const void* const Fs[],
+                                        fastKronOp opFs, int perBatchFs, uint32_t batchCount, uint32_t first, uint32_t last,
+                                        const void* gOut, void* save, void* gIn, void* const gFs[], void* work);
 
 #ifdef __cplusplus
 }

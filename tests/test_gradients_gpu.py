@@ -33,6 +33,16 @@ CASES = [
     ("kmm", 9, [(20, 30)], (), (), True, False),
     ("mkm", 6, [(3, 8), (5, 5)], (3,), (), True, False),              # ... copied to Z, batch folded into rows
     ("kmm", 6, [(3, 8), (5, 5)], (2, 1), (3,), True, False),
+    # steps whose input's gradient is a product of PyTorch's, alone, in front of, behind and between steps that are not
+    ("mkm", 5, [(130, 400)], (), (), False, True),
+    ("kmm", 5, [(40, 400)], (), (), False, False),
+    ("mkm", 3, [(4, 390), (3, 5)], (), (), False, False),
+    ("kmm", 3, [(3, 5), (4, 390)], (), (), False, True),
+    ("mkm", 2, [(2, 3), (5, 387), (3, 2)], (2,), (), True, False),
+    ("kmm", 2, [(2, 3), (5, 387), (3, 2)], (2,), (), False, False),
+    ("kmm", 2, [(3, 385), (2, 385)], (), (2,), False, True),
+    ("mkm", 3, [(7, 385), (2, 2)], (2, 1), (3,), False, False),
+    ("kmm", 1, [(7, 385), (2, 2)], (3,), (), False, False),
 ]
 
 
