@@ -47,8 +47,7 @@ __global__ __launch_bounds__(kGenThreads) void kron_step_generic(const StepArgs 
     __syncthreads();
   };
   if constexpr (AHEAD) {
-    // few waves: eight elements of X in registers ahead of their products, the first eight ahead of the factor's (one
-    // load, one product after the other is one round trip to memory per element)
+    // eight elements of X in registers ahead of their products, the first eight ahead of the factor's
     constexpr int LU = 8;
     T x[LU];
     auto loadX = [&](uint32_t p) {
@@ -118,10 +117,17 @@ static hipError_t launchGenericT(const StepArgs& a, hipStream_t stream) {
   const uint32_t qTiles = (Q + tq - 1) / tq;
   if (tiles * qTiles >= (1ull << 31) || a.batch > 65535) return hipErrorInvalidValue;
   dim3 grid((uint32_t)(tiles * qTiles), 1, a.batch), block(kGenThreads);
-  // Up to four workgroups per CU the loads run ahead (kmm 16 x 16^3 fp64, the single step 9.4 -> about 5 us; 200 x 129 fp64
-  // 21.9 -> 15.0; 100 x 7^5 fp32, 938 workgroups, 37.0 -> 34.8); beyond, the waves of a CU hide each other's round trips and
-  // the plain loop is ahead (27^3 x 21, batch of 10, 1200 workgroups, 40.5 against 42.3 us).
-  const bool ahead = tiles * qTiles * a.batch < 1024;
+  // Loads ahead of the products, up to four workgroups per CU: for short rows, where the first eight leave before the factor
+  // is staged (sgekmm 7^5 x 100 37.0 -> 34.7 us, 17^3 x 200 27.5 -> 24.8, 3^8 x 50 34.3 -> 30.0), and in the KMM layout where
+  // a load takes long: few columns and with them many short pieces (21^3 x 25, batch of 5, 29.0 -> 24.7), or an X of more
+  // than an XCD's L2 has left (dgekmm 129^2 x 60 76 -> 61, 257x40 x 30000 70 -> 55, 300^2 x 7 140 -> 101; with few output
+  // columns per thread, whose products hide little, beyond 32 MB, 512x1 x 30000 57 -> 47).  Elsewhere rows of more than 32
+  // elements run into the staging of the next 32 with nothing gained and the plain loop is ahead (1000x3, one row, 42 us
+  // against 84, 2048x2048, 7 rows, 212 / 316, dgemkm 40x3^3 x 30 20.8 / 24.3), and so it is on full devices, where the waves
+  // of a CU hide each other's round trips (27^3 x 21, batch of 10, 1200 workgroups, 40.5 / 42.3).
+  const uint32_t P = a.p[0];
+  const uint64_t wgs = tiles * qTiles * a.batch, xBytes = (uint64_t)a.M * a.Kin * a.batch * sizeof(T);
+  const bool ahead = wgs < 1024 && (P <= 20 || (LANES_M && (P <= 32 ? a.M < 128 && S > 1 : xBytes >= (tq >= 8 ? 2400000u : 32000000u))));
 #define GEN_LAUNCH(TQ) \
   if (ahead) hipLaunchKernelGGL((kron_step_generic<T, TQ, LANES_M, true>), grid, block, 0, stream, a, qTiles); \
   else       hipLaunchKernelGGL((kron_step_generic<T, TQ, LANES_M, false>), grid, block, 0, stream, a, qTiles);

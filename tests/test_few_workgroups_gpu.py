@@ -54,3 +54,17 @@ def test_plain_step(fk, P, Q, dt):
             assert any(k == plain for _, _, k in fk.last_plan()), fk.last_plan()
     finally:
         fk.set_options(fusion=True)
+
+
+@pytest.mark.parametrize("dt", [np.float32, np.float64], ids=["f", "d"])
+@pytest.mark.parametrize("M,P,Q", [(70000, 33, 16), (70000, 65, 9), (70000, 129, 17), (8, 260, 300), (70000, 16, 17), (3, 1000, 3)])
+def test_plain_step_on_either_side_of_the_rule_for_loads_ahead(fk, M, P, Q, dt):
+    """Rows of more than one staged piece of 32 with the loads ahead (from 256 workgroups on) and without; TOL as above, the
+    sums have at most 1000 terms: sqrt(1000) * u = 1.9e-6."""
+    fk.set_options(fusion=False)
+    try:
+        check(fk, ko.KMM, M, [P], [Q], dt, 7, alpha=1.5, beta=0.5)
+        if M < 100:
+            check(fk, ko.MKM, M, [P], [Q], dt, 8, batch=2)
+    finally:
+        fk.set_options(fusion=True)
