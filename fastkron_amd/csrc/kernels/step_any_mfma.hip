@@ -91,12 +91,14 @@ __global__ __launch_bounds__(kSaThreads, 2) void kron_step_any_kernel(const Step
   auto stageFactor = [&]() {
     const T* F = (const T*)a.f[0] + (size_t)bt * a.f_batch[0];
     const uint32_t perK = g.pcPad * Qp;                // rows pc .. pcPad-1 of a lane group are zero
-    // eight loads of a thread go out before the first LDS write waits for one: a loop of load, wait, write would
+    // several loads of a thread go out before the first LDS write waits for one: a loop of load, wait, write would
     // put one memory round trip per element of a thread in front of the first product.  Divisions by multiplication, and the
     // first tile's loads ahead: on short launches the indexes and the tile's round trip cost as much as the products (two
     // steps each: 1003 x 31x63^2 fp32 23.1 -> 20.6 us, 100 rows 15.0 -> 12.4, dgekmm 20^2 x 50 13.0 -> 10.5; 3000 x 24x48^2
     // 31.2 -> 27.5).
-    constexpr int kBatch = 8;
+    // Four loads of a thread for the narrow forms: with eight beside the first tile they took 74 to 93 registers instead of 54
+    // to 75, two or three workgroups per CU instead of three or four (dgemkm 9 x 12535 x 16x13^2 190 -> 240 us).
+    constexpr int kBatch = PCMAX <= 16 ? 4 : 8;
     for (uint32_t base = 0; base < 4 * perK; base += kBatch * kSaThreads) {
       T v[kBatch];
       uint32_t dst[kBatch];

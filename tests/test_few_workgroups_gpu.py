@@ -68,3 +68,13 @@ def test_plain_step_on_either_side_of_the_rule_for_loads_ahead(fk, M, P, Q, dt):
             check(fk, ko.MKM, M, [P], [Q], dt, 8, batch=2)
     finally:
         fk.set_options(fusion=True)
+
+
+@pytest.mark.parametrize("dt", [np.float32, np.float64], ids=["f", "d"])
+@pytest.mark.parametrize("P,Q", [(12, 13), (16, 400), (33, 90), (64, 300), (65, 16), (128, 70), (129, 33), (200, 13), (256, 512)])
+def test_padded_step_stages_its_factor_in_any_number_of_batches(fk, P, Q, dt):
+    """Factors of one and of many batches of staged elements, the first tile's loads ahead of them and behind, fewer tiles than
+    waves and more; sums of at most 256 terms, sqrt(256) * u = 1e-6."""
+    for mm, M in [(ko.MKM, 3), (ko.KMM, 3), (ko.KMM, 40), (ko.KMM, 3000 if P * Q < 20000 else 300), (ko.MKM, 700 if P * Q < 20000 else 50)]:
+        check(fk, mm, M, [P], [Q], dt, 9, alpha=1.5, beta=0.5)
+        check(fk, mm, M, [P], [Q], dt, 10, batch=2, opX=ko.OP_T, opFs=ko.OP_T)
