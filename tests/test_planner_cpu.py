@@ -467,7 +467,8 @@ def test_whole_rows_of_small_square_factors_run_in_place(online_planner):
     assert blocks("s", 3, [5] * 7) == 15 and blocks("d", 3, [5] * 8) == 75 and blocks("s", 2, [6] * 6) == 12
     assert blocks("s", 1, [7] * 6) == 7 and blocks("s", 2, [9, 2] + [3] * 8) == 36 and blocks("s", 9, [5] * 7, beta=0.5, y_is_z=True) == 45
     assert blocks("s", 3, [3] * 11) is None and blocks("s", 3, [64] + [5] * 3) is None      # three leading ones; short blocks
-    assert blocks("d", 15, [6] * 6) is None and blocks("d", 16, [6] * 6) == 96
+    assert blocks("d", 34, [6] * 6) is None and blocks("d", 35, [6] * 6) == 210      # (the measured crossing)
+    assert blocks("d", 13, [7] * 6) is None and blocks("d", 14, [7] * 6) == 98 and blocks("d", 32, [2, 2] + [6] * 5) is None
     assert blocks("s", 3, [5] * 7, batch=2) is None and blocks("s", 3, [5] * 7, batch=2, strideF=[0] * 7) == 15
 
 
