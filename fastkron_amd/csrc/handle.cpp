@@ -566,7 +566,6 @@ bool Handle::mergeSmallFactors(const KronProblem& p, KronProblem* out, const Cal
 
   const bool pMajor = (p.mm == MMType::MKM) == (p.opF == fastKronOp_N);   // as in makeStepArgs
   MergeArgs ma{};
-  ma.batch = 1;
   KronProblem q = p;
   q.N = ng;
   size_t wsOff = 0;

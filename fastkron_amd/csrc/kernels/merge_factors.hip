@@ -20,16 +20,15 @@ __global__ __launch_bounds__(256) void kron_merge_kernel(const MergeArgs a) {
   const MergeGroup g = a.g[blockIdx.x];
   uint32_t P = 1, Q = 1;
   for (uint32_t j = 0; j < g.count; j++) { P *= g.p[j]; Q *= g.q[j]; }
-  const uint32_t b = blockIdx.y;
-  T* dst = (T*)g.dst + (size_t)b * P * Q;
-  for (uint32_t e = blockIdx.z * 256 + threadIdx.x; e < P * Q; e += gridDim.z * 256) {
+  T* dst = (T*)g.dst;
+  for (uint32_t e = blockIdx.y * 256 + threadIdx.x; e < P * Q; e += gridDim.y * 256) {
     uint32_t p = e / Q, q = e % Q;
     const uint32_t p0 = p, q0 = q;
     T v = (T)1;
     for (int j = (int)g.count - 1; j >= 0; j--) {          // the last source owns the fastest digit
       const uint32_t pj = p % g.p[j], qj = q % g.q[j];
       p /= g.p[j]; q /= g.q[j];
-      v *= ((const T*)g.src[j])[(int64_t)b * (g.p[j] * g.q[j]) + (int64_t)pj * g.sp[j] + (int64_t)qj * g.sq[j]];
+      v *= ((const T*)g.src[j])[(int64_t)pj * g.sp[j] + (int64_t)qj * g.sq[j]];
     }
     dst[(int64_t)p0 * g.dsp + (int64_t)q0 * g.dsq] = v;
   }
@@ -56,7 +55,7 @@ hipError_t launchFill(void* dst, size_t elems, DType dt, hipStream_t stream) {
 }
 
 hipError_t launchMergeFactors(const MergeArgs& a, DType dt, hipStream_t stream) {
-  if (a.groups == 0 || a.groups > kMaxMergeGroups || a.batch == 0 || a.batch > 65535) return hipErrorInvalidValue;
+  if (a.groups == 0 || a.groups > kMaxMergeGroups) return hipErrorInvalidValue;
   // 256 entries per workgroup (in one workgroup, the 16 rounds of a 64x64 product took 22 us)
   uint32_t widest = 1;
   for (uint32_t i = 0; i < a.groups; i++) {
@@ -64,7 +63,7 @@ hipError_t launchMergeFactors(const MergeArgs& a, DType dt, hipStream_t stream) 
     for (uint32_t j = 0; j < a.g[i].count; j++) n *= a.g[i].p[j] * a.g[i].q[j];
     if (n > widest) widest = n;
   }
-  const dim3 grid(a.groups, a.batch, (widest + 255) / 256);
+  const dim3 grid(a.groups, (widest + 255) / 256);
   if (dt == DType::F32) hipLaunchKernelGGL(kron_merge_kernel<float>, grid, dim3(256), 0, stream, a);
   else                  hipLaunchKernelGGL(kron_merge_kernel<double>, grid, dim3(256), 0, stream, a);
   return hipGetLastError();

@@ -104,7 +104,6 @@ struct MergeGroup {
 struct MergeArgs {
   MergeGroup g[kMaxMergeGroups];
   uint32_t groups;
-  uint32_t batch;                      // > 1: sources and products per batch entry, one after the other (P*Q elements apart)
 };
 
 }  // namespace fk
