@@ -18,8 +18,20 @@ CASES = [
     (1100, [3, 3]),          # several rows per workgroup, last one not full
     (2051, [5, 5, 5]), (1031, [7, 7]), (1029, [2, 2, 2, 2, 2]), (4111, [6, 2]), (1057, [4, 4, 4]),
     (13, [8, 8, 8]), (9, [8] * 4), (4, [2, 3, 5, 7, 8]), (3, [8, 7, 5, 3, 2]), (2, [4, 4, 8, 3, 3, 3, 3]),
-    (2, [2, 3, 4, 5, 6, 7, 8]),      # 40320 columns: a whole CU's LDS in fp32
+    (2, [2, 3, 4, 5, 6, 7, 8]),      # few long rows in passes of one digit: not in place
+    (96, [2, 3, 4, 5, 6, 7, 8]), (96, [3, 4, 5, 6, 7, 8]),      # 161280 bytes, a whole CU's LDS, in fp32 and in fp64
+    (96, [7] * 5), (33, [4, 4, 8, 3, 3, 3, 3]),
 ]
+
+
+def runs_in_place(M, Ps, dt, batch, own_factors):
+    """Which calls the kernel is meant for: rows that fit, not few long ones in passes of one digit, and no neighbours that
+    are merged into a larger factor instead (which factors of one batch entry only are not)."""
+    bytes_ = int(np.prod(Ps)) * np.dtype(dt).itemsize
+    one_digit = len(set(Ps)) > 1 or (dt is np.float64 and Ps[-1] >= 6)
+    merged = (2, 4) if dt is np.float32 else (2, 4, 8)
+    return (bytes_ + 16 <= 160 * 1024 and not (one_digit and bytes_ > 65536 and M * batch < 96) and
+            (own_factors or not any(a in merged and b in merged for a, b in zip(Ps, Ps[1:]))))
 
 
 @pytest.fixture(scope="module")
@@ -34,13 +46,16 @@ def fk():
 @pytest.mark.parametrize("M,Ps", CASES, ids=lambda v: str(v) if isinstance(v, int) else "x".join(map(str, v)))
 def test_small_factors_in_place(fk, M, Ps, dt):
     for seed, kw in enumerate([dict(alpha=1.5, beta=0.5), dict(alpha=1.0, beta=0.0, opFs=ko.OP_T),
-                               dict(alpha=1.0, beta=0.0, batch=3), dict(alpha=-2.0, beta=1.0, batch=2, share_f=True)]):
+                               dict(alpha=1.0, beta=0.0, batch=3), dict(alpha=-2.0, beta=1.0, batch=2, share_f=True),
+                               dict(alpha=1.5, beta=0.5, batch=3)]):
         alpha, beta = kw.pop("alpha"), kw.pop("beta")
         batch, share = kw.get("batch", 1), dict(share_f=True) if kw.get("share_f") else {}
         X, Fs, Y = make_case(ko.MKM, M, Ps, Ps, dt, seed=7 + 50 * seed, with_y=beta != 0.0, batch=batch, **share)
         want = oracle_answer(ko.MKM, M, Ps, Ps, X, Fs, Y, alpha, beta, **kw)
         got, e = run_gpu(fk, ko.MKM, M, Ps, Ps, X, Fs, Y, alpha, beta, **kw)
         assert e == 0 and normwise(got, want) <= TOL[dt], (fk.last_plan(), kw)
+        in_place = len(fk.last_plan()) == 1 and "inplace" in fk.last_plan()[0][2]
+        assert in_place == runs_in_place(M, Ps, dt, batch, batch > 1 and not share), (fk.last_plan(), kw)
 
 
 @pytest.mark.parametrize("dt", [np.float32, np.float64], ids=["f", "d"])
@@ -48,7 +63,7 @@ def test_small_factors_in_place(fk, M, Ps, dt):
                          ids=lambda v: str(v) if isinstance(v, int) else "x".join(map(str, v)))
 def test_rows_beyond_the_lds_run_their_trailing_factors_in_place(fk, M, Ps, dt):
     """A two-part plan: blocks of 3^8, 5^6, 6^5 or 7^5 columns in place, the leading factors across the blocks."""
-    few_long_rows = dt is np.float64 and Ps[-1] >= 6 and M < 20       # (fewer than 96 blocks in passes of one digit)
+    few_long_rows = dt is np.float64 and Ps[-1] >= 6 and M < 20       # (few blocks in passes of one digit)
     for seed, kw in enumerate([dict(alpha=1.5, beta=0.5), dict(alpha=1.0, beta=0.0, opFs=ko.OP_T, batch=2, share_f=True)]):
         alpha, beta = kw.pop("alpha"), kw.pop("beta")
         batch, share = kw.get("batch", 1), dict(share_f=True) if kw.get("share_f") else {}
