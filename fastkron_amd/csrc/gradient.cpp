@@ -136,13 +136,17 @@ fastKronError Handle::gradForward(const GradProblem& p, void* Z, void* save) {
   KronProblem q = gp.q;
   q.X = p.X; q.strideX = q.batch > 1 ? p.strideX : 0;
   if (gp.copyX) {
-    if (q.N > 1 && (uint64_t)gp.xBatch * p.M * q.K() <= (uint64_t)q.batch * q.M * q.L()) {
+    // (a first factor beyond the padded step, which the plain kernel runs, is ahead on X as it is stored in the MKM layout: its
+    // lanes then lie along neighbours, sgemkm 200 x 320x320^2 with all gradients 2.7 ms against 3.8; in the KMM layout they
+    // do so on the copy, sgekmm 8x8 (x) 300x300 x 4166 0.78 against 1.02)
+    const bool plainFirst = q.mm == MMType::MKM && (q.P[q.N - 1] > 256 || q.Q[q.N - 1] > 512);
+    if (q.N > 1 && !plainFirst && (uint64_t)gp.xBatch * p.M * q.K() <= (uint64_t)q.batch * q.M * q.L()) {
       // the copy stands in Z, which only the last of the launches writes
       if (!planOnly_ && transposeX(p, Z) != hipSuccess) return fastKronInvalidArgument;
       q.X = Z; q.strideX = q.batch > 1 && gp.xBatch > 1 ? (uint64_t)p.M * q.K() : 0;
       q.xJustWritten = true;
     } else {
-      // no room for it: the first launch reads X as it is stored (entry by entry: not as rows of one problem)
+      // the first launch reads X as it is stored (entry by entry: not as rows of one problem)
       q.M = p.M; q.batch = p.batch;
       q.opX = fastKronOp_T; q.strideX = q.batch > 1 ? p.strideX : 0;
     }

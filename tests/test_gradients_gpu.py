@@ -33,6 +33,8 @@ CASES = [
     ("kmm", 9, [(20, 30)], (), (), True, False),
     ("mkm", 6, [(3, 8), (5, 5)], (3,), (), True, False),              # ... copied to Z, batch folded into rows
     ("kmm", 6, [(3, 8), (5, 5)], (2, 1), (3,), True, False),
+    ("mkm", 5, [(2, 3), (258, 260)], (2,), (), True, False),          # a first factor of the plain kernel: as it is stored
+    ("kmm", 5, [(2, 3), (3, 515)], (), (), True, True),
     # steps whose input's gradient is a product of PyTorch's, alone, in front of, behind and between steps that are not
     ("mkm", 5, [(130, 400)], (), (), False, True),
     ("kmm", 5, [(40, 400)], (), (), False, False),
