@@ -225,6 +225,12 @@ fastKronError Handle::gradBackward(const GradProblem& p, uint32_t first, uint32_
     }
     a.in_batch = inBatch; a.g_batch = gBatch; a.gin_batch = ginBatch;
     if (!wanted[i] && !gin) { g = gin; gBatch = ginBatch; continue; }
+    // a single partial sum is the gradient: written where it goes (2048x2048, 7 rows: the launch that adds them took 38 us to
+    // copy it, the step itself 10)
+    const bool direct = wanted[i] && gp.parts[i] == 1 && (p.perBatchF || q.batch == 1);
+    a.partSp = direct && gp.outTransposed ? 1 : a.Q;
+    a.partSq = direct && gp.outTransposed ? a.P : 1;
+    char* partials = direct ? (char*)gF[i] : wk + gp.workP[i] * es;
     const StepShape sh = stepShape(q, i);
     uint32_t partFirst = 0;
     hipError_t he = hipSuccess;
@@ -247,7 +253,7 @@ fastKronError Handle::gradBackward(const GradProblem& p, uint32_t first, uint32_
         c.g = (const char*)g + ((size_t)b0 * gBatch + gOff) * es;
         c.gin = gin ? (char*)gin + ((size_t)b0 * ginBatch + inOff) * es : nullptr;
         c.f = F + (size_t)b0 * a.f_batch * es;
-        c.partial = wanted[i] ? wk + (gp.workP[i] + (size_t)b0 * gp.parts[i] * c.P * c.Q) * es : nullptr;
+        c.partial = wanted[i] ? partials + (size_t)b0 * gp.parts[i] * c.P * c.Q * es : nullptr;
         auto aligned = [&](const void* ptr, int64_t s1, int64_t s2, uint64_t sb) {
           return (uintptr_t)ptr % 16 == 0 && s1 % ve == 0 && s2 % ve == 0 && sb % ve == 0;
         };
@@ -286,7 +292,7 @@ fastKronError Handle::gradBackward(const GradProblem& p, uint32_t first, uint32_
     return hipSuccess;
   };
   for (int i = (int)first; i <= lastWanted; i++) {
-    if (!wanted[i]) continue;
+    if (!wanted[i] || (gp.parts[i] == 1 && (p.perBatchF || q.batch == 1))) continue;
     GradReduce& r = ra.r[ra.count++];
     r.P = q.P[i]; r.Q = q.Q[i];
     r.count = gp.parts[i] * (p.perBatchF ? 1 : q.batch);

@@ -17,6 +17,7 @@ struct GradStepArgs {
   uint32_t vecIn, vecG, vecOut;                                // 16-byte accesses possible (alignment and Tn, P multiples of 4)
   uint32_t gridX;                                              // workgroups along u = partial sums of this launch
   uint32_t partStride, partFirst;                              // partial sums per batch entry, first one of this launch
+  uint32_t partSp, partSq;                                     // element (p, q) of a partial sum at p*partSp + q*partSq
   uint32_t qChunks, fPitch;                                    // set by the launcher
 };
 

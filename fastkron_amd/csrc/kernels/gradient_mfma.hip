@@ -330,8 +330,8 @@ void kron_grad_step_kernel(const GradStepArgs a) {
     __syncthreads();
     T* part = (T*)a.partial + ((size_t)bt * a.partStride + a.partFirst + blockIdx.x) * ((size_t)P * Q);
     for (uint32_t e = tid; e < N * N; e += kGradThreads) {
-      const uint32_t p = p0 + e / N, q = q0 + e % N;
-      if (p < P && q < Q) part[(size_t)p * Q + q] = fs[N * N + e];
+      const uint32_t pl = a.partSq == 1 ? e / N : e % N, ql = a.partSq == 1 ? e % N : e / N, p = p0 + pl, q = q0 + ql;
+      if (p < P && q < Q) part[(size_t)p * a.partSp + (size_t)q * a.partSq] = fs[N * N + pl * N + ql];
     }
   }
 }
