@@ -2,9 +2,8 @@
 // the entry points, the autograd functions and the messages of refused operands).
 //
 // A product of small operands costs what the host spends on it: in Python the shape rules, three allocations, a dozen
-// ctypes objects and the stream look-up took 27 of the 34.5 us of a vector against 8x8 (x) 8x8 (x) 8x8 (now 7.7 us with
-// its kernel of 5 us; sgemkm 4096 x 32x32^2 with all gradients 175 -> 95 us, dgekmm 8x8^5 x 16 with factor gradients 255
-// -> 123 us).  Everything between the Python call and the C API happens here instead; nothing is kept between calls.
+// ctypes objects and the stream look-up took 27 of the 34.5 us of a vector against 8x8 (x) 8x8 (x) 8x8 (now 7 to 7.5 us with
+// its kernel of 5 us).  Everything between the Python call and the C API happens here instead; nothing is kept between calls.
 // A function returns None for operands that it does not take (the Python side then says why), a fastKronError as a
 // whole number where the library refuses the call, and otherwise its tensors; product returns False for a call that is
 // to be recorded for gradients.
@@ -437,7 +436,7 @@ PyObject* gradBackward(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
     if (product) gIn = wideInputGradient(o, g, i, cols / o.Qs[i], gNow);
     gNow = gIn; cols = k; i = last + 1;
   }
-  if (needX) gx = gNow.view(xs);
+  if (needX) gx = gNow.sizes() == at::IntArrayRef(xs) ? gNow : gNow.view(xs);
   PyObject* out = PyTuple_New(1 + (Py_ssize_t)o.N);
   if (!out) return nullptr;
   auto put = [&](Py_ssize_t at, Tensor t) {

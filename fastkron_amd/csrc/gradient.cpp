@@ -1,9 +1,9 @@
 // Gradients of a GeMKM / GeKMM: a forward pass that keeps every step's input and a backward pass that goes through the
 // steps in the opposite order, one launch per step for the gradients of the step's input and of its factor
-// (kernels/gradient_mfma.hip), one launch that adds the partial sums of all factors.
+// (kernels/gradient_mfma.hip), one launch that adds the partial sums of all factors that have several.
 //
 // Every factor keeps a step of its own: merged to products of up to 64x64, chains of small factors took fewer launches
-// (dgekmm 8x8^5 x 16 nine instead of eleven, 125 against 130 us), but Z and the gradient of X came out with twice the
+// (dgekmm 8x8^5 x 16 nine instead of eleven, 125 against 134 us), but Z and the gradient of X came out with twice the
 // rounding error (8x8^4 in fp32 2.0e-7 against 1.1e-7).
 // The reference chains PyTorch matmuls through the intermediates of its forward family, one factor at a time
 // (reference pyfastkron/fastkrontorch.py:160-217).

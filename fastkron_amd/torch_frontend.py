@@ -14,8 +14,10 @@ broadcast and batching rules):
   pass keeping every step's input and the backward pass through the steps (reference fastkrontorch.py:160-217);
   when only X needs a gradient the backward pass is one fused library call with the transposed factors.
 
-PyTorch supplies memory and streams; the arithmetic of both passes is the library's HIP kernels (a backward pass that
-is itself differentiated, create_graph=True, is composed of PyTorch operations).  CPU tensors and dtypes other than
+PyTorch supplies memory and streams; the arithmetic of both passes is the library's HIP kernels, but for two parts: the
+gradient of the input of a step with a wide factor is PyTorch's product (`wideStep` in csrc/frontend.cpp has the rule and
+the measurements), and a backward pass that is itself differentiated (create_graph=True) or takes a batch of gradients
+(is_grads_batched) is composed of PyTorch operations.  CPU tensors and dtypes other than
 float32 / float64 are errors: there is no fallback path (the reference falls back to a shuffle algorithm
 built from `torch.matmul`, fastkronbase.py:478-518).
 """
@@ -193,12 +195,15 @@ def _forward(mm, ctx, x, fs):
     return z
 
 
+# is_grads_batched, jacobian(vectorize=True): tensors with no address to pass on
+_legacy_batched, _batched = torch._C._functorch.is_legacy_batchedtensor, torch._C._functorch.is_batchedtensor
+
+
 def _backward(mm, ctx, grad_z):
     saved = ctx.saved_tensors
     x, fs = saved[0], saved[1:ctx.nf + 1]
     need_x, need_f = ctx.needs_input_grad[0], ctx.needs_input_grad[1:ctx.nf + 1]
-    # is_grads_batched, jacobian(vectorize=True): tensors with no address to pass on
-    batched = torch._C._functorch.is_legacy_batchedtensor(grad_z) or torch._C._functorch.is_batchedtensor(grad_z)
+    batched = _legacy_batched(grad_z) or _batched(grad_z)
     if not any(need_f) and not batched:
         # one fused library call on the transposed views: dX = dZ (F_0^T (x) ...) for MKM, (F_0^T (x) ...) dZ for KMM
         # (itself recorded where the backward pass is differentiated)
