@@ -458,6 +458,13 @@ PyObject* gradBackward(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
   END_HANDLE_TH_ERRORS
 }
 
+// batched(tensor): under vmap, old or new style, a tensor has no address to pass on
+PyObject* batched(PyObject*, PyObject* t) {
+  if (!THPVariable_Check(t)) Py_RETURN_FALSE;
+  const c10::DispatchKeySet keys = THPVariable_Unpack(t).key_set();
+  return PyBool_FromLong(keys.has(c10::DispatchKey::Batched) || keys.has(c10::DispatchKey::FuncTorchBatched));
+}
+
 // use(addresses of the entry points, in the order of Api)
 PyObject* use(PyObject*, PyObject* addresses) {
   void* a[sizeof(Api) / sizeof(void*)];
@@ -471,6 +478,7 @@ PyObject* use(PyObject*, PyObject* addresses) {
 
 PyMethodDef methods[] = {
     {"use", (PyCFunction)use, METH_O, nullptr},
+    {"batched", (PyCFunction)batched, METH_O, nullptr},
     {"product", (PyCFunction)(void (*)(void))product, METH_FASTCALL, nullptr},
     {"grad_forward", (PyCFunction)(void (*)(void))gradForward, METH_FASTCALL, nullptr},
     {"grad_backward", (PyCFunction)(void (*)(void))gradBackward, METH_FASTCALL, nullptr},

@@ -195,15 +195,11 @@ def _forward(mm, ctx, x, fs):
     return z
 
 
-# is_grads_batched, jacobian(vectorize=True): tensors with no address to pass on
-_legacy_batched, _batched = torch._C._functorch.is_legacy_batchedtensor, torch._C._functorch.is_batchedtensor
-
-
 def _backward(mm, ctx, grad_z):
     saved = ctx.saved_tensors
     x, fs = saved[0], saved[1:ctx.nf + 1]
     need_x, need_f = ctx.needs_input_grad[0], ctx.needs_input_grad[1:ctx.nf + 1]
-    batched = _legacy_batched(grad_z) or _batched(grad_z)
+    batched = _native.batched(grad_z)                      # is_grads_batched, jacobian(vectorize=True)
     if not any(need_f) and not batched:
         # one fused library call on the transposed views: dX = dZ (F_0^T (x) ...) for MKM, (F_0^T (x) ...) dZ for KMM
         # (itself recorded where the backward pass is differentiated)
