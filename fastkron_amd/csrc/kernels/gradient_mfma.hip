@@ -20,9 +20,9 @@
 // A workgroup handles at most 64x64 of the factor; larger factors run as one launch for dF, one 64x64 block of it per
 // grid z, and one for gin, 64 rows of F per grid z with all of Q contracted.
 //
-// Bound: memory for P, Q <= 32, matrix cores above.  sgemkm 4096 x 32x32^2: 16.8 us a step for 35 MB moved (2.1 TB/s, launch
-// included); dgekmm 8x8^5 x 16: 6.9 us a step for 8.7 MB, most of it launch and one tile's round trips.  gin alone falls
-// behind a GEMM beyond 128 rows or columns; the PyTorch front end has products of its own there.
+// Bound: memory for P, Q <= 32, matrix cores above.  sgemkm 4096 x 32x32^2: 16.7 us a step for 52.6 MB (3.1 TB/s); dgekmm
+// 8x8^5 x 16: 7.0 us a step for 12.9 MB, most of it the launch and one tile's round trips.  gin alone falls behind a GEMM
+// beyond 128 rows or columns; the PyTorch front end has products of its own there.
 // The reference leaves this to PyTorch's matmul (reference pyfastkron/fastkrontorch.py:160-217).
 #include <hip/hip_runtime.h>
 #include "../problem.h"
@@ -401,8 +401,8 @@ uint32_t gradWorkgroups(uint32_t P, uint32_t Q, uint64_t U, uint32_t batch) {
   if (big <= 32) {
     if (share < 512) cap = 512 / share;
   } else {
-    // The number for which the last round over 256 CUs is fullest, the smallest of equal ones, within four rounds.  Rounded up
-    // from 256 / blocks, 3x3 blocks had 261 workgroups, which took two rounds (forward pass and factor gradient alone, us:
+    // The number for which the last 256 CUs' worth of workgroups is fullest, the smallest of equal ones, within four times 256.
+    // Rounded up from 256 / blocks, 3x3 blocks had 261 workgroups, which took as long as 512 (forward pass and factor gradient, us:
     // sgekmm 192x192 x 83333 484 -> 353, 96x192 x 83333 271 -> 191, 640x640 x 6250 367 -> 279).
     for (uint64_t c = 1; c * share <= 1024; c++)
       if ((c * share + 255) / 256 * cap < (cap * share + 255) / 256 * c) cap = c;

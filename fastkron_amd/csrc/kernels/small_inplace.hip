@@ -16,8 +16,9 @@
 //            otherwise from LDS.
 //
 // Bound: memory in principle; with two workgroups of 62.5 KB per CU (5^6) their load, arithmetic and store phases
-// overlap little: 4 us of FMAs and 6 us of memory per row and CU.  Measured against two launches of the kernel with two LDS
-// buffers and one factor per pass (fused_small.hip): sgemkm 1001 x 5^6 90.6 -> 45.4 us (2.8 TB/s), 4096 x 5^5 62.4 ->
+// overlap little: 3.9 us of FMAs (9390 cycles by the instruction count) and 5.7 us of memory per row and CU, 37.5 of the
+// 44.5 us of sgemkm 1001 x 5^6 one after the other.  Measured against two launches of the kernel with two LDS
+// buffers and one factor per pass (fused_small.hip): sgemkm 1001 x 5^6 90.6 -> 44.5 us (2.8 TB/s), 4096 x 5^5 62.4 ->
 // 28.6, 1000 x 7^5 128 -> 58, dgemkm 1000 x 3^8 89 -> 28 (3.8 TB/s), 1000 x 6^5 112 -> 48.  Tried and slower: a
 // persistent form with the next rows in registers (45 -> 53 us, spills), a start delay of the CU's second workgroup
 // (no change).
