@@ -15,15 +15,19 @@
 //   store    straight from the registers of the last pass where its lanes cover runs of 64 elements or more,
 //            otherwise from LDS.
 //
-// Bound: memory in principle; with two workgroups of 62.5 KB per CU (5^6) their load, arithmetic and store phases
-// overlap little: 3.9 us of FMAs (9390 cycles by the instruction count) and 5.7 us of memory per row and CU, 37.5 of the
-// 44.5 us of sgemkm 1001 x 5^6 one after the other.  Measured against two launches of the kernel with two LDS
-// buffers and one factor per pass (fused_small.hip): sgemkm 1001 x 5^6 90.6 -> 44.5 us (2.8 TB/s), 4096 x 5^5 62.4 ->
-// 28.6, 1000 x 7^5 128 -> 58, dgemkm 1000 x 3^8 89 -> 28 (3.8 TB/s), 1000 x 6^5 112 -> 48.  Tried and slower: a
-// persistent form with the next rows in registers (45 -> 53 us, spills), a start delay of the CU's second workgroup
-// (no change).
+// Bound: memory in principle.  Two workgroups of 62.5 KB per CU (5^6) that load, multiply and store go through these phases
+// with the whole device: 3.9 us of FMAs (9390 cycles by the instruction count) and 5.7 us of memory per row and CU, 37.5 of
+// the 44.5 us of sgemkm 1001 x 5^6 one after the other.  Long rows of equal factors therefore have a form of their own
+// (kron_rows_inplace_kernel): sgemkm 1001 x 5^6 50.2 -> 38.1 us (3.3 TB/s; cold operands), 8192 x 5^6 322 -> 237 (4.3), 1001 x 7^5
+// 62.9 -> 52.5, 4096 x 5^5 31.7 -> 24.8, dgemkm 1001 x 3^8 33.3 -> 23.3 (4.5), 1001 x 6^5 51.6 -> 30.0, 700 x 7^5 98 -> 70.
+// Measured against two launches of the kernel with two LDS buffers and one factor per pass (fused_small.hip): sgemkm
+// 1001 x 5^6 90.6 -> 44.5 us, 4096 x 5^5 62.4 -> 28.6, 1000 x 7^5 128 -> 58, dgemkm 1000 x 3^8 89 -> 28, 1000 x 6^5 112 -> 48.
+// Tried and slower: the next tile's pieces in registers in the general kernel (45 -> 53 us: its passes of every width leave
+// no registers, 60 spilled); a start delay of a CU's second workgroup, in either form (3 us: 43.4 -> 45.9); 5^6 in passes of
+// three digits, 128 threads per row (1 row 9.5 -> 12.7 us, 8192 rows 237 -> 259; 1001 rows 43.4 -> 40.6).
 // The reference fuses factors in shared memory between two buffers (reference src/kernels/cuda/kernel.cuh:165-219).
 #include <hip/hip_runtime.h>
+#include <algorithm>
 #include <type_traits>
 #include "../problem.h"
 #include "launch.h"
@@ -46,10 +50,11 @@ template <typename T> __device__ __forceinline__ T ipLoad(__amdgpu_buffer_rsrc_t
   if constexpr (sizeof(T) == 4) return __builtin_bit_cast(T, __builtin_amdgcn_raw_buffer_load_b32(from, (int)lane, (int)uniform, 0));
   else return __builtin_bit_cast(T, __builtin_amdgcn_raw_buffer_load_b64(from, (int)lane, (int)uniform, 0));
 }
-template <typename T> __device__ __forceinline__ void ipStore(T v, __amdgpu_buffer_rsrc_t to, uint32_t lane, uint32_t uniform) {
+// ST: non-temporal
+template <bool ST, typename T> __device__ __forceinline__ void ipStore(T v, __amdgpu_buffer_rsrc_t to, uint32_t lane, uint32_t uniform) {
   typedef unsigned int U2 __attribute__((ext_vector_type(2)));
-  if constexpr (sizeof(T) == 4) __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(unsigned int, v), to, (int)lane, (int)uniform, 0);
-  else __builtin_amdgcn_raw_buffer_store_b64(__builtin_bit_cast(U2, v), to, (int)lane, (int)uniform, 0);
+  if constexpr (sizeof(T) == 4) __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(unsigned int, v), to, (int)lane, (int)uniform, ST ? 2 : 0);
+  else __builtin_amdgcn_raw_buffer_store_b64(__builtin_bit_cast(U2, v), to, (int)lane, (int)uniform, ST ? 2 : 0);
 }
 
 // out = alpha * v (+ beta * y)
@@ -66,18 +71,22 @@ struct IpOut {
 
 // S: the distance between the values of the fastest digit when it is known at compile time (the values' addresses are
 // then offsets of one register), 0 otherwise.
-template <typename T, int P, int D, int S, bool HAS_Y>
+// SYNC: a barrier behind the reads of the values (one digit group per thread at most): the rows' LDS is free from there on.
+template <typename T, int P, int D, int S, bool HAS_Y, bool SYNC = false, bool ST = false>
 __device__ __forceinline__ void ipPass(T* __restrict__ rows, const StepArgs& a, const InplacePass& ps, const uint32_t b,
                                        const uint32_t E, const bool vec, const bool toMemory, const IpOut<T, HAS_Y>& o) {
   constexpr int N = ipPow(P, D), VE = 16 / (int)sizeof(T);
   constexpr int U = N >= 16 ? 1 : N >= 6 ? 2 : 4;            // digit groups per thread and round
-  constexpr int kScalars = 64;                               // scalar registers for factor values
+  constexpr int kScalars = D == 3 ? 75 : D == 2 && P == 6 && sizeof(T) == 8 ? 72 : 64;                 // scalar registers for factor values
   constexpr bool kHoist = D * P * P * (int)sizeof(T) / 4 <= kScalars;
   constexpr int TQ0 = kScalars * 4 / (int)sizeof(T) / P, TQ = TQ0 < P ? TQ0 : P;      // columns of a factor at a time
   static_assert(TQ == P || D == 1, "the values read are overwritten after all columns");
   typedef T VT __attribute__((ext_vector_type(VE)));
   typedef const __attribute__((address_space(4))) T* ConstPtr;
+  static_assert(!SYNC || U == 1, "one group per thread");
   const uint32_t s = S ? S : ps.s, groups = E / N, nth = blockDim.x;
+  uint32_t tid = threadIdx.x;
+  if (SYNC) asm volatile("" : "+v"(tid));                     // (what depends on it would be kept in registers from tile to tile)
   // (read-only for the whole launch, the same address in every lane: the constant address space makes these scalar loads)
   auto loadF = [&](int d, int q0, T (&F_)[P][TQ]) {
     uint64_t fa = (uint64_t)((const T*)a.f[ps.f0 + d] + (size_t)b * a.f_batch[ps.f0 + d]);
@@ -116,7 +125,7 @@ __device__ __forceinline__ void ipPass(T* __restrict__ rows, const StepArgs& a, 
 #pragma unroll
     for (int d = 0; d < D; d++) loadF(d, 0, Fk[d]);
   }
-  for (uint32_t g0 = threadIdx.x; g0 < groups; g0 += U * nth) {
+  for (uint32_t g0 = tid; SYNC ? g0 < nth : g0 < groups; g0 += U * nth) {
     uint32_t step = s;
     asm volatile("" : "+s"(step));                             // (its multiples would fill the registers)
     uint32_t e0[U];
@@ -127,7 +136,7 @@ __device__ __forceinline__ void ipPass(T* __restrict__ rows, const StepArgs& a, 
       const uint32_t g = g0 + k * nth;
       const uint32_t hi = S == 1 ? g : S ? g / (uint32_t)(S ? S : 1) : __umulhi(g, ps.magic);
       e0[k] = hi * (s * N) + (g - hi * s);
-      if (U > 1 && g >= groups) continue;
+      if ((U > 1 || SYNC) && g >= groups) continue;
       if (v16) {
 #pragma unroll
         for (int i = 0; i < N / VE; i++) {
@@ -141,6 +150,7 @@ __device__ __forceinline__ void ipPass(T* __restrict__ rows, const StepArgs& a, 
         for (int i = 0; i < N; i++, at += step) x[k][i] = rows[S ? e0[k] + i * S : at];
       }
     }
+    if (SYNC) __syncthreads();
 #pragma unroll
     for (int d = 0; d < D; d++) {
       const int st = ipPow(P, d);
@@ -176,7 +186,7 @@ __device__ __forceinline__ void ipPass(T* __restrict__ rows, const StepArgs& a, 
     }
 #pragma unroll
     for (int k = 0; k < U; k++) {
-      if (U > 1 && g0 + k * nth >= groups) continue;
+      if ((U > 1 || SYNC) && g0 + k * nth >= groups) continue;
       uint32_t at = e0[k];
       if (toMemory) {
         // through buffer descriptors: one address register per group, the values' distances as scalar offsets
@@ -189,7 +199,7 @@ __device__ __forceinline__ void ipPass(T* __restrict__ rows, const StepArgs& a, 
         for (uint32_t i = 0; i < N; i++) {
           T v = x[k][i] * o.alpha;
           if constexpr (HAS_Y) v += o.beta * yv[i];
-          ipStore<T>(v, o.target, e0[k] * sizeof(T), i * step * sizeof(T));
+          ipStore<ST>(v, o.target, e0[k] * sizeof(T), i * step * sizeof(T));
         }
       } else if (v16) {
 #pragma unroll
@@ -296,6 +306,112 @@ void kron_small_inplace_kernel(const StepArgs a, const InplaceTile t) {
   for (uint32_t e = whole * VE + tid; e < E; e += nth) o.put(e, rows[e]);
 }
 
+// Rows of NF equal factors, one row per workgroup at a time and as many workgroups as the device holds at once: the next
+// row's pieces are on their way to registers while this one's digits are multiplied, and go to LDS as soon as the last pass
+// has read its values (its stores follow).
+template <int P, int NF, size_t ES> struct IpRow {
+  static constexpr int VE = 16 / (int)ES, K = ipPow(P, NF);
+  // digits per pass (two of 6 in fp64 need the next factor's values after the first's; two of 7 do not fit); what is left over
+  // is the first pass, so that the last one is wide
+  static constexpr int D = P <= 3 ? 3 : P == 7 && ES == 8 ? 1 : 2, N = ipPow(P, D), R = NF % D ? NF % D : D;
+  static constexpr int groups = K / N, threads = groups <= (int)kIpMaxThreads ? (groups + 63) / 64 * 64 : (int)kIpMaxThreads;
+  static constexpr bool oneRound = groups <= threads;
+  static constexpr int loads = (K / VE + 1 + threads - 1) / threads;             // 16-byte pieces per thread
+  // workgroups per CU: by LDS, and by the registers of the values, of the pieces and of the rest
+  static constexpr int regs = N * (oneRound ? 1 : 2) * (int)ES / 4 + 4 * loads + 40;
+  static constexpr int byLds = (int)kIpLdsMax / (K * (int)ES + 16), byRegs = 4 * (512 / ((regs + 7) / 8 * 8)) / (threads / 64);
+  static constexpr int perCU = byLds < byRegs ? byLds : byRegs, waves = (perCU * threads / 64 + 3) / 4;
+};
+
+template <typename T, int P, int NF, int J, bool HAS_Y, bool ST>
+__device__ __forceinline__ void ipRowPasses(T* rows, const StepArgs& a, const uint32_t b, const bool vec, const IpOut<T, HAS_Y>& o) {
+  using C = IpRow<P, NF, sizeof(T)>;
+  constexpr int F0 = J == 0 ? 0 : C::R + (J - 1) * C::D, D = J == 0 ? C::R : C::D;
+  constexpr bool last = F0 + D == NF;
+  InplacePass ps{};
+  ps.f0 = F0; ps.p = P; ps.d = D; ps.s = ipPow(P, F0);
+  asm volatile("" : "+s"(ps.f0));                              // (factor values of the next row are not this row's to keep)
+  ipPass<T, P, D, ipPow(P, F0), HAS_Y, last && C::oneRound, ST>(rows, a, ps, b, C::K, vec, last, o);
+  if constexpr (!last || !C::oneRound) __syncthreads();
+  if constexpr (!last) {
+    ipRowPasses<T, P, NF, J + 1, HAS_Y, ST>(rows, a, b, vec, o);
+  }
+}
+
+// NT: 0 ordinary accesses, 1 non-temporal loads, 2 non-temporal loads and stores.
+template <typename T, int P, int NF, bool HAS_Y, int NT>
+__global__ __launch_bounds__((IpRow<P, NF, sizeof(T)>::threads), (IpRow<P, NF, sizeof(T)>::waves))
+void kron_rows_inplace_kernel(const StepArgs a, const uint32_t total) {
+  using C = IpRow<P, NF, sizeof(T)>;
+  constexpr uint32_t VE = C::VE, K = C::K;
+  typedef T VT __attribute__((ext_vector_type(C::VE)));
+  extern __shared__ __align__(16) unsigned char ipLds[];
+  VT* chunks = (VT*)ipLds;
+  IpOut<T, HAS_Y> o;
+  o.alpha = a.epilogue ? (T)a.alpha : T(1); o.beta = (T)a.beta;
+
+  // 16-byte pieces that lie inside the row, and the elements before the first and behind the last of them
+  struct Row { const T* src; uint32_t b, m, shift, last; };
+  auto rowAt = [&](uint32_t i) {
+    Row r;
+    r.b = a.batch == 1 ? 0 : i / a.M; r.m = i - r.b * a.M;
+    r.src = (const T*)a.in + (size_t)r.b * a.in_batch + (size_t)r.m * K;
+    r.shift = (uint32_t)((uintptr_t)r.src / sizeof(T)) & (VE - 1);
+    r.last = (r.shift + K) / VE;
+    return r;
+  };
+  VT v[C::loads];
+  T edge = T(0);
+  auto edgeOf = [&](const Row& r, uint32_t tid, uint32_t* e) {
+    const uint32_t behind = r.last * VE - r.shift;             // first element behind the last piece
+    *e = tid < VE ? tid : behind + tid - VE;
+    return tid < 2 * VE && (tid < VE ? r.shift != 0 && tid < VE - r.shift : *e < K);
+  };
+  auto fetch = [&](const Row& r) {
+    uint32_t tid = threadIdx.x, e;
+    asm volatile("" : "+v"(tid));
+    // (beyond `last`, and piece 0 where it begins before the row: outside the descriptor's range, nothing is read)
+    const auto from = streamTarget((void*)(r.src - r.shift), r.last * 16);
+    if (edgeOf(r, tid, &e)) edge = r.src[e];
+    const uint32_t off = tid * 16;
+#pragma unroll
+    for (int k = 0; k < C::loads; k++)
+      v[k] = __builtin_bit_cast(VT, __builtin_amdgcn_raw_buffer_load_b128(from, (int)(k == 0 && tid == 0 && r.shift ? 0x7ffffff0u : off),
+                                                                         k * C::threads * 16, NT ? 2 : 0));
+  };
+
+  uint32_t i = blockIdx.x;
+  Row r = rowAt(i);
+  fetch(r);
+  for (;;) {
+    T* rows = (T*)ipLds + r.shift;
+    const uint32_t b = r.b;
+    o.out = (T*)a.out + (size_t)b * a.out_batch + (size_t)r.m * K;
+    o.y = HAS_Y ? (const T*)a.y + (size_t)b * a.y_batch + (size_t)r.m * K : nullptr;
+    o.target = streamTarget(o.out, K * (uint32_t)sizeof(T));
+    if (HAS_Y) o.yTarget = streamTarget((void*)o.y, K * (uint32_t)sizeof(T));
+    {
+      uint32_t tid = threadIdx.x, e;
+      asm volatile("" : "+v"(tid));
+#pragma unroll
+      for (int k = 0; k < C::loads; k++) {
+        const uint32_t c = tid + k * C::threads;
+        if ((k > 0 || c > 0 || r.shift == 0) && ((k + 1) * C::threads <= (int)(K / VE) || c < r.last)) chunks[c] = v[k];
+      }
+      if (edgeOf(r, tid, &e)) rows[e] = edge;
+    }
+    __syncthreads();
+    const bool vec = r.shift == 0, more = i + gridDim.x < total;
+    if (more) {
+      i += gridDim.x;
+      r = rowAt(i);
+      fetch(r);
+    }
+    ipRowPasses<T, P, NF, 0, HAS_Y, NT == 2>(rows, a, b, vec, o);
+    if (!more) return;
+  }
+}
+
 static bool ipTile(uint32_t nf, const uint32_t* p, const uint32_t* q, uint64_t Kin, uint32_t M, uint32_t batch, DType dt,
                    InplaceTile* t) {
   if (nf < 1 || nf > kMaxFused || M == 0) return false;
@@ -383,9 +499,65 @@ static hipError_t launchIpT(const StepArgs& a, const InplaceTile& t, hipStream_t
   }
 }
 
+template <typename T, int P, int NF, bool HAS_Y, int NT>
+static hipError_t launchIpRowsAs(const StepArgs& a, uint32_t total, uint32_t grid, hipStream_t stream) {
+  using C = IpRow<P, NF, sizeof(T)>;
+  static PerDeviceOnce attrOnce;
+  const int dev = launchDeviceIndex();
+  const auto kernel = kron_rows_inplace_kernel<T, P, NF, HAS_Y, NT>;
+  const size_t lds = C::K * sizeof(T) + 16;
+  if (lds > 65536 && !attrOnce.done(dev)) {
+    if (const hipError_t e = hipFuncSetAttribute((const void*)kernel, hipFuncAttributeMaxDynamicSharedMemorySize, (int)kIpLdsMax); e != hipSuccess) return e;
+    attrOnce.mark(dev);
+  }
+  hipLaunchKernelGGL(kernel, dim3(grid), dim3(C::threads), lds, stream, a, total);
+  return hipGetLastError();
+}
+
+// One row per workgroup at a time, if that is the better form (*taken).  Rows per workgroup slot of the device decide:
+//   against several workgroups that each take a row and end (kron_small_inplace_kernel): better up to 6 rows per slot for every
+//   size (5^5 fp32, 2.7 rows 44.6 -> 37, 8 rows 103 / 109 us; 3^8 fp64, 5 rows 103 -> 92, 13 rows 211 / 216), beyond that where
+//   a CU holds one or two rows (5^6 fp32, 16 rows 322 -> 237) or where this form takes more digits per pass or more registers
+//   per thread than that kernel (6 and 7: 6^5 fp64, 16 rows 307 -> 220; 7^4 fp32, 13 rows 193 -> 162);
+//   streamed operands: non-temporal loads up to 6 rows per slot (4096 x 5^5 fp32 28.0 -> 23.8; beyond 207 / 215), and stores up
+//   to 2 (1001 x 5^6 40.5 -> 38.0, 1001 x 6^5 fp64 33.0 -> 30.0; 7000 x 5^5, 2.7 rows 37 / 45: the runs of a wave begin and end
+//   inside lines, whose other parts come later the further the workgroups of a CU have drifted apart).
+template <typename T, int P, int NF>
+static hipError_t launchIpRows(const StepArgs& a, hipStream_t stream, bool* taken) {
+  using C = IpRow<P, NF, sizeof(T)>;
+  const uint32_t total = a.M * a.batch, resident = (uint32_t)(C::perCU * deviceCUs()), grid = std::min(total, resident);
+  *taken = P >= 6 || C::perCU <= 2 || total / 6 <= resident;
+  if (!*taken) return hipSuccess;
+  const int nt = streamMode(a) < 2 || total / 6 > resident ? 0 : total / 2 > resident ? 1 : 2;
+  const bool y = a.y && a.epilogue;
+#define IP_ROWS(NT) y ? launchIpRowsAs<T, P, NF, true, NT>(a, total, grid, stream) : launchIpRowsAs<T, P, NF, false, NT>(a, total, grid, stream)
+  return nt == 0 ? IP_ROWS(0) : nt == 1 ? IP_ROWS(1) : IP_ROWS(2);
+#undef IP_ROWS
+}
+
+// The sizes of rows of equal factors that have the form above: those of 9 to 160 KB, up to which several rows per workgroup
+// fill its threads better; 3^9 is more factors than a launch takes.
+static hipError_t launchIpRowsAny(const StepArgs& a, const InplaceTile& t, DType dt, hipStream_t stream, bool* taken) {
+  *taken = false;
+  if ((uint64_t)a.M * a.batch >= (1ull << 31)) return hipSuccess;
+  const uint32_t size = t.P * 16 + a.nf;
+#define IP_ROWS(T, P, NF) case P * 16 + NF: return launchIpRows<T, P, NF>(a, stream, taken);
+  if (dt == DType::F32) switch (size) {
+    IP_ROWS(float, 3, 8) IP_ROWS(float, 5, 5) IP_ROWS(float, 5, 6) IP_ROWS(float, 6, 5) IP_ROWS(float, 7, 4) IP_ROWS(float, 7, 5)
+    default: return hipSuccess;
+  }
+  switch (size) {
+    IP_ROWS(double, 3, 8) IP_ROWS(double, 5, 5) IP_ROWS(double, 5, 6) IP_ROWS(double, 6, 5) IP_ROWS(double, 7, 5)
+    default: return hipSuccess;
+  }
+#undef IP_ROWS
+}
+
 hipError_t launchSmallInplace(const StepArgs& a, DType dt, hipStream_t stream) {
   InplaceTile t;
   if (!smallInplaceSupported(a, dt) || !ipTile(a.nf, a.p, a.q, a.Kin, a.M, a.batch, dt, &t)) return hipErrorInvalidValue;
+  bool taken;
+  if (const hipError_t e = launchIpRowsAny(a, t, dt, stream, &taken); taken || e != hipSuccess) return e;
   return dt == DType::F32 ? launchIpT<float>(a, t, stream) : launchIpT<double>(a, t, stream);
 }
 

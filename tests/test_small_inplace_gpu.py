@@ -74,6 +74,26 @@ def test_rows_beyond_the_lds_run_their_trailing_factors_in_place(fk, M, Ps, dt):
         assert few_long_rows or "inplace" in fk.last_plan()[0][2], fk.last_plan()
 
 
+# rows, factors, type: more rows than the device holds at once (workgroups that go from row to row, the next one loaded
+# ahead): a few more, a few less than twice as many, and sizes at which operands are streamed
+MANY = [(515, 5, 6, "f"), (1030, 5, 6, "f"), (258, 5, 6, "d"), (517, 7, 5, "f"), (259, 7, 5, "d"), (1027, 6, 5, "f"), (513, 6, 5, "d"),
+        (1283, 3, 8, "f"), (771, 3, 8, "d"), (2563, 5, 5, "f"), (1539, 5, 5, "d"), (3077, 7, 4, "f"), (2200, 3, 8, "d"), (16000, 5, 5, "f")]
+
+
+@pytest.mark.parametrize("M,P,n,t", MANY, ids=lambda v: str(v))
+def test_more_rows_than_the_device_holds(fk, M, P, n, t):
+    dt = np.float32 if t == "f" else np.float64
+    Ps = [P] * n
+    for seed, (m, kw) in enumerate([(M, dict(alpha=1.5, beta=0.5)), (M, dict(alpha=1.0, beta=0.0, opFs=ko.OP_T)),
+                                    (M // 3 + 1, dict(alpha=-1.0, beta=0.0, batch=3))]):
+        alpha, beta, batch = kw.pop("alpha"), kw.pop("beta"), kw.get("batch", 1)
+        X, Fs, Y = make_case(ko.MKM, m, Ps, Ps, dt, seed=11 + seed, with_y=beta != 0.0, batch=batch)
+        want = oracle_answer(ko.MKM, m, Ps, Ps, X, Fs, Y, alpha, beta, **kw)
+        got, e = run_gpu(fk, ko.MKM, m, Ps, Ps, X, Fs, Y, alpha, beta, **kw)
+        assert e == 0 and normwise(got, want) <= TOL[dt], (fk.last_plan(), kw)
+        assert len(fk.last_plan()) == 1 and "inplace" in fk.last_plan()[0][2], fk.last_plan()
+
+
 def test_rows_off_a_16_byte_boundary(fk):
     """Base addresses that are only 4-byte aligned, of X and of Z, and the in-place epilogue (Y is Z)."""
     import torch
