@@ -226,6 +226,21 @@ fastKronError Handle::tune(const KronProblem& p0, bool haveTemp2, Choice* best) 
       v.c.transposeX = tx != 0;
       if (!(tx && !haveTemp2 && plan.size() != 1)) variants.push_back(v);
     }
+    if (!merge && q.mm == MMType::KMM && useFusion()) {
+      // the digits in place, in the groups of the rule, with the fastest kernel for each
+      Variant v; v.c.columns = true; v.c.transposeX = tx != 0; v.estimate = extra; v.measured = FLT_MAX;
+      bool ok = true;
+      for (auto& s : columnsPlan(q)) {
+        KronProblem part;
+        Plan one;
+        float t = 0;
+        ok = ok && columnsPart(q, s.lo, s.hi, &part) && tuneSingle(*this, onBuffers(part), B, verbose, &one, &t);
+        if (!ok) break;
+        v.c.plan.push_back(PlanStep{s.lo, s.hi, one[0].kernel});
+        v.estimate += t;
+      }
+      if (ok && !v.c.plan.empty() && (haveTemp2 || (v.c.plan.size() <= 2 && !tx))) variants.push_back(v);
+    }
     if (!useFusion() || !haveTemp2) continue;
     for (uint32_t g = 1; g < q.N; g++) {
       KronProblem q1, q2;
@@ -282,7 +297,7 @@ fastKronError Handle::tune(const KronProblem& p0, bool haveTemp2, Choice* best) 
     if (variants[vi].measured != FLT_MAX && (!win || variants[vi].measured < win->measured)) win = &variants[vi];
   if (!win) return fastKronKernelNotFound;
   *best = win->c;
-  db_.storeTuned(p0.str(), win->c.plan, win->measured, win->c.merge ? 1 : 0, win->c.split, win->c.transposeX ? 1 : 0);
+  db_.storeTuned(p0.str(), win->c.plan, win->measured, win->c.columns ? 2 : win->c.merge ? 1 : 0, win->c.split, win->c.transposeX ? 1 : 0);
   if (!dbPath_.empty()) db_.saveFile(dbPath_);
   return fastKronSuccess;
 }

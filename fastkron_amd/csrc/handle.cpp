@@ -442,6 +442,15 @@ bool Handle::transposeFirstOnline(const KronProblem& p, const KronProblem& pn, v
 
 fastKronError Handle::runOnline(KronProblem p, void* temp1, void* temp2, const CallWorkspace* ws) {
   fastKronError e;
+  if (useFusion() && p.mm == MMType::KMM && !p.forward && p.N >= 2 && p.M > 1) {
+    const std::string ck = p.str() + "_columns";
+    auto it = planCache_.find(ck);
+    if (it == planCache_.end()) it = planCache_.emplace(ck, columnsPlan(p)).first;
+    if (!it->second.empty()) {
+      e = runColumns(p, it->second, temp1, temp2);
+      if (e != fastKronKernelNotFound) return e;
+    }
+  }
   {
     KronProblem merged;
     if (useFusion() && mergeSmallFactors(p, &merged, ws)) p = merged;
@@ -726,6 +735,105 @@ uint32_t Handle::chunkRowsForCache(const KronProblem& p, const KronProblem& q2) 
   return rows >= p.M ? p.M : (uint32_t)rows;
 }
 
+// A Kronecker product acts on every digit of the row index by itself, so that a GeKMM may leave the digits where they are:
+// with the factors behind `hi` applied already, the rows are H x K x (Q of those factors), and the factors lo .. hi are a
+// problem of H entries (batch) with K rows and M * Q.. columns.  Nothing moves, the columns are many even when M is not.
+bool Handle::columnsPart(const KronProblem& p, uint32_t lo, uint32_t hi, KronProblem* out) const {
+  uint64_t H = 1, Kg = 1, Lg = 1, C = p.M;
+  for (uint32_t i = 0; i < lo; i++) H *= p.P[i];
+  for (uint32_t i = lo; i <= hi; i++) { Kg *= p.P[i]; Lg *= p.Q[i]; }
+  for (uint32_t i = hi + 1; i < p.N; i++) C *= p.Q[i];
+  if (C >= (1ull << 32) || H * p.batch >= (1ull << 32)) return false;
+  // entries of the problem become H entries each: shared factors, and the caller's operands without gaps
+  if (p.batch > 1 && H > 1) {
+    for (uint32_t i = lo; i <= hi; i++) if (p.strideF[i] != 0) return false;
+    if (hi == p.N - 1 && p.strideX != H * Kg * C) return false;
+  }
+  KronProblem q = p;
+  q.N = hi - lo + 1;
+  for (uint32_t i = 0; i < q.N; i++) { q.P[i] = p.P[lo + i]; q.Q[i] = p.Q[lo + i]; q.F[i] = p.F[lo + i]; q.strideF[i] = p.strideF[lo + i]; }
+  q.M = (uint32_t)C; q.batch = (uint32_t)(H * p.batch); q.strided = q.batch > 1;
+  if (hi < p.N - 1 || H > 1) q.strideX = Kg * C;
+  if (lo > 0) {
+    q.strideZ = Lg * C;
+    q.Y = nullptr; q.strideY = 0; q.alpha = 1.0; q.beta = 0.0;
+    q.zReadNext = true;
+  }
+  if (hi < p.N - 1) q.xJustWritten = true;
+  *out = q;
+  return true;
+}
+
+Plan Handle::columnsPlan(const KronProblem& p) const {
+  if (p.mm != MMType::KMM || p.forward || p.opX != fastKronOp_N || p.N < 2 || p.M < 2) return Plan();
+  Plan plan;
+  bool grouped = false;
+  for (int hi = (int)p.N - 1; hi >= 0;) {
+    int lo = hi;
+    const uint32_t P = p.P[hi], most = p.P[hi] == p.Q[hi] ? colsInplaceMost(P, p.dt) : 0;
+    if (most) {
+      int run = 1;
+      while (run <= hi && p.P[hi - run] == P && p.Q[hi - run] == P) run++;
+      const int groups = (run + (int)most - 1) / (int)most;
+      lo = hi + 1 - (run + groups - 1) / groups;
+    }
+    KronProblem q;
+    if (!columnsPart(p, (uint32_t)lo, (uint32_t)hi, &q)) return Plan();
+    const Plan one = db_.selectOnline(q, dev_, true);
+    if (one.size() != 1) return Plan();
+    plan.push_back(PlanStep{(uint32_t)lo, (uint32_t)hi, one[0].kernel});
+    if (lo < hi) grouped = true;
+    hi = lo - 1;
+  }
+  if (!grouped) return Plan();
+  // against the launches of the chain as it would run otherwise (with merged factors, one more that writes those): fewer is
+  // ahead at every size measured (2 to 10 factors of 2 to 8 rows, 2 to 1024 columns, either type: 1.2 to 4.5 times but for
+  // sgekmm 8^4 x 88, 14.1 / 14.0 us), as many where groups of the kernel with two LDS buffers are among them (1.4 to 2.6 times:
+  // sgekmm 6^6 x 88 58.8 -> 22.2, dgekmm 5^6 x 1024 217 -> 95); as many launches of the register kernels are no slower
+  // (sgekmm 8^5 x 64 19.8, 1024 columns 113)
+  KronProblem q = p;
+  size_t merge = 0;
+  {
+    Handle* self = const_cast<Handle*>(this);
+    const bool was = planOnly_;
+    self->planOnly_ = true;
+    if (self->mergeSmallFactors(p, &q)) merge = 1;
+    self->planOnly_ = was;
+  }
+  const Plan other = db_.selectOnline(q, dev_, true);
+  bool lds = false, merged16 = merge != 0;
+  for (auto& s : other) lds = lds || db_.kernels()[s.kernel].name.find("_small_fused_lds_") != std::string::npos;
+  for (uint32_t i = 0; i < q.N; i++) merged16 = merged16 && q.P[i] <= 16;
+  // (Small fp64 problems of 2x2 and 4x4 factors keep the plan that merges them to 16x16, which is fixed for them: dgekmm 4^6 x 64
+  // 17.1 us against 9.2.)
+  if (merged16 && (uint64_t)p.M * p.K() * p.batch <= (1ull << 18)) return Plan();
+  return plan.size() < merge + other.size() + (lds ? 1 : 0) ? plan : Plan();
+}
+
+fastKronError Handle::runColumns(const KronProblem& p, const Plan& plan, void* temp1, void* temp2) {
+  if (plan.empty() || (plan.size() > 1 && !temp1) || (plan.size() > 2 && !temp2)) return fastKronKernelNotFound;
+  void* tmps[2] = {temp1, temp2};
+  auto run = [&](bool dry) -> fastKronError {
+    const void* x = p.X;
+    for (size_t i = 0; i < plan.size(); i++) {
+      const PlanStep& s = plan[i];
+      KronProblem q;
+      if (s.hi >= p.N || s.lo > s.hi || !columnsPart(p, s.lo, s.hi, &q)) return fastKronKernelNotFound;
+      q.X = x;
+      if (s.lo > 0) q.Z = tmps[i % 2];
+      const Plan one(1, PlanStep{0, s.hi - s.lo, s.kernel});
+      if (const fastKronError e = execute(q, one, nullptr, nullptr, dry); e != fastKronSuccess) return e;
+      x = q.Z;
+    }
+    return fastKronSuccess;
+  };
+  if (run(true) != fastKronSuccess) return fastKronKernelNotFound;
+  lastPlan_ = p.str();
+  for (auto& s : plan) lastPlan_ += ";" + std::to_string(s.lo) + "-" + std::to_string(s.hi) + ":" + db_.kernels()[s.kernel].name;
+  if (planOnly_) launchLog_.clear();
+  return run(planOnly_);
+}
+
 // The online rule for the two-part plan: how many trailing factors one whole-block kernel takes.
 fastKronError Handle::trySplitLeadingTrailing(const KronProblem& p, void* temp1, void* temp2) {
   if (p.mm != MMType::MKM || p.forward || p.opX != fastKronOp_N) return fastKronKernelNotFound;
@@ -796,7 +904,7 @@ bool Handle::lookupChoice(const KronProblem& p, Choice* c) const {
   uint32_t split = 0;
   Plan plan;
   if (!db_.lookupTuned(p.str(), &plan, &merge, &split, &transposeX) || merge < 0) return false;
-  c->merge = merge != 0; c->split = split; c->plan = plan; c->transposeX = transposeX != 0;
+  c->merge = merge == 1; c->columns = merge == 2; c->split = split; c->plan = plan; c->transposeX = transposeX != 0;
   return true;
 }
 
@@ -815,6 +923,14 @@ fastKronError Handle::runChoice(const KronProblem& p0, const Choice& c, void* te
     return e;
   }
   KronProblem p = p0;
+  if (c.columns) {
+    if (p.mm != MMType::KMM || p.forward || p.opX != fastKronOp_N || !db_.orderedPlan(p, c.plan)) return fastKronKernelNotFound;
+    for (auto& s : c.plan) {
+      KronProblem q;
+      if (!columnsPart(p, s.lo, s.hi, &q) || !db_.validPlan(q, Plan(1, PlanStep{0, s.hi - s.lo, s.kernel}), dev_)) return fastKronKernelNotFound;
+    }
+    return runColumns(p, c.plan, temp1, temp2);
+  }
   if (c.merge) {
     KronProblem merged;
     if (!mergeSmallFactors(p0, &merged, ws)) return fastKronKernelNotFound;

@@ -51,7 +51,8 @@ class Handle {
   // What a tuned record prescribes for a problem: merge small factors or not, two-part plan with `split` leading
   // factors or one chain (0), and the launches (numbered in the chain after merging; for a two-part plan the
   // trailing part's steps, on factors >= split, come first).
-  struct Choice { bool transposeX = false; bool merge = false; uint32_t split = 0; Plan plan; };
+  // columns: the steps of a GeKMM run with their digits in place (runColumns).
+  struct Choice { bool transposeX = false; bool merge = false; bool columns = false; uint32_t split = 0; Plan plan; };
   // Times the alternatives for `p` (merged or not, every two-part split, every kernel on every sub-chain), stores the
   // fastest under the problem's own string and returns it.
   fastKronError tune(const KronProblem& p, bool haveTemp2, Choice* best);
@@ -75,6 +76,12 @@ class Handle {
   // M * prod(leading P) virtual rows, leading factors as a batched KMM over the row blocks.
   // Returns fastKronKernelNotFound when the problem does not have that form.
   fastKronError trySplitLeadingTrailing(const KronProblem& p, void* temp1, void* temp2);
+  // GeKMM chains with runs of equal small factors: every group of adjacent factors is applied with its digits in place.
+  // columnsPart: the factors lo .. hi as a problem of their own; columnsPlan: the groups by rule, empty where another plan
+  // is ahead; runColumns: fastKronKernelNotFound when the plan or the buffers do not have that form.
+  bool columnsPart(const KronProblem& p, uint32_t lo, uint32_t hi, KronProblem* q) const;
+  Plan columnsPlan(const KronProblem& p) const;
+  fastKronError runColumns(const KronProblem& p, const Plan& plan, void* temp1, void* temp2);
   // Chains of 2x2 / 4x4 (fp64: also 8x8) factors: adjacent factors are replaced by their Kronecker product
   // (16x16; 64x64 in fp64 when the chain holds 8x8 or 32x32 factors), computed into the handle's workspace by one small launch, so that the
   // kernels for those sizes apply.  Returns false when nothing is merged; on true `out` is the merged problem.

@@ -95,6 +95,22 @@ static bool smallInplaceCanRun(const KernelInfo& k, const KronProblem& p, uint32
 static hipError_t smallInplaceLaunch(const KernelInfo& k, const StepArgs& a, hipStream_t s) { return launchSmallInplace(a, k.dt, s); }
 static bool smallInplaceCheck(const KernelInfo& k, const StepArgs& a) { return smallInplaceSupported(a, k.dt); }
 
+// ---- all rows of equal small factors in the KMM layout, in place ----
+static bool colsInplaceCanRun(const KernelInfo& k, const KronProblem& p, uint32_t lo, uint32_t hi, bool first, bool,
+                              const DeviceInfo& dev) {
+  const uint32_t nf = hi - lo + 1;
+  if (k.dt != p.dt || p.mm != MMType::KMM || p.M < 2 || nf < 2 || nf > kMaxFused || p.forward) return false;
+  if (first && p.opX == 2) return false;
+  // Small fp32 problems of 4x4 and 8x8 factors keep the plans on the register kernels, which are fixed for them (sgekmm
+  // 8^3 x 88 10.2 us against 7.5).
+  if (dev.rulesOfThumb && p.dt == DType::F32 && (p.P[hi] == 4 || p.P[hi] == 8) && (uint64_t)p.M * p.K() * p.batch < (1ull << 16)) return false;
+  uint32_t ps[kMaxFused], qs[kMaxFused];
+  for (uint32_t j = 0; j < nf; j++) { ps[j] = p.P[hi - j]; qs[j] = p.Q[hi - j]; }
+  return dev.ldsPerBlock >= 160 * 1024 && colsInplaceFits(nf, ps, qs, p.colsBefore(hi), p.dt);
+}
+static hipError_t colsInplaceLaunch(const KernelInfo& k, const StepArgs& a, hipStream_t s) { return launchColsInplace(a, k.dt, s); }
+static bool colsInplaceCheck(const KernelInfo& k, const StepArgs& a) { return colsInplaceSupported(a, k.dt); }
+
 // ---- one factor of any shape up to 256x512 on the matrix cores (zero padded) ----
 static bool stepAnyCanRun(const KernelInfo& k, const KronProblem& p, uint32_t lo, uint32_t hi, bool first, bool,
                           const DeviceInfo& dev) {
@@ -134,6 +150,13 @@ void registerGenericKernels(std::vector<KernelInfo>& out) {
     k.name = std::string("mkm_hip_gfx950_640_") + (dt == DType::F32 ? "f" : "d") + "_small_fused_inplace_8";
     k.dt = dt; k.P = 1; k.Q = 1; k.fused = kMaxFused; k.tileM = 0; k.tileK = 0; k.threads = 640; k.variant = 0;
     k.canRun = smallInplaceCanRun; k.launch = smallInplaceLaunch; k.check = smallInplaceCheck;
+    out.push_back(k);
+  }
+  for (DType dt : {DType::F32, DType::F64}) {
+    KernelInfo k{};
+    k.name = std::string("kmm_hip_gfx950_512_") + (dt == DType::F32 ? "f" : "d") + "_small_fused_columns_8";
+    k.dt = dt; k.P = 1; k.Q = 1; k.fused = kMaxFused; k.tileM = 0; k.tileK = 0; k.threads = 512; k.variant = 0;
+    k.canRun = colsInplaceCanRun; k.launch = colsInplaceLaunch; k.check = colsInplaceCheck;
     out.push_back(k);
   }
   for (DType dt : {DType::F32, DType::F64}) {
@@ -671,20 +694,26 @@ Plan KernelDB::selectOnline(const KronProblem& p, const DeviceInfo& dev, bool al
   return plan;
 }
 
-bool KernelDB::validPlan(const KronProblem& p, const Plan& plan, const DeviceInfo& dev) const {
+bool KernelDB::orderedPlan(const KronProblem& p, const Plan& plan) const {
   if (plan.empty() || p.N == 0) return false;
   int64_t expectHi = (int64_t)p.N - 1;
-  for (size_t l = 0; l < plan.size(); l++) {
-    const PlanStep& s = plan[l];
+  for (const PlanStep& s : plan) {
     if (s.kernel < 0 || (size_t)s.kernel >= kernels_.size()) return false;
     if ((int64_t)s.hi != expectHi || s.lo > s.hi || s.hi - s.lo + 1 > kMaxFused) return false;
-    const KernelInfo& k = kernels_[s.kernel];
-    DeviceInfo able = dev;
-    able.rulesOfThumb = false;
-    if (!k.canRun(k, p, s.lo, s.hi, l == 0, s.lo == 0, able)) return false;
     expectHi = (int64_t)s.lo - 1;
   }
   return expectHi == -1;
+}
+
+bool KernelDB::validPlan(const KronProblem& p, const Plan& plan, const DeviceInfo& dev) const {
+  if (!orderedPlan(p, plan)) return false;
+  DeviceInfo able = dev;
+  able.rulesOfThumb = false;
+  for (size_t l = 0; l < plan.size(); l++) {
+    const KernelInfo& k = kernels_[plan[l].kernel];
+    if (!k.canRun(k, p, plan[l].lo, plan[l].hi, l == 0, plan[l].lo == 0, able)) return false;
+  }
+  return true;
 }
 
 bool KernelDB::lookupTuned(const std::string& key, Plan* plan, int* merge, uint32_t* split, int* transposeX) const {
@@ -712,6 +741,7 @@ void KernelDB::storeTuned(const std::string& key, const Plan& plan, float ms, in
 
 // File format, one problem per line:
 //   <problem string> <ms> [M<merge> S<split> [X<transposeX>]] <nsteps> {<lo> <hi> <kernel name>}...
+// (merge 2: the steps run with their digits in place, each as a problem on the columns behind them)
 // (lines without the M / S fields leave both to the online selection)
 bool KernelDB::loadFile(const std::string& path, bool shipped) {
   std::ifstream f(path);
@@ -726,7 +756,8 @@ bool KernelDB::loadFile(const std::string& path, bool shipped) {
     if (!tok.empty() && tok[0] == 'M') {
       std::string stok, ntok;
       if (!(is >> stok >> ntok) || stok.empty() || stok[0] != 'S') continue;
-      t.merge = atoi(tok.c_str() + 1) ? 1 : 0;
+      t.merge = atoi(tok.c_str() + 1);
+      if (t.merge < 0 || t.merge > 2) continue;
       t.split = (uint32_t)strtoul(stok.c_str() + 1, nullptr, 10);
       if (!ntok.empty() && ntok[0] == 'X') {
         t.transposeX = atoi(ntok.c_str() + 1) ? 1 : 0;

@@ -75,8 +75,11 @@ class KernelDB {
   // accepts its factor range (a plan read from a file is not trusted before it passes this).
   bool validPlan(const KronProblem& p, const Plan& plan, const DeviceInfo& dev) const;
 
+  // The first half of that: every factor once, last factor first.
+  bool orderedPlan(const KronProblem& p, const Plan& plan) const;
+
   // Tuned plans, keyed by the problem string.  A record may also say how the chain is to be rewritten before the plan
-  // applies: `merge` (1: adjacent small factors replaced by their Kronecker products, 0: not, -1: unspecified, as the
+  // applies: `merge` (1: adjacent small factors replaced by their Kronecker products, 0: not, 2: the digits of a GeKMM stay in place, -1: unspecified, as the
   // online selection decides) and `split` (g > 0: the plan's steps on factors >= g are the trailing part of a two-part
   // plan, run on the contiguous blocks of the rows, the steps on factors < g the leading part, run across the blocks).
   // `transposeX` (1: op(X) = T is handled by a transposed copy of X ahead of the launches, which then see op(X) = N).

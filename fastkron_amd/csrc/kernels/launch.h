@@ -166,6 +166,12 @@ bool smallInplaceFits(uint32_t nf, const uint32_t* p, const uint32_t* q, uint64_
 bool smallInplaceSupported(const StepArgs& a, DType dt);
 hipError_t launchSmallInplace(const StepArgs& a, DType dt, hipStream_t stream);
 
+// All rows of equal small factors (2 <= P <= 8, at most colsInplaceMost of them) in the KMM layout, in place.
+uint32_t colsInplaceMost(uint32_t P, DType dt);
+bool colsInplaceFits(uint32_t nf, const uint32_t* p, const uint32_t* q, uint64_t Kin, DType dt);
+bool colsInplaceSupported(const StepArgs& a, DType dt);
+hipError_t launchColsInplace(const StepArgs& a, DType dt, hipStream_t stream);
+
 // Kronecker products of adjacent small factors into the handle's workspace, 256 entries per workgroup.
 hipError_t launchMergeFactors(const MergeArgs& a, DType dt, hipStream_t stream);
 // Transposed copy: in is R x C row-major per batch entry, out is C x R.

@@ -62,6 +62,9 @@ template <typename T, bool HAS_Y>
 struct IpOut {
   T* out; const T* y; T alpha, beta;
   __amdgpu_buffer_rsrc_t target, yTarget;                    // the same as buffer descriptors
+  // columns: the operand as well, byte offsets of the lane's column in the three, bytes from a row to the next
+  __amdgpu_buffer_rsrc_t source;
+  uint32_t laneIn, laneOut, laneY, pitch;
   __device__ __forceinline__ void put(uint32_t e, T v) const {
     v *= alpha;
     if (HAS_Y) v += beta * y[e];
@@ -72,7 +75,8 @@ struct IpOut {
 // S: the distance between the values of the fastest digit when it is known at compile time (the values' addresses are
 // then offsets of one register), 0 otherwise.
 // SYNC: a barrier behind the reads of the values (one digit group per thread at most): the rows' LDS is free from there on.
-template <typename T, int P, int D, int S, bool HAS_Y, bool SYNC = false, bool ST = false>
+// TU: 0 for rows; columns otherwise, so many in LDS next to each other, read from memory by the first pass (FIRST).
+template <typename T, int P, int D, int S, bool HAS_Y, bool SYNC = false, bool ST = false, int TU = 0, bool FIRST = false>
 __device__ __forceinline__ void ipPass(T* __restrict__ rows, const StepArgs& a, const InplacePass& ps, const uint32_t b,
                                        const uint32_t E, const bool vec, const bool toMemory, const IpOut<T, HAS_Y>& o) {
   constexpr int N = ipPow(P, D), VE = 16 / (int)sizeof(T);
@@ -137,7 +141,11 @@ __device__ __forceinline__ void ipPass(T* __restrict__ rows, const StepArgs& a, 
       const uint32_t hi = S == 1 ? g : S ? g / (uint32_t)(S ? S : 1) : __umulhi(g, ps.magic);
       e0[k] = hi * (s * N) + (g - hi * s);
       if ((U > 1 || SYNC) && g >= groups) continue;
-      if (v16) {
+      if constexpr (FIRST) {
+        const uint32_t lane = o.laneIn + e0[k] / (TU ? TU : 1) * o.pitch, row = step / (TU ? TU : 1) * o.pitch;
+#pragma unroll
+        for (uint32_t i = 0; i < N; i++) x[k][i] = ipLoad<T>(o.source, lane, i * row);
+      } else if (v16) {
 #pragma unroll
         for (int i = 0; i < N / VE; i++) {
           const VT t = *(const VT*)(rows + e0[k] + i * VE);
@@ -190,16 +198,19 @@ __device__ __forceinline__ void ipPass(T* __restrict__ rows, const StepArgs& a, 
       uint32_t at = e0[k];
       if (toMemory) {
         // through buffer descriptors: one address register per group, the values' distances as scalar offsets
+        const uint32_t to = TU ? o.laneOut + e0[k] / (TU ? TU : 1) * o.pitch : e0[k] * sizeof(T);
+        const uint32_t next = TU ? step / (TU ? TU : 1) * o.pitch : step * sizeof(T);
         T yv[HAS_Y ? N : 1];
         if constexpr (HAS_Y) {
+          const uint32_t from = TU ? to - o.laneOut + o.laneY : to;
 #pragma unroll
-          for (uint32_t i = 0; i < N; i++) yv[i] = ipLoad<T>(o.yTarget, e0[k] * sizeof(T), i * step * sizeof(T));
+          for (uint32_t i = 0; i < N; i++) yv[i] = ipLoad<T>(o.yTarget, from, i * next);
         }
 #pragma unroll
         for (uint32_t i = 0; i < N; i++) {
           T v = x[k][i] * o.alpha;
           if constexpr (HAS_Y) v += o.beta * yv[i];
-          ipStore<ST>(v, o.target, e0[k] * sizeof(T), i * step * sizeof(T));
+          ipStore<ST>(v, o.target, to, i * next);
         }
       } else if (v16) {
 #pragma unroll
@@ -412,6 +423,65 @@ void kron_rows_inplace_kernel(const StepArgs a, const uint32_t total) {
   }
 }
 
+// Columns (KMM layout): all K = P^NF rows of TU neighbouring columns per workgroup.  Batch entries that share the factors
+// count as further columns, so that a few columns per entry fill the lanes as well.  The first pass reads its values from
+// memory, the last one writes its results there, lanes along the columns; LDS holds the values in between (none with a single
+// pass).  Bound: memory; 128 bytes of a row per access, the digits of one or two passes as independent loads per lane.
+// TU is 32 (fp32) and 16 (fp64, 32 for short columns): 44 to 80 KB of LDS, two or three workgroups per CU.
+// Chains of GeKMM run as groups of such launches with their digits left where they are (Handle::runColumns), us before (one
+// plain launch per factor, groups of the kernel with two LDS buffers, or fp64 factors merged to 64x64) -> after: sgekmm
+// 7^6 x 88 117 -> 55 (2 x 1.5 TB/s), 7^5 x 1024 132 -> 61, 5^6 x 1024 115 -> 54, 3^8 x 1024 67 -> 29, 8^5 x 88 27.6 -> 21,
+// dgekmm 8^5 x 88 88 -> 31, 8^3 x 787, 12 entries 76 -> 33, 6^6 x 300 237 -> 101, 5^4 x 1024 18 -> 7.
+template <int P, int NF, size_t ES, bool NARROW> struct IpCols {
+  static constexpr int K = ipPow(P, NF);
+  static constexpr int most = P == 2 ? (ES == 4 ? 6 : 3) : P == 3 ? 3 : P == 4 ? (ES == 4 ? 3 : 2) : P <= 6 || ES == 4 ? 2 : 1;
+  static constexpr int passes = (NF + most - 1) / most, D = (NF + passes - 1) / passes, N = ipPow(P, D);      // digits of every pass but the last
+  static constexpr int U = N >= 16 ? 1 : N >= 6 ? 2 : 4;
+  static constexpr int TU = passes == 1 ? 64 : NARROW ? 8 : K * 32 * (int)ES <= (ES == 4 ? 81920 : 49152) ? 32 : 16;
+  static constexpr int groups = K / N * TU, threads0 = ((groups + U - 1) / U + 63) / 64 * 64, threads = threads0 < 512 ? threads0 : 512;
+  static constexpr int lds = passes == 1 ? 0 : K * TU * (int)ES;
+  static constexpr int regs = N * U * (int)ES / 4 + (N >= 64 ? 90 : 48), byRegs = 512 / ((regs + 7) / 8 * 8);
+  static constexpr int perCU = passes == 1 ? 32 : (int)kIpLdsMax / lds, waves0 = (perCU * threads / 64 + 3) / 4;
+  static constexpr int waves1 = waves0 < byRegs ? waves0 : byRegs, waves = waves1 > 8 ? 8 : waves1;
+};
+
+template <typename T, int P, int NF, int F0, bool HAS_Y, bool NARROW>
+__device__ __forceinline__ void ipColPasses(T* cols, const StepArgs& a, const uint32_t b, const IpOut<T, HAS_Y>& o) {
+  using C = IpCols<P, NF, sizeof(T), NARROW>;
+  constexpr int D = NF - F0 < C::D ? NF - F0 : C::D;
+  constexpr bool last = F0 + D == NF;
+  InplacePass ps{};
+  ps.f0 = F0; ps.p = P; ps.d = D; ps.s = C::TU * ipPow(P, F0);
+  ipPass<T, P, D, C::TU * ipPow(P, F0), HAS_Y, false, false, C::TU, F0 == 0>(cols, a, ps, b, C::K * C::TU, false, last, o);
+  if constexpr (!last) {
+    __syncthreads();
+    ipColPasses<T, P, NF, F0 + D, HAS_Y, NARROW>(cols, a, b, o);
+  }
+}
+
+template <typename T, int P, int NF, bool HAS_Y, bool NARROW>
+__global__ __launch_bounds__((IpCols<P, NF, sizeof(T), NARROW>::threads), (IpCols<P, NF, sizeof(T), NARROW>::waves))
+void kron_cols_inplace_kernel(const StepArgs a, const uint32_t total) {
+  using C = IpCols<P, NF, sizeof(T), NARROW>;
+  constexpr uint32_t ES = sizeof(T);
+  extern __shared__ __align__(16) unsigned char ipLds[];
+  // (a grid dimension for entries with factors of their own)
+  const uint32_t b = blockIdx.y, u0 = blockIdx.x * C::TU, u = u0 + threadIdx.x % C::TU;
+  const uint32_t h0 = u0 / a.M, h = u / a.M, c = u - h * a.M, entries = a.batch / gridDim.y, hEnd = (u0 + C::TU - 1) / a.M;
+  const uint32_t more = (hEnd < entries ? hEnd : entries - 1) - h0;             // entries behind the first that the tile reaches
+  IpOut<T, HAS_Y> o;
+  o.alpha = a.epilogue ? (T)a.alpha : T(1); o.beta = (T)a.beta;
+  o.pitch = a.M * ES;
+  const bool live = u < total;
+  auto lane = [&](uint64_t stride) { return live ? (uint32_t)(((h - h0) * stride + c) * ES) : 0x7ffffff0u; };      // (others: out of range)
+  auto range = [&](uint64_t stride) { return (uint32_t)((more * stride + (uint64_t)C::K * a.M) * ES); };
+  const uint64_t e0 = (uint64_t)b + h0;
+  o.source = streamTarget((T*)a.in + e0 * a.in_batch, range(a.in_batch)); o.laneIn = lane(a.in_batch);
+  o.target = streamTarget((T*)a.out + e0 * a.out_batch, range(a.out_batch)); o.laneOut = lane(a.out_batch);
+  if (HAS_Y) { o.yTarget = streamTarget((T*)a.y + e0 * a.y_batch, range(a.y_batch)); o.laneY = lane(a.y_batch); }
+  ipColPasses<T, P, NF, 0, HAS_Y, NARROW>((T*)ipLds, a, b, o);
+}
+
 static bool ipTile(uint32_t nf, const uint32_t* p, const uint32_t* q, uint64_t Kin, uint32_t M, uint32_t batch, DType dt,
                    InplaceTile* t) {
   if (nf < 1 || nf > kMaxFused || M == 0) return false;
@@ -551,6 +621,78 @@ static hipError_t launchIpRowsAny(const StepArgs& a, const InplaceTile& t, DType
     default: return hipSuccess;
   }
 #undef IP_ROWS
+}
+
+// ---- columns ----
+template <typename T, int P, int NF, bool NARROW>
+static hipError_t launchIpColsAs(const StepArgs& a, hipStream_t stream) {
+  using C = IpCols<P, NF, sizeof(T), NARROW>;
+  static PerDeviceOnce attrOnce;
+  const int dev = launchDeviceIndex();
+  const bool own = a.batch > 1 && a.f_batch[0] != 0, y = a.y && a.epilogue;
+  const uint32_t total = own ? a.M : a.M * a.batch;
+  if (C::lds > 65536 && !attrOnce.done(dev)) {
+    for (const void* k : {(const void*)kron_cols_inplace_kernel<T, P, NF, true, NARROW>, (const void*)kron_cols_inplace_kernel<T, P, NF, false, NARROW>})
+      if (const hipError_t e = hipFuncSetAttribute(k, hipFuncAttributeMaxDynamicSharedMemorySize, (int)kIpLdsMax); e != hipSuccess) return e;
+    attrOnce.mark(dev);
+  }
+  const dim3 grid((total + C::TU - 1) / C::TU, own ? a.batch : 1);
+  if (y) hipLaunchKernelGGL((kron_cols_inplace_kernel<T, P, NF, true, NARROW>), grid, dim3(C::threads), C::lds, stream, a, total);
+  else hipLaunchKernelGGL((kron_cols_inplace_kernel<T, P, NF, false, NARROW>), grid, dim3(C::threads), C::lds, stream, a, total);
+  return hipGetLastError();
+}
+
+template <typename T, int P, int NF>
+static hipError_t launchIpCols(const StepArgs& a, hipStream_t stream) {
+  using C = IpCols<P, NF, sizeof(T), false>;
+  // Fewer than one tile for every second CU: 8 columns per workgroup spread them over four (two) times as many (sgekmm 8^5 x 2
+  // 25.4 -> 15.4 us, 7^6 x 2 17.8 -> 13.0, 5^8 x 5 29 -> 24, dgekmm 8^6 x 2 20.9 -> 18.7); with more, pieces of 32 and 64 bytes
+  // cost more than idle CUs (sgekmm 7^6 x 16 17.9 / 22.3, 6^6 x 24 12.8 / 16.5, 5^8 x 10 29 / 38).
+  if constexpr (C::K >= 200) {
+    const uint64_t columns = (uint64_t)a.M * a.batch;
+    if (2 * columns < (uint64_t)C::TU * deviceCUs()) return launchIpColsAs<T, P, NF, true>(a, stream);
+  }
+  return launchIpColsAs<T, P, NF, false>(a, stream);
+}
+
+// Most equal factors per launch: as many as 64 to 80 KB of LDS hold at 128 bytes per row.
+uint32_t colsInplaceMost(uint32_t P, DType dt) {
+  static const uint32_t most[9] = {0, 0, 6, 5, 4, 4, 3, 3, 3};
+  return P < 2 || P > 8 ? 0 : most[P];
+}
+bool colsInplaceFits(uint32_t nf, const uint32_t* p, const uint32_t* q, uint64_t Kin, DType dt) {
+  uint64_t K = 1;
+  for (uint32_t j = 0; j < nf; j++) {
+    if (p[j] != p[0] || q[j] != p[0]) return false;
+    K *= p[j];
+  }
+  return nf >= 2 && nf <= colsInplaceMost(p[0], dt) && K == Kin;
+}
+bool colsInplaceSupported(const StepArgs& a, DType dt) {
+  if (a.batch == 0 || !colsInplaceFits(a.nf, a.p, a.q, a.Kin, dt) || a.Kin != a.Kout) return false;
+  if (a.in_ldm != 1 || a.out_ldm != 1 || a.in_ldc != (int64_t)a.M || a.out_ldc != (int64_t)a.M) return false;
+  if (a.y && (a.y_ldm != 1 || a.y_ldc != (int64_t)a.M)) return false;
+  uint32_t own = 0;
+  for (uint32_t j = 0; j < a.nf; j++) {
+    if (!(a.f_sq[j] == 1 && a.f_sp[j] == (int64_t)a.q[j]) && !(a.f_sp[j] == 1 && a.f_sq[j] == (int64_t)a.p[j])) return false;
+    if (a.batch > 1 && a.f_batch[j] != 0) own++;
+  }
+  // factors of every entry's own, or none; columns are numbered in 31 bits, offsets inside a tile are
+  if (own != 0 && (own != a.nf || a.batch > 65535)) return false;
+  if ((uint64_t)a.M * (own ? 1 : a.batch) >= (1ull << 31)) return false;
+  const uint64_t widest = std::max({a.in_batch, a.out_batch, a.y ? a.y_batch : 0}), entries = own ? 1 : std::min<uint64_t>(a.batch, 64 / a.M + 2);
+  return ((entries - 1) * widest + a.Kin * a.M) * dtypeSize(dt) < (1ull << 31) - 64;
+}
+hipError_t launchColsInplace(const StepArgs& a, DType dt, hipStream_t stream) {
+  if (!colsInplaceSupported(a, dt)) return hipErrorInvalidValue;
+#define IP_COLS(P, NF) case P * 16 + NF: return dt == DType::F32 ? launchIpCols<float, P, NF>(a, stream) : launchIpCols<double, P, NF>(a, stream);
+  switch (a.p[0] * 16 + a.nf) {
+    IP_COLS(2, 2) IP_COLS(2, 3) IP_COLS(2, 4) IP_COLS(2, 5) IP_COLS(2, 6) IP_COLS(3, 2) IP_COLS(3, 3) IP_COLS(3, 4) IP_COLS(3, 5)
+    IP_COLS(4, 2) IP_COLS(4, 3) IP_COLS(4, 4) IP_COLS(5, 2) IP_COLS(5, 3) IP_COLS(5, 4) IP_COLS(6, 2) IP_COLS(6, 3)
+    IP_COLS(7, 2) IP_COLS(7, 3) IP_COLS(8, 2) IP_COLS(8, 3)
+    default: return hipErrorInvalidValue;
+  }
+#undef IP_COLS
 }
 
 hipError_t launchSmallInplace(const StepArgs& a, DType dt, hipStream_t stream) {

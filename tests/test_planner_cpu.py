@@ -662,3 +662,23 @@ def test_workgroups_of_the_backward_kernel_come_in_multiples_of_the_cus(planner,
     groups = int(step["sums"]) * -(-P // 64) * -(-Q // 64) * batch
     places = -(-groups // 256) * 256
     assert groups >= 0.75 * places, (groups, places)
+
+
+def test_gekmm_chains_of_small_factors_keep_their_digits_in_place(online_planner):
+    """Groups of equal small factors as problems on the columns behind them: their row counts, strides and batch entries; other
+    plans where factors differ per entry, X has gaps, or as many launches of the register kernels do."""
+    def groups(dt, M, Ps, **kw):
+        e, names, launches = plan(online_planner, "kmm", dt, M, Ps, Ps, **kw)
+        assert e == capi.SUCCESS
+        return [(int(l["M"]), int(l["batch"])) for l in launches] if any("columns" in n for n in names) else None
+    for dt in ("s", "d"):
+        assert groups(dt, 88, [7] * 6) == [(88, 343), (88 * 343, 1)]
+        assert groups(dt, 10, [7] * 6, batch=3, strideF=[0] * 6) == [(10, 3 * 343), (10 * 343, 3)]
+        assert groups(dt, 10, [7] * 6, batch=3) is None                                          # factors of each entry's own
+        assert groups(dt, 10, [7] * 6, batch=3, strideF=[0] * 6, strides={"x": 10 * 7 ** 6 + 8}) is None
+        assert groups(dt, 10, [7] * 3, batch=3) == [(10, 3)]                                      # whole problems: own factors as well
+        assert groups(dt, 5, [6, 6, 16, 3, 3, 3]) == [(5, 576), (5 * 27, 36), (5 * 432, 1)]
+        assert groups(dt, 9, [5] * 7, beta=0.5, y_is_z=True) == [(9, 125), (9 * 625, 1)]
+        assert groups(dt, 9, [5] * 9, temp2=False) is None                                       # three groups need two temporaries
+    assert groups("s", 1024, [8] * 5) is None and groups("s", 2048, [4] * 6) is None
+    assert groups("d", 16, [16] * 3) is None and groups("d", 3, [9, 9]) is None
