@@ -15,7 +15,7 @@ CASES = [
     (2, [7] * 3, 1), (33, [7] * 3, 1), (64, [7] * 2, 1), (65, [8] * 3, None), (130, [8] * 3, 1), (3, [8] * 5, 2), (31, [6] * 3, 1), (500, [5] * 4, 1),
     (17, [5] * 4, 1), (9, [3] * 5, 1), (70, [3] * 3, 1), (5, [4] * 4, None), (13, [4] * 3, None), (6, [2] * 6, None), (11, [2] * 5, None),
     (10, [7] * 6, 2), (88, [7] * 4, 2), (4, [5] * 7, 2), (150, [6] * 5, 2), (7, [3] * 8, 2), (23, [8] * 4, 2), (3, [7, 7, 24], 2),
-    (12, [24, 5, 5, 5], 2), (5, [6, 6, 16, 3, 3, 3], 3), (2200, [7] * 3, 1), (4100, [5] * 4, 1), (2, [3] * 10, 2),
+    (12, [24, 5, 5, 5], 2), (5, [6, 6, 16, 3, 3, 3], 3), (2200, [7] * 3, 1), (4100, [5] * 4, 1), (2, [3] * 10, 2), (40, [7] * 7, 3),
 ]
 
 
