@@ -41,6 +41,7 @@ void Handle::setPlanOnly(bool on) {
   }
   if (on && !dev_.valid) {
     // the device the library is written for: 256 compute units, 160 KB of LDS per workgroup
+    selectCache_.clear();
     dev_.cus = 256; dev_.ldsPerBlock = 160 * 1024; dev_.waveSize = 64; dev_.xcdRoundRobin = true;
   }
   if (on && !mergeWs_) {
@@ -69,6 +70,7 @@ fastKronError Handle::ensureDevice() {
   dev_.clockKHz = prop.clockRate;
   strncpy(dev_.arch, prop.gcnArchName, sizeof(dev_.arch) - 1);
   dev_.valid = true;
+  selectCache_.clear();
   if (logLevel() >= 1)
     printf("[fastkron] device %d %s: %d CUs, %d B LDS per workgroup, wave %d, %d kHz\n", d, dev_.arch,
            dev_.cus, dev_.ldsPerBlock, dev_.waveSize, dev_.clockKHz);
@@ -446,15 +448,32 @@ bool Handle::transposeFirstOnline(const KronProblem& p, const KronProblem& pn, v
   return true;
 }
 
+// What the kernels' rules look at, as bytes.
+static std::string selectionKey(const KronProblem& p, uint32_t more = 0) {
+  uint32_t key[8 + 2 * kMaxFactors];
+  uint64_t own = 0;
+  for (uint32_t i = 0; i < p.N; i++) {
+    key[8 + 2 * i] = p.P[i]; key[9 + 2 * i] = p.Q[i];
+    if (p.batch > 1 && p.strideF[i] != 0) own |= 1ull << i;
+  }
+  key[0] = (uint32_t)p.mm; key[1] = (uint32_t)p.dt | more << 8; key[2] = (uint32_t)p.opX | (p.forward ? 256u : 0u);
+  key[3] = p.M; key[4] = p.N; key[5] = p.batch; key[6] = (uint32_t)own; key[7] = (uint32_t)(own >> 32);
+  return std::string((const char*)key, sizeof(uint32_t) * (8 + 2 * p.N));
+}
+
 fastKronError Handle::runOnline(KronProblem p, void* temp1, void* temp2, const CallWorkspace* ws) {
   fastKronError e;
   if (useFusion() && p.mm == MMType::KMM && !p.forward && p.N >= 2 && p.M > 1) {
-    const std::string ck = p.str() + "_columns";
-    auto it = planCache_.find(ck);
-    if (it == planCache_.end()) it = planCache_.emplace(ck, columnsPlan(p)).first;
-    if (!it->second.empty()) {
-      e = runColumns(p, it->second, temp1, temp2);
-      if (e != fastKronKernelNotFound) return e;
+    bool pairs = false;                  // (neighbours that a group could hold)
+    for (uint32_t i = 1; i < p.N; i++) pairs = pairs || (p.P[i] <= 8 && p.P[i] == p.P[i - 1] && p.P[i] == p.Q[i] && p.P[i] == p.Q[i - 1]);
+    if (pairs) {
+      const std::string ck = selectionKey(p, p.strideX == (uint64_t)p.M * p.K() ? 1 : 2);
+      auto it = selectCache_.find(ck);
+      if (it == selectCache_.end()) it = selectCache_.emplace(ck, columnsPlan(p)).first;
+      if (!it->second.empty()) {
+        e = runColumns(p, it->second, temp1, temp2);
+        if (e != fastKronKernelNotFound) return e;
+      }
     }
   }
   {
@@ -519,6 +538,13 @@ fastKronError Handle::runOnline(KronProblem p, void* temp1, void* temp2, const C
   return execute(p, plan, temp1, temp2);
 }
 
+const Plan& Handle::select(const KronProblem& p) const {
+  const std::string key = selectionKey(p);
+  auto it = selectCache_.find(key);
+  if (it == selectCache_.end()) it = selectCache_.emplace(key, db_.selectOnline(p, dev_, true)).first;
+  return it->second;
+}
+
 static bool isPow2(uint32_t v) { return v && !(v & (v - 1)); }
 
 bool Handle::mergeSmallFactors(const KronProblem& p, KronProblem* out, const CallWorkspace* ws) {
@@ -538,7 +564,7 @@ bool Handle::mergeSmallFactors(const KronProblem& p, KronProblem* out, const Cal
     bool all8 = true;
     for (uint32_t i = 0; i < p.N; i++) all8 = all8 && p.P[i] == 8 && p.Q[i] == 8;
     if (all8) {
-      const Plan whole = db_.selectOnline(p, dev_, true);
+      const Plan& whole = select(p);
       if (whole.size() == 1 && whole[0].lo == 0 && whole[0].hi == 4) return false;
     }
   }
@@ -785,7 +811,7 @@ Plan Handle::columnsPlan(const KronProblem& p) const {
     }
     KronProblem q;
     if (!columnsPart(p, (uint32_t)lo, (uint32_t)hi, &q)) return Plan();
-    const Plan one = db_.selectOnline(q, dev_, true);
+    const Plan& one = select(q);
     if (one.size() != 1) return Plan();
     plan.push_back(PlanStep{(uint32_t)lo, (uint32_t)hi, one[0].kernel});
     if (lo < hi) grouped = true;
@@ -806,7 +832,7 @@ Plan Handle::columnsPlan(const KronProblem& p) const {
     if (self->mergeSmallFactors(p, &q)) merge = 1;
     self->planOnly_ = was;
   }
-  const Plan other = db_.selectOnline(q, dev_, true);
+  const Plan& other = select(q);
   bool lds = false, merged16 = merge != 0;
   for (auto& s : other) lds = lds || db_.kernels()[s.kernel].name.find("_small_fused_lds_") != std::string::npos;
   for (uint32_t i = 0; i < q.N; i++) merged16 = merged16 && q.P[i] <= 16;
@@ -848,18 +874,23 @@ fastKronError Handle::trySplitLeadingTrailing(const KronProblem& p, void* temp1,
   // fp32 8x8 (five), 16x16 (four), 32x32 (three), 64x64 (two); fp64 16x16 (three), 32x32 or 64x64 (two);
   // 9x9 ... 15x15 (three, either type); 3x3, 5x5, 6x6, 7x7 (eight, six, five, five, either type)
   const uint32_t tp = p.P[p.N - 1], tq = p.Q[p.N - 1];
-  if (tq != tp) {
-    // two trailing rectangular factors of a shape the pair kernel has exact tiles for (32x64, 64x32)
-    if (p.P[p.N - 2] != tp || p.Q[p.N - 2] != tq) return fastKronKernelNotFound;
+  // two trailing factors of other shapes on one of the pair kernels (exact tiles for 32x64 and 64x32, padded ones up to 64), where
+  // that takes fewer launches: (31x63)^3 on one row 18.3 -> 11.3 us, 10 x 50^3 31.7 -> 21.8, 80 x 63^3 176 -> 130, 10 x 6x6x50x50
+  // 28.9 -> 17.2.  Not with fewer than 256 columns for the leading factors to run along (80 x 50x2x50 21.7 / 26.9), and not for
+  // many blocks of 33 to 47 rows a side, which the padded step reads in whole pieces (80 x 40^3 49.2 / 52.0, 500 x 36^3 174 / 191).
+  auto trailingPair = [&]() -> fastKronError {
     const uint32_t g2 = p.N - 2;
     KronProblem r1, r2;
     if (!buildSplit(p, g2, temp1, temp2, &r1, &r2)) return fastKronKernelNotFound;
-    Plan rp1 = db_.selectOnline(r1, dev_, true);
+    if (r2.M < 256 || (tp == tq && tp > 32 && tp < 48 && (uint64_t)r1.M * r1.batch >= 2048)) return fastKronKernelNotFound;
+    const Plan& rp1 = select(r1);
     if (rp1.size() != 1 || db_.kernels()[rp1[0].kernel].fused != 2 || db_.kernels()[rp1[0].kernel].P == 0)
       return fastKronKernelNotFound;
-    Plan rp2 = db_.selectOnline(r2, dev_, true);
+    const Plan& rp2 = select(r2);
+    if (1 + rp2.size() >= select(p).size()) return fastKronKernelNotFound;
     return runSplit(p, g2, r1, rp1, r2, rp2, temp2);
-  }
+  };
+  if (tq != tp || p.P[p.N - 2] != tp || p.Q[p.N - 2] != tq || (tp > 32 && tp < 64)) return trailingPair();
   uint32_t maxT = 0;
   if (tp == 32 && p.dt == DType::F32) maxT = 3;      // three 32x32 fp32 factors fused per 32768-column block
   else if (tp == 32 || tp == 64)      maxT = 2;
@@ -898,9 +929,9 @@ fastKronError Handle::trySplitLeadingTrailing(const KronProblem& p, void* temp1,
   const uint32_t g = p.N - nT;
   KronProblem q1, q2;
   if (!buildSplit(p, g, temp1, temp2, &q1, &q2)) return fastKronKernelNotFound;
-  Plan plan1 = db_.selectOnline(q1, dev_, true);
+  const Plan& plan1 = select(q1);
   if (plan1.size() != 1 || db_.kernels()[plan1[0].kernel].P == 0) return fastKronKernelNotFound;
-  Plan plan2 = db_.selectOnline(q2, dev_, true);
+  const Plan& plan2 = select(q2);
   return runSplit(p, g, q1, plan1, q2, plan2, temp2);
 }
 

@@ -81,6 +81,9 @@ class Handle {
   // is ahead; runColumns: fastKronKernelNotFound when the plan or the buffers do not have that form.
   bool columnsPart(const KronProblem& p, uint32_t lo, uint32_t hi, KronProblem* q) const;
   Plan columnsPlan(const KronProblem& p) const;
+  // The online selection with fusion, kept per problem as its rules see it (the parts of two-part plans are asked for on every
+  // call: sgemkm 1 x 24^3 spent 5 us there).
+  const Plan& select(const KronProblem& p) const;
   fastKronError runColumns(const KronProblem& p, const Plan& plan, void* temp1, void* temp2);
   // Chains of 2x2 / 4x4 (fp64: also 8x8) factors: adjacent factors are replaced by their Kronecker product
   // (16x16; 64x64 in fp64 when the chain holds 8x8 or 32x32 factors), computed into the handle's workspace by one small launch, so that the
@@ -129,6 +132,7 @@ class Handle {
   DeviceInfo dev_;
   KernelDB db_;
   std::unordered_map<std::string, Plan> planCache_;   // online selections, per problem string
+  mutable std::unordered_map<std::string, Plan> selectCache_;   // ... per what the kernels' rules look at
   std::unordered_map<std::string, bool> transposeCache_;   // op(X) = T: transpose first or not, per problem string
   std::string dbPath_;
   std::string lastPlan_;

@@ -1,4 +1,5 @@
 #include "kernel_db.h"
+#include <algorithm>
 
 #include <dlfcn.h>
 
@@ -136,7 +137,38 @@ static hipError_t stepAnyLaunch(const KernelInfo& k, const StepArgs& a, hipStrea
 }
 static bool stepAnyCheck(const KernelInfo& k, const StepArgs& a) { return stepAnyMfmaSupported(a, k.dt); }
 
+// ---- two factors of any sizes up to 64x64 on the matrix cores (zero padded), whole rows ----
+static bool pairAnyCanRun(const KernelInfo& k, const KronProblem& p, uint32_t lo, uint32_t hi, bool first, bool,
+                          const DeviceInfo& dev) {
+  if (k.dt != p.dt || p.mm != MMType::MKM || hi - lo + 1 != 2 || p.forward) return false;
+  if (first && p.opX == 2) return false;
+  const uint32_t ps[2] = {p.P[hi], p.P[lo]}, qs[2] = {p.Q[hi], p.Q[lo]};
+  if (dev.rulesOfThumb) {
+    // Ahead of a launch per factor at every size measured (0.25 to 0.9 of their time, 1 to 20000 rows, either type), except:
+    // factors of at most 8 rows and columns, which go through LDS together with more of their kind;
+    if (std::max({ps[0], ps[1], qs[0], qs[1]}) <= 8) return false;
+    // 64x64 and (fp64) 64x32, whose single steps have kernels and plans of their own;
+    if (ps[0] == 64 && ps[1] == 64 && qs[0] == qs[1] && (qs[0] == 64 || (qs[0] == 32 && p.dt == DType::F64))) return false;
+    // many rows of which most of the padded products are for nothing (33x33: 2.7 times the real ones; sgemkm 5000 rows 48.6 ->
+    // 45.7 us, 20000 rows 146 / 161; with factors of one block of 16 the products are not what bounds it).
+    auto blocks = [](uint32_t n) { return (uint64_t)(n + 15) / 16; };
+    const uint64_t padded = 1024 * blocks(ps[1]) * blocks(qs[0]) * ((ps[0] + 3) / 4 + 4 * blocks(qs[1]));
+    const uint64_t real = (uint64_t)ps[1] * qs[0] * (ps[0] + qs[1]);
+    if ((uint64_t)p.M * p.batch >= 8192 && 2 * padded > 5 * real && std::max(ps[0], ps[1]) > 16) return false;
+  }
+  return dev.ldsPerBlock >= 160 * 1024 && pairAnyFits(2, ps, qs, p.colsBefore(hi));
+}
+static hipError_t pairAnyLaunch(const KernelInfo& k, const StepArgs& a, hipStream_t s) { return launchPairAny(a, k.dt, s); }
+static bool pairAnyCheck(const KernelInfo& k, const StepArgs& a) { return pairAnySupported(a, k.dt); }
+
 void registerGenericKernels(std::vector<KernelInfo>& out) {
+  for (DType dt : {DType::F32, DType::F64}) {
+    KernelInfo k{};
+    k.name = std::string("mkm_hip_gfx950_256_") + (dt == DType::F32 ? "f" : "d") + "_anyxany_64x64_2_1xany_mfma16x16x4";
+    k.dt = dt; k.P = 1; k.Q = 1; k.fused = 2; k.tileM = 0; k.tileK = 0; k.threads = 256; k.variant = 0;
+    k.canRun = pairAnyCanRun; k.launch = pairAnyLaunch; k.check = pairAnyCheck;
+    out.push_back(k);
+  }
   for (DType dt : {DType::F32, DType::F64}) {
     KernelInfo k{};
     k.name = std::string("gekmm_hip_gfx950_512_") + (dt == DType::F32 ? "f" : "d") + "_anyxany_256x512_1_16xany_mfma16x16x4";

@@ -103,6 +103,11 @@ hipError_t launchRow32x3p(const StepArgs& a, hipStream_t stream);
 bool pairMfmaSupported(const StepArgs& a, DType dt);
 hipError_t launchPairMfma(const StepArgs& a, DType dt, hipStream_t stream);
 
+// Two fused factors of any sizes up to 64 on rows of exactly P1*P2 columns (MKM layout), fp32 or fp64.
+bool pairAnyFits(uint32_t nf, const uint32_t* p, const uint32_t* q, uint64_t Kin);
+bool pairAnySupported(const StepArgs& a, DType dt);
+hipError_t launchPairAny(const StepArgs& a, DType dt, hipStream_t stream);
+
 // Three fused 8x8 fp32 factors in the KMM layout, 512 rows by 64 columns per workgroup.
 bool kmm8x3Supported(const StepArgs& a);
 hipError_t launchKmm8x3(const StepArgs& a, hipStream_t stream);
