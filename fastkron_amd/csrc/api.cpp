@@ -305,6 +305,22 @@ fastKronError fastKronGradSizes(fastKronHandle handle, int mkm, int dbl, uint32_
                                           batchCount), saveElems, workElems);
 }
 
+fastKronError fastKronProductOuter(fastKronHandle handle, int mkm, int dbl, uint32_t M, uint32_t N, const uint32_t Ps[], const uint32_t Qs[],
+                                   const void* X, fastKronOp opX, const uint64_t strideX[2], const void* const Fs[], fastKronOp opFs, void* Z,
+                                   const uint64_t strideZ[2], double alpha, double beta, const uint32_t count[2], const void* Y,
+                                   const uint64_t strideY[2], void* temp1, void* temp2) {
+  if (!handle || !Fs || !Ps || !Qs || !strideX || !strideZ || !count || (Y && !strideY)) return fastKronInvalidArgument;
+  if (N == 0 || N > kMaxFactors) return fastKronInvalidKMMProblem;
+  KronProblem p{};
+  p.mm = mkm ? MMType::MKM : MMType::KMM; p.dt = dbl ? DType::F64 : DType::F32;
+  p.M = M; p.N = N;
+  for (uint32_t i = 0; i < N; i++) { p.P[i] = Ps[i]; p.Q[i] = Qs[i]; p.F[i] = Fs[i]; p.strideF[i] = (uint64_t)Ps[i] * Qs[i]; }
+  p.X = X; p.opX = opX; p.opF = opFs; p.Z = Z; p.Y = Y;
+  p.strideX = strideX[1]; p.strideZ = strideZ[1]; p.strideY = Y ? strideY[1] : 0;
+  p.alpha = alpha; p.beta = beta; p.batch = count[1]; p.strided = true;
+  return H(handle)->xgemmOuter(p, count[0], strideX[0], strideZ[0], Y ? strideY[0] : 0, fastKronBackend_HIP, temp1, temp2);
+}
+
 fastKronError fastKronGradForward(fastKronHandle handle, int mkm, int dbl, uint32_t M, uint32_t N, const uint32_t Ps[],
                                   const uint32_t Qs[], const void* X, fastKronOp opX, uint64_t strideX, const void* const Fs[],
                                   fastKronOp opFs, int perBatchFs, uint32_t batchCount, void* Z, void* save) {

@@ -9,7 +9,8 @@
 // to be recorded for gradients.
 //
 // Rules (reference pyfastkron/fastkronbase.py:104-518): leading dimensions are batches, broadcast between X, the factors
-// and Y; the innermost batch dimension is one strided-batched call (stride 0 = shared operand), outer ones a loop; a
+// and Y; neighbouring ones that all operands have alike are one; one dimension is a strided-batched call (stride 0 = shared
+// operand), two of which the factors have one a call with both, otherwise the largest is the call's and the others a loop; a
 // batch of X against shared factors is more rows of one problem (MKM); transposed views are passed as their buffer.
 #include <Python.h>
 #include <torch/csrc/Exceptions.h>
@@ -37,6 +38,7 @@ struct Api {
   decltype(&sgemkmStridedBatched) sgemkmB; decltype(&dgemkmStridedBatched) dgemkmB;
   decltype(&sgekmmStridedBatched) sgekmmB; decltype(&dgekmmStridedBatched) dgekmmB;
   decltype(&gekmmSizes) sizes; decltype(&fastKronSetStream) setStream;
+  decltype(&fastKronProductOuter) productOuter;
   decltype(&fastKronGradSizes) gradSizes; decltype(&fastKronGradForward) gradForward; decltype(&fastKronGradBackwardSteps) gradSteps;
 } api;
 
@@ -214,13 +216,42 @@ PyObject* product(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
   const bool fold = o.folds() && (!y.defined() || yb == o.zb);
   const int64_t M = fold ? o.M * prod(o.zb) : o.M;
   const bool one = fold || o.zb.empty();
-  const int64_t inner = one ? 1 : o.zb.back();
-  if (inner > kMaxCount) return failed(fastKronInvalidKMMProblem);
+  // batch dimensions as steps of every operand in entries, neighbours merged where all operands go on in one
+  struct Dim { int64_t n, x, f, y, z; };
+  c10::SmallVector<Dim, 8> dims;
+  if (!one) {
+    if (o.zb.back() > kMaxCount) return failed(fastKronInvalidKMMProblem);
+    int64_t x = 1, f = 1, s = 1, zz = 1;
+    auto step = [](const Dims& b, size_t fromBack, int64_t* run) {
+      if (fromBack >= b.size() || b[b.size() - 1 - fromBack] == 1) return (int64_t)0;
+      const int64_t r = *run;
+      *run *= b[b.size() - 1 - fromBack];
+      return r;
+    };
+    for (size_t i = 0; i < o.zb.size(); i++) {
+      const int64_t n = o.zb[o.zb.size() - 1 - i];
+      Dim d{n, step(o.xb, i, &x), step(o.fb, i, &f), step(yb, i, &s), zz};
+      zz *= n;
+      if (!dims.empty() && prod(o.zb) > 0) {
+        Dim& in = dims.back();
+        if (n == 1) continue;
+        if (in.n == 1) { in = d; continue; }
+        if (d.x == in.x * in.n && d.f == in.f * in.n && d.y == in.y * in.n && in.n * n <= kMaxCount) { in.n *= n; continue; }
+      }
+      dims.push_back(d);
+    }
+  }
+  size_t largest = 0;
+  for (size_t i = 1; i < dims.size(); i++) if (dims[i].n > dims[largest].n && prod(o.zb) > 0 && dims[i].n <= kMaxCount) largest = i;
+  const int64_t inner = one ? 1 : dims[largest].n;
   size_t ye = 0, te = 0;
   fastKronError e = api.sizes(c.handle, (uint32_t)M, o.N, o.Ps, o.Qs, &ye, &te);
   if (e != fastKronSuccess) return failed(e);
   // both temporaries in one allocation, each on a 256-byte boundary
-  const size_t tn = te * (size_t)inner, off = (tn * es + 255) / 256 * 256 / es;
+  // (two dimensions at once only while the temporaries stay small beside the operands)
+  const size_t withF = dims.size() == 2 ? (dims[0].f != 0) + (dims[1].f != 0) : 0;
+  const bool both = withF == 1 && prod(o.zb) > 0 && prod(o.zb) <= 65535 && te * (size_t)prod(o.zb) * es <= (size_t)256 << 20;
+  const size_t tn = te * (size_t)(both ? prod(o.zb) : inner), off = (tn * es + 255) / 256 * 256 / es;
   Tensor temp = at::empty({(int64_t)(off + tn)}, o.x.options());
   char* t1 = (char*)temp.data_ptr();
   char* t2 = t1 ? t1 + off * es : nullptr;
@@ -233,28 +264,33 @@ PyObject* product(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
       for (uint32_t i = 0; i < o.N; i++) f[i] = o.f[i].data_ptr();
       return call(c, o, (uint32_t)M, o.x.data_ptr(), f, z.data_ptr(), alpha, beta, y.defined() ? y.data_ptr() : nullptr, t1, t2);
     }
-    const size_t d = o.zb.size();
-    // element offset of the entry `idx` (innermost index 0) of an operand with batch dimensions `b` broadcast to zb's
-    auto entry = [&](const Dims& b, const Dims& idx) {
-      int64_t lin = 0;
-      for (size_t i = 0; i < b.size(); i++) lin = lin * b[i] + (b[i] > 1 ? idx[d - b.size() + i] : 0);
-      return lin;
-    };
-    auto step = [&](const Dims& b) { return !b.empty() && b.back() > 1 ? 1 : 0; };
     const int64_t xblk = o.M * o.K, zblk = o.M * o.L;
+    if (both) {
+      const Dim& in = dims[dims[0].f != 0 ? 0 : 1], & out = dims[dims[0].f != 0 ? 1 : 0];
+      const uint64_t sx[2] = {(uint64_t)(out.x * xblk), (uint64_t)(in.x * xblk)}, sz[2] = {(uint64_t)(out.z * zblk), (uint64_t)(in.z * zblk)};
+      const uint64_t sy[2] = {(uint64_t)(out.y * zblk), (uint64_t)(in.y * zblk)};
+      const uint32_t count[2] = {(uint32_t)out.n, (uint32_t)in.n};
+      for (uint32_t i = 0; i < o.N; i++) f[i] = o.f[i].data_ptr();
+      return api.productOuter(c.handle, mkm, o.f64(), (uint32_t)o.M, o.N, o.Ps, o.Qs, o.x.data_ptr(), o.opX, sx, f, o.opF, z.data_ptr(), sz, alpha,
+                              beta, count, y.defined() ? y.data_ptr() : nullptr, sy, t1, t2);
+    }
+    const Dim in = dims[largest];
     uint64_t sf[kMaxFactors];
-    for (uint32_t i = 0; i < o.N; i++) sf[i] = step(o.fb) ? (uint64_t)o.Ps[i] * o.Qs[i] : 0;
-    const int64_t outer = prod(at::IntArrayRef(o.zb.data(), d - 1));
-    Dims idx(d, 0);
+    for (uint32_t i = 0; i < o.N; i++) sf[i] = (uint64_t)in.f * o.Ps[i] * o.Qs[i];
+    int64_t outer = 1;
+    for (size_t i = 0; i < dims.size(); i++) if (i != largest) outer *= dims[i].n;
     for (int64_t lin = 0; lin < outer; lin++) {
-      int64_t rem = lin;
-      for (size_t i = d - 1; i-- > 0;) { idx[i] = rem % o.zb[i]; rem /= o.zb[i]; }
-      const int64_t fo = entry(o.fb, idx);
+      int64_t rem = lin, xo = 0, fo = 0, yo = 0, zo = 0;
+      for (size_t i = 0; i < dims.size(); i++) {
+        if (i == largest) continue;
+        const int64_t k = rem % dims[i].n;
+        rem /= dims[i].n;
+        xo += k * dims[i].x; fo += k * dims[i].f; yo += k * dims[i].y; zo += k * dims[i].z;
+      }
       for (uint32_t i = 0; i < o.N; i++) f[i] = (char*)o.f[i].data_ptr() + (size_t)fo * o.Ps[i] * o.Qs[i] * es;
-      e = callBatched(c, o, (char*)o.x.data_ptr() + (size_t)(entry(o.xb, idx) * xblk) * es, step(o.xb) ? xblk : 0, f, sf,
-                      (char*)z.data_ptr() + (size_t)(entry(o.zb, idx) * zblk) * es, zblk, alpha, beta, (uint32_t)inner,
-                      y.defined() ? (char*)y.data_ptr() + (size_t)(entry(yb, idx) * zblk) * es : nullptr, y.defined() && step(yb) ? zblk : 0, t1,
-                      t2);
+      e = callBatched(c, o, (char*)o.x.data_ptr() + (size_t)(xo * xblk) * es, in.x * xblk, f, sf, (char*)z.data_ptr() + (size_t)(zo * zblk) * es,
+                      in.z * zblk, alpha, beta, (uint32_t)inner, y.defined() ? (char*)y.data_ptr() + (size_t)(yo * zblk) * es : nullptr,
+                      y.defined() ? in.y * zblk : 0, t1, t2);
       if (e != fastKronSuccess) return e;
     }
     return e;

@@ -254,6 +254,83 @@ fastKronError Handle::xgemm(KronProblem p, fastKronBackend backend, void* temp1,
   return runOnline(p, temp1, temp2, ws);
 }
 
+fastKronError Handle::xgemmOuter(const KronProblem& p, uint32_t outer, uint64_t outerX, uint64_t outerZ, uint64_t outerY,
+                                 fastKronBackend backend, void* temp1, void* temp2) {
+  if (outer == 0) return fastKronInvalidKMMProblem;
+  if (outer > 1) {
+    const fastKronError e = runOuter(p, outer, outerX, outerZ, outerY, temp1, temp2);
+    if (e != fastKronKernelNotFound) return e;
+  }
+  const size_t es = dtypeSize(p.dt);
+  if (outer > p.batch) {
+    // fewer factors than outer entries: a call for each of them, the outer dimension as its batch
+    for (uint32_t i = 0; i < p.batch; i++) {
+      KronProblem q = p;
+      q.batch = outer;
+      q.X = (const char*)p.X + (size_t)i * p.strideX * es; q.strideX = outerX;
+      q.Z = (char*)p.Z + (size_t)i * p.strideZ * es; q.strideZ = outerZ;
+      if (p.Y) { q.Y = (const char*)p.Y + (size_t)i * p.strideY * es; q.strideY = outerY; }
+      for (uint32_t j = 0; j < p.N && j < kMaxFactors; j++) {
+        if (p.F[j]) q.F[j] = (const char*)p.F[j] + (size_t)i * p.strideF[j] * es;
+        q.strideF[j] = 0;
+      }
+      if (const fastKronError e = xgemm(q, backend, temp1, temp2); e != fastKronSuccess) return e;
+    }
+    return fastKronSuccess;
+  }
+  for (uint32_t o = 0; o < outer; o++) {
+    KronProblem q = p;
+    q.X = (const char*)p.X + (size_t)o * outerX * es;
+    q.Z = (char*)p.Z + (size_t)o * outerZ * es;
+    if (p.Y) q.Y = (const char*)p.Y + (size_t)o * outerY * es;
+    if (const fastKronError e = xgemm(q, backend, temp1, temp2); e != fastKronSuccess) return e;
+  }
+  return fastKronSuccess;
+}
+
+// fastKronKernelNotFound: not in this form (nothing has been launched).
+fastKronError Handle::runOuter(const KronProblem& p0, uint32_t outer, uint64_t outerX, uint64_t outerZ, uint64_t outerY, void* temp1, void* temp2) {
+  KronProblem p = p0;
+  if (!p.X || !p.Z || !temp1 || !temp2 || p.N == 0 || p.N > kMaxFactors || p.M == 0 || p.batch == 0 || p.forward || !useFusion() || canTune())
+    return fastKronKernelNotFound;
+  if ((uint64_t)outer * p.batch > 65535) return fastKronKernelNotFound;
+  for (uint32_t i = 0; i < p.N; i++) if (p.P[i] == 0 || p.Q[i] == 0 || !p.F[i] || p.strideF[i] == 0) return fastKronKernelNotFound;
+  if (p.mm == MMType::KMM && (p.M == 1 || p.opX == fastKronOp_T || viaMKMOnline(p))) return fastKronKernelNotFound;
+  Choice tuned;
+  if (lookupChoice(p, &tuned)) return fastKronKernelNotFound;
+  if (const fastKronError e = planOnly_ ? fastKronSuccess : ensureDevice(); e != fastKronSuccess) return e;
+  callWs_ = false;
+  const uint32_t inner = p.batch;
+  KronProblem x = p;                       // the transposed copy: X's own entries only
+  bool copy = false;
+  if (p.opX == fastKronOp_T) {
+    KronProblem pn;
+    void* xt = nullptr;
+    if (!transposedProblem(p, temp1, temp2, &pn, &xt)) return fastKronKernelNotFound;
+    if (transposeFirstOnline(p, pn, temp1, temp2, nullptr)) {
+      if (inner > 1 && p.strideX != 0 && outerX != inner * p.strideX) return fastKronKernelNotFound;
+      copy = true;
+      x.batch = inner > 1 && p.strideX != 0 ? outer * inner : outer;
+      x.strideX = x.batch > outer ? p.strideX : outerX;
+      p = pn;
+      outerX = (uint64_t)p.M * p.K() * (x.batch / outer);
+    }
+  }
+  p.inner = inner; p.batch = outer * inner; p.strided = true;
+  p.outerX = outerX; p.outerZ = outerZ; p.outerY = outerY;
+  KronProblem flat = p;
+  const Plan& plan = select(flat);
+  if (execute(p, plan, temp1, temp2, true) != fastKronSuccess) return fastKronKernelNotFound;
+  lastPlan_ = p.str();
+  for (auto& s : plan) lastPlan_ += ";" + std::to_string(s.lo) + "-" + std::to_string(s.hi) + ":" + db_.kernels()[s.kernel].name;
+  launchLog_.clear();
+  if (planOnly_) return execute(p, plan, temp1, temp2, true);
+  if (copy && launchTransposeX(x, const_cast<void*>(p.X), (uint64_t)p.M * p.K()) != hipSuccess) return fastKronInvalidArgument;
+  const fastKronError e = execute(p, plan, temp1, temp2);
+  if (e == fastKronSuccess && copy) noteTranspose(x);
+  return e;
+}
+
 // Online rule for a GeKMM with op(X) = T: as the GeMKM of the same buffer plus a transposition of the result.
 // FASTKRON_KMM_VIA_MKM=0 / 1 forces the answer.
 bool Handle::viaMKMOnline(const KronProblem& p) const {
@@ -1062,6 +1139,7 @@ fastKronError Handle::execute(const KronProblem& p, const Plan& plan, void* temp
     if (s.hi - s.lo + 1 > kMaxFused) return fastKronKernelNotFound;
     StepArgs a = makeStepArgs(p, s.lo, s.hi, first, last);
     a.in = in; a.in_batch = inBatch;
+    if (p.inner && !k.outer) { if (refused) *refused = s.kernel; return fastKronKernelNotFound; }
     if (last) {
       a.out = p.Z; a.out_batch = p.strideZ;
     } else if (p.forward) {
@@ -1077,6 +1155,12 @@ fastKronError Handle::execute(const KronProblem& p, const Plan& plan, void* temp
         if (p.batch > 1) a.out_batch = p.strideZ;
       }
       if (a.out == nullptr) return fastKronInvalidArgument;
+    }
+    if (p.inner) {
+      a.inner = p.inner;
+      a.outer.in = first ? p.outerX : p.inner * a.in_batch;
+      a.outer.out = last ? p.outerZ : p.inner * a.out_batch;
+      a.outer.y = p.outerY;
     }
     {
       // Non-temporal hints (StepArgs::stream_in / stream_out).  Measured: an intermediate of 134 MB is read back
@@ -1117,7 +1201,9 @@ fastKronError Handle::execute(const KronProblem& p, const Plan& plan, void* temp
       for (uint32_t j = 0; j < a.nf && j < kMaxFused; j++)
         c.f[j] = (const char*)a.f[j] + (size_t)b0 * a.f_batch[j] * es;
       if (dryRun) {
-        if (k.check && !k.check(k, c)) {                                // every chunk: its base pointers differ
+        StepArgs c2 = c;                                                // (alignment of both batch dimensions)
+        if (c.inner) { c2.in_batch = c.outer.in; c2.out_batch = c.outer.out; c2.y_batch = c.outer.y; }
+        if (k.check && (!k.check(k, c) || (c.inner && !k.check(k, c2)))) {  // every chunk: its base pointers differ
           if (refused) *refused = s.kernel;
           return fastKronKernelNotFound;
         }

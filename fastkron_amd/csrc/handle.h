@@ -44,6 +44,13 @@ class Handle {
   struct CallWorkspace { void* merge; size_t mergeBytes; };
   fastKronError xgemm(KronProblem p, fastKronBackend backend, void* temp1, void* temp2, const CallWorkspace* ws = nullptr);
 
+  // The same with a second batch dimension: `outer` times the problem p with X, Z and Y that many elements on each time, the
+  // factors the same.  One series of launches where every kernel takes both dimensions, otherwise one call per outer entry;
+  // the temporaries hold outer * p.batch entries.
+  fastKronError xgemmOuter(const KronProblem& p, uint32_t outer, uint64_t outerX, uint64_t outerZ, uint64_t outerY, fastKronBackend backend,
+                           void* temp1, void* temp2);
+  fastKronError runOuter(const KronProblem& p, uint32_t outer, uint64_t outerX, uint64_t outerZ, uint64_t outerY, void* temp1, void* temp2);
+
   // Runs `plan` on the stream; temps may be null when the plan has a single launch.
   // dryRun: only the kernels' checks of the concrete buffers run; *refused then names the kernel that said no
   fastKronError execute(const KronProblem& p, const Plan& plan, void* temp1, void* temp2, bool dryRun = false,

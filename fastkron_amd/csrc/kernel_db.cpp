@@ -1,5 +1,6 @@
 #include "kernel_db.h"
 #include <algorithm>
+#include <charconv>
 
 #include <dlfcn.h>
 
@@ -13,27 +14,30 @@
 
 namespace fk {
 
+// (Every call looks its problem up: put together in a buffer, as a stream the name took 1 us of host time each time.)
 std::string KronProblem::str() const {
-  std::ostringstream o;
+  char buf[48 * kMaxFactors / 2 + 192], *c = buf, *const end = buf + sizeof(buf);
+  auto num = [&](uint64_t v) { c = std::to_chars(c, end, v).ptr; };
+  auto text = [&](const char* t) { while (*t) *c++ = *t++; };
   auto facs = [&]() {
-    if (sameShapes(0, N - 1)) o << P[0] << "x" << Q[0] << "^" << N;
-    else for (uint32_t i = 0; i < N; i++) { o << P[i] << "x" << Q[i]; if (i + 1 < N) o << "(x)"; }
+    if (sameShapes(0, N - 1)) { num(P[0]); text("x"); num(Q[0]); text("^"); num(N); }
+    else for (uint32_t i = 0; i < N; i++) { num(P[i]); text("x"); num(Q[i]); if (i + 1 < N) text("(x)"); }
   };
-  if (mm == MMType::MKM) { o << M << "x" << K() << "*("; facs(); o << ")"; }
-  else                   { o << "("; facs(); o << ")*" << K() << "x" << M; }
-  o << "_" << (opX == 2 ? "T" : "N") << (opF == 2 ? "T" : "N") << "_" << (dt == DType::F32 ? "f" : "d");
+  if (mm == MMType::MKM) { num(M); text("x"); num(K()); text("*("); facs(); text(")"); }
+  else                   { text("("); facs(); text(")*"); num(K()); text("x"); num(M); }
+  text("_"); text(opX == 2 ? "T" : "N"); text(opF == 2 ? "T" : "N"); text("_"); text(dt == DType::F32 ? "f" : "d");
   if (strided) {
-    o << "_stridedBatched_" << batch;
+    text("_stridedBatched_"); num(batch);
     // the stride class: a shared X and shared factors change which kernels and rewritings apply (merging, the
     // two-part plan), so plans of one class are not looked up for another.  Per-batch operands carry no suffix.
     if (batch > 1) {
-      if (strideX == 0) o << "_Xs";
+      if (strideX == 0) text("_Xs");
       uint64_t shared = 0;
       for (uint32_t i = 0; i < N; i++) if (strideF[i] == 0) shared |= 1ull << i;
-      if (shared) o << "_Fs" << std::hex << shared << std::dec;
+      if (shared) { text("_Fs"); c = std::to_chars(c, end, shared, 16).ptr; }
     }
   }
-  return o.str();
+  return std::string(buf, c);
 }
 
 static bool genericCanRun(const KernelInfo& k, const KronProblem& p, uint32_t lo, uint32_t hi, bool, bool,
@@ -666,6 +670,10 @@ void registerRowKernels(std::vector<KernelInfo>& out) {
 KernelDB::KernelDB() {
   registerRowKernels(kernels_);
   registerGenericKernels(kernels_);
+  // (those with a grid dimension for the outer entries)
+  for (KernelInfo& k : kernels_)
+    for (LaunchFn f : {(LaunchFn)genericLaunch, (LaunchFn)row8Launch, (LaunchFn)pairAnyLaunch, (LaunchFn)smallInplaceLaunch})
+      k.outer = k.outer || k.launch == f;
 }
 
 int KernelDB::findByName(const std::string& name) const {

@@ -47,6 +47,7 @@ struct KernelInfo {
   uint32_t threads;
   uint32_t variant;       // kernel-family specific
   bool     tunerOnly;     // a candidate for the tuner, never chosen by the online selection
+  bool     outer;         // takes two batch dimensions (StepArgs::inner)
   bool     usesSync;      // synchronises its workgroups through the handle's counter area (StepArgs::sync)
   CanRunFn canRun;
   LaunchFn launch;

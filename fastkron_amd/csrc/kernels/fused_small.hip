@@ -139,7 +139,7 @@ __device__ __forceinline__ void fsLocalStep(const T* __restrict__ src, T* __rest
 }
 
 template <typename T, int MODE, bool HAS_Y>
-__global__ __launch_bounds__(kFsThreads, 4) void kron_fused_small_kernel(const StepArgs a, const FusedTile t) {
+__global__ __launch_bounds__(kFsThreads, 4) void kron_fused_small_kernel(const KernelArgs a, const FusedTile t) {
   extern __shared__ __align__(16) unsigned char fsLds[];
   T* const lds = (T*)fsLds;                  // two buffers of t.bufElems elements
   const uint32_t tid = threadIdx.x;

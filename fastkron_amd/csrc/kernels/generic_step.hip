@@ -17,16 +17,16 @@ constexpr int kGenThreads = 256;
 constexpr int kGenTP = 32;
 
 template <typename T, int TQ, bool LANES_M, bool AHEAD>
-__global__ __launch_bounds__(kGenThreads) void kron_step_generic(const StepArgs a, const uint32_t qTiles) {
+__global__ __launch_bounds__(kGenThreads) void kron_step_generic(const KernelArgs a, const uint32_t qTiles, const OuterStrides outer) {
   __shared__ T fs[kGenTP][TQ];
   const uint32_t P = a.p[0], Q = a.q[0];
   const uint64_t S = a.Kin / P;
   const uint64_t tile = blockIdx.x / qTiles;
   const uint32_t q0 = (blockIdx.x % qTiles) * TQ;
   const uint32_t b = blockIdx.z;
-  const T* in = (const T*)a.in + (size_t)b * a.in_batch;
-  T* out = (T*)a.out + (size_t)b * a.out_batch;
-  const T* y = a.y ? (const T*)a.y + (size_t)b * a.y_batch : nullptr;
+  const T* in = (const T*)a.in + (size_t)b * a.in_batch + (size_t)blockIdx.y * outer.in;
+  T* out = (T*)a.out + (size_t)b * a.out_batch + (size_t)blockIdx.y * outer.out;
+  const T* y = a.y ? (const T*)a.y + (size_t)b * a.y_batch + (size_t)blockIdx.y * outer.y : nullptr;
   const T* F = (const T*)a.f[0] + (size_t)b * a.f_batch[0];
 
   const uint64_t g = tile * kGenThreads + threadIdx.x;
@@ -116,7 +116,7 @@ static hipError_t launchGenericT(const StepArgs& a, hipStream_t stream) {
   while (tq > 4 && tiles * ((Q + tq - 1) / tq) * a.batch < 128) tq /= 2;
   const uint32_t qTiles = (Q + tq - 1) / tq;
   if (tiles * qTiles >= (1ull << 31) || a.batch > 65535) return hipErrorInvalidValue;
-  dim3 grid((uint32_t)(tiles * qTiles), 1, a.batch), block(kGenThreads);
+  dim3 grid((uint32_t)(tiles * qTiles), outerEntries(a), innerEntries(a)), block(kGenThreads);
   // Loads ahead of the products, up to four workgroups per CU: for short rows, where the first eight leave before the factor
   // is staged (sgekmm 7^5 x 100 37.0 -> 34.7 us, 17^3 x 200 27.5 -> 24.8, 3^8 x 50 34.3 -> 30.0), and in the KMM layout where
   // a load takes long: few columns and with them many short pieces (21^3 x 25, batch of 5, 29.0 -> 24.7), or an X of more
@@ -129,8 +129,8 @@ static hipError_t launchGenericT(const StepArgs& a, hipStream_t stream) {
   const uint64_t wgs = tiles * qTiles * a.batch, xBytes = (uint64_t)a.M * a.Kin * a.batch * sizeof(T);
   const bool ahead = wgs < 1024 && (P <= 20 || (LANES_M && (P <= 32 ? a.M < 128 && S > 1 : xBytes >= (tq >= 8 ? 2400000u : 32000000u))));
 #define GEN_LAUNCH(TQ) \
-  if (ahead) hipLaunchKernelGGL((kron_step_generic<T, TQ, LANES_M, true>), grid, block, 0, stream, a, qTiles); \
-  else       hipLaunchKernelGGL((kron_step_generic<T, TQ, LANES_M, false>), grid, block, 0, stream, a, qTiles);
+  if (ahead) hipLaunchKernelGGL((kron_step_generic<T, TQ, LANES_M, true>), grid, block, 0, stream, a, qTiles, a.outer); \
+  else       hipLaunchKernelGGL((kron_step_generic<T, TQ, LANES_M, false>), grid, block, 0, stream, a, qTiles, a.outer);
   switch (tq) {
     case 1:  GEN_LAUNCH(1) break;
     case 2:  GEN_LAUNCH(2) break;

@@ -51,7 +51,7 @@ constexpr int kK2Win = 3;              // k0 slices of a tile in flight
 // them as one 8-byte element, and a quarter wave covers a whole 128-byte line per row where JW = 1 covers half of
 // one; the two columns go through the matrix cores as two column blocks.
 template <typename T, bool HAS_Y, bool EXACT, int JW>
-__global__ __launch_bounds__(256, 2) void kron_kmm16x2_kernel(const StepArgs a, const uint32_t mTiles,
+__global__ __launch_bounds__(256, 2) void kron_kmm16x2_kernel(const KernelArgs a, const uint32_t mTiles,
                                                               const uint32_t totalTiles, const uint32_t qSplit) {
   using MF = K2Mfma<T>;
   using Acc = typename MF::Acc;

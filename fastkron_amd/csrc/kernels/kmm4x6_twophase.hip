@@ -95,7 +95,7 @@ __device__ __forceinline__ uint32_t t6L2Load(uint32_t* p, uint32_t zero) {
 #define T6_WAIT_VM(n) __builtin_amdgcn_s_waitcnt(0x0F70 | ((n) & 15) | (((n) >> 4) << 14))
 
 template <bool HAS_Y>
-__global__ __launch_bounds__(256) void kron_kmm4x6_twophase_kernel(const StepArgs a, const uint32_t blocksPerEntry,
+__global__ __launch_bounds__(256) void kron_kmm4x6_twophase_kernel(const KernelArgs a, const uint32_t blocksPerEntry,
                                                                    const uint32_t totalBlocks, const uint32_t helpAfter,
                                                                    const uint32_t zero) {
   __shared__ int shared[2];

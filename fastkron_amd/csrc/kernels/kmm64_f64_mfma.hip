@@ -36,7 +36,7 @@ constexpr int kKmm64Waves = 4;
 // a 2 KB wide strip of every entry (the leading 64x64 factor of dgemkm 256 x 64^3, 256 entries of 64 x 4096: 225 ->
 // 208 us; memory accesses alone take 176 us in this order and 208 us entry by entry, the products alone 127 us)
 template <bool HAS_Y, int NT, bool FLAT>
-__global__ __launch_bounds__(256, 1) void kron_kmm64_f64_kernel(const StepArgs a, const uint32_t mBlocks,
+__global__ __launch_bounds__(256, 1) void kron_kmm64_f64_kernel(const KernelArgs a, const uint32_t mBlocks,
                                                                 const uint32_t tilesPerEntry, const uint32_t totalTiles) {
   constexpr int P = 64;
   __shared__ double fB[P * P];                       // F[p][q] at p*64 + (q ^ 4*(p%4))
@@ -205,7 +205,7 @@ hipError_t launchKmm64F64(const StepArgs& a, hipStream_t stream) {
   if (wgs == 0) wgs = 1;
   dim3 grid(wgs, flat ? 1 : a.batch), block(256);
   const bool y = a.y && a.epilogue, nt = a.stream_in && a.stream_out;
-  using Kernel = void (*)(const StepArgs, const uint32_t, const uint32_t, const uint32_t);
+  using Kernel = void (*)(const KernelArgs, const uint32_t, const uint32_t, const uint32_t);
   static const Kernel kernels[2][2][2] = {
       {{kron_kmm64_f64_kernel<false, 0, false>, kron_kmm64_f64_kernel<false, 0, true>},
        {kron_kmm64_f64_kernel<false, 2, false>, kron_kmm64_f64_kernel<false, 2, true>}},

@@ -70,7 +70,7 @@ __device__ __forceinline__ void k83ContractSecond(float (&x)[8][8], const float 
 
 // NT: 0 = ordinary accesses, 2 = non-temporal loads of X and stores (sgekmm 1024 x 8^6: 873 -> 832 us; small problems lose)
 template <bool HAS_Y, int NT>
-__global__ __launch_bounds__(512, 4) void kron_kmm8x3_kernel(const StepArgs a, const uint32_t mTiles) {
+__global__ __launch_bounds__(512, 4) void kron_kmm8x3_kernel(const KernelArgs a, const uint32_t mTiles) {
   extern __shared__ __align__(16) float k83Lds[];
   float* fl = k83Lds + 8 * 32 * 64;              // factors: fl[f*64 + p*8 + q]; f = 0 is F1 (slowest digit)
   const int tid = threadIdx.x;
@@ -181,7 +181,7 @@ hipError_t launchKmm8x3(const StepArgs& a, hipStream_t stream) {
   static PerDeviceOnce attrOnce;
   const int devIdx = launchDeviceIndex();
   const size_t ldsBytes = kK83LdsWords * sizeof(float);
-  using Kernel = void (*)(const StepArgs, const uint32_t);
+  using Kernel = void (*)(const KernelArgs, const uint32_t);
   static const Kernel kernels[2][2] = {{kron_kmm8x3_kernel<false, 0>, kron_kmm8x3_kernel<false, 2>},
                                        {kron_kmm8x3_kernel<true, 0>, kron_kmm8x3_kernel<true, 2>}};
   if (!attrOnce.done(devIdx)) {

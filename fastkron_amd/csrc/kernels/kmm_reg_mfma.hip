@@ -34,7 +34,7 @@ constexpr int kKmmWaves = 4;
 
 // NT: 0 = ordinary, 2 = non-temporal loads of X and stores (sgekmm 1024 x 8^6: 1175 -> 1127 us)
 template <int P, int NF, bool HAS_Y, int NT>
-__global__ __launch_bounds__(256, HAS_Y ? 3 : 4) void kron_kmm_reg_kernel(const StepArgs a, const uint32_t mTiles,
+__global__ __launch_bounds__(256, HAS_Y ? 3 : 4) void kron_kmm_reg_kernel(const KernelArgs a, const uint32_t mTiles,
                                                               const uint32_t totalTiles) {
   constexpr int G = KmmRegCfg<P, NF>::G;
   constexpr int QQ = P / 4;

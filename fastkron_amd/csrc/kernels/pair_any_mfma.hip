@@ -63,7 +63,7 @@ constexpr uint32_t paItems(int PB) { return PB == 2 ? 4 : 2; }
 
 // PB, QB: 16-wide blocks of an input / output digit (2: up to 32, 4: up to 64)
 template <typename T, int PB, int QB, bool HAS_Y>
-__global__ __launch_bounds__(kPaThreads, 2) void kron_pair_any_kernel(const StepArgs a, const PairAnyTile t) {
+__global__ __launch_bounds__(kPaThreads, 2) void kron_pair_any_kernel(const KernelArgs a, const PairAnyTile t, const OuterStrides outer) {
   using MF = PaMfma<T>;
   using Acc = typename MF::Acc;
   constexpr uint32_t ES = sizeof(T), VE = 16 / ES;
@@ -81,13 +81,16 @@ __global__ __launch_bounds__(kPaThreads, 2) void kron_pair_any_kernel(const Step
   VT* pieces = (VT*)paLds;
   T* f1Lds = (T*)paLds;                                             // (behind the tile: see below)
 
+  const T* const inB = (const T*)a.in + (size_t)b * a.in_batch + (size_t)blockIdx.z * outer.in;
+  T* const outB = (T*)a.out + (size_t)b * a.out_batch + (size_t)blockIdx.z * outer.out;
+  T* const yB = HAS_Y ? (T*)a.y + (size_t)b * a.y_batch + (size_t)blockIdx.z * outer.y : nullptr;
   struct Tile { const T* src; uint32_t n, E, shift, last; };
   auto tileAt = [&](uint32_t i) {
     Tile r;
     const uint32_t m0 = i * t.items;
     r.n = a.M - m0 < t.items ? a.M - m0 : t.items;
     r.E = r.n * rowIn;
-    r.src = (const T*)a.in + (size_t)b * a.in_batch + (size_t)m0 * rowIn;
+    r.src = inB + (size_t)m0 * rowIn;
     r.shift = (uint32_t)((uintptr_t)r.src / ES) & (VE - 1);
     r.last = (r.shift + r.E) / VE;
     return r;
@@ -195,8 +198,8 @@ __global__ __launch_bounds__(kPaThreads, 2) void kron_pair_any_kernel(const Step
     }
     __syncthreads();                                              // the tile has been read
     if (work) {
-      const auto out = streamTarget((T*)a.out + (size_t)b * a.out_batch + (size_t)row * rowOut, rowOut * ES);
-      const auto y = HAS_Y ? streamTarget((T*)a.y + (size_t)b * a.y_batch + (size_t)row * rowOut, rowOut * ES) : out;
+      const auto out = streamTarget(outB + (size_t)row * rowOut, rowOut * ES);
+      const auto y = HAS_Y ? streamTarget(yB + (size_t)row * rowOut, rowOut * ES) : out;
       const uint32_t q2 = 16 * jb + lo, lane = q2 < t.Q2 ? (MF::rowLane(hi) * t.Q2 + q2) * ES : kPaNowhere;
 #pragma unroll
       for (int u = 0; u < QB; u++)
@@ -267,7 +270,7 @@ static hipError_t launchPairAnyAs(const StepArgs& a, hipStream_t stream) {
   }
   // two waves per SIMD, four of the kernels that need few registers
   const uint32_t resident = (sizeof(T) == 4 && PB == 2 ? 4 : 2) * (uint32_t)deviceCUs(), perBatch = (resident + a.batch - 1) / a.batch;
-  hipLaunchKernelGGL(kernel, dim3(std::min(t.tiles, perBatch), a.batch), dim3(kPaThreads), lds, stream, a, t);
+  hipLaunchKernelGGL(kernel, dim3(std::min(t.tiles, perBatch), innerEntries(a), outerEntries(a)), dim3(kPaThreads), lds, stream, a, t, a.outer);
   return hipGetLastError();
 }
 template <typename T, int PB, int QB>

@@ -75,7 +75,7 @@ template <> struct PairMfma<float> {
 // the 16-wide blocks of output columns q_a (few rows: more waves than rows, and the products of a block are one
 // dependent chain).
 template <typename T, int P, bool HAS_Y, bool EXACT = true, int Q = P, bool SPLIT = false>
-__global__ __launch_bounds__(256, 2) void kron_pair_kernel(const StepArgs a, const uint32_t splitArg) {
+__global__ __launch_bounds__(256, 2) void kron_pair_kernel(const KernelArgs a, const uint32_t splitArg) {
   const uint32_t splitShift = SPLIT ? splitArg : 0;   // a constant in the kernels of whole rows
   static_assert(EXACT || P == Q, "the zero-padded form is square");
   using MF = PairMfma<T>;
@@ -330,7 +330,7 @@ constexpr size_t kPair64LdsBytes = (2 * kP64 * kP64 + kPair64Waves * kPair64XWor
 // of a row in one wave are latency bound, about 35 us whatever else runs).  Columns of group g and lane n: with
 // GN >= 2 the pairs 32*(g/2) + 2n + g%2 (128-bit accesses), with GN = 1 the 16 neighbours 16*g + n.
 template <bool HAS_Y, int NT, int GN = 4>
-__global__ __launch_bounds__(512, 2) void kron_pair64_f64_kernel(const StepArgs a) {
+__global__ __launch_bounds__(512, 2) void kron_pair64_f64_kernel(const KernelArgs a) {
   constexpr int P = kP64;
   constexpr int HN = GN >= 2 ? GN / 2 : 1;          // 128-bit column pairs (GN = 1: the one column) per lane
   constexpr uint32_t SHARE = 4 / GN;                // waves per row
@@ -580,7 +580,7 @@ static hipError_t launchPairT(const StepArgs& a, hipStream_t stream) {
   const int devIdx = launchDeviceIndex();
   const bool y = a.y && a.epilogue;
   if (!attrOnce[y].done(devIdx)) {
-    using Kernel = void (*)(const StepArgs, const uint32_t);
+    using Kernel = void (*)(const KernelArgs, const uint32_t);
     const Kernel all[4] = {kron_pair_kernel<T, P, false, EXACT, Q, false>, kron_pair_kernel<T, P, false, EXACT, Q, true>,
                            kron_pair_kernel<T, P, true, EXACT, Q, false>, kron_pair_kernel<T, P, true, EXACT, Q, true>};
     for (int k = 2 * y; k < 2 * y + 2; k++) {
@@ -612,7 +612,7 @@ static hipError_t launchPair64(const StepArgs& a, hipStream_t stream) {
   dim3 grid(wgs, a.batch), block(64 * kPair64Waves);
   static PerDeviceOnce attrOnce;
   const int devIdx = launchDeviceIndex();
-  using Kernel = void (*)(const StepArgs);
+  using Kernel = void (*)(const KernelArgs);
   // (the shared forms run on rows that stay in the caches: ordinary loads and stores)
   static const Kernel kernels[2][5] = {
       {kron_pair64_f64_kernel<false, 0>, kron_pair64_f64_kernel<false, 1>, kron_pair64_f64_kernel<false, 2>,

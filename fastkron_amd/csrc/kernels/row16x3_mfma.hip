@@ -56,7 +56,7 @@ template <typename T> struct R3Depth { static constexpr int ahead = sizeof(T) ==
 // wave instruction writing 1 KB in one piece (instead of 64-byte pieces 4 bytes per lane); results that nothing reads
 // back soon go out at system scope (sgemkm 4096 x 16^3: 33.9 -> 24.6 us, 16384 x 16^3: 107.5 -> 104.6 us).
 template <typename T, bool HAS_Y, bool EXACT, bool WIDE>
-__global__ __launch_bounds__(256, 2) void kron_row16x3_kernel(const StepArgs a, const uint32_t blocksPerBatch,
+__global__ __launch_bounds__(256, 2) void kron_row16x3_kernel(const KernelArgs a, const uint32_t blocksPerBatch,
                                                               const uint32_t totalBlocks) {
   using MF = R3Mfma<T>;
   using Acc = typename MF::Acc;

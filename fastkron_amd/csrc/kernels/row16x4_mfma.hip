@@ -62,7 +62,7 @@ constexpr int kLdsWords = 2 * kQuarterWords + 4 * kFacWords + 256;   // two quar
 // 16-byte stores at system scope through a buffer descriptor of the row (sgemkm 1024 x 16^4: 103.7 us with
 // non-temporal stores, 99.1 us with these).
 template <bool HAS_Y, int NT>
-__global__ __launch_bounds__(1024, 1) void kron_row16x4_kernel(const StepArgs a, const uint32_t blocksPerBatch,
+__global__ __launch_bounds__(1024, 1) void kron_row16x4_kernel(const KernelArgs a, const uint32_t blocksPerBatch,
                                                                const uint32_t totalItems, const uint32_t staggerTicks) {
   extern __shared__ __align__(16) float lds[];
   const int tid = threadIdx.x;
@@ -294,7 +294,7 @@ hipError_t launchRow16x4(const StepArgs& a, hipStream_t stream, bool staggered) 
   static PerDeviceOnce attrOnce;
   const int devIdx = launchDeviceIndex();
   const size_t ldsBytes = kLdsWords * sizeof(float);
-  using Kernel = void (*)(const StepArgs, const uint32_t, const uint32_t, const uint32_t);
+  using Kernel = void (*)(const KernelArgs, const uint32_t, const uint32_t, const uint32_t);
   static const Kernel kernels[2][3] = {
       {kron_row16x4_kernel<false, 0>, kron_row16x4_kernel<false, 1>, kron_row16x4_kernel<false, 2>},
       {kron_row16x4_kernel<true, 0>, kron_row16x4_kernel<true, 1>, kron_row16x4_kernel<true, 2>}};

@@ -44,7 +44,7 @@ constexpr int kW8LdsWords = 32768;          // 128 KB: one half of a block
 constexpr int kW8Early = 16;                // (v,t) register blocks of the next item requested when stage 2 starts
 
 template <bool HAS_Y>
-__global__ __launch_bounds__(512, 2) void kron_row16x4w8_kernel(const StepArgs a, const uint32_t blocksPerBatch,
+__global__ __launch_bounds__(512, 2) void kron_row16x4w8_kernel(const KernelArgs a, const uint32_t blocksPerBatch,
                                                                 const uint32_t totalItems) {
   extern __shared__ __align__(16) float lds[];
   const int tid = threadIdx.x;

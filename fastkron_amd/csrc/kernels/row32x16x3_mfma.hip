@@ -32,7 +32,7 @@ constexpr int kRow32LdsWords = 8192;
 // lane: Z is written and Y read 16 bytes per lane (rows of Z and Y 16-byte aligned), streamed results at system
 // scope (8 x 512 x (32x16)^3 with beta = 1: 120.9 -> 117.9 us)
 template <bool HAS_Y, int NT, bool WIDE>
-__global__ __launch_bounds__(512, 4) void kron_row32x16x3_kernel(const StepArgs a) {
+__global__ __launch_bounds__(512, 4) void kron_row32x16x3_kernel(const KernelArgs a) {
   extern __shared__ __align__(16) float lds[];
   const int tid = threadIdx.x;
   const int l = tid & 63;
@@ -179,7 +179,7 @@ hipError_t launchRow32x16x3(const StepArgs& a, hipStream_t stream) {
   // rows of Z (and Y) on 16-byte boundaries: results 16 bytes per lane
   const bool wide = !(((uintptr_t)a.out & 15) || (a.out_ldm & 3) || (a.out_batch & 3)) &&
                     !(y && (((uintptr_t)a.y & 15) || (a.y_ldm & 3) || (a.y_batch & 3)));
-  using Kernel = void (*)(const StepArgs);
+  using Kernel = void (*)(const KernelArgs);
   static const Kernel kernels[2][2][2] = {
       {{kron_row32x16x3_kernel<false, 0, false>, kron_row32x16x3_kernel<false, 0, true>},
        {kron_row32x16x3_kernel<false, 1, false>, kron_row32x16x3_kernel<false, 1, true>}},

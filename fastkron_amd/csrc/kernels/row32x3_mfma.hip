@@ -37,7 +37,7 @@ constexpr int kR32LdsWords = 2 * kR32QuarterWords + 3 * 1024;      // two quarte
 // NT: 0 = ordinary stores, 1 = streaming stores (1024 x 32^3: 85.0 -> 78.0 us with non-temporal stores, non-temporal loads
 // of X as well: 81.6; at system scope through a descriptor of the row: 4096 rows 286 -> 279 us)
 template <bool HAS_Y, int NT>
-__global__ __launch_bounds__(512, 4) void kron_row32x3_kernel(const StepArgs a) {
+__global__ __launch_bounds__(512, 4) void kron_row32x3_kernel(const KernelArgs a) {
   extern __shared__ __align__(16) float r32lds[];
   float* const fl = r32lds + 2 * kR32QuarterWords;                 // fl[j*1024 + p*32 + q]; j = 0: F3, 1: F2, 2: F1
   const int tid = threadIdx.x;
@@ -203,7 +203,7 @@ hipError_t launchRow32x3(const StepArgs& a, hipStream_t stream) {
   static PerDeviceOnce attrOnce;
   const int devIdx = launchDeviceIndex();
   const size_t ldsBytes = kR32LdsWords * sizeof(float);
-  using Kernel = void (*)(const StepArgs);
+  using Kernel = void (*)(const KernelArgs);
   static const Kernel kernels[2][2] = {{kron_row32x3_kernel<false, 0>, kron_row32x3_kernel<false, 1>},
                                        {kron_row32x3_kernel<true, 0>, kron_row32x3_kernel<true, 1>}};
   if (!attrOnce.done(devIdx)) {

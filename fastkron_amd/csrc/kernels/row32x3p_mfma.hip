@@ -49,7 +49,7 @@ constexpr int kP3LdsWords = 4 * kP3QuarterWords + 3 * 1024;        // the four q
 
 // NT: 0 = ordinary stores, 1 = streaming stores (16 bytes at system scope through a descriptor of the row)
 template <bool HAS_Y, int NT>
-__global__ __launch_bounds__(1024, 1) void kron_row32x3p_kernel(const StepArgs a, const uint32_t totalItems) {
+__global__ __launch_bounds__(1024, 1) void kron_row32x3p_kernel(const KernelArgs a, const uint32_t totalItems) {
   extern __shared__ __align__(16) float p3lds[];
   float* const fl = p3lds + 4 * kP3QuarterWords;                   // fl[j*1024 + p*32 + q]; j = 0: F3, 1: F2, 2: F1
   const int tid = threadIdx.x;
@@ -249,7 +249,7 @@ hipError_t launchRow32x3p(const StepArgs& a, hipStream_t stream) {
   static PerDeviceOnce attrOnce;
   const int devIdx = launchDeviceIndex();
   const size_t ldsBytes = kP3LdsWords * sizeof(float);
-  using Kernel = void (*)(const StepArgs, const uint32_t);
+  using Kernel = void (*)(const KernelArgs, const uint32_t);
   static const Kernel kernels[2][2] = {{kron_row32x3p_kernel<false, 0>, kron_row32x3p_kernel<false, 1>},
                                        {kron_row32x3p_kernel<true, 0>, kron_row32x3p_kernel<true, 1>}};
   if (!attrOnce.done(devIdx)) {

@@ -139,7 +139,7 @@ __device__ __forceinline__ void contractSecond(double (&x)[8][8], const Factor8&
 
 // PMAJOR: the factors are stored with q fastest (element (p,q) at 8p + q), otherwise with p fastest (the other op)
 template <bool HAS_Y, int NT, bool PMAJOR>
-__global__ __launch_bounds__(512) void kron_row8x5_f64_kernel(const StepArgs a, const uint32_t firstRound,
+__global__ __launch_bounds__(512) void kron_row8x5_f64_kernel(const KernelArgs a, const uint32_t firstRound,
                                                               const uint32_t staggerGroups, const uint32_t staggerTicks) {
   extern __shared__ __align__(16) double ldsd[];
   const int tid = threadIdx.x;
@@ -290,7 +290,7 @@ hipError_t launchRow8x5F64(const StepArgs& a, hipStream_t stream) {
   static PerDeviceOnce attrOnce;
   const int devIdx = launchDeviceIndex();
   const size_t ldsBytes = kRow8dLdsDoubles * sizeof(double);
-  using Kernel = void (*)(const StepArgs, const uint32_t, const uint32_t, const uint32_t);
+  using Kernel = void (*)(const KernelArgs, const uint32_t, const uint32_t, const uint32_t);
   static const Kernel kernels[2][2][3] = {
       {{kron_row8x5_f64_kernel<false, 0, false>, kron_row8x5_f64_kernel<false, 1, false>, kron_row8x5_f64_kernel<false, 2, false>},
        {kron_row8x5_f64_kernel<true, 0, false>, kron_row8x5_f64_kernel<true, 1, false>, kron_row8x5_f64_kernel<true, 2, false>}},

@@ -78,7 +78,8 @@ __device__ __forceinline__ void contractSecond(float (&x)[8][8], const float (&f
 }
 
 template <bool HAS_Y, int NT>
-__global__ __launch_bounds__(512, 4) void kron_row8x5_kernel(const StepArgs a, const uint32_t firstRound, const uint32_t delayTicks) {
+__global__ __launch_bounds__(512, 4) void kron_row8x5_kernel(const KernelArgs a, const uint32_t firstRound, const uint32_t delayTicks,
+                                                                const OuterStrides outer) {
   extern __shared__ __align__(16) float lds[];
   float* fl = lds + 16384;                       // factors: fl[f*64 + p*8 + q], f = 0 is F1
   const int tid = threadIdx.x;
@@ -87,8 +88,8 @@ __global__ __launch_bounds__(512, 4) void kron_row8x5_kernel(const StepArgs a, c
   const uint32_t m = blockIdx.x, bt = blockIdx.y;
 
   // m counts blocks of 32768 contiguous elements: one row for five factors, 8^(5-nf) rows otherwise
-  const float* X = (const float*)a.in + (size_t)bt * a.in_batch + (size_t)m * kRow8Len;
-  float* Z = (float*)a.out + (size_t)bt * a.out_batch + (size_t)m * kRow8Len;
+  const float* X = (const float*)a.in + (size_t)bt * a.in_batch + (size_t)blockIdx.z * outer.in + (size_t)m * kRow8Len;
+  float* Z = (float*)a.out + (size_t)bt * a.out_batch + (size_t)blockIdx.z * outer.out + (size_t)m * kRow8Len;
 
   // factors to LDS, ahead of the row loads (vector memory operations retire in order, so these small
   // loads must not queue behind 128 KB of row data).  a.f[0] is the last factor F5 ... a.f[nf-1] the first.  With fewer than five
@@ -205,7 +206,7 @@ __global__ __launch_bounds__(512, 4) void kron_row8x5_kernel(const StepArgs a, c
 
   // ---- epilogue and store ----
   const float alpha = (float)a.alpha, beta = (float)a.beta;
-  const float* Y = HAS_Y ? (const float*)a.y + (size_t)bt * a.y_batch + (size_t)m * kRow8Len : nullptr;
+  const float* Y = HAS_Y ? (const float*)a.y + (size_t)bt * a.y_batch + (size_t)blockIdx.z * outer.y + (size_t)m * kRow8Len : nullptr;
   const int lo = (l & 31), q2b = l >> 5;
 #pragma unroll
   for (int q3 = 0; q3 < 8; q3++)
@@ -245,7 +246,7 @@ hipError_t launchRow8x5(const StepArgs& a, hipStream_t stream, int schedule) {
   const int devIdx = launchDeviceIndex();
   const size_t ldsMax = 96 * 1024;
   const size_t ldsBytes = schedule == 1 ? ldsMax : kRow8LdsWords * sizeof(float);
-  using Kernel = void (*)(const StepArgs, const uint32_t, const uint32_t);
+  using Kernel = void (*)(const KernelArgs, const uint32_t, const uint32_t, const OuterStrides);
   static const Kernel kernels[2][3] = {
       {kron_row8x5_kernel<false, 0>, kron_row8x5_kernel<false, 1>, kron_row8x5_kernel<false, 2>},
       {kron_row8x5_kernel<true, 0>, kron_row8x5_kernel<true, 1>, kron_row8x5_kernel<true, 2>}};
@@ -257,10 +258,10 @@ hipError_t launchRow8x5(const StepArgs& a, hipStream_t stream, int schedule) {
       }
     attrOnce.mark(devIdx);
   }
-  dim3 grid(a.M / row8Rows(a), a.batch), block(512);
+  dim3 grid(a.M / row8Rows(a), innerEntries(a), outerEntries(a)), block(512);
   const uint32_t firstRound = 2u * (uint32_t)deviceCUs();
   hipLaunchKernelGGL(kernels[(a.y && a.epilogue) ? 1 : 0][streamMode(a)], grid, block, ldsBytes, stream, a, firstRound,
-                     schedule == 0 ? kRow8SlotDelayTicks : 0u);
+                     schedule == 0 ? kRow8SlotDelayTicks : 0u, a.outer);
   return hipGetLastError();
 }
 

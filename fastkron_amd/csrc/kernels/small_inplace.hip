@@ -77,7 +77,7 @@ struct IpOut {
 // SYNC: a barrier behind the reads of the values (one digit group per thread at most): the rows' LDS is free from there on.
 // TU: 0 for rows; columns otherwise, so many in LDS next to each other, read from memory by the first pass (FIRST).
 template <typename T, int P, int D, int S, bool HAS_Y, bool SYNC = false, bool ST = false, int TU = 0, bool FIRST = false>
-__device__ __forceinline__ void ipPass(T* __restrict__ rows, const StepArgs& a, const InplacePass& ps, const uint32_t b,
+__device__ __forceinline__ void ipPass(T* __restrict__ rows, const KernelArgs& a, const InplacePass& ps, const uint32_t b,
                                        const uint32_t E, const bool vec, const bool toMemory, const IpOut<T, HAS_Y>& o) {
   constexpr int N = ipPow(P, D), VE = 16 / (int)sizeof(T);
   constexpr int U = N >= 16 ? 1 : N >= 6 ? 2 : 4;            // digit groups per thread and round
@@ -198,19 +198,19 @@ __device__ __forceinline__ void ipPass(T* __restrict__ rows, const StepArgs& a, 
       uint32_t at = e0[k];
       if (toMemory) {
         // through buffer descriptors: one address register per group, the values' distances as scalar offsets
-        const uint32_t to = TU ? o.laneOut + e0[k] / (TU ? TU : 1) * o.pitch : e0[k] * sizeof(T);
-        const uint32_t next = TU ? step / (TU ? TU : 1) * o.pitch : step * sizeof(T);
+        const uint32_t row = TU ? e0[k] / (TU ? TU : 1) * o.pitch : 0, next = TU ? step / (TU ? TU : 1) * o.pitch : 0;
         T yv[HAS_Y ? N : 1];
         if constexpr (HAS_Y) {
-          const uint32_t from = TU ? to - o.laneOut + o.laneY : to;
 #pragma unroll
-          for (uint32_t i = 0; i < N; i++) yv[i] = ipLoad<T>(o.yTarget, from, i * next);
+          for (uint32_t i = 0; i < N; i++)
+            yv[i] = TU ? ipLoad<T>(o.yTarget, o.laneY + row, i * next) : ipLoad<T>(o.yTarget, e0[k] * sizeof(T), i * step * sizeof(T));
         }
 #pragma unroll
         for (uint32_t i = 0; i < N; i++) {
           T v = x[k][i] * o.alpha;
           if constexpr (HAS_Y) v += o.beta * yv[i];
-          ipStore<ST>(v, o.target, to, i * next);
+          if (TU) ipStore<ST>(v, o.target, o.laneOut + row, i * next);
+          else ipStore<ST>(v, o.target, e0[k] * sizeof(T), i * step * sizeof(T));
         }
       } else if (v16) {
 #pragma unroll
@@ -230,7 +230,7 @@ __device__ __forceinline__ void ipPass(T* __restrict__ rows, const StepArgs& a, 
 
 // The pass with its distance as a constant where the chain is one of equal factors (1, P^D, P^2D) or begins it.
 template <typename T, int P, int D, bool HAS_Y>
-__device__ __forceinline__ void ipPassAny(T* __restrict__ rows, const StepArgs& a, const InplacePass& ps, const uint32_t b,
+__device__ __forceinline__ void ipPassAny(T* __restrict__ rows, const KernelArgs& a, const InplacePass& ps, const uint32_t b,
                                           const uint32_t E, const bool vec, const bool toMemory, const IpOut<T, HAS_Y>& o) {
   constexpr int N = ipPow(P, D);
   if (ps.s == 1) return ipPass<T, P, D, 1, HAS_Y>(rows, a, ps, b, E, vec, false, o);
@@ -250,20 +250,20 @@ constexpr int ipWaves(int p, size_t es) { return es == 8 || p == 7 ? 3 : p == 6 
 // P: all factors are PxP; 0: any mix, one digit per pass.
 template <typename T, int P, bool HAS_Y>
 __global__ __launch_bounds__(kIpMaxThreads, ipWaves(P, sizeof(T)))
-void kron_small_inplace_kernel(const StepArgs a, const InplaceTile t) {
+void kron_small_inplace_kernel(const KernelArgs a, const InplaceTile t, const OuterStrides outer) {
   constexpr uint32_t VE = 16 / sizeof(T);
   typedef T VT __attribute__((ext_vector_type(VE)));
   extern __shared__ __align__(16) unsigned char ipLds[];
   const uint32_t tid = threadIdx.x, nth = blockDim.x, b = blockIdx.y;
   const uint32_t m0 = blockIdx.x * t.rows;
   const uint32_t E = (a.M - m0 < t.rows ? a.M - m0 : t.rows) * t.K;
-  const T* src = (const T*)a.in + (size_t)b * a.in_batch + (size_t)m0 * t.K;
+  const T* src = (const T*)a.in + (size_t)b * a.in_batch + (size_t)blockIdx.z * outer.in + (size_t)m0 * t.K;
   const uint32_t shift = (uint32_t)((uintptr_t)src / sizeof(T)) & (VE - 1);
   VT* chunks = (VT*)ipLds;
   T* rows = (T*)ipLds + shift;
   IpOut<T, HAS_Y> o;
-  o.out = (T*)a.out + (size_t)b * a.out_batch + (size_t)m0 * t.K;
-  o.y = HAS_Y ? (const T*)a.y + (size_t)b * a.y_batch + (size_t)m0 * t.K : nullptr;
+  o.out = (T*)a.out + (size_t)b * a.out_batch + (size_t)blockIdx.z * outer.out + (size_t)m0 * t.K;
+  o.y = HAS_Y ? (const T*)a.y + (size_t)b * a.y_batch + (size_t)blockIdx.z * outer.y + (size_t)m0 * t.K : nullptr;
   o.target = streamTarget(o.out, E * (uint32_t)sizeof(T));
   if (HAS_Y) o.yTarget = streamTarget((void*)o.y, E * (uint32_t)sizeof(T));
   o.alpha = a.epilogue ? (T)a.alpha : T(1); o.beta = (T)a.beta;
@@ -335,7 +335,7 @@ template <int P, int NF, size_t ES> struct IpRow {
 };
 
 template <typename T, int P, int NF, int J, bool HAS_Y, bool ST>
-__device__ __forceinline__ void ipRowPasses(T* rows, const StepArgs& a, const uint32_t b, const bool vec, const IpOut<T, HAS_Y>& o) {
+__device__ __forceinline__ void ipRowPasses(T* rows, const KernelArgs& a, const uint32_t b, const bool vec, const IpOut<T, HAS_Y>& o) {
   using C = IpRow<P, NF, sizeof(T)>;
   constexpr int F0 = J == 0 ? 0 : C::R + (J - 1) * C::D, D = J == 0 ? C::R : C::D;
   constexpr bool last = F0 + D == NF;
@@ -352,7 +352,7 @@ __device__ __forceinline__ void ipRowPasses(T* rows, const StepArgs& a, const ui
 // NT: 0 ordinary accesses, 1 non-temporal loads, 2 non-temporal loads and stores.
 template <typename T, int P, int NF, bool HAS_Y, int NT>
 __global__ __launch_bounds__((IpRow<P, NF, sizeof(T)>::threads), (IpRow<P, NF, sizeof(T)>::waves))
-void kron_rows_inplace_kernel(const StepArgs a, const uint32_t total) {
+void kron_rows_inplace_kernel(const KernelArgs a, const uint32_t total) {
   using C = IpRow<P, NF, sizeof(T)>;
   constexpr uint32_t VE = C::VE, K = C::K;
   typedef T VT __attribute__((ext_vector_type(C::VE)));
@@ -446,7 +446,7 @@ template <int P, int NF, size_t ES, bool NARROW> struct IpCols {
 };
 
 template <typename T, int P, int NF, int F0, bool HAS_Y, bool NARROW>
-__device__ __forceinline__ void ipColPasses(T* cols, const StepArgs& a, const uint32_t b, const IpOut<T, HAS_Y>& o) {
+__device__ __forceinline__ void ipColPasses(T* cols, const KernelArgs& a, const uint32_t b, const IpOut<T, HAS_Y>& o) {
   using C = IpCols<P, NF, sizeof(T), NARROW>;
   constexpr int D = NF - F0 < C::D ? NF - F0 : C::D;
   constexpr bool last = F0 + D == NF;
@@ -461,7 +461,7 @@ __device__ __forceinline__ void ipColPasses(T* cols, const StepArgs& a, const ui
 
 template <typename T, int P, int NF, bool HAS_Y, bool NARROW>
 __global__ __launch_bounds__((IpCols<P, NF, sizeof(T), NARROW>::threads), (IpCols<P, NF, sizeof(T), NARROW>::waves))
-void kron_cols_inplace_kernel(const StepArgs a, const uint32_t total) {
+void kron_cols_inplace_kernel(const KernelArgs a, const uint32_t total) {
   using C = IpCols<P, NF, sizeof(T), NARROW>;
   constexpr uint32_t ES = sizeof(T);
   extern __shared__ __align__(16) unsigned char ipLds[];
@@ -553,8 +553,8 @@ static hipError_t launchIpP(const StepArgs& a, const InplaceTile& t, hipStream_t
     if (e != hipSuccess) return e;
     attrOnce.mark(dev);
   }
-  hipLaunchKernelGGL((kron_small_inplace_kernel<T, P, HAS_Y>), dim3(t.tiles, a.batch), dim3(t.threads), lds,
-                     stream, a, t);
+  hipLaunchKernelGGL((kron_small_inplace_kernel<T, P, HAS_Y>), dim3(t.tiles, innerEntries(a), outerEntries(a)), dim3(t.threads), lds,
+                     stream, a, t, a.outer);
   return hipGetLastError();
 }
 
@@ -609,7 +609,7 @@ static hipError_t launchIpRows(const StepArgs& a, hipStream_t stream, bool* take
 // fill its threads better; 3^9 is more factors than a launch takes.
 static hipError_t launchIpRowsAny(const StepArgs& a, const InplaceTile& t, DType dt, hipStream_t stream, bool* taken) {
   *taken = false;
-  if ((uint64_t)a.M * a.batch >= (1ull << 31)) return hipSuccess;
+  if (a.inner || (uint64_t)a.M * a.batch >= (1ull << 31)) return hipSuccess;
   const uint32_t size = t.P * 16 + a.nf;
 #define IP_ROWS(T, P, NF) case P * 16 + NF: return launchIpRows<T, P, NF>(a, stream, taken);
   if (dt == DType::F32) switch (size) {

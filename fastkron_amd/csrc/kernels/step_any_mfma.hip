@@ -68,7 +68,7 @@ struct StepAnyGeom {
 // NBT > 0: every slab has exactly NBT full 16-column blocks (Q a multiple of 16) and P is a multiple of 4; the tile loop
 // then has no conditional memory operation (see there).  NBT = 0: anything.
 template <typename T, int PCMAX, bool HAS_Y, bool PREFETCH, int NBT>
-__global__ __launch_bounds__(kSaThreads, 2) void kron_step_any_kernel(const StepArgs a, const StepAnyGeom g) {
+__global__ __launch_bounds__(kSaThreads, 2) void kron_step_any_kernel(const KernelArgs a, const StepAnyGeom g) {
   using MF = SaMfma<T>;
   using Acc = typename MF::Acc;
   extern __shared__ __align__(16) unsigned char saLds[];

@@ -56,7 +56,7 @@ constexpr int kStepWaves = 4;            // waves per workgroup
 // tile is then 16 consecutive m of one slice, the B operand lane 16*k + m reads in[(s*P + p)*M + m] (16
 // consecutive elements per quarter wave and product), and the stores are the same 16-element runs.
 template <typename T, int P, int Q, int QS, bool HAS_Y, bool KMM>
-__global__ __launch_bounds__(256, 2) void kron_step_mfma_kernel(const StepArgs a, const uint32_t tilesPerRow,
+__global__ __launch_bounds__(256, 2) void kron_step_mfma_kernel(const KernelArgs a, const uint32_t tilesPerRow,
                                                                 const uint32_t totalTiles) {
   using M16 = Mfma16<T>;
   using Acc = typename M16::Acc;

@@ -75,7 +75,7 @@ template <typename V> struct SwLane<V, 1> {
 template <int CPS> __device__ __forceinline__ int swSlot(int s) { return CPS < 16 ? s ^ ((s >> 5) & 1) : s; }
 
 template <typename T, int P, bool KMM, bool HAS_Y, bool STREAM>
-__global__ __launch_bounds__(256, 2) void kron_step_wide_kernel(const StepArgs a, const uint32_t tilesPerLine,
+__global__ __launch_bounds__(256, 2) void kron_step_wide_kernel(const KernelArgs a, const uint32_t tilesPerLine,
                                                                 const uint32_t totalTiles) {
   using ST = SwType<T>;
   using Acc = typename ST::Acc;
@@ -276,7 +276,7 @@ static hipError_t launchStepWideT(const StepArgs& a, hipStream_t stream, int max
   // streamed results at system scope: 16 bytes per lane (not the 128x128 form), one batch entry, tiles spanning < 2 GB
   const uint64_t qStride = KMM ? (a.Kin / P) * (uint64_t)a.out_ldc : a.Kin / P;
   const bool streamOut = P != 128 && a.stream_out && a.batch == 1 && (uint64_t)P * qStride * sizeof(T) < (1ull << 31);
-  using Kernel = void (*)(const StepArgs, const uint32_t, const uint32_t);
+  using Kernel = void (*)(const KernelArgs, const uint32_t, const uint32_t);
   static const Kernel kernels[2][2] = {
       {kron_step_wide_kernel<T, P, KMM, false, false>, kron_step_wide_kernel<T, P, KMM, false, P != 128>},
       {kron_step_wide_kernel<T, P, KMM, true, false>, kron_step_wide_kernel<T, P, KMM, true, P != 128>}};

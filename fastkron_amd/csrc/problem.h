@@ -37,6 +37,10 @@ struct KronProblem {
   void* inter[kMaxFactors];           // forward only: inter[j] = output of the step of factor j+1
   uint64_t strideInter[kMaxFactors];
   bool haveStrideInter;
+  // Two batch dimensions: entry b is (o, i) = (b / inner, b % inner), with X, Z and Y at o * outer.. + i * stride.. and the i-th
+  // factors.  0: one dimension.
+  uint32_t inner;
+  uint64_t outerX, outerZ, outerY;
   // Set for the parts of a call that the library runs as problems of their own: X was written by a launch of this
   // call just before (a transposed copy, the first part of a two-part plan) / Z is read by the next launch.
   bool xJustWritten, zReadNext;
@@ -63,7 +67,7 @@ struct KronProblem {
 };
 
 // Arguments of one launch.  f[0] is the factor applied first (the highest-numbered one of the group).
-struct StepArgs {
+struct KernelArgs {
   const void* in;  void* out;  const void* y;
   const void* f[kMaxFused];
   uint64_t f_batch[kMaxFused];
@@ -86,6 +90,17 @@ struct StepArgs {
   void*    scratch;
   uint64_t scratch_elems;
   void*    sync;
+};
+
+// With a second batch dimension: entry (o, i) begins at i * .._batch + o * these (0 with one dimension).  An argument of its own
+// of the kernels that take two: 32 bytes more in the middle of everybody's arguments cost the shortest launches up to 0.5 us
+// (dgemkm 2000 x 5^4 9.0 / 9.7).
+struct OuterStrides { uint64_t in, out, y; };
+
+// What the host knows of a launch: `inner` != 0 entries of the first dimension where there are two.
+struct StepArgs : KernelArgs {
+  OuterStrides outer;
+  uint32_t inner;
 };
 
 // Merging of adjacent small factors into their Kronecker product (kernels/merge_factors.hip).

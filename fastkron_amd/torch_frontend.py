@@ -5,8 +5,9 @@ Mirrors the reference's `pyfastkron` interface (reference pyfastkron/fastkrontor
 broadcast and batching rules):
 
 * operands may carry leading batch dimensions, broadcast between X, the factors and Y the NumPy way; the
-  innermost batch dimension becomes one strided-batched library call (stride 0 = shared operand), outer
-  ones a host loop; a batch of X against shared factors (MKM) is folded into the row count instead;
+  batch dimensions become one strided-batched library call (stride 0 = shared operand) where one remains after neighbours
+  that all operands have alike are merged, or two of which the factors have one; further ones a host loop; a batch of X
+  against shared factors (MKM) is folded into the row count instead;
 * a tensor whose last two dimensions are a transposed view of a row-major buffer is passed as that buffer
   with `fastKronOp_T` instead of being copied (reference fastkrontorch.py:66-76);
 * 1-D X is a single row (MKM) or column (KMM);
@@ -45,7 +46,7 @@ def _load_native():
     loader.exec_module(m)
     lib = capi.load()
     names = ["sgemkm", "dgemkm", "sgekmm", "dgekmm", "sgemkmStridedBatched", "dgemkmStridedBatched", "sgekmmStridedBatched",
-             "dgekmmStridedBatched", "gekmmSizes", "fastKronSetStream", "fastKronGradSizes", "fastKronGradForward",
+             "dgekmmStridedBatched", "gekmmSizes", "fastKronSetStream", "fastKronProductOuter", "fastKronGradSizes", "fastKronGradForward",
              "fastKronGradBackwardSteps"]                 # the order of csrc/frontend.cpp
     m.use(tuple(ctypes.cast(getattr(lib, n), ctypes.c_void_p).value for n in names))
     return m

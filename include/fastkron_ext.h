@@ -81,6 +81,18 @@ fastKronError fastKronProbeCopyPattern(fastKronHandle handle, int pattern, const
                                        float* T, uint32_t M);
 
 /*
+ * A product with two batch dimensions of which the factors have the second one only (X of shape (a, 1), factors of shape
+ * (b) ...): entry (o, i) of count[0] x count[1] takes X at o * strideX[0] + i * strideX[1] elements, the i-th factors (P*Q
+ * elements apart) and Y and Z likewise.  mkm, dbl as below; the temporaries hold count[0] * count[1] entries of the size that
+ * gekmmSizes gives.  Results are those of count[0] strided-batched calls.  (The reference loops over outer batch dimensions
+ * in Python, reference pyfastkron/fastkronbase.py:104-518.)
+ */
+fastKronError fastKronProductOuter(fastKronHandle handle, int mkm, int dbl, uint32_t M, uint32_t N, const uint32_t Ps[], const uint32_t Qs[],
+                                   const void* X, fastKronOp opX, const uint64_t strideX[2], const void* const Fs[], fastKronOp opFs, void* Z,
+                                   const uint64_t strideZ[2], double alpha, double beta, const uint32_t count[2], const void* Y,
+                                   const uint64_t strideY[2], void* temp1, void* temp2);
+
+/*
  * Gradients.  fastKronGradForward computes Z like the forward family of include/fastkron.h (alpha = 1, no Y) and keeps in
  * `save` what the backward pass needs; fastKronGradBackward takes the gradient gZ of Z (laid out like Z, batch entries
  * one after the other) and writes the gradient of X to gX (row-major M x K for MKM, K x M for KMM, one per batch entry,
