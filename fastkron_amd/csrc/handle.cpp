@@ -993,7 +993,7 @@ fastKronError Handle::trySplitLeadingTrailing(const KronProblem& p, void* temp1,
   if (nT < 2 || nT == p.N) return fastKronKernelNotFound;         // a chain of nT factors alone is a whole-row problem
   // (sgemkm 1000 x 5^7 527 -> 342 us, 1 x 5^7 26 -> 14, 1000 x 3^9 128 -> 76, 1000 x 6^6 313 -> 177, 200 x 7^6 183 -> 120,
   // dgemkm 100 x 7^6 185 -> 126, all against groups of the kernel with two LDS buffers.  Three and more leading factors lose,
-  // 50 x 3^11 87 -> 125.  fp64 blocks of 6^5 and 7^5 go through passes of one digit and take a CU each: 7^6 is ahead from 96
+  // 50 x 3^11 87 -> 125.  fp64 blocks of 6^5 and 7^5 take a CU each (these figures in passes of one digit; 6^5 has two a pass since): 7^6 is ahead from 96
   // blocks on (14 rows 50 -> 39 us, 13 rows 37 / 37), 6^6 only where the groups' pieces no longer fit the CUs at once, from 208
   // on (16 rows 19.5 / 22.5, 33 rows 27.1 / 27.3, 38 rows 38.6 / 29.0; 32 x 2x2x6^5 25.0 / 31.1, 57 rows 40.8 / 37.0).)
   if (inplace && (nT != maxT || p.N - nT > 2)) return fastKronKernelNotFound;
