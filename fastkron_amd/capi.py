@@ -31,7 +31,7 @@ EXPORTS = [
 EXT_EXPORTS = ["fastKronGetLastPlan", "fastKronSetTunedDB", "fastKronSetPlanOnly", "fastKronGetLastLaunches",
                "sgemkmStaticScratch", "fastKronGetSyncError", "fastKronSetSyncHelpAfter",
                "fastKronProbeCopyPattern", "fastKronGradSizes", "fastKronGradForward", "fastKronGradBackward",
-               "fastKronGradBackwardSteps"]     # include/fastkron_ext.h
+               "fastKronGradBackwardSteps", "fastKronProductOuter"]     # include/fastkron_ext.h
 
 _lib = None
 
@@ -103,6 +103,8 @@ def load():
                                          vp, vpp, vp]
     lib.fastKronGradBackwardSteps.argtypes = [vp, cint, cint, u32, u32, u32p, u32p, vp, cint, u64, vpp, cint, cint, u32, u32, u32, vp, vp,
                                               vp, vpp, vp]
+    lib.fastKronProductOuter.argtypes = [vp, cint, cint, u32, u32, u32p, u32p, vp, cint, u64p, vpp, cint, vp, u64p, ctypes.c_double,
+                                         ctypes.c_double, u32p, vp, u64p, vp, vp]
     lib.fastKronSetPlanOnly.argtypes = [vp, cint]
     lib.fastKronGetLastLaunches.argtypes = [vp, ctypes.c_char_p, ctypes.c_size_t]
     lib.fastKronGetLastLaunches.restype = ctypes.c_size_t

@@ -174,14 +174,6 @@ fastKronError run(fastKronHandle handle, fastKronBackend backend, const Call& c,
       if (c.strideInter) { p.strideInter[i] = c.strideInter[i]; p.haveStrideInter = true; }
     }
   }
-  // A strided-batched call with a single batch entry never uses its strides: they are cleared here so that no
-  // plan that re-views the rows of one problem as batch entries of another (the two-part plan does) can carry a
-  // caller's stride into a batch index of its own.
-  if (p.batch == 1) {
-    p.strideX = p.strideZ = p.strideY = 0;
-    for (uint32_t i = 0; i < c.N; i++) { p.strideF[i] = 0; p.strideInter[i] = 0; }
-    p.haveStrideInter = false;
-  }
   return H(handle)->xgemm(p, backend, t1, t2);
 }
 

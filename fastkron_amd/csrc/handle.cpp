@@ -197,6 +197,14 @@ fastKronError Handle::xgemm(KronProblem p, fastKronBackend backend, void* temp1,
   if (p.X == nullptr) return fastKronInvalidArgument;
   if (p.forward && p.N > 1)
     for (uint32_t i = 0; i + 1 < p.N; i++) if (!p.inter[i]) return fastKronInvalidArgument;
+  // A call with a single batch entry never uses its strides: they are cleared here, for every entry point, so that no
+  // plan that re-views the rows of one problem as batch entries of another (the two-part plan and the digits of a GeKMM
+  // in place do) can carry a caller's stride into a batch index of its own.
+  if (p.batch == 1) {
+    p.strideX = p.strideZ = p.strideY = 0;
+    for (uint32_t i = 0; i < p.N; i++) p.strideF[i] = p.strideInter[i] = 0;
+    p.haveStrideInter = false;
+  }
 
   // A KMM with a single column is the MKM of the same vector with transposed factors
   // (reference src/handle/handle.cpp:134-138).
@@ -257,7 +265,7 @@ fastKronError Handle::xgemm(KronProblem p, fastKronBackend backend, void* temp1,
 fastKronError Handle::xgemmOuter(const KronProblem& p, uint32_t outer, uint64_t outerX, uint64_t outerZ, uint64_t outerY,
                                  fastKronBackend backend, void* temp1, void* temp2) {
   if (outer == 0) return fastKronInvalidKMMProblem;
-  if (outer > 1) {
+  if (outer > 1 && p.batch > 1) {              // (one entry of factors: they are shared, a strided batch of X)
     const fastKronError e = runOuter(p, outer, outerX, outerZ, outerY, temp1, temp2);
     if (e != fastKronKernelNotFound) return e;
   }

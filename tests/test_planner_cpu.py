@@ -682,3 +682,45 @@ def test_gekmm_chains_of_small_factors_keep_their_digits_in_place(online_planner
         assert groups(dt, 9, [5] * 9, temp2=False) is None                                       # three groups need two temporaries
     assert groups("s", 1024, [8] * 5) is None and groups("s", 2048, [4] * 6) is None
     assert groups("d", 16, [16] * 3) is None and groups("d", 3, [9, 9]) is None
+
+
+# ---- products with two batch dimensions ----
+def outer_plan(planner, mm, dt, M, Ps, Qs, count, opX=capi.OP_N, opF=capi.OP_N, sx=None, beta=0.0, y_is_z=False):
+    """fastKronProductOuter in plan-only mode; the strides are those of compact operands unless sx gives X's."""
+    lib, h = planner
+    K, L = 1, 1
+    for p, q in zip(Ps, Qs):
+        K, L = K * p, L * q
+    ptr = [ctypes.c_void_p(BASE + i * GAP) for i in range(5)]            # x, z, y, t1, t2
+    fs = capi.arr_ptr([BASE + (8 + i) * GAP for i in range(len(Ps))])
+    sz = capi.arr_u64([count[1] * M * L, M * L])
+    e = lib.fastKronProductOuter(h, mm == "mkm", dt == "d", M, len(Ps), capi.arr_u32(Ps), capi.arr_u32(Qs), ptr[0], opX,
+                                 capi.arr_u64(sx if sx is not None else [count[1] * M * K, M * K]), fs, opF, ptr[1], sz, 1.0, beta,
+                                 capi.arr_u32(count), (ptr[1] if y_is_z else ptr[2]) if beta else None, sz, ptr[3], ptr[4])
+    buf = ctypes.create_string_buffer(1 << 16)
+    lib.fastKronGetLastPlan(h, buf, len(buf))
+    names = [s.split(":")[1] for s in buf.value.decode().split(";")[1:]]
+    lib.fastKronGetLastLaunches(h, buf, len(buf))
+    launches = []
+    for line in buf.value.decode().splitlines():
+        rec = dict(kv.split("=", 1) for kv in line.split())
+        rec["f_batch"] = [int(v) for v in rec["f_batch"].split(",")]
+        launches.append(rec)
+    return e, names, launches
+
+
+@pytest.mark.parametrize("mm,dt,M,P,N", [("kmm", "s", 88, 7, 6), ("kmm", "d", 16, 8, 5), ("mkm", "s", 8, 16, 5), ("mkm", "d", 2, 64, 3),
+                                         ("mkm", "s", 1, 31, 3), ("kmm", "s", 5, 9, 4)])
+def test_one_entry_of_two_dimensions_is_the_plain_call(online_planner, mm, dt, M, P, N):
+    """Blocks of one problem's rows become batch entries of a launch: no stride of the caller's may reach them."""
+    plain = plan(online_planner, mm, dt, M, [P] * N, [P] * N)
+    e, names, launches = outer_plan(online_planner, mm, dt, M, [P] * N, [P] * N, (1, 1))
+    assert e == plain[0] == capi.SUCCESS and names == plain[1]
+    for rec in launches:
+        assert rec["f_batch"] == [0] * len(rec["f_batch"]), rec
+    # one entry of factors for several of X: the batch with shared factors
+    shared = plan(online_planner, mm, dt, M, [P] * N, [P] * N, batch=3, strideF=[0] * N)
+    e, names, launches = outer_plan(online_planner, mm, dt, M, [P] * N, [P] * N, (3, 1))
+    assert e == shared[0] == capi.SUCCESS and names == shared[1]
+    assert [r["batch"] for r in launches] == [r["batch"] for r in shared[2]]
+    assert all(r["f_batch"] == [0] * len(r["f_batch"]) for r in launches)
