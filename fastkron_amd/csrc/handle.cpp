@@ -316,12 +316,13 @@ fastKronError Handle::runOuter(const KronProblem& p0, uint32_t outer, uint64_t o
     void* xt = nullptr;
     if (!transposedProblem(p, temp1, temp2, &pn, &xt)) return fastKronKernelNotFound;
     if (transposeFirstOnline(p, pn, temp1, temp2, nullptr)) {
-      if (inner > 1 && p.strideX != 0 && outerX != inner * p.strideX) return fastKronKernelNotFound;
+      if (p.strideX != 0 && outerX != inner * p.strideX) return fastKronKernelNotFound;
       copy = true;
-      x.batch = inner > 1 && p.strideX != 0 ? outer * inner : outer;
-      x.strideX = x.batch > outer ? p.strideX : outerX;
+      // an X that both dimensions share is copied once and read by all of them
+      x.batch = p.strideX != 0 ? outer * inner : outerX != 0 ? outer : 1;
+      x.strideX = p.strideX != 0 ? p.strideX : outerX;
       p = pn;
-      outerX = (uint64_t)p.M * p.K() * (x.batch / outer);
+      outerX = x.batch > 1 ? (uint64_t)p.M * p.K() * (x.batch / outer) : 0;
     }
   }
   p.inner = inner; p.batch = outer * inner; p.strided = true;
@@ -332,9 +333,8 @@ fastKronError Handle::runOuter(const KronProblem& p0, uint32_t outer, uint64_t o
   lastPlan_ = p.str();
   for (auto& s : plan) lastPlan_ += ";" + std::to_string(s.lo) + "-" + std::to_string(s.hi) + ":" + db_.kernels()[s.kernel].name;
   launchLog_.clear();
-  if (planOnly_) return execute(p, plan, temp1, temp2, true);
-  if (copy && launchTransposeX(x, const_cast<void*>(p.X), (uint64_t)p.M * p.K()) != hipSuccess) return fastKronInvalidArgument;
-  const fastKronError e = execute(p, plan, temp1, temp2);
+  if (copy && !planOnly_ && launchTransposeX(x, const_cast<void*>(p.X), (uint64_t)p.M * p.K()) != hipSuccess) return fastKronInvalidArgument;
+  const fastKronError e = execute(p, plan, temp1, temp2, planOnly_);
   if (e == fastKronSuccess && copy) noteTranspose(x);
   return e;
 }
@@ -1225,6 +1225,9 @@ fastKronError Handle::execute(const KronProblem& p, const Plan& plan, void* temp
           launchLog_.append(line, n > 0 ? (size_t)n : 0);
           for (uint32_t j = 0; j < c.nf && j < kMaxFused; j++)
             launchLog_ += (j ? "," : "") + std::to_string(c.f_batch[j]);
+          if (c.inner)
+            launchLog_ += " inner=" + std::to_string(c.inner) + " outer_in=" + std::to_string(c.outer.in) + " outer_out=" +
+                          std::to_string(c.outer.out) + " outer_y=" + std::to_string(c.outer.y);
           launchLog_ += "\n";
         }
         continue;

@@ -32,7 +32,9 @@ fastKronError fastKronSetTunedDB(fastKronHandle handle, const char* path);
  * an MI355X is assumed when none has been initialised.  fastKronGetLastPlan then names the kernels and
  * fastKronGetLastLaunches lists the launches the call would have made, one text line per launch:
  *   "kernel=<name> lo=<lo> hi=<hi> M=<rows> batch=<n> Kin=<cols> Kout=<cols> in=<ptr> out=<ptr> y=<ptr>
- *    in_batch=<elems> out_batch=<elems> y_batch=<elems> f_batch=<elems>,<elems>,..."
+ *    in_batch=<elems> out_batch=<elems> y_batch=<elems> stream_in=<0|1> stream_out=<0|1> f_batch=<elems>,<elems>,..."
+ * with " inner=<n> outer_in=<elems> outer_out=<elems> outer_y=<elems>" behind it for two batch dimensions (batch entry b is
+ * entry b % inner of the first and b / inner of the second).
  * fastKronGradForward is such a call; for fastKronGradBackward the lines are kernel=gradient_step, one per step of the chain,
  * and kernel=gradient_sum.
  * Meant for host-side tests of the planner and for inspecting what a call will do.  The reference has no such

@@ -724,3 +724,21 @@ def test_one_entry_of_two_dimensions_is_the_plain_call(online_planner, mm, dt, M
     assert e == shared[0] == capi.SUCCESS and names == shared[1]
     assert [r["batch"] for r in launches] == [r["batch"] for r in shared[2]]
     assert all(r["f_batch"] == [0] * len(r["f_batch"]) for r in launches)
+
+
+@pytest.mark.parametrize("count,sx,outer_in,entries", [((2, 3), "shared", 0, 1), ((2, 3), "own", None, 6), ((2, 3), "outer", None, 2)])
+def test_transposed_copies_of_two_dimensions_are_those_that_are_read(online_planner, count, sx, outer_in, entries):
+    """X of op T in front of the rows of five 8x8 factors is copied first: as many entries as differ, and the launch reads those."""
+    M, K = 32, 8 ** 5
+    strides = {"shared": [0, 0], "own": [count[1] * M * K, M * K], "outer": [M * K, 0]}[sx]
+    e, names, launches = outer_plan(online_planner, "mkm", "s", M, [8] * 5, [8] * 5, count, opX=capi.OP_T, sx=strides)
+    assert e == capi.SUCCESS and names[0].startswith("transpose_") and len(launches) == 1, (names, launches)
+    rec = launches[0]
+    lib, h = online_planner
+    buf = ctypes.create_string_buffer(1 << 12)
+    lib.fastKronGetLastPlan(h, buf, len(buf))
+    copied = buf.value.decode().split(";")[0].split("_stridedBatched_")[1]                # the problem whose X is copied
+    assert int(rec["batch"]) == count[0] * count[1] and int(rec["inner"]) == count[1] and int(copied) == entries
+    # the last entry that the launch reads is the last one that the copy has written
+    last = (count[0] - 1) * int(rec["outer_in"]) + (count[1] - 1) * int(rec["in_batch"])
+    assert last == (entries - 1) * M * K and (outer_in is None or int(rec["outer_in"]) == outer_in), rec
