@@ -264,7 +264,7 @@ fastKronError Handle::xgemm(KronProblem p, fastKronBackend backend, void* temp1,
 
 fastKronError Handle::xgemmOuter(const KronProblem& p, uint32_t outer, uint64_t outerX, uint64_t outerZ, uint64_t outerY,
                                  fastKronBackend backend, void* temp1, void* temp2) {
-  if (outer == 0) return fastKronInvalidKMMProblem;
+  if (outer == 0 || p.batch == 0) return fastKronInvalidKMMProblem;
   if (outer > 1 && p.batch > 1) {              // (one entry of factors: they are shared, a strided batch of X)
     const fastKronError e = runOuter(p, outer, outerX, outerZ, outerY, temp1, temp2);
     if (e != fastKronKernelNotFound) return e;

@@ -742,3 +742,10 @@ def test_transposed_copies_of_two_dimensions_are_those_that_are_read(online_plan
     # the last entry that the launch reads is the last one that the copy has written
     last = (count[0] - 1) * int(rec["outer_in"]) + (count[1] - 1) * int(rec["in_batch"])
     assert last == (entries - 1) * M * K and (outer_in is None or int(rec["outer_in"]) == outer_in), rec
+
+
+def test_two_dimensions_without_entries_are_refused(online_planner):
+    """As a strided batch of no entries is."""
+    for count in [(3, 0), (0, 3), (1, 0), (0, 0)]:
+        e, _, _ = outer_plan(online_planner, "mkm", "s", 4, [8, 8], [8, 8], count)
+        assert e == capi.INVALID_KMM_PROBLEM, count
