@@ -9,7 +9,8 @@
 // the B operand of the second one, whose contraction index is permuted to match (as in pair_mfma.hip): T never leaves the
 // registers.  X arrives as whole 16-byte pieces whatever its alignment, the next tile's on their way while this one is
 // multiplied, and goes through LDS to the waves of a row; elements beyond P2 and rows beyond P1 are selected to zero as they
-// are read (a product with a zero factor would make NaN of an infinity).  Results go out by quarter waves of 16 consecutive
+// are read, and the rows beyond P1 of the first product once more (padding with zeros alone would make NaN of an infinity in X
+// or F2).  Results go out by quarter waves of 16 consecutive
 // elements through a descriptor of the row's result, which drops rows beyond Q1.
 //
 // Bound: memory for large row counts, for few rows one chain of load, products and store per workgroup.
@@ -194,6 +195,14 @@ __global__ __launch_bounds__(kPaThreads, 2) void kron_pair_any_kernel(const Kern
 #pragma unroll
               for (int c = 0; c < 4; c++) d1[g] = MF::mma(4 * cg + c < limit[g] ? xv[c] : T(0), f2[4 * cg + c], d1[g]);
             }
+        }
+      // rows beyond P1 are zero times F2, NaN where that is infinite: they are zero in the second product as well
+#pragma unroll
+      for (int g = 0; g < PB; g++)
+        if (16 * g < (int)t.P1 && 16 * g + 16 > (int)t.P1) {
+#pragma unroll
+          for (int k = 0; k < 4; k++)
+            if (16 * g + MF::rowLane(hi) + MF::rowReg(k) >= (int)t.P1) d1[g][k] = T(0);
         }
     }
     __syncthreads();                                              // the tile has been read

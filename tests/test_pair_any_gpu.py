@@ -82,3 +82,24 @@ def test_infinities_stay_in_their_rows_and_operands_off_a_16_byte_boundary(fk):
         rows = [i for i in range(M) if i != 20]
         assert normwise(got[rows], want[rows]) <= TOL[np.float32]
         assert bool((z[:off] == 77.0).all()) and bool((z[off + M * L:] == 77.0).all())
+
+
+@pytest.mark.parametrize("dt", [np.float32, np.float64], ids=["f", "d"])
+@pytest.mark.parametrize("M,a,b", [(3, (31, 63), (31, 63)), (7, (50, 50), (50, 50)), (2100, (24, 48), (24, 48)), (2, (12, 20), (12, 20)), (5, (33, 17), (9, 12)),
+                                   (2, (63, 31), (47, 49)), (40, (2, 33), (5, 48)), (2, (17, 64), (64, 17))],
+                         ids=lambda v: str(v) if isinstance(v, int) else "%dx%d" % v)
+def test_infinities_of_the_factors_reach_their_columns_only(fk, M, a, b, dt):
+    """One infinity in either factor, everything else positive: infinite results in its columns, no NaN, the others as they were."""
+    import torch
+    Ps, Qs = [a[0], b[0]], [a[1], b[1]]
+    X, Fs, _ = make_case(ko.MKM, M, Ps, Qs, dt, seed=7, with_y=False, integer=True)
+    want = oracle_answer(ko.MKM, M, Ps, Qs, X, Fs, None, 1.0, 0.0).reshape(M, Qs[0], Qs[1])
+    for which, (p, q) in [(0, (0, 1)), (0, (a[0] - 1, a[1] - 1)), (1, (0, 0)), (1, (b[0] - 1, b[1] - 1))]:
+        fs = [f.copy() for f in Fs]
+        fs[which].reshape(Ps[which], Qs[which])[p, q] = np.inf
+        got, e = run_gpu(fk, ko.MKM, M, Ps, Qs, X, fs, None, 1.0, 0.0)
+        got = got.reshape(M, Qs[0], Qs[1])
+        hit = np.zeros((Qs[0], Qs[1]), bool)
+        (hit if which == 0 else hit.T)[q] = True
+        assert e == 0 and "_anyxany_64x64_2_" in fk.last_plan()[0][2], fk.last_plan()
+        assert np.all(np.isposinf(got[:, hit])) and normwise(got[:, ~hit], want[:, ~hit]) <= TOL[dt], (which, p, q)
