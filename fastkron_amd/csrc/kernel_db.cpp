@@ -142,23 +142,60 @@ static hipError_t stepAnyLaunch(const KernelInfo& k, const StepArgs& a, hipStrea
 static bool stepAnyCheck(const KernelInfo& k, const StepArgs& a) { return stepAnyMfmaSupported(a, k.dt); }
 
 // ---- two factors of any sizes up to 64x64 on the matrix cores (zero padded), whole rows ----
+// One launch against the two factors one by one (behindCopy: behind a transposed copy of X, against steps that read X as it is
+// stored).  Both sides as times fitted to 6700 calls of 1 to 60000 rows in either type (us; four of five within 0.8 to 1.2): a
+// workgroup of the pair kernel needs its 1 to 2.5 us for a row or a few however small they are, so that many rows of little work
+// lose against launches at the memory's rate (dgemkm 250000 rows of 2x2, 9x9 203 / 41, 22000 rows of 3x20, 43x57 82 / 45, sgemkm
+// 7000 of 8x64 53 / 33; 1100 rows of 50x40, 12x20 10.3 / 15.0, 515 of (48x64)^2 12.3 / 19.5).
+bool pairAnyAhead(const uint32_t* ps, const uint32_t* qs, uint64_t M, uint32_t batch, DType dt, const DeviceInfo& dev, bool behindCopy) {
+  const double rows = (double)M * batch, mrows = rows * 1e-6, es = (double)dtypeSize(dt);
+  if (!behindCopy && rows <= 256) return true;                     // (one row a workgroup: 0.5 to 0.9 of the steps' time)
+  const bool f64 = dt == DType::F64;
+  auto blocks = [](uint32_t n) { return (double)((n + 15) / 16); };
+  const double in = (double)ps[0] * ps[1] * es, mid = (double)ps[1] * qs[0] * es, out = (double)qs[0] * qs[1] * es;
+  // first round's latency; per round a chain, its products, its bytes (KB)
+  static const double fit[2][2][2][4] = {{{{4.0, 1.15, .016, .12}, {3.0, 1.4, .05, .046}}, {{4.2, 1.25, .017, .065}, {3.7, 1.65, .027, .066}}},
+                                         {{{3.7, 1.0, .037, .053}, {3.0, 1.6, .042, .034}}, {{4.2, 2.0, .03, .08}, {3.9, 2.5, .04, .05}}}};
+  const double* t = fit[f64][std::max(ps[0], ps[1]) > 32][std::max(qs[0], qs[1]) > 32];
+  const PairAnyWork w = pairAnyWork(ps, qs, M, batch, dt, (uint32_t)dev.cus);
+  const double products = blocks(ps[1]) * 4 * (((ps[0] + 3) / 4 + 3) / 4) + 4 * blocks(qs[1]) * blocks(ps[1]);
+  double pair = t[0] + (batch > 1 ? 0.6 : 0) + (double)w.rounds * (t[1] + t[2] * products + t[3] * w.rows * (in + out) / 1024);
+  if (!behindCopy && ps[0] <= 8 && ps[1] <= 8)                     // one launch of the kernel with two LDS buffers
+    return pair < 5.8 + .096 * qs[1] + .11 * qs[0] + mrows * ((in + out) * (f64 ? .3 : .57) + (double)ps[0] * ps[1] * qs[0] * (f64 ? .28 : .02) +
+                                                              (double)ps[1] * qs[0] * qs[1] * (f64 ? 1.0 : .26));
+  double apart = 0;
+  for (int j = 0; j < 2; j++) {
+    const double bytes = mrows * (j ? mid + out : in + mid), slices = mrows * (j ? qs[0] : ps[1]);
+    const double padded = slices * blocks(ps[j]) * blocks(qs[j]) * 256, real = slices * ps[j] * qs[j];
+    const bool asStored = behindCopy && j == 0;
+    if (ps[j] * qs[j] >= (f64 ? 144u : 256u))                      // the padded step, or one of the exact ones
+      apart += 4.5 + (asStored ? padded * (f64 ? .15 : .09) : bytes * (f64 ? .056 : .105) + padded * (f64 ? .063 : .03));
+    else                                                           // the plain step
+      apart += 4.2 + (!asStored ? bytes * .21 + real * .05 : f64 ? bytes * .3 + real * 1.25 : bytes * 1.5);
+  }
+  if (!behindCopy) return pair < apart;
+  apart += std::max(0.0, mrows * in - 4) * (f64 ? .6 : 1.0);       // (an X beyond one L2)
+  return pair + 4.5 + mrows * in * .6 < .9 * apart;
+}
 static bool pairAnyCanRun(const KernelInfo& k, const KronProblem& p, uint32_t lo, uint32_t hi, bool first, bool,
                           const DeviceInfo& dev) {
   if (k.dt != p.dt || p.mm != MMType::MKM || hi - lo + 1 != 2 || p.forward) return false;
   if (first && p.opX == 2) return false;
   const uint32_t ps[2] = {p.P[hi], p.P[lo]}, qs[2] = {p.Q[hi], p.Q[lo]};
   if (dev.rulesOfThumb) {
-    // Ahead of a launch per factor at every size measured (0.25 to 0.9 of their time, 1 to 20000 rows, either type), except:
-    // factors of at most 8 rows and columns, which go through LDS together with more of their kind;
+    // Not for factors of at most 8 rows and columns, which go through LDS together with more of their kind;
     if (std::max({ps[0], ps[1], qs[0], qs[1]}) <= 8) return false;
     // 64x64 and (fp64) 64x32, whose single steps have kernels and plans of their own;
     if (ps[0] == 64 && ps[1] == 64 && qs[0] == qs[1] && (qs[0] == 64 || (qs[0] == 32 && p.dt == DType::F64))) return false;
     // many rows of which most of the padded products are for nothing (33x33: 2.7 times the real ones; sgemkm 5000 rows 48.6 ->
-    // 45.7 us, 20000 rows 146 / 161; with factors of one block of 16 the products are not what bounds it).
+    // 45.7 us, 20000 rows 146 / 161; with factors of one block of 16 the products are not what bounds it);
     auto blocks = [](uint32_t n) { return (uint64_t)(n + 15) / 16; };
     const uint64_t padded = 1024 * blocks(ps[1]) * blocks(qs[0]) * ((ps[0] + 3) / 4 + 4 * blocks(qs[1]));
     const uint64_t real = (uint64_t)ps[1] * qs[0] * (ps[0] + qs[1]);
     if ((uint64_t)p.M * p.batch >= 8192 && 2 * padded > 5 * real && std::max(ps[0], ps[1]) > 16) return false;
+    // and where the factors one by one are faster.  (Equal square ones of 17x17 ... 31x31 have the padded pair instead.)
+    const bool square = ps[0] == qs[0] && ps[0] == ps[1] && ps[0] == qs[1] && ps[0] >= 17 && ps[0] < 32;
+    if (!square && !pairAnyAhead(ps, qs, p.M, p.batch, p.dt, dev, false)) return false;
   }
   return dev.ldsPerBlock >= 160 * 1024 && pairAnyFits(2, ps, qs, p.colsBefore(hi));
 }

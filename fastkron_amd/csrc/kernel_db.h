@@ -54,6 +54,9 @@ struct KernelInfo {
   CheckFn  check;
 };
 
+// Rule of the kernel for two factors of any sizes (p[0], q[0] the one applied first): M rows of p[0]*p[1] columns.
+bool pairAnyAhead(const uint32_t* p, const uint32_t* q, uint64_t M, uint32_t batch, DType dt, const DeviceInfo& dev, bool behindCopy);
+
 struct PlanStep { uint32_t lo, hi; int kernel; };   // factors [lo, hi], hi applied first
 using Plan = std::vector<PlanStep>;
 

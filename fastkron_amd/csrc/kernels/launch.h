@@ -112,6 +112,9 @@ hipError_t launchPairMfma(const StepArgs& a, DType dt, hipStream_t stream);
 bool pairAnyFits(uint32_t nf, const uint32_t* p, const uint32_t* q, uint64_t Kin);
 bool pairAnySupported(const StepArgs& a, DType dt);
 hipError_t launchPairAny(const StepArgs& a, DType dt, hipStream_t stream);
+// How a device with so many CUs runs it: rows per workgroup at a time, and how often a workgroup takes some.
+struct PairAnyWork { uint32_t rows; uint64_t rounds; };
+PairAnyWork pairAnyWork(const uint32_t* p, const uint32_t* q, uint64_t M, uint32_t batch, DType dt, uint32_t cus);
 
 // Three fused 8x8 fp32 factors in the KMM layout, 512 rows by 64 columns per workgroup.
 bool kmm8x3Supported(const StepArgs& a);

@@ -255,17 +255,37 @@ bool pairAnySupported(const StepArgs& a, DType dt) {
   return true;
 }
 
+static uint32_t paWaves(int PB, uint32_t Q2) {
+  const uint32_t blocks = (Q2 + 15) / 16, waves = blocks > 2 ? 4 : blocks;
+  return std::max(waves, 4 / paItems(PB));
+}
+// (several rows per workgroup only where there are rows for all CUs twice over)
+static uint32_t paRows(uint32_t waves, uint64_t rows, uint32_t cus) {
+  uint32_t items = 4 / waves;
+  while (items > 1 && rows < 2ull * items * cus) items /= 2;
+  return items;
+}
+// Workgroups at once per batch entry: two waves per SIMD, four of the kernels that need few registers.
+static uint32_t paWorkgroups(int PB, size_t es, uint32_t batch, uint32_t cus) {
+  return ((es == 4 && PB == 2 ? 4 : 2) * cus + batch - 1) / batch;
+}
+PairAnyWork pairAnyWork(const uint32_t* p, const uint32_t* q, uint64_t M, uint32_t batch, DType dt, uint32_t cus) {
+  const int PB = std::max(p[0], p[1]) > 32 ? 4 : 2;
+  PairAnyWork w;
+  w.rows = paRows(paWaves(PB, q[0]), M * batch, cus);
+  const uint64_t tiles = (M + w.rows - 1) / w.rows, at = std::min<uint64_t>(tiles, paWorkgroups(PB, dtypeSize(dt), batch, cus));
+  w.rounds = (tiles + at - 1) / at;
+  return w;
+}
+
 template <typename T, int PB, int QB, bool HAS_Y>
 static hipError_t launchPairAnyAs(const StepArgs& a, hipStream_t stream) {
   constexpr uint32_t VE = 16 / sizeof(T);
   PairAnyTile t{};
   t.P2 = a.p[0]; t.Q2 = a.q[0]; t.P1 = a.p[1]; t.Q1 = a.q[1];
-  const uint32_t blocks = (t.Q2 + 15) / 16;
-  t.waves = blocks > 2 ? 4 : blocks;
-  if (4 / t.waves > paItems(PB)) t.waves = 4 / paItems(PB);
-  // several rows per workgroup only where there are rows for all CUs twice over
-  t.items = 4 / t.waves;
-  while (t.items > 1 && (uint64_t)a.M * a.batch < 2ull * t.items * deviceCUs()) t.items /= 2;
+  const uint32_t cus = (uint32_t)deviceCUs();
+  t.waves = paWaves(PB, t.Q2);
+  t.items = paRows(t.waves, (uint64_t)a.M * a.batch, cus);
   t.tiles = (a.M + t.items - 1) / t.items;
   t.pitchedMagic = t.P2 % VE == 0 && t.P2 > VE ? (uint32_t)((1ull << 32) / (t.P2 / VE)) + 1 : 0;       // (pieces are below 2^12)
   constexpr bool f1Lds = sizeof(T) == 8 && PB == 4;
@@ -277,9 +297,7 @@ static hipError_t launchPairAnyAs(const StepArgs& a, hipStream_t stream) {
     if (const hipError_t e = hipFuncSetAttribute((const void*)kernel, hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024); e != hipSuccess) return e;
     attrOnce.mark(dev);
   }
-  // two waves per SIMD, four of the kernels that need few registers
-  const uint32_t resident = (sizeof(T) == 4 && PB == 2 ? 4 : 2) * (uint32_t)deviceCUs(), perBatch = (resident + a.batch - 1) / a.batch;
-  hipLaunchKernelGGL(kernel, dim3(std::min(t.tiles, perBatch), innerEntries(a), outerEntries(a)), dim3(kPaThreads), lds, stream, a, t, a.outer);
+  hipLaunchKernelGGL(kernel, dim3(std::min(t.tiles, paWorkgroups(PB, sizeof(T), a.batch, cus)), innerEntries(a), outerEntries(a)), dim3(kPaThreads), lds, stream, a, t, a.outer);
   return hipGetLastError();
 }
 template <typename T, int PB, int QB>

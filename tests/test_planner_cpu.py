@@ -684,6 +684,30 @@ def test_gekmm_chains_of_small_factors_keep_their_digits_in_place(online_planner
     assert groups("d", 16, [16] * 3) is None and groups("d", 3, [9, 9]) is None
 
 
+PAIR = "_anyxany_64x64_2_1xany_"
+
+
+@pytest.mark.parametrize("dt,M,a,b,pair", [
+    # one launch (us against the two steps): few rows always, many where a row is enough work
+    ("s", 1, (31, 63), (31, 63), True), ("s", 256, (2, 2), (9, 9), True), ("s", 1100, (50, 40), (12, 20), True), ("d", 2500, (33, 17), (9, 12), True),
+    ("d", 1003, (31, 63), (31, 63), True), ("d", 515, (48, 64), (48, 64), True),
+    # the two steps: dgemkm 203 / 41, 82 / 45, sgemkm 53 / 33, and the kernel with two LDS buffers 35.7 / 14.8
+    ("d", 251160, (2, 2), (9, 9), False), ("d", 7300, (3, 20), (43, 57), False), ("s", 7038, (8, 8), (64, 64), False), ("d", 44884, (2, 10), (7, 5), False)])
+def test_two_factors_are_one_launch_where_that_is_faster(online_planner, dt, M, a, b, pair):
+    for opF in (capi.OP_N, capi.OP_T):
+        e, names, _ = plan(online_planner, "mkm", dt, M, [a[0], b[0]], [a[1], b[1]], opF=opF)
+        assert e == capi.SUCCESS and any(PAIR in n for n in names) == pair, names
+
+
+@pytest.mark.parametrize("dt,M,a,b,copied", [
+    # sgemkm 59 / 144 and 15 / 18 with the copy; 33 / 19, 15.5 / 13.9 and 11.3 / 9.6 with it, without
+    ("s", 7936, (62, 62), (20, 20), True), ("s", 26247, (14, 14), (12, 12), True), ("d", 6685, (2, 1), (32, 40), False), ("s", 284, (33, 33), (33, 33), False),
+    ("s", 40, (33, 33), (50, 50), False), ("s", 100, (31, 31), (31, 31), True)])
+def test_transposed_x_is_copied_for_the_pair_only_where_that_is_faster(online_planner, dt, M, a, b, copied):
+    e, names, _ = plan(online_planner, "mkm", dt, M, [a[0], b[0]], [a[1], b[1]], opX=capi.OP_T)
+    assert e == capi.SUCCESS and names[0].startswith("transpose_") == copied, names
+
+
 # ---- products with two batch dimensions ----
 def outer_plan(planner, mm, dt, M, Ps, Qs, count, opX=capi.OP_N, opF=capi.OP_N, sx=None, beta=0.0, y_is_z=False):
     """fastKronProductOuter in plan-only mode; the strides are those of compact operands unless sx gives X's."""
