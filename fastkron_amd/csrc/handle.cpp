@@ -522,14 +522,11 @@ bool Handle::transposeFirstOnline(const KronProblem& p, const KronProblem& pn, v
     const bool copyOnTie = p.mm == MMType::MKM || p.M >= 64 || p.P[p.N - 1] < 16;
     yes = okN && (!okT || (copyOnTie ? 1 + nN <= nT : 1 + nN < nT));
     // where the copy makes the last two factors a launch of the pair of any sizes, that one's rule decides (opX = T, us: sgemkm
-    // 284 rows of 33x33 13.9 without the copy / 15.5, dgemkm 6685 rows of 2x1, 32x40 18.9 / 33.2; factors of at most 8 rows
-    // are transposed for the kernel with two LDS buffers anyway, equal ones of 17x17 ... 31x31 for the padded pair)
+    // 284 rows of 33x33 13.9 without the copy / 15.5, dgemkm 6685 rows of 2x1, 32x40 18.9 / 33.2)
     const size_t n0 = planN.second.find(':');
     if (yes && okT && 1 + nN == nT && p.N >= 2 && n0 != std::string::npos && planN.second.find("_anyxany_64x64_2_", n0) < planN.second.find(';', n0)) {
       const uint32_t ps[2] = {p.P[p.N - 1], p.P[p.N - 2]}, qs[2] = {p.Q[p.N - 1], p.Q[p.N - 2]};
-      const bool square = ps[0] == qs[0] && ps[0] == ps[1] && ps[0] == qs[1] && ps[0] >= 17 && ps[0] < 32;
-      if (!square && (ps[0] > 8 || ps[1] > 8))
-        yes = pairAnyAhead(ps, qs, (uint64_t)p.M * (p.K() / ((uint64_t)ps[0] * ps[1])), p.batch, p.dt, dev_, true);
+      yes = pairAnyAhead(ps, qs, (uint64_t)p.M * (p.K() / ((uint64_t)ps[0] * ps[1])), p.batch, p.dt, dev_, true);
     }
     transposeCache_[ck] = yes;           // the preference of the shape; the buffers of each call are checked below
   }

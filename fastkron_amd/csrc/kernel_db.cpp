@@ -142,6 +142,16 @@ static hipError_t stepAnyLaunch(const KernelInfo& k, const StepArgs& a, hipStrea
 static bool stepAnyCheck(const KernelInfo& k, const StepArgs& a) { return stepAnyMfmaSupported(a, k.dt); }
 
 // ---- two factors of any sizes up to 64x64 on the matrix cores (zero padded), whole rows ----
+// Two equal square factors of 17x17 ... 31x31: the padded pair, but for many rows in fp32 the kernel that reads them in whole
+// pieces (us: sgemkm 5000 x 24^2 16.2 -> 11.6, 31^2 18.0 -> 13.6, 20000 x 20^2 40.0 -> 32.4; 1003 x 31^2 6.1 / 6.8, dgemkm
+// 5000 x 20^2 18.2 / 18.5, 20000 rows 53.6 / 60.1).
+static bool paddedPairSize(const uint32_t* ps, const uint32_t* qs) {
+  return ps[0] == qs[0] && ps[0] == ps[1] && ps[0] == qs[1] && ps[0] >= 17 && ps[0] < 32;
+}
+static bool paddedPairInPieces(const KronProblem& p, const DeviceInfo& dev) {
+  return p.dt == DType::F32 && (uint64_t)p.M * p.batch >= 2048 && dev.ldsPerBlock >= 160 * 1024;
+}
+
 // One launch against the two factors one by one (behindCopy: behind a transposed copy of X, against steps that read X as it is
 // stored).  Both sides as times fitted to 6700 calls of 1 to 60000 rows in either type (us; four of five within 0.8 to 1.2): a
 // workgroup of the pair kernel needs its 1 to 2.5 us for a row or a few however small they are, so that many rows of little work
@@ -150,6 +160,8 @@ static bool stepAnyCheck(const KernelInfo& k, const StepArgs& a) { return stepAn
 bool pairAnyAhead(const uint32_t* ps, const uint32_t* qs, uint64_t M, uint32_t batch, DType dt, const DeviceInfo& dev, bool behindCopy) {
   const double rows = (double)M * batch, mrows = rows * 1e-6, es = (double)dtypeSize(dt);
   if (!behindCopy && rows <= 256) return true;                     // (one row a workgroup: 0.5 to 0.9 of the steps' time)
+  // (the padded pair and the kernel with two LDS buffers would want the copy as well)
+  if (behindCopy && (paddedPairSize(ps, qs) || (ps[0] <= 8 && ps[1] <= 8))) return true;
   const bool f64 = dt == DType::F64;
   auto blocks = [](uint32_t n) { return (double)((n + 15) / 16); };
   const double in = (double)ps[0] * ps[1] * es, mid = (double)ps[1] * qs[0] * es, out = (double)qs[0] * qs[1] * es;
@@ -187,15 +199,16 @@ static bool pairAnyCanRun(const KernelInfo& k, const KronProblem& p, uint32_t lo
     if (std::max({ps[0], ps[1], qs[0], qs[1]}) <= 8) return false;
     // 64x64 and (fp64) 64x32, whose single steps have kernels and plans of their own;
     if (ps[0] == 64 && ps[1] == 64 && qs[0] == qs[1] && (qs[0] == 64 || (qs[0] == 32 && p.dt == DType::F64))) return false;
+    // equal ones of 17x17 ... 31x31 where the padded pair is faster;
+    if (paddedPairSize(ps, qs)) return paddedPairInPieces(p, dev) && pairAnyFits(2, ps, qs, p.colsBefore(hi));
     // many rows of which most of the padded products are for nothing (33x33: 2.7 times the real ones; sgemkm 5000 rows 48.6 ->
     // 45.7 us, 20000 rows 146 / 161; with factors of one block of 16 the products are not what bounds it);
     auto blocks = [](uint32_t n) { return (uint64_t)(n + 15) / 16; };
     const uint64_t padded = 1024 * blocks(ps[1]) * blocks(qs[0]) * ((ps[0] + 3) / 4 + 4 * blocks(qs[1]));
     const uint64_t real = (uint64_t)ps[1] * qs[0] * (ps[0] + qs[1]);
     if ((uint64_t)p.M * p.batch >= 8192 && 2 * padded > 5 * real && std::max(ps[0], ps[1]) > 16) return false;
-    // and where the factors one by one are faster.  (Equal square ones of 17x17 ... 31x31 have the padded pair instead.)
-    const bool square = ps[0] == qs[0] && ps[0] == ps[1] && ps[0] == qs[1] && ps[0] >= 17 && ps[0] < 32;
-    if (!square && !pairAnyAhead(ps, qs, p.M, p.batch, p.dt, dev, false)) return false;
+    // and where the factors one by one are faster
+    if (!pairAnyAhead(ps, qs, p.M, p.batch, p.dt, dev, false)) return false;
   }
   return dev.ldsPerBlock >= 160 * 1024 && pairAnyFits(2, ps, qs, p.colsBefore(hi));
 }
@@ -401,6 +414,7 @@ static bool pairCanRun(const KernelInfo& k, const KronProblem& p, uint32_t lo, u
   for (uint32_t i = lo; i <= hi; i++) if (p.P[i] != P || p.Q[i] != P) return false;
   if (p.colsBefore(hi) != (uint64_t)P * P) return false;
   if (first && p.opX == 2) return false;
+  if (dev.rulesOfThumb && P < 32 && paddedPairInPieces(p, dev)) return false;
   // one wave per 64x64 block: with few blocks two single-factor launches, whose tiles are 16 times smaller, fill the
   // device better (tuned plans at 256 blocks: 1.4 times faster in fp32, 1.9 times in fp64; at 1024 blocks the pair wins)
   // fp64, a block per wave and two waves per SIMD: from 8 blocks per CU on; with up to 4 per CU two or four waves share a

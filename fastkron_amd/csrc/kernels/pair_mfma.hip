@@ -639,12 +639,7 @@ hipError_t launchPairMfma(const StepArgs& a, DType dt, hipStream_t stream) {
     if (dt == DType::F64) return launchPairT<double, 32, true, 64>(a, stream);
     return a.p[0] == 32 ? launchPairT<float, 32, true, 64>(a, stream) : launchPairT<float, 64, true, 32>(a, stream);
   }
-  if (a.p[0] < 32) {
-    // many rows in fp32: the kernel that reads them in whole pieces (5000 x 24^2 16.2 -> 11.6 us, 31^2 18.0 -> 13.6, 20000 x 20^2
-    // 40.0 -> 32.4; 1003 rows of 31^2 6.1 / 6.8, and in fp64 5000 x 20^2 18.2 / 18.5, 20000 rows 53.6 / 60.1)
-    if (dt == DType::F32 && (uint64_t)a.M * a.batch >= 2048 && pairAnySupported(a, dt)) return launchPairAny(a, dt, stream);
-    return dt == DType::F64 ? launchPairT<double, 32, false>(a, stream) : launchPairT<float, 32, false>(a, stream);
-  }
+  if (a.p[0] < 32) return dt == DType::F64 ? launchPairT<double, 32, false>(a, stream) : launchPairT<float, 32, false>(a, stream);
   if (dt == DType::F64) return a.p[0] == 64 ? launchPair64(a, stream) : launchPairT<double, 32>(a, stream);
   return a.p[0] == 64 ? launchPairT<float, 64>(a, stream) : launchPairT<float, 32>(a, stream);
 }

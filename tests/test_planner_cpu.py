@@ -708,6 +708,21 @@ def test_transposed_x_is_copied_for_the_pair_only_where_that_is_faster(online_pl
     assert e == capi.SUCCESS and names[0].startswith("transpose_") == copied, names
 
 
+def test_padded_pairs_of_many_rows_name_the_kernel_that_runs(planner, tmp_path):
+    """Equal factors of 17x17 ... 31x31 on 2048 rows and more, fp32: the pair of any sizes by rule, the padded pair by record."""
+    padded = "mkm_hip_gfx950_256_f_32x32_32x32_2_1x1024_mfma16x16x4_NN_strided_0_3"
+    for P in (17, 20, 24, 31):
+        for dt, M, batch, any_size in [("s", 2047, None, False), ("s", 2048, None, True), ("s", 30000, None, True), ("s", 700, 3, True), ("d", 30000, None, False)]:
+            e, names, _ = plan(planner, "mkm", dt, M, [P] * 2, [P] * 2, batch=batch)
+            assert e == capi.SUCCESS and len(names) == 1 and ((PAIR if any_size else "_32x32_32x32_2_1x1024_") in names[0]), (P, dt, M, names)
+    lib, h = planner
+    db = tmp_path / "plans.txt"
+    db.write_text(f"5000x576*(24x24^2)_NN_f 0.01 M0 S0 1 0 1 {padded}\n")
+    lib.fastKronSetTunedDB(h, str(db).encode())
+    e, names, _ = plan(planner, "mkm", "s", 5000, [24] * 2, [24] * 2)
+    assert e == capi.SUCCESS and names == [padded]
+
+
 # ---- products with two batch dimensions ----
 def outer_plan(planner, mm, dt, M, Ps, Qs, count, opX=capi.OP_N, opF=capi.OP_N, sx=None, beta=0.0, y_is_z=False):
     """fastKronProductOuter in plan-only mode; the strides are those of compact operands unless sx gives X's."""
