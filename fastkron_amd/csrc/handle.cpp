@@ -556,7 +556,18 @@ static std::string selectionKey(const KronProblem& p, uint32_t more = 0) {
 
 fastKronError Handle::runOnline(KronProblem p, void* temp1, void* temp2, const CallWorkspace* ws) {
   fastKronError e;
-  if (useFusion() && p.mm == MMType::KMM && !p.forward && p.N >= 2 && p.M > 1) {
+  // (records without the merge / split fields are keyed by the chain as the online rules rewrite it, and are asked before them)
+  auto recorded = [&](const KronProblem& q, Plan* plan) {
+    int merge = -1;
+    return !q.forward && db_.openRecords() && db_.lookupTuned(q.str(), plan, &merge) && merge < 0 && db_.validPlan(q, *plan, dev_);
+  };
+  auto recordedMerged = [&]() {
+    KronProblem q;
+    MergeArgs unused;
+    Plan plan;
+    return db_.openRecords() && recorded(mergedProblem(p, &q, &unused, ws) ? q : p, &plan);
+  };
+  if (useFusion() && p.mm == MMType::KMM && !p.forward && p.N >= 2 && p.M > 1 && !recordedMerged()) {
     bool pairs = false;                  // (neighbours that a group could hold)
     for (uint32_t i = 1; i < p.N; i++) pairs = pairs || (p.P[i] <= 8 && p.P[i] == p.P[i - 1] && p.P[i] == p.Q[i] && p.P[i] == p.Q[i - 1]);
     if (pairs) {
@@ -576,12 +587,7 @@ fastKronError Handle::runOnline(KronProblem p, void* temp1, void* temp2, const C
 
   Plan plan;
   const std::string key = p.str();
-  bool have = false;
-  // (records without the merge / split fields are keyed by the chain as the online rules rewrite it)
-  if (!p.forward) {
-    int merge = -1;
-    have = db_.lookupTuned(key, &plan, &merge) && merge < 0 && db_.validPlan(p, plan, dev_);
-  }
+  const bool have = recorded(p, &plan);
   // chains longer than one whole-block kernel: the two-part plan, when the problem and the buffers allow it
   if (!have && useFusion()) {
     e = trySplitLeadingTrailing(p, temp1, temp2);
@@ -640,7 +646,7 @@ const Plan& Handle::select(const KronProblem& p) const {
 
 static bool isPow2(uint32_t v) { return v && !(v & (v - 1)); }
 
-bool Handle::mergeSmallFactors(const KronProblem& p, KronProblem* out, const CallWorkspace* ws) {
+bool Handle::mergedProblem(const KronProblem& p, KronProblem* out, MergeArgs* args, const CallWorkspace* ws) const {
   void* const wsBase = ws ? ws->merge : mergeWs_;
   const size_t wsBytes = ws ? ws->mergeBytes : mergeWsBytes_;
   if (!wsBase || p.forward || p.N < 2) return false;
@@ -699,7 +705,7 @@ bool Handle::mergeSmallFactors(const KronProblem& p, KronProblem* out, const Cal
   if (mergedGroups == 0 || mergedGroups > kMaxMergeGroups) return false;
 
   const bool pMajor = (p.mm == MMType::MKM) == (p.opF == fastKronOp_N);   // as in makeStepArgs
-  MergeArgs ma{};
+  MergeArgs& ma = *args = MergeArgs{};
   KronProblem q = p;
   q.N = ng;
   size_t wsOff = 0;
@@ -726,6 +732,14 @@ bool Handle::mergeSmallFactors(const KronProblem& p, KronProblem* out, const Cal
     wsOff += (bytes + 255) & ~(size_t)255;
     q.P[g] = G.size; q.Q[g] = G.size; q.F[g] = mg.dst;
   }
+  *out = q;
+  return true;
+}
+
+bool Handle::mergeSmallFactors(const KronProblem& p, KronProblem* out, const CallWorkspace* ws) {
+  MergeArgs ma;
+  KronProblem q;
+  if (!mergedProblem(p, &q, &ma, ws)) return false;
   if (!planOnly_) {
     if (!ws && mergeWsUsed_ && mergeWsStream_ != stream_) orderWorkspaceBehind(stream_);
     if (launchMergeFactors(ma, p.dt, stream_) != hipSuccess) return false;
@@ -917,14 +931,8 @@ Plan Handle::columnsPlan(const KronProblem& p) const {
   // sgekmm 6^6 x 88 58.8 -> 22.2, dgekmm 5^6 x 1024 217 -> 95); as many launches of the register kernels are no slower
   // (sgekmm 8^5 x 64 19.8, 1024 columns 113)
   KronProblem q = p;
-  size_t merge = 0;
-  {
-    Handle* self = const_cast<Handle*>(this);
-    const bool was = planOnly_;
-    self->planOnly_ = true;
-    if (self->mergeSmallFactors(p, &q)) merge = 1;
-    self->planOnly_ = was;
-  }
+  MergeArgs unused;
+  const size_t merge = mergedProblem(p, &q, &unused) ? 1 : 0;
   const Plan& other = select(q);
   bool lds = false, merged16 = merge != 0;
   for (auto& s : other) lds = lds || db_.kernels()[s.kernel].name.find("_small_fused_lds_") != std::string::npos;

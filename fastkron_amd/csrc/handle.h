@@ -96,6 +96,8 @@ class Handle {
   // (16x16; 64x64 in fp64 when the chain holds 8x8 or 32x32 factors), computed into the handle's workspace by one small launch, so that the
   // kernels for those sizes apply.  Returns false when nothing is merged; on true `out` is the merged problem.
   bool mergeSmallFactors(const KronProblem& p, KronProblem* out, const CallWorkspace* ws = nullptr);
+  // The same without the launch: the merged problem and what the launch would be given.
+  bool mergedProblem(const KronProblem& p, KronProblem* out, MergeArgs* args, const CallWorkspace* ws = nullptr) const;
 
   // Forward pass that keeps what the backward pass needs, and the backward pass (gradient.cpp).
   struct GradProblem {

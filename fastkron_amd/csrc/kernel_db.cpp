@@ -828,6 +828,7 @@ void KernelDB::storeTuned(const std::string& key, const Plan& plan, float ms, in
   t.ms = ms; t.merge = merge; t.split = split; t.transposeX = transposeX;
   for (auto& s : plan) t.steps.push_back({{s.lo, s.hi}, kernels_[s.kernel].name});
   tuned_[key] = t;
+  openRecords_ = openRecords_ || merge < 0;
 }
 
 // File format, one problem per line:
@@ -869,7 +870,9 @@ bool KernelDB::loadFile(const std::string& path, bool shipped) {
       if (!(is >> lo >> hi >> name)) { ok = false; break; }
       t.steps.push_back({{lo, hi}, name});
     }
-    if (ok) tuned_[key] = t;
+    if (!ok) continue;
+    tuned_[key] = t;
+    openRecords_ = openRecords_ || t.merge < 0;
   }
   return true;
 }

@@ -89,6 +89,8 @@ class KernelDB {
   // `transposeX` (1: op(X) = T is handled by a transposed copy of X ahead of the launches, which then see op(X) = N).
   bool lookupTuned(const std::string& key, Plan* plan, int* merge = nullptr, uint32_t* split = nullptr,
                    int* transposeX = nullptr) const;
+  // Whether any record leaves both to the online selection (merge -1).
+  bool openRecords() const { return openRecords_; }
   void storeTuned(const std::string& key, const Plan& plan, float ms, int merge = -1, uint32_t split = 0,
                   int transposeX = 0);
   // `shipped`: the records come from the file that ships with the library; saveFile leaves those out, so that a
@@ -109,6 +111,7 @@ class KernelDB {
     bool shipped = false;
   };
   std::map<std::string, Tuned> tuned_;
+  bool openRecords_ = false;
 };
 
 // Filled in by each kernel family's translation unit.

@@ -788,3 +788,19 @@ def test_two_dimensions_without_entries_are_refused(online_planner):
     for count in [(3, 0), (0, 3), (1, 0), (0, 0)]:
         e, _, _ = outer_plan(online_planner, "mkm", "s", 4, [8, 8], [8, 8], count)
         assert e == capi.INVALID_KMM_PROBLEM, count
+
+
+# ---- records and caches of a handle ----
+@pytest.mark.parametrize("dt,M,P,N,key,steps", [("s", 88, 7, 4, "(7x7^4)*2401x88_NN_f", 4), ("d", 88, 7, 4, "(7x7^4)*2401x88_NN_d", 4),
+                                                ("d", 1000, 4, 5, "(4x4(x)16x16(x)16x16)*1024x1000_NN_d", 3)])
+def test_records_without_rewriting_fields_come_before_the_rules_for_columns(online_planner, tmp_path, dt, M, P, N, key, steps):
+    """Plan files written before records said how a chain is rewritten hold it as the rules rewrote it (the last one: merged)."""
+    lib, h = online_planner
+    e, names, _ = plan(online_planner, "kmm", dt, M, [P] * N, [P] * N)
+    assert e == capi.SUCCESS and any("columns" in n for n in names), names
+    generic = "gekmm_hip_gfx950_256_%s_generic_1" % ("f" if dt == "s" else "d")
+    f = tmp_path / "open.db"
+    f.write_text(f"{key} 0.01 {steps} " + " ".join(f"{i} {i} {generic}" for i in reversed(range(steps))) + "\n")
+    lib.fastKronSetTunedDB(h, str(f).encode())
+    e, names, _ = plan(online_planner, "kmm", dt, M, [P] * N, [P] * N)
+    assert e == capi.SUCCESS and names == [generic] * steps, names
