@@ -298,6 +298,7 @@ fastKronError Handle::xgemmOuter(const KronProblem& p, uint32_t outer, uint64_t 
 
 // fastKronKernelNotFound: not in this form (nothing has been launched).
 fastKronError Handle::runOuter(const KronProblem& p0, uint32_t outer, uint64_t outerX, uint64_t outerZ, uint64_t outerY, void* temp1, void* temp2) {
+  trimCaches();
   KronProblem p = p0;
   if (!p.X || !p.Z || !temp1 || !temp2 || p.N == 0 || p.N > kMaxFactors || p.M == 0 || p.batch == 0 || p.forward || !useFusion() || canTune())
     return fastKronKernelNotFound;
@@ -541,6 +542,13 @@ bool Handle::transposeFirstOnline(const KronProblem& p, const KronProblem& pn, v
   return true;
 }
 
+// (Called where nothing refers to an entry.)
+void Handle::trimCaches() {
+  if (planCache_.size() > kMaxCached) planCache_.clear();
+  if (selectCache_.size() > kMaxCached) selectCache_.clear();
+  if (transposeCache_.size() > kMaxCached) transposeCache_.clear();
+}
+
 // What the kernels' rules look at, as bytes.
 static std::string selectionKey(const KronProblem& p, uint32_t more = 0) {
   uint32_t key[8 + 2 * kMaxFactors];
@@ -555,6 +563,7 @@ static std::string selectionKey(const KronProblem& p, uint32_t more = 0) {
 }
 
 fastKronError Handle::runOnline(KronProblem p, void* temp1, void* temp2, const CallWorkspace* ws) {
+  trimCaches();
   fastKronError e;
   // (records without the merge / split fields are keyed by the chain as the online rules rewrite it, and are asked before them)
   auto recorded = [&](const KronProblem& q, Plan* plan) {

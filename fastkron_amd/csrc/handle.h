@@ -140,6 +140,9 @@ class Handle {
   bool hipInit_ = false;
   DeviceInfo dev_;
   KernelDB db_;
+  // What the rules said of a problem.  A program with ever new sizes would fill them without end: a full one begins anew.
+  static constexpr size_t kMaxCached = 4096;
+  void trimCaches();
   std::unordered_map<std::string, Plan> planCache_;   // online selections, per problem string
   mutable std::unordered_map<std::string, Plan> selectCache_;   // ... per what the kernels' rules look at
   std::unordered_map<std::string, bool> transposeCache_;   // op(X) = T: transpose first or not, per problem string

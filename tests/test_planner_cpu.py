@@ -804,3 +804,20 @@ def test_records_without_rewriting_fields_come_before_the_rules_for_columns(onli
     lib.fastKronSetTunedDB(h, str(f).encode())
     e, names, _ = plan(online_planner, "kmm", dt, M, [P] * N, [P] * N)
     assert e == capi.SUCCESS and names == [generic] * steps, names
+
+
+def test_a_handle_keeps_a_bounded_number_of_plans(online_planner):
+    """Calls with ever new row counts: what the handle remembers of them stops growing (50000 problems took 34 MB)."""
+    import os
+    lib, h = online_planner
+    page = os.sysconf("SC_PAGE_SIZE")
+    resident = lambda: int(open("/proc/self/statm").read().split()[1]) * page
+    def calls(lo, hi):
+        ps, x = capi.arr_u32([24] * 3), ctypes.c_void_p(BASE)
+        fs = capi.arr_ptr([BASE] * 3)
+        for M in range(lo, hi):
+            assert lib.sgemkm(h, capi.BACKEND_HIP, M, 3, ps, ps, x, capi.OP_T, fs, capi.OP_N, x, ctypes.c_float(1), ctypes.c_float(0), None, x, x) == 0
+    calls(1, 12000)
+    before = resident()
+    calls(12000, 62000)
+    assert resident() - before < 8 << 20
