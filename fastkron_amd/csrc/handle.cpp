@@ -352,13 +352,14 @@ bool Handle::viaMKMOnline(const KronProblem& p) const {
     // 32 x 8^6, 33 MB: no difference, 48 x 16^4, 13 MB: 23 -> 37 us; fp64 loses 1.1 to 1.6 times)
     if (p.dt != DType::F32 || p.M >= 64 || (uint64_t)p.M * p.K() * 4 < (64ull << 20)) return false;
     // (groups of small factors whose digits stay in place need no transposition: sgekmm 30 x 7^7 239 -> 159 us, 40 x 5^9
-    // 1014 -> 562, 50 x 4^10 419 -> 285; chains with 8x8 factors keep this plan, which is fixed for them, 16 x 8^8 1532 / 1130)
+    // 1014 -> 562, 50 x 4^10 419 -> 285; chains with 8x8 factors keep this plan, which is fixed for them, 16 x 8^8 1532 / 1130;
+    // chains without such groups, 2 x 17 columns of 4x3x7x6x3x6x5x6x4 551 / 688)
     bool small = true;
     for (uint32_t i = 0; i < p.N; i++) {
       if (p.P[i] != p.Q[i] || p.P[i] > 32) return false;
       small = small && p.P[i] < 8;
     }
-    return !small;
+    return !small || columnsPlan(p).empty();
   }
   // Measured on the reference's published shapes with both operands transposed.  Square factors up to 32x32 gain 1.3
   // to 2.8 times in fp32 (sgekmm 1024 x 8^5 171 -> 112 us, 16 x 8^8 3.34 -> 1.20 ms) and up to 1.2 times in fp64.  With

@@ -790,6 +790,18 @@ def test_two_dimensions_without_entries_are_refused(online_planner):
         assert e == capi.INVALID_KMM_PROBLEM, count
 
 
+def test_gekmm_of_small_factors_runs_as_a_gemkm_where_no_digits_stay_in_place(online_planner):
+    """fp32, few columns, 64 MB of X and more: no equal neighbours, or batches whose factors or gaps rule the groups out."""
+    def via(M, Ps, **kw):
+        e, names, _ = plan(online_planner, "kmm", "s", M, Ps, Ps, **kw)
+        assert e == capi.SUCCESS
+        return names[0].startswith("transpose_") and names[-1].startswith("transpose_")
+    mixed, equal = [4, 3, 7, 6, 3, 6, 5, 6, 4], [7] * 7
+    assert via(17, mixed) and via(17, mixed, batch=2) and via(17, mixed, batch=2, strideF=[0] * 9)
+    assert not via(30, equal) and not via(30, equal, batch=2, strideF=[0] * 7)
+    assert via(30, equal, batch=2) and via(30, equal, batch=2, strideF=[0] * 7, strides={"x": 30 * 7 ** 7 + 32})
+
+
 # ---- records and caches of a handle ----
 @pytest.mark.parametrize("dt,M,P,N,key,steps", [("s", 88, 7, 4, "(7x7^4)*2401x88_NN_f", 4), ("d", 88, 7, 4, "(7x7^4)*2401x88_NN_d", 4),
                                                 ("d", 1000, 4, 5, "(4x4(x)16x16(x)16x16)*1024x1000_NN_d", 3)])
