@@ -216,11 +216,17 @@ PyObject* product(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
   const bool fold = o.folds() && (!y.defined() || yb == o.zb);
   const int64_t M = fold ? o.M * prod(o.zb) : o.M;
   const bool one = fold || o.zb.empty();
+  if (!one && o.zb.back() > kMaxCount) return failed(fastKronInvalidKMMProblem);
+  size_t ye = 0, te = 0;
+  fastKronError e = api.sizes(c.handle, (uint32_t)M, o.N, o.Ps, o.Qs, &ye, &te);
+  if (e != fastKronSuccess) return failed(e);
+  // more entries in a call than the innermost dimension has only while the temporaries stay small beside the operands (X of
+  // (64, 1) entries and factors of (2): two temporaries of 64 entries would be as much as Z again)
+  auto room = [&](int64_t entries) { return entries <= o.zb.back() || te * (size_t)entries * es <= (size_t)256 << 20; };
   // batch dimensions as steps of every operand in entries, neighbours merged where all operands go on in one
   struct Dim { int64_t n, x, f, y, z; };
   c10::SmallVector<Dim, 8> dims;
   if (!one) {
-    if (o.zb.back() > kMaxCount) return failed(fastKronInvalidKMMProblem);
     int64_t x = 1, f = 1, s = 1, zz = 1;
     auto step = [](const Dims& b, size_t fromBack, int64_t* run) {
       if (fromBack >= b.size() || b[b.size() - 1 - fromBack] == 1) return (int64_t)0;
@@ -235,22 +241,18 @@ PyObject* product(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
       if (!dims.empty() && prod(o.zb) > 0) {
         Dim& in = dims.back();
         if (n == 1) continue;
-        if (in.n == 1) { in = d; continue; }
-        if (d.x == in.x * in.n && d.f == in.f * in.n && d.y == in.y * in.n && in.n * n <= kMaxCount) { in.n *= n; continue; }
+        if (in.n == 1 && room(n)) { in = d; continue; }
+        if (d.x == in.x * in.n && d.f == in.f * in.n && d.y == in.y * in.n && in.n * n <= kMaxCount && room(in.n * n)) { in.n *= n; continue; }
       }
       dims.push_back(d);
     }
   }
   size_t largest = 0;
-  for (size_t i = 1; i < dims.size(); i++) if (dims[i].n > dims[largest].n && prod(o.zb) > 0 && dims[i].n <= kMaxCount) largest = i;
+  for (size_t i = 1; i < dims.size(); i++) if (dims[i].n > dims[largest].n && prod(o.zb) > 0 && dims[i].n <= kMaxCount && room(dims[i].n)) largest = i;
   const int64_t inner = one ? 1 : dims[largest].n;
-  size_t ye = 0, te = 0;
-  fastKronError e = api.sizes(c.handle, (uint32_t)M, o.N, o.Ps, o.Qs, &ye, &te);
-  if (e != fastKronSuccess) return failed(e);
   // both temporaries in one allocation, each on a 256-byte boundary
-  // (two dimensions at once only while the temporaries stay small beside the operands)
   const size_t withF = dims.size() == 2 ? (dims[0].f != 0) + (dims[1].f != 0) : 0;
-  const bool both = withF == 1 && prod(o.zb) > 0 && prod(o.zb) <= 65535 && te * (size_t)prod(o.zb) * es <= (size_t)256 << 20;
+  const bool both = withF == 1 && prod(o.zb) > 0 && prod(o.zb) <= 65535 && room(prod(o.zb));
   const size_t tn = te * (size_t)(both ? prod(o.zb) : inner), off = (tn * es + 255) / 256 * 256 / es;
   Tensor temp = at::empty({(int64_t)(off + tn)}, o.x.options());
   char* t1 = (char*)temp.data_ptr();

@@ -63,3 +63,24 @@ def test_empty_dimensions_as_before():
     assert fk.gemkm(torch.randn(0, 1, 5, 16, device="cuda"), fs).shape == (0, 3, 5, 16)
     with pytest.raises(fk.FastKronError):
         fk.gemkm(torch.randn(3, 0, 5, 16, device="cuda"), [torch.randn(0, 4, 4, device="cuda") for _ in range(2)])
+
+
+@pytest.mark.parametrize("xb,fb,entries", [((6, 1), (2,), 2), ((3, 2), (3, 2), 2), ((6, 1), (6, 1), 1)])
+def test_temporaries_of_large_entries_stay_those_of_the_innermost_dimension(xb, fb, entries):
+    """Entries of 64 MB: two temporaries of as many as the innermost dimension has, not of all that could be one call."""
+    import torch
+    import fastkron_amd as fk
+    x = torch.randn(xb + (4096, 4096), device="cuda")
+    fs = [torch.randn(fb + (64, 64), device="cuda") / 8 for _ in range(2)]
+    torch.cuda.synchronize()
+    torch.cuda.empty_cache()
+    torch.cuda.reset_peak_memory_stats()
+    before = torch.cuda.memory_allocated()
+    z = fk.gemkm(x, fs)
+    torch.cuda.synchronize()
+    entry = 4096 * 4096 * 4
+    assert torch.cuda.max_memory_allocated() - before <= z.numel() * 4 + max(2 * entries * entry, 512 << 20) + (8 << 20)
+    last = tuple(n - 1 for n in z.shape[:-2])
+    at = lambda t: t[tuple(min(i, n - 1) for i, n in zip(last[len(last) - t.dim() + 2:], t.shape[:-2]))]
+    want = fk.gemkm(at(x).contiguous(), [at(f).contiguous() for f in fs])
+    assert (z[last] - want).abs().max() <= 1e-5 * want.abs().max()
