@@ -352,14 +352,17 @@ bool Handle::viaMKMOnline(const KronProblem& p) const {
     // 32 x 8^6, 33 MB: no difference, 48 x 16^4, 13 MB: 23 -> 37 us; fp64 loses 1.1 to 1.6 times)
     if (p.dt != DType::F32 || p.M >= 64 || (uint64_t)p.M * p.K() * 4 < (64ull << 20)) return false;
     // (groups of small factors whose digits stay in place need no transposition: sgekmm 30 x 7^7 239 -> 159 us, 40 x 5^9
-    // 1014 -> 562, 50 x 4^10 419 -> 285; chains with 8x8 factors keep this plan, which is fixed for them, 16 x 8^8 1532 / 1130;
-    // chains without such groups, 2 x 17 columns of 4x3x7x6x3x6x5x6x4 551 / 688)
+    // 1014 -> 562, 50 x 4^10 419 -> 285; chains with 8x8 factors keep this plan, which is fixed for them, 16 x 8^8 1532 / 1130)
     bool small = true;
     for (uint32_t i = 0; i < p.N; i++) {
       if (p.P[i] != p.Q[i] || p.P[i] > 32) return false;
       small = small && p.P[i] < 8;
     }
-    return !small || columnsPlan(p).empty();
+    if (!small) return true;
+    // Without such groups (no equal neighbours, factors or gaps of every entry's own) chains of many launches gain (53 columns of
+    // 7x7x6x7x5x7x6x3 1264 -> 869, 54 of 7x7x2x3x7x6x4x3x5 629 -> 535, six launches 0.98 to 1.06), and those of 8 to 23 columns (17 of
+    // 5x3x6x5x4x5x6x6x5 499 -> 401); others lose (63 columns in three launches 725 / 1069, 4 columns of 7^8, 4 entries, 1302 / 1900).
+    return p.M >= 8 && columnsPlan(p).empty() && (p.M < 24 || select(p).size() >= 6);
   }
   // Measured on the reference's published shapes with both operands transposed.  Square factors up to 32x32 gain 1.3
   // to 2.8 times in fp32 (sgekmm 1024 x 8^5 171 -> 112 us, 16 x 8^8 3.34 -> 1.20 ms) and up to 1.2 times in fp64.  With
@@ -931,6 +934,14 @@ Plan Handle::columnsPlan(const KronProblem& p) const {
     const Plan& one = select(q);
     if (one.size() != 1) return Plan();
     plan.push_back(PlanStep{(uint32_t)lo, (uint32_t)hi, one[0].kernel});
+    // A last factor of its own on the plain or padded step runs on the caller's columns, an entry for every block of its rows: many
+    // entries of few columns cost more than the groups behind it save (us: sgekmm 2 columns of 8x7^3x12^3 222 / 643, 6 columns of
+    // 8x8x6x7x4x7x3 44 / 121, 47 columns of 6x7x7x2x3x3x7x6x2 285 / 448, dgekmm 5 columns of 8x3x7^3x6x3, 2 entries, 65 / 153; with
+    // fewer entries or more columns 0.6 to 0.95 of the time).
+    if (lo == hi && hi == (int)p.N - 1 && db_.kernels()[one[0].kernel].P <= 1) {
+      const uint32_t wide = p.dt == DType::F32 ? 64 : 16;
+      if (q.batch >= 16384 ? p.M <= wide : q.batch >= 4096 && p.M <= (p.dt == DType::F32 ? 16u : 8u)) return Plan();
+    }
     if (lo < hi) grouped = true;
     hi = lo - 1;
   }

@@ -724,7 +724,7 @@ def test_padded_pairs_of_many_rows_name_the_kernel_that_runs(planner, tmp_path):
 
 
 # ---- products with two batch dimensions ----
-def outer_plan(planner, mm, dt, M, Ps, Qs, count, opX=capi.OP_N, opF=capi.OP_N, sx=None, beta=0.0, y_is_z=False):
+def outer_plan(planner, mm, dt, M, Ps, Qs, count, opX=capi.OP_N, opF=capi.OP_N, sx=None, sz=None, beta=0.0, y_is_z=False):
     """fastKronProductOuter in plan-only mode; the strides are those of compact operands unless sx gives X's."""
     lib, h = planner
     K, L = 1, 1
@@ -732,7 +732,7 @@ def outer_plan(planner, mm, dt, M, Ps, Qs, count, opX=capi.OP_N, opF=capi.OP_N, 
         K, L = K * p, L * q
     ptr = [ctypes.c_void_p(BASE + i * GAP) for i in range(5)]            # x, z, y, t1, t2
     fs = capi.arr_ptr([BASE + (8 + i) * GAP for i in range(len(Ps))])
-    sz = capi.arr_u64([count[1] * M * L, M * L])
+    sz = capi.arr_u64(sz if sz is not None else [count[1] * M * L, M * L])
     e = lib.fastKronProductOuter(h, mm == "mkm", dt == "d", M, len(Ps), capi.arr_u32(Ps), capi.arr_u32(Qs), ptr[0], opX,
                                  capi.arr_u64(sx if sx is not None else [count[1] * M * K, M * K]), fs, opF, ptr[1], sz, 1.0, beta,
                                  capi.arr_u32(count), (ptr[1] if y_is_z else ptr[2]) if beta else None, sz, ptr[3], ptr[4])
@@ -790,8 +790,9 @@ def test_two_dimensions_without_entries_are_refused(online_planner):
         assert e == capi.INVALID_KMM_PROBLEM, count
 
 
-def test_gekmm_of_small_factors_runs_as_a_gemkm_where_no_digits_stay_in_place(online_planner):
-    """fp32, few columns, 64 MB of X and more: no equal neighbours, or batches whose factors or gaps rule the groups out."""
+def test_gekmm_of_small_factors_runs_as_a_gemkm_where_that_is_faster(online_planner):
+    """fp32, few columns, 64 MB of X and more: no equal neighbours, or batches whose factors or gaps rule the groups out, in six
+    launches and more or on 8 to 23 columns (2 x 17 columns of 4x3x7x6x3x6x5x6x4 551 us, 688 without)."""
     def via(M, Ps, **kw):
         e, names, _ = plan(online_planner, "kmm", "s", M, Ps, Ps, **kw)
         assert e == capi.SUCCESS
@@ -800,6 +801,18 @@ def test_gekmm_of_small_factors_runs_as_a_gemkm_where_no_digits_stay_in_place(on
     assert via(17, mixed) and via(17, mixed, batch=2) and via(17, mixed, batch=2, strideF=[0] * 9)
     assert not via(30, equal) and not via(30, equal, batch=2, strideF=[0] * 7)
     assert via(30, equal, batch=2) and via(30, equal, batch=2, strideF=[0] * 7, strides={"x": 30 * 7 ** 7 + 32})
+    assert not via(4, [7] * 8, batch=4) and not via(63, [3, 4, 4, 6, 4, 6, 4, 2, 7], batch=3)
+
+
+def test_a_last_factor_of_its_own_keeps_the_digits_in_place_only_with_columns_enough(online_planner):
+    """Us with the groups against without: 643 / 222, 153 / 65, 121 / 44; 51 / 75 (few entries), 0.7 to 0.9 (many columns)."""
+    def inplace(dt, M, Ps, **kw):
+        e, names, launches = plan(online_planner, "kmm", dt, M, Ps, Ps, **kw)
+        assert e == capi.SUCCESS
+        return int(launches[0]["batch"]) > kw.get("batch", 1)
+    assert not inplace("s", 2, [8, 7, 7, 7, 12, 12, 12]) and not inplace("d", 5, [8, 3, 7, 7, 7, 6, 3], batch=2, strideF=[0] * 7)
+    assert not inplace("s", 6, [8, 8, 6, 7, 4, 7, 3]) and not inplace("s", 47, [6, 7, 7, 2, 3, 3, 7, 6, 2])
+    assert inplace("s", 6, [7, 7, 7, 10]) and inplace("d", 10, [7, 7, 7, 10]) and inplace("s", 300, [7, 7, 7, 7, 7, 3])
 
 
 # ---- records and caches of a handle ----
