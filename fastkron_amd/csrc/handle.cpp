@@ -530,8 +530,12 @@ bool Handle::transposeFirstOnline(const KronProblem& p, const KronProblem& pn, v
     // 284 rows of 33x33 13.9 without the copy / 15.5, dgemkm 6685 rows of 2x1, 32x40 18.9 / 33.2)
     const size_t n0 = planN.second.find(':');
     if (yes && okT && 1 + nN == nT && p.N >= 2 && n0 != std::string::npos && planN.second.find("_anyxany_64x64_2_", n0) < planN.second.find(';', n0)) {
-      const uint32_t ps[2] = {p.P[p.N - 1], p.P[p.N - 2]}, qs[2] = {p.Q[p.N - 1], p.Q[p.N - 2]};
-      yes = pairAnyAhead(ps, qs, (uint64_t)p.M * (p.K() / ((uint64_t)ps[0] * ps[1])), p.batch, p.dt, dev_, true);
+      // (of the chain as it is merged: sgemkm 1673 rows of 2x2^5 10.7 without the copy / 14.8, dgemkm 213 rows of 4x4^4 10.7 / 13.8)
+      KronProblem m;
+      MergeArgs unused;
+      if (!mergedProblem(pn, &m, &unused, ws)) m = pn;
+      const uint32_t ps[2] = {m.P[m.N - 1], m.P[m.N - 2]}, qs[2] = {m.Q[m.N - 1], m.Q[m.N - 2]};
+      yes = m.N < 2 || pairAnyAhead(ps, qs, (uint64_t)m.M * (m.K() / ((uint64_t)ps[0] * ps[1])), m.batch, m.dt, dev_, true);
     }
     transposeCache_[ck] = yes;           // the preference of the shape; the buffers of each call are checked below
   }

@@ -815,6 +815,13 @@ def test_a_last_factor_of_its_own_keeps_the_digits_in_place_only_with_columns_en
     assert inplace("s", 6, [7, 7, 7, 10]) and inplace("d", 10, [7, 7, 7, 10]) and inplace("s", 300, [7, 7, 7, 7, 7, 3])
 
 
+def test_the_pair_behind_a_copy_is_judged_by_its_merged_factors(online_planner):
+    """Us without the copy / with it: 10.7 / 14.8, 10.7 / 13.8, 10.4 / 12.0."""
+    for dt, M, Ps in [("s", 1673, [2] * 5), ("d", 213, [4] * 4), ("d", 548, [4] * 3)]:
+        e, names, _ = plan(online_planner, "mkm", dt, M, Ps, Ps, opX=capi.OP_T)
+        assert e == capi.SUCCESS and not any(n.startswith("transpose_") for n in names), (dt, M, Ps, names)
+
+
 # ---- records and caches of a handle ----
 @pytest.mark.parametrize("dt,M,P,N,key,steps", [("s", 88, 7, 4, "(7x7^4)*2401x88_NN_f", 4), ("d", 88, 7, 4, "(7x7^4)*2401x88_NN_d", 4),
                                                 ("d", 1000, 4, 5, "(4x4(x)16x16(x)16x16)*1024x1000_NN_d", 3)])
