@@ -815,6 +815,14 @@ def test_a_last_factor_of_its_own_keeps_the_digits_in_place_only_with_columns_en
     assert inplace("s", 6, [7, 7, 7, 10]) and inplace("d", 10, [7, 7, 7, 10]) and inplace("s", 300, [7, 7, 7, 7, 7, 3])
 
 
+def test_copies_of_a_transposed_x_are_not_made_for_one_row(online_planner):
+    """A row is stored the same either way: where the copy's plan is the better one it runs on X itself."""
+    for dt, Ps in [("d", [57] * 4), ("s", [6, 36, 6]), ("s", [8] * 5), ("s", [16] * 4)]:
+        plain = plan(online_planner, "mkm", dt, 1, Ps, Ps)
+        e, names, launches = plan(online_planner, "mkm", dt, 1, Ps, Ps, opX=capi.OP_T)
+        assert e == capi.SUCCESS and names == plain[1] and launches[0]["in"] == plain[2][0]["in"], (dt, Ps, names)
+
+
 def test_the_pair_behind_a_copy_is_judged_by_its_merged_factors(online_planner):
     """Us without the copy / with it: 10.7 / 14.8, 10.7 / 13.8, 10.4 / 12.0."""
     for dt, M, Ps in [("s", 1673, [2] * 5), ("d", 213, [4] * 4), ("d", 548, [4] * 3)]:
