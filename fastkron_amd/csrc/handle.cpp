@@ -574,7 +574,7 @@ static std::string selectionKey(const KronProblem& p, uint32_t more = 0) {
     key[8 + 2 * i] = p.P[i]; key[9 + 2 * i] = p.Q[i];
     if (p.batch > 1 && p.strideF[i] != 0) own |= 1ull << i;
   }
-  key[0] = (uint32_t)p.mm; key[1] = (uint32_t)p.dt | more << 8; key[2] = (uint32_t)p.opX | (p.forward ? 256u : 0u);
+  key[0] = (uint32_t)p.mm; key[1] = (uint32_t)p.dt | more << 8; key[2] = (uint32_t)p.opX | (p.forward ? 256u : 0u) | (p.xJustWritten ? 512u : 0u);
   key[3] = p.M; key[4] = p.N; key[5] = p.batch; key[6] = (uint32_t)own; key[7] = (uint32_t)(own >> 32);
   return std::string((const char*)key, sizeof(uint32_t) * (8 + 2 * p.N));
 }
@@ -620,7 +620,7 @@ fastKronError Handle::runOnline(KronProblem p, void* temp1, void* temp2, const C
     if (e != fastKronKernelNotFound) return e;
   }
   if (!have) {
-    const std::string ck = key + (p.forward ? "_fwd" : "") + (useFusion() ? "" : "_nofuse");
+    const std::string ck = key + (p.forward ? "_fwd" : "") + (p.xJustWritten ? "_copy" : "") + (useFusion() ? "" : "_nofuse");
     auto it = planCache_.find(ck);
     if (it != planCache_.end()) plan = it->second;
     else {
@@ -649,7 +649,7 @@ fastKronError Handle::runOnline(KronProblem p, void* temp1, void* temp2, const C
     }
     refusedKernels.push_back(refused);
     // (cached like the first selection, under the problem and the kernels left out)
-    std::string rk = key + (p.forward ? "_fwd" : "") + (useFusion() ? "" : "_nofuse") + "|without";
+    std::string rk = key + (p.forward ? "_fwd" : "") + (p.xJustWritten ? "_copy" : "") + (useFusion() ? "" : "_nofuse") + "|without";
     for (int k : refusedKernels) rk += ":" + std::to_string(k);
     auto it = planCache_.find(rk);
     if (it != planCache_.end()) plan = it->second;
