@@ -1022,7 +1022,18 @@ fastKronError Handle::trySplitLeadingTrailing(const KronProblem& p, void* temp1,
     if (rp1.size() != 1 || db_.kernels()[rp1[0].kernel].fused != 2 || db_.kernels()[rp1[0].kernel].P == 0)
       return fastKronKernelNotFound;
     const Plan& rp2 = select(r2);
-    if (1 + rp2.size() >= select(p).size()) return fastKronKernelNotFound;
+    const Plan& apart = select(p);
+    if (1 + rp2.size() >= apart.size()) return fastKronKernelNotFound;
+    // nor, from 1024 blocks on in fp64, where leading factors that make rows at least twice as long come from the padded step to the
+    // plain one (dgemkm 242 x 6x50^3 70 / 86, 1071 x 7x28^3 61 / 75, 3 x 9x20^5 54 / 62; other factors 0.9 of the time; behind a
+    // transposed copy the pair is what made the copy worth while)
+    const uint64_t blocks = (uint64_t)r1.M * r1.batch;
+    if (p.dt == DType::F64 && blocks >= 1024 && !p.xJustWritten) {
+      const int plain = db_.genericKernel(p.dt);
+      for (auto& s : rp2)
+        if (s.kernel == plain && p.Q[s.lo] >= 2 * p.P[s.lo])
+          for (auto& t : apart) if (t.lo <= s.lo && s.lo <= t.hi && t.kernel != plain) return fastKronKernelNotFound;
+    }
     return runSplit(p, g2, r1, rp1, r2, rp2, temp2);
   };
   if (tq != tp || p.P[p.N - 2] != tp || p.Q[p.N - 2] != tq || (tp > 32 && tp < 64)) return trailingPair();

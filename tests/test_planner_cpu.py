@@ -826,6 +826,15 @@ def test_pairs_of_33_to_47_rows_a_side_end_where_the_padded_step_reads_whole_pie
     assert e == capi.SUCCESS and len(names) == 2 and names[0].startswith("transpose_") and PAIR in names[1], names
 
 
+@pytest.mark.parametrize("M,P,Q,opX,pair", [(242, 6, 50, capi.OP_N, False), (60, 6, 50, capi.OP_N, True), (1071, 7, 28, capi.OP_N, False),
+                                            (200, 50, 50, capi.OP_N, True), (7, 7, 44, capi.OP_T, True)])
+def test_trailing_pairs_leave_no_long_rows_to_the_plain_step(online_planner, M, P, Q, opX, pair):
+    """fp64, from 1024 blocks on: leading factors whose rows grow stay with the padded step, but behind a transposed copy."""
+    N = 4 if opX == capi.OP_T else 3
+    e, names, _ = plan(online_planner, "mkm", "d", M, [P] * N, [Q] * N, opX=opX)
+    assert e == capi.SUCCESS and any(PAIR in n for n in names) == pair, names
+
+
 def test_copies_of_a_transposed_x_are_not_made_for_one_row(online_planner):
     """A row is stored the same either way: where the copy's plan is the better one it runs on X itself."""
     for dt, Ps in [("d", [57] * 4), ("s", [6, 36, 6]), ("s", [8] * 5), ("s", [16] * 4)]:
