@@ -268,6 +268,13 @@ fastKronError Handle::xgemm(KronProblem p, fastKronBackend backend, void* temp1,
   return runOnline(p, temp1, temp2, ws);
 }
 
+// How many launches the last planned call makes (entries of lastPlan_).
+static size_t countLaunches(const std::string& plan) {
+  size_t n = 0;
+  for (char ch : plan) if (ch == ';') n++;
+  return n;
+}
+
 fastKronError Handle::xgemmOuter(const KronProblem& p, uint32_t outer, uint64_t outerX, uint64_t outerZ, uint64_t outerY,
                                  fastKronBackend backend, void* temp1, void* temp2) {
   if (outer == 0 || p.batch == 0) return fastKronInvalidKMMProblem;
@@ -275,31 +282,64 @@ fastKronError Handle::xgemmOuter(const KronProblem& p, uint32_t outer, uint64_t 
     const fastKronError e = runOuter(p, outer, outerX, outerZ, outerY, temp1, temp2);
     if (e != fastKronKernelNotFound) return e;
   }
-  const size_t es = dtypeSize(p.dt);
-  if (outer > p.batch) {
-    // fewer factors than outer entries: a call for each of them, the outer dimension as its batch
-    for (uint32_t i = 0; i < p.batch; i++) {
-      KronProblem q = p;
-      q.batch = outer;
-      q.X = (const char*)p.X + (size_t)i * p.strideX * es; q.strideX = outerX;
-      q.Z = (char*)p.Z + (size_t)i * p.strideZ * es; q.strideZ = outerZ;
-      if (p.Y) { q.Y = (const char*)p.Y + (size_t)i * p.strideY * es; q.strideY = outerY; }
-      for (uint32_t j = 0; j < p.N && j < kMaxFactors; j++) {
-        if (p.F[j]) q.F[j] = (const char*)p.F[j] + (size_t)i * p.strideF[j] * es;
-        q.strideF[j] = 0;
-      }
-      if (const fastKronError e = xgemm(q, backend, temp1, temp2); e != fastKronSuccess) return e;
-    }
-    return fastKronSuccess;
-  }
-  for (uint32_t o = 0; o < outer; o++) {
-    KronProblem q = p;
-    q.X = (const char*)p.X + (size_t)o * outerX * es;
-    q.Z = (char*)p.Z + (size_t)o * outerZ * es;
-    if (p.Y) q.Y = (const char*)p.Y + (size_t)o * outerY * es;
+  const bool perFactors = outer > p.batch;
+  for (uint32_t i = 0; i < (perFactors ? p.batch : outer); i++) {
+    const KronProblem q = outerCall(p, outer, outerX, outerZ, outerY, i);
     if (const fastKronError e = xgemm(q, backend, temp1, temp2); e != fastKronSuccess) return e;
   }
   return fastKronSuccess;
+}
+
+// Call i of the loop: with fewer factors than outer entries one for each of them, the outer dimension as its batch; otherwise
+// one for each outer entry.
+KronProblem Handle::outerCall(const KronProblem& p, uint32_t outer, uint64_t outerX, uint64_t outerZ, uint64_t outerY, uint32_t i) {
+  const size_t es = dtypeSize(p.dt);
+  const bool perFactors = outer > p.batch;
+  KronProblem q = p;
+  q.X = (const char*)p.X + (size_t)i * (perFactors ? p.strideX : outerX) * es;
+  q.Z = (char*)p.Z + (size_t)i * (perFactors ? p.strideZ : outerZ) * es;
+  if (p.Y) q.Y = (const char*)p.Y + (size_t)i * (perFactors ? p.strideY : outerY) * es;
+  if (perFactors) {
+    q.batch = outer; q.strideX = outerX; q.strideZ = outerZ; q.strideY = outerY;
+    for (uint32_t j = 0; j < p.N && j < kMaxFactors; j++) {
+      if (p.F[j]) q.F[j] = (const char*)p.F[j] + (size_t)i * p.strideF[j] * es;
+      q.strideF[j] = 0;
+    }
+  }
+  return q;
+}
+
+// One series of `launches` against the loop's calls, whose plan is another one: merged factors, parts of rows and groups of columns
+// are only there.  Passes over the operands decide, and what a launch costs beside them.  Of 1600 products (2 to 40 by 2 to 16
+// entries, 0.1 to 240 MB, either type and layout) the series is faster in half, in 4 % the loop; 7 of those are left, by 1.1 to 1.3.
+bool Handle::outerSeriesAhead(const KronProblem& p, uint32_t outer, uint64_t outerX, uint64_t outerZ, uint64_t outerY, size_t launches, void* temp1,
+                              void* temp2) {
+  // (whether the loop's operands have gaps decides on its plan)
+  std::string ck = p.str() + "_outer" + std::to_string(outer);
+  for (const uint64_t stride : {p.strideX, p.strideZ, p.strideY, outerX, outerZ, outerY}) ck += "_" + std::to_string(stride);
+  if (auto it = outerCache_.find(ck); it != outerCache_.end()) return it->second;
+  const KronProblem q = outerCall(p, outer, outerX, outerZ, outerY, 0);
+  const bool wasPlanOnly = planOnly_;
+  const std::string savedPlan = lastPlan_, savedLog = launchLog_;
+  planOnly_ = true;
+  const bool ok = xgemm(q, fastKronBackend_HIP, temp1, temp2) == fastKronSuccess;
+  const size_t loop = countLaunches(lastPlan_);
+  planOnly_ = wasPlanOnly;
+  lastPlan_ = savedPlan; launchLog_ = savedLog;
+  const double calls = std::min(outer, p.batch);
+  const double mb = (double)(p.K() + p.L()) * p.M * outer * p.batch * dtypeSize(p.dt) * 1e-6;
+  bool yes = true;
+  if (ok && launches > loop) {
+    // more passes, for fewer launches: a launch costs as much as 40 MB of a pass, 10 of the plain steps on columns in fp32 (us, series / loop:
+    // sgemkm 460 x 14^3, 10 by 4 374 / 143, sgekmm 50 x 7^5, 9 by 7 505 / 257, 2 x 8^6, 8 by 3 179 / 101; sgemkm 32 x 13^3, 19 by 3
+    // 41 / 54, dgemkm 20 x 11^3, 25 by 9 85 / 164)
+    yes = (double)(launches - loop) * mb < calls * (double)loop * (p.mm == MMType::MKM || p.dt == DType::F64 ? 40 : 10);
+  } else if (ok && launches >= 3 && mb > 256 && mb > 120 * calls) {
+    // as many passes, and one of the loop's calls keeps what it writes in the 256 MB memory-side cache for its next launch without
+    // being short of work (sgemkm 17 x 12^5, 4 by 3 575 / 471; with 30 to 100 MB a call 0.6 to 0.9)
+    yes = false;
+  }
+  return outerCache_[ck] = yes;
 }
 
 // fastKronKernelNotFound: not in this form (nothing has been launched).
@@ -311,11 +351,14 @@ fastKronError Handle::runOuter(const KronProblem& p0, uint32_t outer, uint64_t o
   if ((uint64_t)outer * p.batch > 65535) return fastKronKernelNotFound;
   for (uint32_t i = 0; i < p.N; i++) if (p.P[i] == 0 || p.Q[i] == 0 || !p.F[i] || p.strideF[i] == 0) return fastKronKernelNotFound;
   if (p.mm == MMType::KMM && (p.M == 1 || p.opX == fastKronOp_T || viaMKMOnline(p))) return fastKronKernelNotFound;
+  // (records say what a call of the loop runs)
   Choice tuned;
-  if (lookupChoice(p, &tuned)) return fastKronKernelNotFound;
+  if (db_.openRecords() || lookupChoice(p, &tuned) || lookupChoice(outerCall(p, outer, outerX, outerZ, outerY, 0), &tuned)) return fastKronKernelNotFound;
   if (const fastKronError e = planOnly_ ? fastKronSuccess : ensureDevice(); e != fastKronSuccess) return e;
   callWs_ = false;
   const uint32_t inner = p.batch;
+  const KronProblem call = p;
+  const uint64_t callX = outerX;
   KronProblem x = p;                       // the transposed copy: X's own entries only
   bool copy = false;
   if (p.opX == fastKronOp_T) {
@@ -338,8 +381,9 @@ fastKronError Handle::runOuter(const KronProblem& p0, uint32_t outer, uint64_t o
   p.inner = inner; p.batch = outer * inner; p.strided = true;
   p.outerX = outerX; p.outerZ = outerZ; p.outerY = outerY;
   KronProblem flat = p;
-  const Plan& plan = select(flat);
+  const Plan plan = select(flat);          // (a copy: the loop's plan is laid out before it runs)
   if (execute(p, plan, temp1, temp2, true) != fastKronSuccess) return fastKronKernelNotFound;
+  if (!outerSeriesAhead(call, outer, callX, outerZ, outerY, plan.size() + (copy ? 1 : 0), temp1, temp2)) return fastKronKernelNotFound;
   lastPlan_ = p.str();
   for (auto& s : plan) lastPlan_ += ";" + std::to_string(s.lo) + "-" + std::to_string(s.hi) + ":" + db_.kernels()[s.kernel].name;
   launchLog_.clear();
@@ -441,13 +485,6 @@ fastKronError Handle::runViaMKM(const KronProblem& p, fastKronBackend backend, v
     if (he != hipSuccess) return fastKronInvalidArgument;
   }
   return fastKronSuccess;
-}
-
-// How many launches the last planned call makes (entries of lastPlan_).
-static size_t countLaunches(const std::string& plan) {
-  size_t n = 0;
-  for (char ch : plan) if (ch == ';') n++;
-  return n;
 }
 
 // The problem with X already transposed into `xt` (temp2, or temp1 when there is no temp2): false when X does not
@@ -564,6 +601,7 @@ void Handle::trimCaches() {
   if (planCache_.size() > kMaxCached) planCache_.clear();
   if (selectCache_.size() > kMaxCached) selectCache_.clear();
   if (transposeCache_.size() > kMaxCached) transposeCache_.clear();
+  if (outerCache_.size() > kMaxCached) outerCache_.clear();
 }
 
 // What the kernels' rules look at, as bytes.

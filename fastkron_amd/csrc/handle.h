@@ -49,6 +49,9 @@ class Handle {
   // the temporaries hold outer * p.batch entries.
   fastKronError xgemmOuter(const KronProblem& p, uint32_t outer, uint64_t outerX, uint64_t outerZ, uint64_t outerY, fastKronBackend backend,
                            void* temp1, void* temp2);
+  static KronProblem outerCall(const KronProblem& p, uint32_t outer, uint64_t outerX, uint64_t outerZ, uint64_t outerY, uint32_t i);
+  bool outerSeriesAhead(const KronProblem& p, uint32_t outer, uint64_t outerX, uint64_t outerZ, uint64_t outerY, size_t launches, void* temp1,
+                        void* temp2);
   fastKronError runOuter(const KronProblem& p, uint32_t outer, uint64_t outerX, uint64_t outerZ, uint64_t outerY, void* temp1, void* temp2);
 
   // Runs `plan` on the stream; temps may be null when the plan has a single launch.
@@ -146,6 +149,7 @@ class Handle {
   std::unordered_map<std::string, Plan> planCache_;   // online selections, per problem string
   mutable std::unordered_map<std::string, Plan> selectCache_;   // ... per what the kernels' rules look at
   std::unordered_map<std::string, bool> transposeCache_;   // op(X) = T: transpose first or not, per problem string
+  std::unordered_map<std::string, bool> outerCache_;   // two batch dimensions: one series of launches or not
   std::string dbPath_;
   std::string lastPlan_;
   void* mergeWs_ = nullptr;                           // device memory for merged factors, allocated by initHIP

@@ -783,6 +783,48 @@ def test_transposed_copies_of_two_dimensions_are_those_that_are_read(online_plan
     assert last == (entries - 1) * M * K and (outer_in is None or int(rec["outer_in"]) == outer_in), rec
 
 
+@pytest.mark.parametrize("mm,dt,M,P,N,count,opX,series", [
+    # launches of the series (all entries) against the loop's: us series / loop 374 / 143, 505 / 257, 649 / 264, 174 / 89, 179 / 101
+    ("mkm", "s", 460, 14, 3, (10, 4), capi.OP_N, False), ("kmm", "s", 50, 7, 5, (9, 7), capi.OP_N, False), ("kmm", "d", 2, 7, 6, (39, 3), capi.OP_N, False),
+    ("mkm", "d", 245, 11, 3, (8, 5), capi.OP_N, False), ("kmm", "s", 2, 8, 6, (8, 3), capi.OP_N, False), ("mkm", "s", 17, 12, 5, (4, 3), capi.OP_N, False),
+    # 41 / 54, 85 / 164, one launch either way, and a copy ahead of both
+    ("mkm", "s", 32, 13, 3, (19, 3), capi.OP_N, True), ("mkm", "d", 20, 11, 3, (25, 9), capi.OP_N, True), ("mkm", "s", 1001, 5, 6, (2, 3), capi.OP_N, True),
+    ("mkm", "s", 32, 8, 5, (2, 3), capi.OP_T, True), ("mkm", "d", 5, 12, 2, (2, 3), capi.OP_N, True), ("mkm", "s", 3, 5, 3, (2, 3), capi.OP_N, True)])
+def test_two_dimensions_are_one_series_where_that_is_no_slower(online_planner, mm, dt, M, P, N, count, opX, series):
+    K = M * P ** N
+    perF = count[0] > count[1]                        # the loop's calls: one entry of factors with all of X, or one of X with all factors
+    for _ in range(2):                                # decided, and remembered
+        e, names, launches = outer_plan(online_planner, mm, dt, M, [P] * N, [P] * N, count, opX=opX, sx=[K, 0])
+        assert e == capi.SUCCESS and all(("inner" in l) == series for l in launches), names
+        if series:
+            assert all(int(l["batch"]) == count[0] * count[1] for l in launches)
+        else:
+            plain = plan(online_planner, mm, dt, M, [P] * N, [P] * N, batch=max(count), strideF=[0] * N if perF else None,
+                         strides={"x": K if perF else 0, "z": (count[1] if perF else 1) * K})
+            assert names == plain[1] and [l["batch"] for l in launches] == [l["batch"] for l in plain[2]]
+
+
+@pytest.mark.parametrize("dt,M,P,N", [("s", 64, 10, 4), ("s", 16, 9, 5)])
+def test_two_dimensions_with_the_factors_outside_are_the_calls_with_shared_factors(online_planner, dt, M, P, N):
+    """X of (12) entries and factors of (3, 1): three calls, whose entries lie without gaps, in two parts each."""
+    K = M * P ** N
+    shared = plan(online_planner, "mkm", dt, M, [P] * N, [P] * N, batch=12, strideF=[0] * N)
+    e, names, launches = outer_plan(online_planner, "mkm", dt, M, [P] * N, [P] * N, (12, 3), sx=[K, 0], sz=[K, 12 * K])
+    assert e == capi.SUCCESS and names == shared[1] and all("inner" not in l for l in launches), names
+
+
+def test_records_of_the_loops_calls_are_what_two_dimensions_run(online_planner, tmp_path):
+    lib, h = online_planner
+    generic = "gekmm_hip_gfx950_256_f_generic_1"
+    e, names, launches = outer_plan(online_planner, "mkm", "s", 32, [13] * 2, [13] * 2, (19, 3), sx=[32 * 169, 0])
+    assert e == capi.SUCCESS and "inner" in launches[0]
+    f = tmp_path / "plans.txt"
+    f.write_text(f"32x169*(13x13^2)_NN_f_stridedBatched_19_Fs3 0.01 M0 S0 2 1 1 {generic} 0 0 {generic}\n")
+    lib.fastKronSetTunedDB(h, str(f).encode())
+    e, names, launches = outer_plan(online_planner, "mkm", "s", 32, [13] * 2, [13] * 2, (19, 3), sx=[32 * 169, 0])
+    assert e == capi.SUCCESS and names == [generic] * 2 and all(l["batch"] == "19" and "inner" not in l for l in launches), launches
+
+
 def test_two_dimensions_without_entries_are_refused(online_planner):
     """As a strided batch of no entries is."""
     for count in [(3, 0), (0, 3), (1, 0), (0, 0)]:
