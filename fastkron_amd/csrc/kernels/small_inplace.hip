@@ -317,6 +317,9 @@ void kron_small_inplace_kernel(const KernelArgs a, const InplaceTile t, const Ou
   for (uint32_t e = whole * VE + tid; e < E; e += nth) o.put(e, rows[e]);
 }
 
+struct InplaceNoOuter {};
+struct InplaceOuter { OuterStrides outer; uint32_t inner; };
+
 // Rows of NF equal factors, one row per workgroup at a time and as many workgroups as the device holds at once: the next
 // row's pieces are on their way to registers while this one's digits are multiplied, and go to LDS as soon as the last pass
 // has read its values (its stores follow).
@@ -349,10 +352,11 @@ __device__ __forceinline__ void ipRowPasses(T* rows, const KernelArgs& a, const 
   }
 }
 
-// NT: 0 ordinary accesses, 1 non-temporal loads, 2 non-temporal loads and stores.
-template <typename T, int P, int NF, bool HAS_Y, int NT>
+// NT: 0 ordinary accesses, 1 non-temporal loads, 2 non-temporal loads and stores.  OUTER: two batch dimensions (asked for at run
+// time, the second one cost the form with one of them 1 us of 37, 1001 x 5^6 fp32).
+template <typename T, int P, int NF, bool HAS_Y, int NT, bool OUTER>
 __global__ __launch_bounds__((IpRow<P, NF, sizeof(T)>::threads), (IpRow<P, NF, sizeof(T)>::waves))
-void kron_rows_inplace_kernel(const KernelArgs a, const uint32_t total) {
+void kron_rows_inplace_kernel(const KernelArgs a, const uint32_t total, const std::conditional_t<OUTER, InplaceOuter, InplaceNoOuter> two) {
   using C = IpRow<P, NF, sizeof(T)>;
   constexpr uint32_t VE = C::VE, K = C::K;
   typedef T VT __attribute__((ext_vector_type(C::VE)));
@@ -362,11 +366,13 @@ void kron_rows_inplace_kernel(const KernelArgs a, const uint32_t total) {
   o.alpha = a.epilogue ? (T)a.alpha : T(1); o.beta = (T)a.beta;
 
   // 16-byte pieces that lie inside the row, and the elements before the first and behind the last of them
-  struct Row { const T* src; uint32_t b, m, shift, last; };
+  struct Row { const T* src; uint32_t b, o, m, shift, last; };
   auto rowAt = [&](uint32_t i) {
     Row r;
-    r.b = a.batch == 1 ? 0 : i / a.M; r.m = i - r.b * a.M;
+    r.b = a.batch == 1 ? 0 : i / a.M; r.m = i - r.b * a.M; r.o = 0;
+    if constexpr (OUTER) { r.o = r.b / two.inner; r.b -= r.o * two.inner; }
     r.src = (const T*)a.in + (size_t)r.b * a.in_batch + (size_t)r.m * K;
+    if constexpr (OUTER) r.src += (size_t)r.o * two.outer.in;
     r.shift = (uint32_t)((uintptr_t)r.src / sizeof(T)) & (VE - 1);
     r.last = (r.shift + K) / VE;
     return r;
@@ -399,6 +405,10 @@ void kron_rows_inplace_kernel(const KernelArgs a, const uint32_t total) {
     const uint32_t b = r.b;
     o.out = (T*)a.out + (size_t)b * a.out_batch + (size_t)r.m * K;
     o.y = HAS_Y ? (const T*)a.y + (size_t)b * a.y_batch + (size_t)r.m * K : nullptr;
+    if constexpr (OUTER) {
+      o.out += (size_t)r.o * two.outer.out;
+      if (HAS_Y) o.y += (size_t)r.o * two.outer.y;
+    }
     o.target = streamTarget(o.out, K * (uint32_t)sizeof(T));
     if (HAS_Y) o.yTarget = streamTarget((void*)o.y, K * (uint32_t)sizeof(T));
     {
@@ -569,18 +579,19 @@ static hipError_t launchIpT(const StepArgs& a, const InplaceTile& t, hipStream_t
   }
 }
 
-template <typename T, int P, int NF, bool HAS_Y, int NT>
+template <typename T, int P, int NF, bool HAS_Y, int NT, bool OUTER>
 static hipError_t launchIpRowsAs(const StepArgs& a, uint32_t total, uint32_t grid, hipStream_t stream) {
   using C = IpRow<P, NF, sizeof(T)>;
   static PerDeviceOnce attrOnce;
   const int dev = launchDeviceIndex();
-  const auto kernel = kron_rows_inplace_kernel<T, P, NF, HAS_Y, NT>;
+  const auto kernel = kron_rows_inplace_kernel<T, P, NF, HAS_Y, NT, OUTER>;
   const size_t lds = C::K * sizeof(T) + 16;
   if (lds > 65536 && !attrOnce.done(dev)) {
     if (const hipError_t e = hipFuncSetAttribute((const void*)kernel, hipFuncAttributeMaxDynamicSharedMemorySize, (int)kIpLdsMax); e != hipSuccess) return e;
     attrOnce.mark(dev);
   }
-  hipLaunchKernelGGL(kernel, dim3(grid), dim3(C::threads), lds, stream, a, total);
+  if constexpr (OUTER) hipLaunchKernelGGL(kernel, dim3(grid), dim3(C::threads), lds, stream, a, total, InplaceOuter{a.outer, a.inner});
+  else hipLaunchKernelGGL(kernel, dim3(grid), dim3(C::threads), lds, stream, a, total, InplaceNoOuter{});
   return hipGetLastError();
 }
 
@@ -600,16 +611,18 @@ static hipError_t launchIpRows(const StepArgs& a, hipStream_t stream, bool* take
   if (!*taken) return hipSuccess;
   const int nt = streamMode(a) < 2 || total / 6 > resident ? 0 : total / 2 > resident ? 1 : 2;
   const bool y = a.y && a.epilogue;
-#define IP_ROWS(NT) y ? launchIpRowsAs<T, P, NF, true, NT>(a, total, grid, stream) : launchIpRowsAs<T, P, NF, false, NT>(a, total, grid, stream)
-  return nt == 0 ? IP_ROWS(0) : nt == 1 ? IP_ROWS(1) : IP_ROWS(2);
+#define IP_ROWS(NT, OUTER) y ? launchIpRowsAs<T, P, NF, true, NT, OUTER>(a, total, grid, stream) : launchIpRowsAs<T, P, NF, false, NT, OUTER>(a, total, grid, stream)
+  if (a.inner) return nt == 0 ? IP_ROWS(0, true) : IP_ROWS(1, true);
+  return nt == 0 ? IP_ROWS(0, false) : nt == 1 ? IP_ROWS(1, false) : IP_ROWS(2, false);
 #undef IP_ROWS
 }
 
-// The sizes of rows of equal factors that have the form above: those of 9 to 160 KB, up to which several rows per workgroup
-// fill its threads better; 3^9 is more factors than a launch takes.
+// The sizes of rows of equal factors that have the form above: of those of 9 to 160 KB (below, several rows per workgroup fill its
+// threads better) the ones that were measured in it; fp64 rows of 3^7, 6^4 and 7^4 (10 to 19 KB) were not and stay with the general
+// kernel.  3^9 is more factors than a launch takes.
 static hipError_t launchIpRowsAny(const StepArgs& a, const InplaceTile& t, DType dt, hipStream_t stream, bool* taken) {
   *taken = false;
-  if (a.inner || (uint64_t)a.M * a.batch >= (1ull << 31)) return hipSuccess;
+  if ((uint64_t)a.M * a.batch >= (1ull << 31)) return hipSuccess;
   const uint32_t size = t.P * 16 + a.nf;
 #define IP_ROWS(T, P, NF) case P * 16 + NF: return launchIpRows<T, P, NF>(a, stream, taken);
   if (dt == DType::F32) switch (size) {

@@ -14,7 +14,8 @@ pytestmark = pytest.mark.gpu
 
 PROBLEMS = [  # layout, rows or columns, factors (P, Q)
     (ko.MKM, 8, [(8, 8)] * 5), (ko.MKM, 5, [(5, 5)] * 3), (ko.MKM, 7, [(31, 18), (9, 20)]), (ko.MKM, 3, [(3, 4), (4, 2)]), (ko.MKM, 2, [(10, 10)] * 3),
-    (ko.KMM, 9, [(7, 7)] * 4), (ko.KMM, 3, [(4, 3), (5, 6)]), (ko.KMM, 2, [(50, 40)]), (ko.KMM, 1, [(6, 6)] * 3), (ko.MKM, 4, [(4, 4)] * 6)]
+    (ko.KMM, 9, [(7, 7)] * 4), (ko.KMM, 3, [(4, 3), (5, 6)]), (ko.KMM, 2, [(50, 40)]), (ko.KMM, 1, [(6, 6)] * 3), (ko.MKM, 4, [(4, 4)] * 6),
+    (ko.MKM, 5, [(7, 7)] * 4), (ko.MKM, 2, [(5, 5)] * 6), (ko.MKM, 1, [(9, 9)] * 3)]
 # entries of the two dimensions, which of them X and Y have
 CALLS = [((1, 1), (1, 1), (1, 1)), ((3, 1), (1, 0), (1, 0)), ((1, 3), (0, 1), (0, 0)), ((2, 3), (1, 0), (1, 1)), ((2, 3), (0, 0), (1, 1)),
          ((3, 2), (1, 1), (0, 1)), ((4, 2), (0, 1), (1, 0)), ((3, 1), (0, 0), (1, 1))]
