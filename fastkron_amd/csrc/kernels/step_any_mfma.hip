@@ -76,8 +76,8 @@ struct StepAnyGeom {
 // exact j / wide for j < 2^31: wide > 1 in (2^(b-1), 2^b], wideMagic = ceil(2^(31+b) / wide), wideShift = b - 1
 __device__ __forceinline__ int64_t saWide(uint32_t j, const StepAnyGeom& g) { return __umulhi(j, g.wideMagic) >> g.wideShift; }
 
-// NBT > 0: every slab has exactly NBT full 16-column blocks (Q a multiple of 16) and P is a multiple of 4; the tile loop
-// then has no conditional memory operation (see there).  NBT = 0: anything.
+// NBT > 0: every slab has exactly NBT full 16-column blocks (Q a multiple of 16) and P = 4 * PCMAX (128: the loop reads 4 * PCMAX
+// contraction indices without a condition); the tile loop then has no conditional memory operation (see there).  NBT = 0: anything.
 template <typename T, int PCMAX, bool HAS_Y, bool PREFETCH, int NBT, bool WIDE>
 __global__ __launch_bounds__(kSaThreads, 2) void kron_step_any_kernel(const KernelArgs a, const StepAnyGeom g) {
   using MF = SaMfma<T>;
