@@ -49,19 +49,26 @@ def test_columns_in_place(fk, M, Ps, groups, dt):
             assert len(fk.last_plan()) == groups and any("columns" in s[2] for s in fk.last_plan()), fk.last_plan()
 
 
-def test_tuned_record_of_groups_in_place(tmp_path):
-    """A record says that the digits stay in place (M2), and a handle that does not tune runs it as it was stored."""
+@pytest.mark.parametrize("tune", [False, True])
+def test_records_of_groups_in_place(tmp_path, tune):
+    """A record says that the digits stay in place (M2), in other groups than the rule's: that is what runs.  A handle that tunes
+    stores what it runs, and one that does not runs it from the file."""
     import fastkron_amd
-    db = str(tmp_path / "plans.txt")
-    M, Ps = 5, [7] * 5
+    db = tmp_path / "plans.txt"
+    M, Ps, k = 5, [7] * 5, "kmm_hip_gfx950_512_d_small_fused_columns_8"
     X, Fs, Y = make_case(ko.KMM, M, Ps, Ps, np.float64, seed=5)
     want = oracle_answer(ko.KMM, M, Ps, Ps, X, Fs, Y, 1.5, 0.5)
+    if not tune:
+        db.write_text(f"(7x7^5)*16807x5_NN_d 0.01 M2 S0 2 3 4 {k} 0 2 {k}\n")
     plans = []
-    for tune in (True, False):
-        h = fastkron_amd.FastKron(tune=tune)
-        h.set_tuned_db(db)
+    for t in ([True, False] if tune else [False]):
+        h = fastkron_amd.FastKron(tune=t)
+        h.set_tuned_db(str(db))
         got, e = run_gpu(h, ko.KMM, M, Ps, Ps, X, Fs, Y, 1.5, 0.5)
         assert e == 0 and normwise(got, want) <= TOL[np.float64], h.last_plan()
         plans.append(h.last_plan())
         h.close()
-    assert plans[0] == plans[1] and (" M2 " in open(db).read()) == any("columns" in s[2] for s in plans[0])
+    if tune:
+        assert plans[0] == plans[1] and (" M2 " in db.read_text()) == any("columns" in s[2] for s in plans[0])
+    else:
+        assert plans == [[(3, 4, k), (0, 2, k)]]

@@ -908,6 +908,39 @@ def test_records_without_rewriting_fields_come_before_the_rules_for_columns(onli
     assert e == capi.SUCCESS and names == [generic] * steps, names
 
 
+COLUMNS = "kmm_hip_gfx950_512_%s_small_fused_columns_8"
+
+
+@pytest.mark.parametrize("dt", ["s", "d"])
+def test_records_of_groups_in_place_run_those_groups(online_planner, tmp_path, dt):
+    """M2: the steps as problems on the columns behind them; records that do not fit a call leave it to the rules."""
+    lib, h = online_planner
+    k, t = COLUMNS % ("f" if dt == "s" else "d"), "f" if dt == "s" else "d"
+    key = "(7x7^5)*16807x5_NN_" + t
+    other = plan(online_planner, "kmm", dt, 5, [7] * 5, [7] * 5)[1]
+    f = tmp_path / "groups.db"
+    def run(line, **kw):
+        f.write_text(line + "\n")
+        lib.fastKronSetTunedDB(h, str(f).encode())
+        e, names, launches = plan(online_planner, "kmm", dt, 5, [7] * 5, [7] * 5, **kw)
+        assert e == capi.SUCCESS
+        return names, [(int(l["M"]), int(l["batch"])) for l in launches]
+    # other groups than the rule's (2 and 3 factors), so that the record is what runs
+    assert run(f"{key} 0.01 M2 S0 2 2 4 {k} 0 1 {k}") == ([k] * 2, [(5, 49), (5 * 343, 1)])
+    assert run(f"{key} 0.01 M2 S0 2 3 4 {k} 0 2 {k}") == ([k] * 2, [(5, 343), (5 * 49, 1)])
+    for bad in ("2 0 1 %s 2 4 %s" % (k, k), "2 2 4 %s 1 1 %s" % (k, k), "1 2 4 %s" % k, "2 1 4 %s 0 0 %s" % (k, k), "2 2 4 nothing 0 1 %s" % k):
+        assert run(f"{key} 0.01 M2 S0 {bad}")[0] == other, bad
+    # one temporary holds what two launches pass on; factors of each entry's own and gaps in X rule the groups out
+    assert run(f"{key} 0.01 M2 S0 2 2 4 {k} 0 1 {k}", temp2=False)[0] == [k] * 2
+    batched = "(7x7^5)*16807x5_NN_%s_stridedBatched_2" % t
+    assert run(f"{batched} 0.01 M2 S0 2 2 4 {k} 0 1 {k}", batch=2)[0] == plan(online_planner, "kmm", dt, 5, [7] * 5, [7] * 5, batch=2)[1]
+    own, _ = run(f"{batched} 0.01 M2 S0 2 2 4 {k} 0 1 {k}", batch=2)
+    assert k not in own
+    gaps, _ = run(f"{batched}_Fs1f 0.01 M2 S0 2 2 4 {k} 0 1 {k}", batch=2, strideF=[0] * 5, strides={"x": 5 * 7 ** 5 + 8})
+    assert k not in gaps
+    assert run(f"{batched}_Fs1f 0.01 M2 S0 2 2 4 {k} 0 1 {k}", batch=2, strideF=[0] * 5)[1] == [(5, 98), (5 * 343, 2)]
+
+
 def test_a_handle_keeps_a_bounded_number_of_plans(online_planner):
     """Calls with ever new row counts: what the handle remembers of them stops growing (50000 problems took 34 MB)."""
     import os

@@ -56,6 +56,19 @@ def test_both_dimensions_are_one_series_of_launches():
             assert torch.equal(z[i, j], fk.gemkm(x[i, 0].contiguous(), [f[j].contiguous() for f in fs]))
 
 
+@pytest.mark.parametrize("ps,m,kernel", [([8] * 3, 8, "_small_fused_inplace_"), ([5] * 3, 3, "_small_fused_inplace_"), ([9, 14], 5, "_anyxany_64x64_2_"),
+                                         ([3, 4], 2, "_small_fused_inplace_"), ([13] * 3, 4, "_generic_")], ids=lambda v: str(v))
+def test_the_kernels_of_two_dimensions_run_them_as_one_call(ps, m, kernel):
+    import ctypes
+    import torch
+    import fastkron_amd as fk
+    h = fk.default_handle()
+    fk.gemkm(torch.randn(2, 1, m, int(np.prod(ps)), device="cuda"), [torch.randn(3, p, p, device="cuda") for p in ps])
+    buf = ctypes.create_string_buffer(4096)
+    h.lib.fastKronGetLastPlan(h.h, buf, 4096)
+    assert "_stridedBatched_6" in buf.value.decode() and kernel in buf.value.decode(), buf.value
+
+
 def test_empty_dimensions_as_before():
     import torch
     import fastkron_amd as fk
