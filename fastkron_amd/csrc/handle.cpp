@@ -444,7 +444,8 @@ fastKronError Handle::runViaMKM(const KronProblem& p, fastKronBackend backend, v
   q.Y = nullptr; q.strideY = 0; q.beta = 0.0;
   q.zReadNext = true;
   const bool zFree = !(p.Y == p.Z && p.beta != 0.0);
-  void* zTemp = (zFree && tmpElems <= ML && (p.batch == 1 || p.strideZ >= ML)) ? p.Z : nullptr;
+  // (the entries of a temporary lie side by side: what lies between those of Z is not this call's)
+  void* zTemp = (zFree && tmpElems <= ML && (p.batch == 1 || p.strideZ == ML)) ? p.Z : nullptr;
   fastKronError e;
   const bool copyX = p.opX != fastKronOp_T;
   if (copyX) {

@@ -354,6 +354,24 @@ def test_gekmm_with_transposed_x_runs_as_the_gemkm_of_that_buffer(online_planner
     assert e == capi.SUCCESS and not names[-1].endswith("_z"), names
 
 
+@pytest.mark.parametrize("dt,M,Ps,opX", [("d", 3, [5] * 7, capi.OP_T), ("d", 73, [6, 4, 2, 8, 7], capi.OP_T), ("s", 16, [16] * 5, capi.OP_N)])
+@pytest.mark.parametrize("own", [False, True])
+def test_gekmm_as_a_gemkm_leaves_what_lies_between_the_entries_of_z(online_planner, dt, M, Ps, opX, own):
+    """Z is a temporary of the GeMKM only where its entries lie side by side; otherwise other results may lie between them."""
+    L = 1
+    for p in Ps:
+        L *= p
+    es = 4 if dt == "s" else 8
+    for gap in (0, 8, 4 * M * L):
+        e, names, launches = plan(online_planner, "kmm", dt, M, Ps, Ps, batch=5, opX=opX, strideF=None if own else [0] * len(Ps),
+                                  strides={"z": M * L + gap})
+        assert e == capi.SUCCESS
+        z = BASE + GAP                                                          # (x, z, y, t1, t2)
+        written = [int(l["out"], 16) for l in launches]
+        inZ = [w for w in written if z <= w < z + 5 * (M * L + gap) * es]
+        assert gap == 0 or not names[-1].startswith("transpose_") or not inZ, (names, launches)
+
+
 def test_transposed_x_is_read_in_place_when_a_copy_does_not_pay_or_does_not_fit(planner):
     # one small factor: the plain kernel reads the transposed X directly, a copy would add a pass
     e, names, _ = plan(planner, "mkm", "s", 64, [8], [8], opX=capi.OP_T)

@@ -56,6 +56,26 @@ def test_both_dimensions_are_one_series_of_launches():
             assert torch.equal(z[i, j], fk.gemkm(x[i, 0].contiguous(), [f[j].contiguous() for f in fs]))
 
 
+@pytest.mark.parametrize("xb,fb", [((5, 1), (2,)), ((2,), (5, 1)), ((3, 1), (4,)), ((4,), (3, 1))])
+@pytest.mark.parametrize("dt,m,ps", [("float64", 3, [5] * 6), ("float64", 30, [6, 4, 2, 8, 7]), ("float32", 5, [7, 3, 9, 5, 4])], ids=lambda v: str(v))
+def test_gekmm_of_a_transposed_x_keeps_to_its_entries_of_the_result(dt, m, ps, xb, fb):
+    """The calls' entries lie between those of other calls, in chains whose GeMKM takes several launches."""
+    import torch
+    import fastkron_amd as fk
+    dtype, k = getattr(torch, dt), int(np.prod(ps))
+    x = torch.randn(xb + (m, k), device="cuda", dtype=dtype).mT
+    fs = [torch.randn(fb + (p, p), device="cuda", dtype=dtype) / p ** 0.5 for p in ps]
+    z = fk.gekmm(fs, x)
+    zb = tuple(torch.broadcast_shapes(xb, fb))
+    X, F = x.expand(zb + (k, m)), [f.expand(zb + f.shape[-2:]) for f in fs]
+    for at in np.ndindex(*zb):
+        want = X[at].double()
+        for i, f in enumerate(F):
+            v = want.reshape(int(np.prod(ps[:i])), ps[i], -1)
+            want = torch.matmul(f[at].double(), v).reshape(k, m)
+        assert normwise(z[at].cpu().numpy(), want.cpu().numpy()) <= (1e-5 if dt == "float32" else 1e-12), at
+
+
 @pytest.mark.parametrize("ps,m,kernel", [([8] * 3, 8, "_small_fused_inplace_"), ([5] * 3, 3, "_small_fused_inplace_"), ([9, 14], 5, "_anyxany_64x64_2_"),
                                          ([3, 4], 2, "_small_fused_inplace_"), ([13] * 3, 4, "_generic_")], ids=lambda v: str(v))
 def test_the_kernels_of_two_dimensions_run_them_as_one_call(ps, m, kernel):
