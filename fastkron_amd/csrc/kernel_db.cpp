@@ -207,16 +207,11 @@ static bool pairAnyCanRun(const KernelInfo& k, const KronProblem& p, uint32_t lo
     const uint64_t padded = 1024 * blocks(ps[1]) * blocks(qs[0]) * ((ps[0] + 3) / 4 + 4 * blocks(qs[1]));
     const uint64_t real = (uint64_t)ps[1] * qs[0] * (ps[0] + qs[1]);
     if ((uint64_t)p.M * p.batch >= 8192 && 2 * padded > 5 * real && std::max(ps[0], ps[1]) > 16) return false;
-    // factors of 33 to 47 a side, which the padded step reads in whole pieces: fp64 from 2048 rows on (own factors: of 400 rows an entry),
-    // fp32 with factors of each entry's own from 4096 on (of 1000) (us: dgemkm 513 x 34^2, 12 entries 102 / 138, 692 x 42^2, 9 entries
-    // 121 / 144, sgemkm 2467 x 45^2, 3 entries 80 / 99; 179 x 40^2, 32 entries 126 / 95, sgemkm with shared factors 0.75 to 1.08; behind
-    // a transposed copy the steps would read X as it is stored, 13415 rows of 46^2, 2 entries 1003 / 356);
+    // fp64 factors of 33 to 47 a side on 4096 rows and more, which the padded step reads in whole pieces (us: dgemkm 8056 x 36^2
+    // 120 / 102, 6941 rows 109 / 97; behind a transposed copy the steps would read X as it is stored, 9710 rows of 39^2 216 / 338);
     const uint32_t least = std::min({ps[0], ps[1], qs[0], qs[1]}), widest = std::max({ps[0], ps[1], qs[0], qs[1]});
-    if (!p.xJustWritten && least > 32 && widest < 48) {
-      const bool own = p.batch > 1 && (p.strideF[lo] != 0 || p.strideF[hi] != 0);
-      const uint64_t rows = (uint64_t)p.M * p.batch;
-      if (p.dt == DType::F64 ? rows >= 2048 && (!own || p.M >= 400) : own && rows >= 4096 && p.M >= 1000) return false;
-    }
+    const bool own = p.batch > 1 && (p.strideF[lo] != 0 || p.strideF[hi] != 0);
+    if (p.dt == DType::F64 && !own && !p.xJustWritten && least > 32 && widest < 48 && (uint64_t)p.M * p.batch >= 4096) return false;
     // and where the factors one by one are faster
     if (!pairAnyAhead(ps, qs, p.M, p.batch, p.dt, dev, false)) return false;
   }

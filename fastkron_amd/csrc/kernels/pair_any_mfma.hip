@@ -265,15 +265,15 @@ static uint32_t paRows(uint32_t waves, uint64_t rows, uint32_t cus) {
   while (items > 1 && rows < 2ull * items * cus) items /= 2;
   return items;
 }
-// Workgroups at once per batch entry: two waves per SIMD, four of the kernels that need few registers.
-static uint32_t paWorkgroups(int PB, size_t es, uint32_t batch, uint32_t cus) {
-  return ((es == 4 && PB == 2 ? 4 : 2) * cus + batch - 1) / batch;
+// Workgroups per batch entry: two waves per SIMD at once, four of the kernels that need few registers.
+static uint32_t paWorkgroups(int PB, size_t es, uint32_t tiles, uint32_t batch, uint32_t cus) {
+  return persistentWorkgroups(tiles, batch, (es == 4 && PB == 2 ? 4 : 2) * cus);
 }
 PairAnyWork pairAnyWork(const uint32_t* p, const uint32_t* q, uint64_t M, uint32_t batch, DType dt, uint32_t cus) {
   const int PB = std::max(p[0], p[1]) > 32 ? 4 : 2;
   PairAnyWork w;
   w.rows = paRows(paWaves(PB, q[0]), M * batch, cus);
-  const uint64_t tiles = (M + w.rows - 1) / w.rows, at = std::min<uint64_t>(tiles, paWorkgroups(PB, dtypeSize(dt), batch, cus));
+  const uint64_t tiles = (M + w.rows - 1) / w.rows, at = paWorkgroups(PB, dtypeSize(dt), (uint32_t)std::min<uint64_t>(tiles, UINT32_MAX), batch, cus);
   w.rounds = (tiles + at - 1) / at;
   return w;
 }
@@ -297,7 +297,7 @@ static hipError_t launchPairAnyAs(const StepArgs& a, hipStream_t stream) {
     if (const hipError_t e = hipFuncSetAttribute((const void*)kernel, hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024); e != hipSuccess) return e;
     attrOnce.mark(dev);
   }
-  hipLaunchKernelGGL(kernel, dim3(std::min(t.tiles, paWorkgroups(PB, sizeof(T), a.batch, cus)), innerEntries(a), outerEntries(a)), dim3(kPaThreads), lds, stream, a, t, a.outer);
+  hipLaunchKernelGGL(kernel, dim3(paWorkgroups(PB, sizeof(T), t.tiles, a.batch, cus), innerEntries(a), outerEntries(a)), dim3(kPaThreads), lds, stream, a, t, a.outer);
   return hipGetLastError();
 }
 template <typename T, int PB, int QB>

@@ -352,17 +352,6 @@ bool stepAnyMfmaSupported(const StepArgs& a, DType dt) {
   return stepAnyGeometry(a, dt, &g);
 }
 
-// Workgroups per slab and batch entry (`share` of those) for `need` groups of tiles, where the device holds `places` at once: as many
-// as fit, or one more of each where the tiles then go through in less time although the device takes two rounds.  Equal slabs make the
-// difference: 86 workgroups for each of three slabs are 258 on 256 CUs, and the last two took as long again as all others (us: sgekmm
-// 3285 x 192x192(x)36x36 340 -> 257, dgekmm 45 x 96x256^2, 7 entries 298 -> 202).
-static uint32_t stepAnyWorkgroups(uint32_t need, uint32_t share, uint32_t places) {
-  const uint64_t fit = places / share > 1 ? places / share : 1, more = (places + share - 1) / share;
-  auto time = [&](uint64_t w) { return (w * share + places - 1) / places * ((need + w - 1) / w); };
-  const uint64_t wgs = time(more) < time(fit) ? more : fit;
-  return wgs < need ? (uint32_t)wgs : need > 0 ? need : 1;
-}
-
 template <typename T, int PCMAX, int NBT, bool WIDE>
 static hipError_t launchStepAnyW(const StepArgs& a, const StepAnyGeom& g, hipStream_t stream) {
   // the tile of the next iteration is held in registers too unless the two copies would not fit (fp64, P > 128)
@@ -398,7 +387,8 @@ static hipError_t launchStepAnyW(const StepArgs& a, const StepAnyGeom& g, hipStr
   uint32_t wgs = (uint32_t)cus * (uint32_t)occ;
   const uint32_t share = a.batch * g.nSlabs;                  // the other two grid dimensions
   const uint32_t need = (g.totalTiles + kSaWaves - 1) / kSaWaves;
-  wgs = stepAnyWorkgroups(need, share, wgs);
+  // (us, slabs and entries rounded up before: sgekmm 3285 x 192x192(x)36x36 340 -> 257, dgekmm 45 x 96x256^2, 7 entries 298 -> 202)
+  wgs = persistentWorkgroups(need, share, wgs);
   dim3 grid(wgs, a.batch, g.nSlabs), block(kSaThreads);
   if (a.y && a.epilogue)
     hipLaunchKernelGGL((kron_step_any_kernel<T, PCMAX, true, PF, NBT, WIDE>), grid, block, ldsBytes, stream, a, g);
