@@ -199,6 +199,8 @@ static bool pairAnyCanRun(const KernelInfo& k, const KronProblem& p, uint32_t lo
     if (std::max({ps[0], ps[1], qs[0], qs[1]}) <= 8) return false;
     // 64x64 and (fp64) 64x32, whose single steps have kernels and plans of their own;
     if (ps[0] == 64 && ps[1] == 64 && qs[0] == qs[1] && (qs[0] == 64 || (qs[0] == 32 && p.dt == DType::F64))) return false;
+    // nor, in fp64, 32x32 and 64x64 (us: dgemkm 8 entries of one row 8.5 / 6.2, 64x64(x)32x32 behind a GeKMM of 235 columns 27 / 24);
+    if (p.dt == DType::F64 && ps[0] == qs[0] && ps[1] == qs[1] && ps[0] + ps[1] == 96 && std::max(ps[0], ps[1]) == 64) return false;
     // equal ones of 17x17 ... 31x31 where the padded pair is faster;
     if (paddedPairSize(ps, qs)) return paddedPairInPieces(p, dev) && pairAnyFits(2, ps, qs, p.colsBefore(hi));
     // many rows of which most of the padded products are for nothing (33x33: 2.7 times the real ones; sgemkm 5000 rows 48.6 ->

@@ -893,6 +893,13 @@ def test_trailing_pairs_leave_no_long_rows_to_the_plain_step(online_planner, M, 
     assert e == capi.SUCCESS and any(PAIR in n for n in names) == pair, names
 
 
+@pytest.mark.parametrize("dt,M,a,b,batch,pair", [("d", 1, 32, 64, 8, False), ("d", 235, 64, 32, 1, False), ("d", 235, 16, 64, 1, True),
+                                                 ("s", 235, 24, 64, 1, True)])
+def test_pairs_of_32_and_64_in_fp64_are_two_exact_steps(online_planner, dt, M, a, b, batch, pair):
+    e, names, _ = plan(online_planner, "mkm", dt, M, [a, b], [a, b], batch=batch if batch > 1 else None, strideF=[0] * 2)
+    assert e == capi.SUCCESS and any(PAIR in n for n in names) == pair, names
+
+
 def test_copies_of_a_transposed_x_are_not_made_for_one_row(online_planner):
     """A row is stored the same either way: where the copy's plan is the better one it runs on X itself."""
     for dt, Ps in [("d", [57] * 4), ("s", [6, 36, 6]), ("s", [8] * 5), ("s", [16] * 4)]:
