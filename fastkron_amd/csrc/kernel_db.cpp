@@ -162,6 +162,9 @@ bool pairAnyAhead(const uint32_t* ps, const uint32_t* qs, uint64_t M, uint32_t b
   if (!behindCopy && rows <= 256) return true;                     // (one row a workgroup: 0.5 to 0.9 of the steps' time)
   // (the padded pair and the kernel with two LDS buffers would want the copy as well)
   if (behindCopy && (paddedPairSize(ps, qs) || (ps[0] <= 8 && ps[1] <= 8))) return true;
+  // (the copy is a launch more than it saves of small factors on a small X: sgemkm 7304 transposed rows of 9^2 13.5 / 10.9, 2653 of
+  // 11^2 11.0 / 8.6, dgemkm 1926 of 11^2, 5 entries, 23.3 / 19.0)
+  if (behindCopy && std::max({ps[0], ps[1], qs[0], qs[1]}) <= 16 && mrows * (double)ps[0] * ps[1] * es < 10) return false;
   const bool f64 = dt == DType::F64;
   auto blocks = [](uint32_t n) { return (double)((n + 15) / 16); };
   const double in = (double)ps[0] * ps[1] * es, mid = (double)ps[1] * qs[0] * es, out = (double)qs[0] * qs[1] * es;

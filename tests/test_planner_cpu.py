@@ -900,6 +900,12 @@ def test_pairs_of_32_and_64_in_fp64_are_two_exact_steps(online_planner, dt, M, a
     assert e == capi.SUCCESS and any(PAIR in n for n in names) == pair, names
 
 
+@pytest.mark.parametrize("dt,M,P,copied", [("s", 7304, 9, False), ("s", 2653, 11, False), ("d", 3963, 9, False), ("s", 60000, 12, True), ("d", 60000, 12, True)])
+def test_small_transposed_x_of_small_factors_is_read_as_it_is_stored(online_planner, dt, M, P, copied):
+    e, names, _ = plan(online_planner, "mkm", dt, M, [P] * 2, [P] * 2, opX=capi.OP_T)
+    assert e == capi.SUCCESS and names[0].startswith("transpose_") == copied, names
+
+
 def test_copies_of_a_transposed_x_are_not_made_for_one_row(online_planner):
     """A row is stored the same either way: where the copy's plan is the better one it runs on X itself."""
     for dt, Ps in [("d", [57] * 4), ("s", [6, 36, 6]), ("s", [8] * 5), ("s", [16] * 4)]:
