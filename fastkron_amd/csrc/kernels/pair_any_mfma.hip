@@ -197,6 +197,7 @@ __global__ __launch_bounds__(kPaThreads, 2) void kron_pair_any_kernel(const Kern
             }
         }
       // rows beyond P1 are zero times F2, NaN where that is infinite: they are zero in the second product as well
+      // (1003 rows of 31x63^2 10.1 -> 10.4 us; only where a factor is not finite, or without the condition: the same)
 #pragma unroll
       for (int g = 0; g < PB; g++)
         if (16 * g < (int)t.P1 && 16 * g + 16 > (int)t.P1) {
@@ -266,6 +267,8 @@ static uint32_t paRows(uint32_t waves, uint64_t rows, uint32_t cus) {
   return items;
 }
 // Workgroups per batch entry: two waves per SIMD at once, four of the kernels that need few registers.
+// (us, rounded up before: sgemkm 4979 x 29x29(x)49x49, 6 entries 315 -> 204, 3954 x 44^2, 3 entries 167 -> 110, dgemkm 513 x 34^2,
+// 12 entries 138 -> 70)
 static uint32_t paWorkgroups(int PB, size_t es, uint32_t tiles, uint32_t batch, uint32_t cus) {
   return persistentWorkgroups(tiles, batch, (es == 4 && PB == 2 ? 4 : 2) * cus);
 }
