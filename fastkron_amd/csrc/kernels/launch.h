@@ -29,6 +29,17 @@ __device__ __forceinline__ void streamStore16(V v, __amdgpu_buffer_rsrc_t target
   __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(StreamU4, v), target, (int)byteOffset, 0, 19);
 }
 
+// One element at a lane's byte offset plus a wave-uniform one (elements beyond the descriptor's range: zero, dropped).
+template <typename T> __device__ __forceinline__ T bufferLoad(__amdgpu_buffer_rsrc_t from, uint32_t lane, uint32_t uniform) {
+  if constexpr (sizeof(T) == 4) return __builtin_bit_cast(T, __builtin_amdgcn_raw_buffer_load_b32(from, (int)lane, (int)uniform, 0));
+  else return __builtin_bit_cast(T, __builtin_amdgcn_raw_buffer_load_b64(from, (int)lane, (int)uniform, 0));
+}
+// ST: non-temporal
+template <bool ST = false, typename T> __device__ __forceinline__ void bufferStore(T v, __amdgpu_buffer_rsrc_t to, uint32_t lane, uint32_t uniform) {
+  typedef unsigned int U2 __attribute__((ext_vector_type(2)));
+  if constexpr (sizeof(T) == 4) __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(unsigned int, v), to, (int)lane, (int)uniform, ST ? 2 : 0);
+  else __builtin_amdgcn_raw_buffer_store_b64(__builtin_bit_cast(U2, v), to, (int)lane, (int)uniform, ST ? 2 : 0);
+}
 
 // Two batch dimensions are two grid dimensions (a division of one index in front of a kernel's first load cost the shortest
 // launches 0.5 us, 20 x 5^4 5.7 / 6.2).

@@ -48,15 +48,6 @@ template <> struct PaMfma<float> {
   static constexpr int rowReg(int r) { return r; }
 };
 
-template <typename T> __device__ __forceinline__ T paLoad(__amdgpu_buffer_rsrc_t from, uint32_t lane, uint32_t uniform) {
-  if constexpr (sizeof(T) == 4) return __builtin_bit_cast(T, __builtin_amdgcn_raw_buffer_load_b32(from, (int)lane, (int)uniform, 0));
-  else return __builtin_bit_cast(T, __builtin_amdgcn_raw_buffer_load_b64(from, (int)lane, (int)uniform, 0));
-}
-template <typename T> __device__ __forceinline__ void paStore(T v, __amdgpu_buffer_rsrc_t to, uint32_t lane, uint32_t uniform) {
-  typedef unsigned int U2 __attribute__((ext_vector_type(2)));
-  if constexpr (sizeof(T) == 4) __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(unsigned int, v), to, (int)lane, (int)uniform, 0);
-  else __builtin_amdgcn_raw_buffer_store_b64(__builtin_bit_cast(U2, v), to, (int)lane, (int)uniform, 0);
-}
 constexpr uint32_t kPaNowhere = 0x7ffffff0u;         // an offset outside every descriptor here
 
 // Rows per workgroup at a time, at most: four waves on 32-wide inputs, two rows of 64-wide ones.
@@ -130,13 +121,13 @@ __global__ __launch_bounds__(kPaThreads, 2) void kron_pair_any_kernel(const Kern
     for (int c = 0; c < PC; c++) {
       const uint32_t p = pc2 * hi + c;
       const bool in = (uint32_t)c < pc2 && p < t.P2 && q2 < t.Q2;
-      f2[c] = paLoad<T>(F2, in ? (uint32_t)(p * a.f_sp[0] + q2 * a.f_sq[0]) * ES : kPaNowhere, 0);
+      f2[c] = bufferLoad<T>(F2, in ? (uint32_t)(p * a.f_sp[0] + q2 * a.f_sq[0]) * ES : kPaNowhere, 0);
     }
     if constexpr (kF1Lds) {
       f1Lds = (T*)(paLds + t.items * t.P1 * (t.P2 + VE) * ES + 64);
       for (uint32_t k = tid; k < 64 * 64; k += kPaThreads) {
         const uint32_t p = k / 64, q = k % 64;
-        f1Lds[k] = paLoad<T>(F1, p < t.P1 && q < t.Q1 ? (uint32_t)(p * a.f_sp[1] + q * a.f_sq[1]) * ES : kPaNowhere, 0);
+        f1Lds[k] = bufferLoad<T>(F1, p < t.P1 && q < t.Q1 ? (uint32_t)(p * a.f_sp[1] + q * a.f_sq[1]) * ES : kPaNowhere, 0);
       }
     } else {
 #pragma unroll
@@ -146,7 +137,7 @@ __global__ __launch_bounds__(kPaThreads, 2) void kron_pair_any_kernel(const Kern
 #pragma unroll
           for (int k = 0; k < 4; k++) {
             const uint32_t p = 16 * g + MF::rowLane(hi) + MF::rowReg(k), q = 16 * u + lo;
-            f1[u][g][k] = paLoad<T>(F1, p < t.P1 && q < t.Q1 ? (uint32_t)(p * a.f_sp[1] + q * a.f_sq[1]) * ES : kPaNowhere, 0);
+            f1[u][g][k] = bufferLoad<T>(F1, p < t.P1 && q < t.Q1 ? (uint32_t)(p * a.f_sp[1] + q * a.f_sq[1]) * ES : kPaNowhere, 0);
           }
     }
   }
@@ -217,7 +208,7 @@ __global__ __launch_bounds__(kPaThreads, 2) void kron_pair_any_kernel(const Kern
           Acc z = {0, 0, 0, 0};
           T yv[4];
 #pragma unroll
-          for (int k = 0; k < 4; k++) yv[k] = HAS_Y ? paLoad<T>(y, lane, (16 * u + MF::rowReg(k)) * t.Q2 * ES) : T(0);
+          for (int k = 0; k < 4; k++) yv[k] = HAS_Y ? bufferLoad<T>(y, lane, (16 * u + MF::rowReg(k)) * t.Q2 * ES) : T(0);
 #pragma unroll
           for (int g = 0; g < PB; g++)
             if (g == 0 || 16 * g < (int)t.P1) {
@@ -233,7 +224,7 @@ __global__ __launch_bounds__(kPaThreads, 2) void kron_pair_any_kernel(const Kern
           for (int k = 0; k < 4; k++) {
             T o = z[k] * alpha;
             if (HAS_Y) o += beta * yv[k];
-            paStore<T>(o, out, lane, (16 * u + MF::rowReg(k)) * t.Q2 * ES);
+            bufferStore(o, out, lane, (16 * u + MF::rowReg(k)) * t.Q2 * ES);
           }
         }
     }

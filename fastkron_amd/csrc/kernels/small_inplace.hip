@@ -46,17 +46,6 @@ struct InplaceTile {
 
 constexpr int ipPow(int p, int d) { return d == 0 ? 1 : p * ipPow(p, d - 1); }
 
-template <typename T> __device__ __forceinline__ T ipLoad(__amdgpu_buffer_rsrc_t from, uint32_t lane, uint32_t uniform) {
-  if constexpr (sizeof(T) == 4) return __builtin_bit_cast(T, __builtin_amdgcn_raw_buffer_load_b32(from, (int)lane, (int)uniform, 0));
-  else return __builtin_bit_cast(T, __builtin_amdgcn_raw_buffer_load_b64(from, (int)lane, (int)uniform, 0));
-}
-// ST: non-temporal
-template <bool ST, typename T> __device__ __forceinline__ void ipStore(T v, __amdgpu_buffer_rsrc_t to, uint32_t lane, uint32_t uniform) {
-  typedef unsigned int U2 __attribute__((ext_vector_type(2)));
-  if constexpr (sizeof(T) == 4) __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(unsigned int, v), to, (int)lane, (int)uniform, ST ? 2 : 0);
-  else __builtin_amdgcn_raw_buffer_store_b64(__builtin_bit_cast(U2, v), to, (int)lane, (int)uniform, ST ? 2 : 0);
-}
-
 // out = alpha * v (+ beta * y)
 template <typename T, bool HAS_Y>
 struct IpOut {
@@ -144,7 +133,7 @@ __device__ __forceinline__ void ipPass(T* __restrict__ rows, const KernelArgs& a
       if constexpr (FIRST) {
         const uint32_t lane = o.laneIn + e0[k] / (TU ? TU : 1) * o.pitch, row = step / (TU ? TU : 1) * o.pitch;
 #pragma unroll
-        for (uint32_t i = 0; i < N; i++) x[k][i] = ipLoad<T>(o.source, lane, i * row);
+        for (uint32_t i = 0; i < N; i++) x[k][i] = bufferLoad<T>(o.source, lane, i * row);
       } else if (v16) {
 #pragma unroll
         for (int i = 0; i < N / VE; i++) {
@@ -203,14 +192,14 @@ __device__ __forceinline__ void ipPass(T* __restrict__ rows, const KernelArgs& a
         if constexpr (HAS_Y) {
 #pragma unroll
           for (uint32_t i = 0; i < N; i++)
-            yv[i] = TU ? ipLoad<T>(o.yTarget, o.laneY + row, i * next) : ipLoad<T>(o.yTarget, e0[k] * sizeof(T), i * step * sizeof(T));
+            yv[i] = TU ? bufferLoad<T>(o.yTarget, o.laneY + row, i * next) : bufferLoad<T>(o.yTarget, e0[k] * sizeof(T), i * step * sizeof(T));
         }
 #pragma unroll
         for (uint32_t i = 0; i < N; i++) {
           T v = x[k][i] * o.alpha;
           if constexpr (HAS_Y) v += o.beta * yv[i];
-          if (TU) ipStore<ST>(v, o.target, o.laneOut + row, i * next);
-          else ipStore<ST>(v, o.target, e0[k] * sizeof(T), i * step * sizeof(T));
+          if (TU) bufferStore<ST>(v, o.target, o.laneOut + row, i * next);
+          else bufferStore<ST>(v, o.target, e0[k] * sizeof(T), i * step * sizeof(T));
         }
       } else if (v16) {
 #pragma unroll
