@@ -119,16 +119,6 @@ hipError_t launchRow32x3p(const StepArgs& a, hipStream_t stream);
 bool pairMfmaSupported(const StepArgs& a, DType dt);
 hipError_t launchPairMfma(const StepArgs& a, DType dt, hipStream_t stream);
 
-// Workgroups that go from tile to tile, for each of `share` parts of a launch (batch entries, slabs) with `need` tiles, where the
-// device holds `places` at once: as many as fit, or one more of each where the tiles then go through in less time although the device
-// takes two rounds.  86 workgroups for each of three equal parts are 258 on 256 places, and the last two take as long again as all others.
-inline uint32_t persistentWorkgroups(uint32_t need, uint32_t share, uint32_t places) {
-  const uint64_t fit = places / share > 1 ? places / share : 1, more = ((uint64_t)places + share - 1) / share;
-  auto time = [&](uint64_t w) { return (w * share + places - 1) / places * ((need + w - 1) / w); };
-  const uint64_t wgs = time(more) < time(fit) ? more : fit;
-  return wgs < need ? (uint32_t)wgs : need > 0 ? need : 1;
-}
-
 // Two fused factors of any sizes up to 64 on rows of exactly P1*P2 columns (MKM layout), fp32 or fp64.
 bool pairAnyFits(uint32_t nf, const uint32_t* p, const uint32_t* q, uint64_t Kin);
 bool pairAnySupported(const StepArgs& a, DType dt);

@@ -985,3 +985,28 @@ def test_a_handle_keeps_a_bounded_number_of_plans(online_planner):
     before = resident()
     calls(12000, 62000)
     assert resident() - before < 8 << 20
+
+
+def test_workgroups_that_go_from_tile_to_tile_make_no_second_round_for_a_few(tmp_path):
+    """persistentWorkgroups (csrc/problem.h) on its own: as many per part as fit, or one more each where that ends earlier."""
+    import os
+    import subprocess
+    src = tmp_path / "count.cpp"
+    src.write_text("""
+#include <cstdio>
+#include "problem.h"
+int main() {
+  unsigned need, share, places;
+  while (scanf("%u %u %u", &need, &share, &places) == 3) printf("%u\\n", fk::persistentWorkgroups(need, share, places));
+}
+""")
+    csrc = os.path.join(os.path.dirname(os.path.dirname(os.path.abspath(__file__))), "fastkron_amd", "csrc")
+    subprocess.run(["g++", "-std=c++17", "-I", csrc, str(src), "-o", str(tmp_path / "count")], check=True)
+    cases = [(need, share, places) for places in (256, 512, 1024) for share in (1, 2, 3, 5, 7, 12, 36, 255, 256, 300, 4000) for need in (1, 2, 9, 85, 86, 97, 927, 20000)]
+    out = subprocess.run([str(tmp_path / "count")], input="\n".join("%d %d %d" % c for c in cases), capture_output=True, text=True, check=True).stdout
+    up = lambda a, b: -(-a // b)
+    for (need, share, places), w in zip(cases, map(int, out.split())):
+        time = lambda n: up(n * share, places) * up(need, n)
+        assert 1 <= w <= need and time(w) <= time(min(need, max(1, places // share))) and time(w) <= time(min(need, up(places, share))), (need, share, places, w)
+    answer = dict(zip(cases, map(int, out.split())))
+    assert answer[(927, 3, 256)] == 85 and answer[(20000, 7, 512)] == 73 and answer[(1, 1, 256)] == 1 and answer[(9, 1, 256)] == 9
